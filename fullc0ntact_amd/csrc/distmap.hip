@@ -2,6 +2,8 @@
 // queries (plain and rigidly transformed), and the exact point-mesh builder.
 #include "fc_internal.hpp"
 #include "distmap.hpp"
+#include "mesh_distance.hpp"
+#include "mesh_tree.hpp"
 
 #include <cfloat>
 #include <charconv>
@@ -203,187 +205,122 @@ __global__ __launch_bounds__(kBlock) void k_integrate_distmap(fc_sim_params P, D
 // Builder: exact signed distance of every lattice vertex to a closed mesh.
 // ---------------------------------------------------------------------------
 
-// Squared distance from q to triangle (B, V1, V2) and the closest point, by
-// the region method of D. Eberly, "Distance Between Point and Triangle in
-// 3D" (Geometric Tools), in binary64.  (The reference's variant,
-// distance/distancetriangle.cpp:55-190, departs from it in regions 4 and 6.)
-__device__ __forceinline__ double point_triangle_dist2(const double q[3], const double* B,
-                                                       const double* V1, const double* V2,
-                                                       double cp[3]) {
-  double E0[3], E1[3], D[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    E0[k] = V1[k] - B[k];
-    E1[k] = V2[k] - B[k];
-    D[k] = B[k] - q[k];
-  }
-  const double a = E0[0] * E0[0] + E0[1] * E0[1] + E0[2] * E0[2];
-  const double b = E0[0] * E1[0] + E0[1] * E1[1] + E0[2] * E1[2];
-  const double c = E1[0] * E1[0] + E1[1] * E1[1] + E1[2] * E1[2];
-  const double d = E0[0] * D[0] + E0[1] * D[1] + E0[2] * D[2];
-  const double e = E1[0] * D[0] + E1[1] * D[1] + E1[2] * D[2];
-  const double det = a * c - b * b;
-  double s = b * e - c * d, t = b * d - a * e;
-  if (s + t <= det) {
-    if (s < 0.0) {
-      if (t < 0.0) {  // region 4
-        if (d < 0.0) {
-          t = 0.0;
-          s = (-d >= a) ? 1.0 : -d / a;
-        } else {
-          s = 0.0;
-          t = (e >= 0.0) ? 0.0 : ((-e >= c) ? 1.0 : -e / c);
-        }
-      } else {  // region 3
-        s = 0.0;
-        t = (e >= 0.0) ? 0.0 : ((-e >= c) ? 1.0 : -e / c);
-      }
-    } else if (t < 0.0) {  // region 5
-      t = 0.0;
-      s = (d >= 0.0) ? 0.0 : ((-d >= a) ? 1.0 : -d / a);
-    } else {  // region 0
-      const double inv = 1.0 / det;
-      s *= inv;
-      t *= inv;
-    }
-  } else {
-    if (s < 0.0) {  // region 2
-      const double tmp0 = b + d, tmp1 = c + e;
-      if (tmp1 > tmp0) {
-        const double numer = tmp1 - tmp0, denom = a - 2.0 * b + c;
-        s = (numer >= denom) ? 1.0 : numer / denom;
-        t = 1.0 - s;
-      } else {
-        s = 0.0;
-        t = (tmp1 <= 0.0) ? 1.0 : ((e >= 0.0) ? 0.0 : -e / c);
-      }
-    } else if (t < 0.0) {  // region 6
-      const double tmp0 = b + e, tmp1 = a + d;
-      if (tmp1 > tmp0) {
-        const double numer = tmp1 - tmp0, denom = a - 2.0 * b + c;
-        t = (numer >= denom) ? 1.0 : numer / denom;
-        s = 1.0 - t;
-      } else {
-        t = 0.0;
-        s = (tmp1 <= 0.0) ? 1.0 : ((d >= 0.0) ? 0.0 : -d / a);
-      }
-    } else {  // region 1
-      const double numer = (c + e) - (b + d);
-      if (numer <= 0.0) {
-        s = 0.0;
-      } else {
-        const double denom = a - 2.0 * b + c;
-        s = (numer >= denom) ? 1.0 : numer / denom;
-      }
-      t = 1.0 - s;
-    }
-  }
-  double r2 = 0.0;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    cp[k] = (B[k] + s * E0[k]) + t * E1[k];
-    const double diff = cp[k] - q[k];
-    r2 += diff * diff;
-  }
-  return r2;
-}
-
-// Solid angle of a triangle seen from q (Van Oosterom & Strackee 1983).
-__device__ __forceinline__ double solid_angle(const double q[3], const double* A, const double* B,
-                                              const double* C) {
-  double a[3], b[3], c[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    a[k] = A[k] - q[k];
-    b[k] = B[k] - q[k];
-    c[k] = C[k] - q[k];
-  }
-  const double la = sqrt(a[0] * a[0] + a[1] * a[1] + a[2] * a[2]);
-  const double lb = sqrt(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]);
-  const double lc = sqrt(c[0] * c[0] + c[1] * c[1] + c[2] * c[2]);
-  const double det = a[0] * (b[1] * c[2] - b[2] * c[1]) - a[1] * (b[0] * c[2] - b[2] * c[0]) +
-                     a[2] * (b[0] * c[1] - b[1] * c[0]);
-  const double ab = a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
-  const double bc = b[0] * c[0] + b[1] * c[1] + b[2] * c[2];
-  const double ca = c[0] * a[0] + c[1] * a[1] + c[2] * a[2];
-  const double den = la * lb * lc + ab * lc + bc * la + ca * lb;
-  return 2.0 * atan2(det, den);
-}
-
 constexpr int kTriTile = 128;
 
 // One lane per query point (lattice vertex or free point); triangles are
 // streamed through LDS in tiles that every lane of the block reads
 // (broadcast reads, no bank conflicts).  Minimum over triangles in order
 // (first minimum wins), sign from the generalized winding number.
+// For small problems, and for meshes that the triangle tree does not take:
+// with `info` the kernel leaves those that it does take (mesh_closed).
+// Blocks walk the points with the grid's stride, so that a launch that finds
+// nothing to do is short.
+constexpr unsigned kSdfMaxBlocks = 4096;
+
 template <bool kLattice>
 __global__ __launch_bounds__(kBlock) void k_mesh_sdf(
-    const double* __restrict__ verts, uint32_t nv, const uint32_t* __restrict__ tris, uint32_t nt,
-    uint64_t npts, const double* __restrict__ pts, int cx, int cy, double bx, double by,
-    double bz, double cs, float4* __restrict__ cpd, float4* __restrict__ nrm,
-    double* __restrict__ sdfOut, double* __restrict__ cpOut) {
+    const MeshInfo* __restrict__ info, const double* __restrict__ verts, uint32_t nv,
+    const uint32_t* __restrict__ tris, uint32_t nt, uint64_t npts, const double* __restrict__ pts,
+    int cx, int cy, double bx, double by, double bz, double cs, float4* __restrict__ cpd,
+    float4* __restrict__ nrm, double* __restrict__ sdfOut, double* __restrict__ cpOut) {
   __shared__ double s_tri[kTriTile][9];
-  const uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-  const bool valid = v < npts;
-  double q[3] = {0.0, 0.0, 0.0};
-  if (valid) {
-    if (kLattice) {
-      const uint64_t ix = (uint64_t)cx + 1, islice = ix * ((uint64_t)cy + 1);
-      const uint64_t iz = v / islice, rem = v - iz * islice, iy = rem / ix, ixx = rem - iy * ix;
-      q[0] = bx + (double)ixx * cs;
-      q[1] = by + (double)iy * cs;
-      q[2] = bz + (double)iz * cs;
-    } else {
-      q[0] = pts[3 * v];
-      q[1] = pts[3 * v + 1];
-      q[2] = pts[3 * v + 2];
-    }
-  }
-  double best = DBL_MAX, bcp[3] = {0.0, 0.0, 0.0}, w = 0.0;
-  for (uint32_t t0 = 0; t0 < nt; t0 += kTriTile) {
-    __syncthreads();
-    for (int k = threadIdx.x; k < kTriTile * 3; k += kBlock) {
-      const uint32_t t = t0 + k / 3;
-      if (t < nt) {
-        uint32_t vi = tris[3 * t + k % 3];
-        if (vi >= nv) vi = nv - 1;  // out-of-range indices must not read past the mesh
-        s_tri[k / 3][3 * (k % 3)] = verts[3 * vi];
-        s_tri[k / 3][3 * (k % 3) + 1] = verts[3 * vi + 1];
-        s_tri[k / 3][3 * (k % 3) + 2] = verts[3 * vi + 2];
+  if (info != nullptr && mesh_closed(*info)) return;
+  for (uint64_t base = (uint64_t)blockIdx.x * kBlock; base < npts;
+       base += (uint64_t)gridDim.x * kBlock) {
+    const uint64_t v = base + threadIdx.x;
+    const bool valid = v < npts;
+    double q[3] = {0.0, 0.0, 0.0};
+    if (valid) {
+      if (kLattice) {
+        const uint64_t ix = (uint64_t)cx + 1, islice = ix * ((uint64_t)cy + 1);
+        const uint64_t iz = v / islice, rem = v - iz * islice, iy = rem / ix, ixx = rem - iy * ix;
+        q[0] = bx + (double)ixx * cs;
+        q[1] = by + (double)iy * cs;
+        q[2] = bz + (double)iz * cs;
+      } else {
+        q[0] = pts[3 * v];
+        q[1] = pts[3 * v + 1];
+        q[2] = pts[3 * v + 2];
       }
     }
-    __syncthreads();
+    double best = DBL_MAX, bcp[3] = {0.0, 0.0, 0.0}, w = 0.0;
+    for (uint32_t t0 = 0; t0 < nt; t0 += kTriTile) {
+      __syncthreads();
+      for (int k = threadIdx.x; k < kTriTile * 3; k += kBlock) {
+        const uint32_t t = t0 + k / 3;
+        if (t < nt) {
+          uint32_t vi = tris[3 * t + k % 3];
+          if (vi >= nv) vi = nv - 1;  // out-of-range indices must not read past the mesh
+          s_tri[k / 3][3 * (k % 3)] = verts[3 * vi];
+          s_tri[k / 3][3 * (k % 3) + 1] = verts[3 * vi + 1];
+          s_tri[k / 3][3 * (k % 3) + 2] = verts[3 * vi + 2];
+        }
+      }
+      __syncthreads();
+      if (!valid) continue;
+      const uint32_t cnt = (nt - t0) < (uint32_t)kTriTile ? (nt - t0) : (uint32_t)kTriTile;
+      for (uint32_t t = 0; t < cnt; ++t) {
+        const double* T = s_tri[t];
+        double c3[3];
+        const double d2 = point_triangle_dist2(q, T, T + 3, T + 6, c3);
+        if (d2 < best) {
+          best = d2;
+          bcp[0] = c3[0];
+          bcp[1] = c3[1];
+          bcp[2] = c3[2];
+        }
+        w += solid_angle(q, T, T + 3, T + 6);
+      }
+    }
     if (!valid) continue;
-    const uint32_t cnt = (nt - t0) < (uint32_t)kTriTile ? (nt - t0) : (uint32_t)kTriTile;
-    for (uint32_t t = 0; t < cnt; ++t) {
-      const double* T = s_tri[t];
-      double c3[3];
-      const double d2 = point_triangle_dist2(q, T, T + 3, T + 6, c3);
-      if (d2 < best) {
-        best = d2;
-        bcp[0] = c3[0];
-        bcp[1] = c3[1];
-        bcp[2] = c3[2];
+    w /= 4.0 * 3.14159265358979323846;
+    const double dist = sqrt(best);
+    const double sd = (w > 0.5) ? -dist : dist;
+    if (kLattice) {
+      cpd[v] = make_float4((float)bcp[0], (float)bcp[1], (float)bcp[2], (float)sd);
+      nrm[v] = make_float4((float)(q[0] - bcp[0]), (float)(q[1] - bcp[1]), (float)(q[2] - bcp[2]),
+                           0.0f);
+    } else {
+      sdfOut[v] = sd;
+      if (cpOut) {
+        cpOut[3 * v] = bcp[0];
+        cpOut[3 * v + 1] = bcp[1];
+        cpOut[3 * v + 2] = bcp[2];
       }
-      w += solid_angle(q, T, T + 3, T + 6);
     }
   }
-  if (!valid) return;
-  w /= 4.0 * 3.14159265358979323846;
-  const double dist = sqrt(best);
-  const double sd = (w > 0.5) ? -dist : dist;
-  if (kLattice) {
-    cpd[v] = make_float4((float)bcp[0], (float)bcp[1], (float)bcp[2], (float)sd);
-    nrm[v] = make_float4((float)(q[0] - bcp[0]), (float)(q[1] - bcp[1]), (float)(q[2] - bcp[2]),
-                         0.0f);
-  } else {
-    sdfOut[v] = sd;
-    if (cpOut) {
-      cpOut[3 * v] = bcp[0];
-      cpOut[3 * v + 1] = bcp[1];
-      cpOut[3 * v + 2] = bcp[2];
-    }
+}
+
+unsigned sdf_blocks(uint64_t npts) {
+  const unsigned g = grid_for(npts, kBlock);
+  return g < kSdfMaxBlocks ? g : kSdfMaxBlocks;
+}
+
+// The tree's scratch, grown to the largest mesh the context has seen (about
+// 130 bytes a triangle); false when there is no memory for it, or inside a
+// graph capture, where it could not grow.  The callers then take the brute
+// force alone.
+bool tree_scratch(fc_context* ctx, uint32_t nt, size_t extra) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+    return false;
+  if (ensure_sort_capacity(ctx, nt) != FC_SUCCESS) {
+    (void)hipGetLastError();
+    return false;
   }
+  const size_t need = mesh_tree_bytes(nt) + extra;
+  if (ctx->meshCapacity >= need) return true;
+  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+  (void)hipFree(ctx->meshScratch);
+  ctx->meshScratch = nullptr;
+  ctx->meshCapacity = 0;
+  if (hipMalloc(&ctx->meshScratch, need) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->meshScratch = nullptr;
+    return false;
+  }
+  ctx->meshCapacity = need;
+  return true;
 }
 
 }  // namespace
@@ -396,13 +333,19 @@ hipError_t launch_integrate_distmap(hipStream_t s, const fc_sim_params& P, const
   return hipGetLastError();
 }
 
-hipError_t launch_mesh_sdf_points(hipStream_t s, const double* verts, uint32_t nv,
-                                  const uint32_t* tris,
-                                  uint32_t nt, const double* pts, uint64_t np, double* sdf,
-                                  double* cp) {
+hipError_t launch_mesh_sdf_points(fc_context* ctx, const double* verts, uint32_t nv,
+                                  const uint32_t* tris, uint32_t nt, const double* pts,
+                                  uint64_t np, double* sdf, double* cp) {
   if (np == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_mesh_sdf<false>, dim3(grid_for(np, kBlock)), dim3(kBlock), 0, s, verts, nv,
-                     tris, nt, np, pts, 0, 0, 0.0, 0.0, 0.0, 0.0, nullptr, nullptr, sdf, cp);
+  hipStream_t s = ctx->stream;
+  MeshTree T;
+  if (mesh_tree_pays(nt, np) && tree_scratch(ctx, nt, 0)) {
+    hipError_t e = launch_mesh_tree(ctx, verts, nv, tris, nt, ctx->meshScratch, &T);
+    if (e == hipSuccess) e = launch_tree_points(s, T, verts, nv, tris, nt, pts, np, sdf, cp);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(k_mesh_sdf<false>, dim3(sdf_blocks(np)), dim3(kBlock), 0, s, T.info, verts,
+                     nv, tris, nt, np, pts, 0, 0, 0.0, 0.0, 0.0, 0.0, nullptr, nullptr, sdf, cp);
   return hipGetLastError();
 }
 
@@ -847,10 +790,18 @@ fc_status fc_distmap_build(fc_context* ctx, const double* vertices, uint32_t num
   if (e == hipSuccess) e = hipMemcpyAsync(m->xs, ax[0].data(), ax[0].size() * 4, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipMemcpyAsync(m->ys, ax[1].data(), ax[1].size() * 4, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipMemcpyAsync(m->zs, ax[2].data(), ax[2].size() * 4, hipMemcpyHostToDevice, st);
+  MeshTree T;
+  if (e == hipSuccess && mesh_tree_pays(numTriangles, m->V) && tree_lattice_fits(cells) &&
+      tree_scratch(ctx, numTriangles, 0)) {
+    e = launch_mesh_tree(ctx, dv, numVertices, dt, numTriangles, ctx->meshScratch, &T);
+    if (e == hipSuccess)
+      e = launch_tree_lattice(st, T, dv, numVertices, dt, numTriangles, m->cells, b, cs, m->cpd,
+                              m->nrm);
+  }
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_mesh_sdf<true>, dim3(grid_for(m->V, kBlock)), dim3(kBlock), 0, st, dv,
-                       numVertices, dt, numTriangles, (uint64_t)m->V, nullptr, cells[0], cells[1], b[0], b[1],
-                       b[2], cs, m->cpd, m->nrm, nullptr, nullptr);
+    hipLaunchKernelGGL(k_mesh_sdf<true>, dim3(sdf_blocks(m->V)), dim3(kBlock), 0, st, T.info, dv,
+                       numVertices, dt, numTriangles, (uint64_t)m->V, nullptr, cells[0], cells[1],
+                       b[0], b[1], b[2], cs, m->cpd, m->nrm, nullptr, nullptr);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -1016,8 +967,8 @@ fc_status fc_mesh_signed_distance(fc_context* ctx, const double* vertices, uint3
   if (numPoints == 0) return FC_SUCCESS;
   if (numTriangles == 0) return set_error(FC_ERROR_INVALID_VALUE, "empty mesh");
   if (numVertices == 0) return set_error(FC_ERROR_INVALID_VALUE, "empty mesh");
-  hipError_t e = launch_mesh_sdf_points(ctx->stream, vertices, numVertices, triangles,
-                                        numTriangles, points, numPoints, sdf, closest);
+  hipError_t e = launch_mesh_sdf_points(ctx, vertices, numVertices, triangles, numTriangles,
+                                        points, numPoints, sdf, closest);
   if (e != hipSuccess) return hip_error(e, "mesh signed distance");
   return FC_SUCCESS;
 }

@@ -336,6 +336,7 @@ fc_status fc_context_destroy(fc_context* ctx) {
   hipFree(ctx->statsScratch);
   hipFree(ctx->rowsVel);
   hipFree(ctx->rowsQ);
+  hipFree(ctx->meshScratch);
   if (ctx->stream) hipStreamDestroy(ctx->stream);
   delete ctx;
   return FC_SUCCESS;

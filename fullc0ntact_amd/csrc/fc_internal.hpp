@@ -329,6 +329,10 @@ struct fc_context {
   float4* rowsVel = nullptr;
   uint2* rowsQ = nullptr;
   uint32_t rowsCapacity = 0;
+  // Triangle tree of the mesh distances (mesh_tree.hip), grown to the
+  // largest mesh seen.
+  void* meshScratch = nullptr;
+  size_t meshCapacity = 0;
 };
 
 namespace fc {
