@@ -28,6 +28,7 @@ struct SceneCollide {
   v3f invCell;
   float contactD2;
   uint32_t qThreshold;
+  uint32_t cutWraps;  // the walls keep the scene inside its grid
 };
 }  // namespace fc
 
@@ -191,8 +192,9 @@ __device__ __forceinline__ T scene_block(const T* p, uint32_t s) {
 // of a wave take their scenes one at a time (nearly every wave holds one
 // scene), each with its parameters in scalar registers, which keeps them
 // out of the vector registers the walk needs.
+constexpr int kBatchWavesPerSimd = 4;
 template <int BS>
-__global__ __launch_bounds__(BS) void k_batch_collide_rows(
+__global__ __launch_bounds__(BS, kBatchWavesPerSimd) void k_batch_collide_rows(
     const fc_sim_params* __restrict__ prm, const SceneCollide* __restrict__ sc, int cellBits,
     uint32_t C, float4* __restrict__ newVel, const float4* __restrict__ sortedPos,
     const float4* __restrict__ sortedVel, const uint2* __restrict__ sortedQ,
@@ -217,8 +219,8 @@ __global__ __launch_bounds__(BS) void k_batch_collide_rows(
     const v3f force = add_collider(
         P, pos, vel, P.particleRadius,
         collide_one_rows<false, BS>(P, c.invCell, c.contactD2, k, pos, vel, P.particleRadius,
-                                    sortedPos, sortedVel, sortedQ, c.qThreshold,
-                                    cellStart + base, cellEnd + base, n, s_list));
+                                    sortedPos, sortedVel, sortedQ, RowFilter{c.qThreshold, 0.0f},
+                                    c.cutWraps != 0u, cellStart + base, cellEnd + base, n, s_list));
     newVel[index[k]] = make_float4(vel.x + force.x, vel.y + force.y, vel.z + force.z, 0.0f);
   }
 }
@@ -232,7 +234,7 @@ __global__ __launch_bounds__(BS) void k_batch_collide_rows(
 // keys' digit-0 histogram for the next sort.  kLast (the run's last step):
 // newVel and the positions go back to the ids instead.
 template <int BS, bool kLast>
-__global__ __launch_bounds__(BS) void k_batch_collide_run(
+__global__ __launch_bounds__(BS, kBatchWavesPerSimd) void k_batch_collide_run(
     const fc_sim_params* __restrict__ prm, const SceneCollide* __restrict__ sc, int cellBits,
     uint32_t C, float4* __restrict__ pos, float4* __restrict__ vel,
     const float4* __restrict__ sortedPos, const float4* __restrict__ sortedVel,
@@ -269,8 +271,8 @@ __global__ __launch_bounds__(BS) void k_batch_collide_run(
     const v3f force = add_collider(
         P, p0, v0, P.particleRadius,
         collide_one_rows<false, BS>(P, c.invCell, c.contactD2, k, p0, v0, P.particleRadius,
-                                    sortedPos, sortedVel, sortedQ, c.qThreshold,
-                                    cellStart + base, cellEnd + base, n, s_list));
+                                    sortedPos, sortedVel, sortedQ, RowFilter{c.qThreshold, 0.0f},
+                                    c.cutWraps != 0u, cellStart + base, cellEnd + base, n, s_list));
     const uint32_t orig = index[k];
     const v3f nv = make_v3(v0.x + force.x, v0.y + force.y, v0.z + force.z);
     if (kLast) {
@@ -653,6 +655,7 @@ fc_status upload_batch_params(fc_batch* b) {
     sc[s].invCell = inv_cell(P);
     sc[s].contactD2 = d2[s];
     sc[s].qThreshold = quant_threshold(P.particleRadius + P.particleRadius, batch_frame().scale);
+    sc[s].cutWraps = wraps_out_of_reach(P) && walls_inside_grid(P) ? 1u : 0u;
   }
   FC_HIP_TRY(hipMemcpyAsync(b->dSceneCollide, sc.data(), b->S * sizeof(SceneCollide),
                             hipMemcpyHostToDevice, b->ctx->stream));

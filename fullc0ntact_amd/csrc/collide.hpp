@@ -243,6 +243,14 @@ __device__ __forceinline__ uint32_t quant_d2(uint2 a, uint2 b) {
   return (uint32_t)__builtin_amdgcn_sdot2(dxy, dxy, __mul24(dz, dz), false);
 }
 
+// Bounds of the candidate filter: on the squared fixed-point distance of a
+// pair in contact (units of 1/scale) for the largest contact distance, and
+// the scale for a sphere's own.
+struct RowFilter {
+  uint32_t threshold;
+  float scale;
+};
+
 // Row-range variant of collide_one_v3 for grids with every dimension >= 4,
 // numCells <= 2^30 and n < 2^28, on the arrays of a sort that gathered the
 // state (SortGather): sortedVel[j].w holds the bits of sphere j's sorted
@@ -278,10 +286,23 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
                                                 float rA, const float4* __restrict__ sortedPos,
                                                 const float4* __restrict__ sortedVel,
                                                 const uint2* __restrict__ sortedQ,
-                                                uint32_t qThreshold,
+                                                RowFilter filter, bool cutWraps,
                                                 const uint32_t* __restrict__ cellStart,
                                                 const uint32_t* __restrict__ cellEnd, uint32_t n,
                                                 uint32_t (*s_list)[BS]) {
+  // Equal radii: the launch's bounds for the contact distance 2 r.  With
+  // radii of their own, no neighbour is larger than particleRadius, so this
+  // sphere's contacts lie within rA + particleRadius: on a log-normal bed
+  // (3x clip) 11 instead of 20 candidates pass, and 7 % of the waves instead
+  // of 64 % hold a list that overflows.
+  uint32_t qThreshold = filter.threshold;
+  if (kPoly) {
+    const float reach = rA + P.particleRadius;
+    const float b = reach * filter.scale + 2.51f;  // quant_threshold, in binary32
+    if (b < 32000.0f && reach > 0.0f)
+      qThreshold = min(qThreshold, (uint32_t)ceilf(b * b * (1.0f + 0x1p-20f)));
+    contactD2 = fminf(contactD2, reach * reach * (1.0f + 0x1p-20f));
+  }
   const v3f q = cell_quotients(P, invCell, pos);
   const int gx = cell_of_quotient(q.x), gy = cell_of_quotient(q.y), gz = cell_of_quotient(q.z);
   const uint32_t Gx = P.gridSize.x, Gy = P.gridSize.y;
@@ -329,6 +350,19 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
     const float lz = fmaxf(fz - uz, 0.0f) * P.cellSize.z, hz = fmaxf(1.0f - fz - uz, 0.0f) * P.cellSize.z;
     lo2 = make_v3(lx * lx, ly * ly, lz * lz);
     hi2 = make_v3(hx * hx, hy * hy, hz * hz);
+  }
+  // cutWraps: every sphere's cell index lies inside the grid, so the cells
+  // reached by wrapping hold spheres of the opposite side only, G - 2 cells
+  // away, out of contact (wraps_out_of_reach).  Cutting them keeps the lanes
+  // at a wall out of the direct loop below, which a row of two runs takes:
+  // where the grid covers the box exactly, as the class defaults do, most
+  // waves hold such a lane.  500,009 spheres in a 128^3 grid: TIMES_STAGES.
+  if (cutWraps) {
+    const uint32_t yc = (uint32_t)gy & my, zc = (uint32_t)gz & mz;
+    lo2 = make_v3(xc == 0u ? INFINITY : lo2.x, yc == 0u ? INFINITY : lo2.y,
+                  zc == 0u ? INFINITY : lo2.z);
+    hi2 = make_v3(xc == mx ? INFINITY : hi2.x, yc == my ? INFINITY : hi2.y,
+                  zc == mz ? INFINITY : hi2.z);
   }
 
   const bool wrapLo = xc == 0u, wrapHi = xc == mx;
@@ -442,12 +476,13 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
     }
     force = make_v3(force.x + cf.x, force.y + cf.y, force.z + cf.z);
   } else if (!split) {
-    // The list overflowed (a densely packed bed: up to ~60 contacts): walk
-    // the nine row ranges as one flattened sequence, kPairBatch candidates
-    // per iteration with their loads in flight together, each candidate
-    // through the exact pair force (non-touching ones add +0), the cell
-    // partial added when the sorted hash changes -- the list path's terms
-    // in the list path's order.
+    // The list overflowed (a densely packed bed: up to ~60 contacts; cells
+    // of 50 and more where spheres pile up): walk the nine row ranges again
+    // as one flattened sequence, filling the list and emptying it through
+    // the exact pair force in turns, the lanes of the wave together -- the
+    // list path's terms in the list path's order.  Only what passes the
+    // filter reaches the pair force (a walk that sent every candidate
+    // through it took TIMES_KNOT).
     uint32_t B[9], Q[9];  // slots before row r; slot t of row r is sphere t + Q[r]
     uint32_t total = 0;
 #pragma unroll
@@ -458,33 +493,54 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
     }
     v3f cf = make_v3(0.0f, 0.0f, 0.0f);
     uint32_t curHash = 0xffffffffu;
+    uint32_t t = 0;
 #pragma unroll 1
-    for (uint32_t t = 0; t < total; t += kPairBatch) {
-      uint32_t jj[kPairBatch];
-      float4 qp[kPairBatch], qv[kPairBatch];
+    while (t < total) {
+      cnt = 0;
+#pragma unroll 1
+      while (t < total && cnt <= (uint32_t)(kListCap - kPairBatch)) {
+        uint32_t jj[kPairBatch];
+        uint2 c[kPairBatch];
 #pragma unroll
-      for (int u = 0; u < kPairBatch; ++u) {
-        const uint32_t tu = t + (uint32_t)u < total ? t + (uint32_t)u : total - 1u;
-        uint32_t qr = Q[0];
+        for (int u = 0; u < kPairBatch; ++u) {
+          const uint32_t tu = t + (uint32_t)u < total ? t + (uint32_t)u : total - 1u;
+          uint32_t qr = Q[0];
 #pragma unroll
-        for (int r = 1; r < 9; ++r) qr = tu >= B[r] ? Q[r] : qr;
-        jj[u] = tu + qr;
-        qp[u] = sortedPos[jj[u]];
-        qv[u] = sortedVel[jj[u]];  // .w holds the sorted hash
+          for (int r = 1; r < 9; ++r) qr = tu >= B[r] ? Q[r] : qr;
+          jj[u] = tu + qr;
+          c[u] = sortedQ[jj[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < kPairBatch; ++u) {
+          s_list[cnt][threadIdx.x] = jj[u];
+          const bool in = t + (uint32_t)u < total && jj[u] != k;
+          cnt += (quant_d2(c[u], me) < qThreshold && in) ? 1u : 0u;
+        }
+        t += kPairBatch;
       }
+#pragma unroll 1
+      for (uint32_t i = 0; i < cnt; i += kPairBatch) {
+        float4 qp[kPairBatch], qv[kPairBatch];
 #pragma unroll
-      for (int u = 0; u < kPairBatch; ++u) {
-        if (t + (uint32_t)u < total && jj[u] != k) {
-          const uint32_t hu = __float_as_uint(qv[u].w);
-          if (hu != curHash) {
-            force = make_v3(force.x + cf.x, force.y + cf.y, force.z + cf.z);
-            cf = make_v3(0.0f, 0.0f, 0.0f);
-            curHash = hu;
+        for (int u = 0; u < kPairBatch; ++u) {
+          const uint32_t j = i + (uint32_t)u < cnt ? s_list[i + (uint32_t)u][threadIdx.x] : k;
+          qp[u] = load_off(sortedPos, j << 4);
+          qv[u] = load_off(sortedVel, j << 4);  // .w holds the sorted hash
+        }
+#pragma unroll
+        for (int u = 0; u < kPairBatch; ++u) {
+          if (i + (uint32_t)u < cnt) {
+            const uint32_t hu = __float_as_uint(qv[u].w);
+            if (hu != curHash) {
+              force = make_v3(force.x + cf.x, force.y + cf.y, force.z + cf.z);
+              cf = make_v3(0.0f, 0.0f, 0.0f);
+              curHash = hu;
+            }
+            v3f f = collide_spheres_fast(pos, xyz(qp[u]), vel, xyz(qv[u]), rA,
+                                         kPoly ? qp[u].w : rA, P.spring, P.damping, P.shear,
+                                         P.attraction);
+            cf = make_v3(cf.x + f.x, cf.y + f.y, cf.z + f.z);
           }
-          v3f f = collide_spheres_fast(pos, xyz(qp[u]), vel, xyz(qv[u]), rA,
-                                       kPoly ? qp[u].w : rA, P.spring, P.damping, P.shear,
-                                       P.attraction);
-          cf = make_v3(cf.x + f.x, cf.y + f.y, cf.z + f.z);
         }
       }
     }

@@ -84,16 +84,24 @@ __global__ __launch_bounds__(kBlock) void k_calc_hash(fc_sim_params P, uint32_t*
 // sorted sphere's velocity with the bits of its cell hash in w (the hash of
 // its position, as calcHash computes it, so the hash it was sorted by when
 // the arrays come from reorderDataAndFindCellStart of those hashes), and its
-// 16-bit coordinates in `frame`.
+// 16-bit coordinates in `frame`; *outside = epoch when a sphere's cell index
+// lies outside the grid.
 __global__ __launch_bounds__(kBlock) void k_rows_state(fc_sim_params P, QuantFrame frame,
                                                        const float4* __restrict__ sortedPos,
                                                        const float4* __restrict__ sortedVel,
                                                        uint32_t n, float4* __restrict__ velOut,
-                                                       uint2* __restrict__ qOut) {
+                                                       uint2* __restrict__ qOut,
+                                                       uint32_t* __restrict__ outside,
+                                                       uint32_t epoch) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   const float4 p = sortedPos[i], v = sortedVel[i];
-  velOut[i] = make_float4(v.x, v.y, v.z, __uint_as_float(hash_of(P, p.x, p.y, p.z)));
+  const int gx = cell_coord(p.x, P.worldOrigin.x, P.cellSize.x);
+  const int gy = cell_coord(p.y, P.worldOrigin.y, P.cellSize.y);
+  const int gz = cell_coord(p.z, P.worldOrigin.z, P.cellSize.z);
+  if ((uint32_t)gx >= P.gridSize.x || (uint32_t)gy >= P.gridSize.y || (uint32_t)gz >= P.gridSize.z)
+    *outside = epoch;
+  velOut[i] = make_float4(v.x, v.y, v.z, __uint_as_float(grid_hash(gx, gy, gz, P.gridSize)));
   qOut[i] = quantize_pos(frame, p.x, p.y, p.z);
 }
 
@@ -293,7 +301,8 @@ __global__ __launch_bounds__(kBlock) void k_collide_v2(
 // pre-filter are sized by particleRadius).
 // kRows selects the row-range neighbour walk (collide_one_rows), which
 // needs the sorted hashes in sortedVel.w and the fixed-point coordinates
-// sortedQ with their filter bound qThreshold.
+// sortedQ with their filter bounds, and leaves out the cells reached by
+// wrapping where `wraps` allows it.
 // forceOut != nullptr (not fused) is evalForces_launcher
 // (particledem_um.cu:538-589): no cursor sphere, and the force also stored
 // as float3 at the original index.
@@ -307,6 +316,14 @@ __global__ __launch_bounds__(kBlock) void k_collide_v2(
 // VGPRs; the fused launch on the settled 1M-sphere bed measured 91.0 us
 // against 94.3 us.
 constexpr int kCollideWavesPerSimd = 5;
+
+// Whether the wrapped cells may be cut (collide_one_rows): known by the
+// launch, or unless the arrays' check wrote `epoch` (GatheredState).
+struct WrapCut {
+  uint32_t cut = 0, epoch = 0;
+  const uint32_t* outside = nullptr;
+};
+
 template <bool kFuse, bool kPoly, bool kRows>
 __global__ __launch_bounds__(kBlock, kCollideWavesPerSimd) void k_collide_v3(
     fc_sim_params P, BoundaryArg B, float contactD2, float4* __restrict__ newVel,
@@ -315,9 +332,11 @@ __global__ __launch_bounds__(kBlock, kCollideWavesPerSimd) void k_collide_v3(
     const uint32_t* __restrict__ cellEnd, uint32_t n, uint32_t xcdGroup, float4* __restrict__ pos,
     float dt, uint32_t* __restrict__ keysOut, int passes, uint32_t* gHist, uint32_t* counters,
     uint32_t* devFlags, uint32_t* __restrict__ slotOf, uint32_t* __restrict__ idOfSlot,
-    v3f invCell, const uint2* __restrict__ sortedQ, uint32_t qThreshold,
+    v3f invCell, const uint2* __restrict__ sortedQ, RowFilter filter, WrapCut wraps,
     float* __restrict__ forceOut, int slotKeys, RowHists rows) {
   __shared__ uint32_t s_list[kListCap + 1][kBlock];
+  const bool cutWraps =
+      wraps.cut != 0u && (wraps.outside == nullptr || *wraps.outside != wraps.epoch);
   __shared__ uint32_t s_hist[kFuse ? RS_RADIX : 1];
   const uint32_t k = xcd_grouped_block(blockIdx.x, gridDim.x, xcdGroup) * kBlock + threadIdx.x;
   const bool valid = k < n;
@@ -338,7 +357,7 @@ __global__ __launch_bounds__(kBlock, kCollideWavesPerSimd) void k_collide_v3(
     const v3f pos0 = xyz(p4), vel0 = xyz(v4);
     v3f force =
         kRows ? collide_one_rows<kPoly, kBlock>(P, invCell, contactD2, k, pos0, vel0, rA,
-                                                sortedPos, sortedVel, sortedQ, qThreshold,
+                                                sortedPos, sortedVel, sortedQ, filter, cutWraps,
                                                 cellStart, cellEnd, n, s_list)
               : collide_one_v3<kPoly, kBlock>(P, contactD2, k, pos0, vel0, rA, sortedPos,
                                               sortedVel, cellStart, cellEnd, n, s_list);
@@ -504,10 +523,10 @@ hipError_t launch_integrate(hipStream_t s, const fc_sim_params& P, float4* pos, 
 
 hipError_t launch_rows_state(hipStream_t s, const fc_sim_params& P, const QuantFrame& frame,
                              const float4* sortedPos, const float4* sortedVel, uint32_t n,
-                             float4* velOut, uint2* qOut) {
+                             float4* velOut, uint2* qOut, uint32_t* outside, uint32_t epoch) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_rows_state, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, s, P, frame,
-                     sortedPos, sortedVel, n, velOut, qOut);
+                     sortedPos, sortedVel, n, velOut, qOut, outside, epoch);
   return hipGetLastError();
 }
 
@@ -605,6 +624,45 @@ uint32_t quant_threshold(float R, float scale) {
   return (uint32_t)std::ceil(b * b);
 }
 
+bool wraps_out_of_reach(const fc_sim_params& P) {
+  const uint32_t G[3] = {P.gridSize.x, P.gridSize.y, P.gridSize.z};
+  const float cs[3] = {P.cellSize.x, P.cellSize.y, P.cellSize.z};
+  for (int a = 0; a < 3; ++a) {
+    if (G[a] < 4u) return false;
+    // relative margin for the rounding of the spheres' cell quotients (2^-24
+    // of up to G cells each) and of their distance
+    const double apart = ((double)G[a] - 2.0 - 1e-6 * (double)G[a]) * (double)cs[a];
+    if (!(apart > 2.0 * (double)P.particleRadius * (1.0 + 1e-6))) return false;
+  }
+  return true;
+}
+
+bool walls_inside_grid(const fc_sim_params& P) {
+  // integrate_box's bounds, and the quotients of cell_coord: both ends in
+  // the same float operations, monotone in between
+  const float hi = 1.0f - P.particleRadius, lo = -1.0f + P.particleRadius;
+  const float top = hi > lo ? hi : lo, low = hi > lo ? lo : hi;
+  const float org[3] = {P.worldOrigin.x, P.worldOrigin.y, P.worldOrigin.z};
+  const float cs[3] = {P.cellSize.x, P.cellSize.y, P.cellSize.z};
+  const uint32_t G[3] = {P.gridSize.x, P.gridSize.y, P.gridSize.z};
+  for (int a = 0; a < 3; ++a)
+    if (!((low - org[a]) / cs[a] >= 0.0f && (top - org[a]) / cs[a] < (float)G[a])) return false;
+  return true;
+}
+
+static WrapCut wrap_cut(const fc_sim_params& P, const GatheredState& gs) {
+  WrapCut w;
+  if (!wraps_out_of_reach(P)) return w;
+  if (gs.walled && walls_inside_grid(P)) {
+    w.cut = 1u;
+  } else if (gs.outside != nullptr) {
+    w.cut = 1u;
+    w.outside = gs.outside;
+    w.epoch = gs.epoch;
+  }
+  return w;
+}
+
 // Systems up to this many spheres take the row-split collide (k_collide_split).
 #ifndef FC_SPLIT_MAX_SPHERES
 #define FC_SPLIT_MAX_SPHERES 16384
@@ -633,13 +691,15 @@ static void launch_v3(hipStream_t s, const GatheredState* gs, dim3 g, dim3 b,
                        sortedPos, sortedVel, index, cellStart, cellEnd, n, kCollideXcdGroup, pos,
                        dt, keysOut, passes, gHist, counters, devFlags, slotOf, idOfSlot,
                        inv_cell(P), gs->sortedQ,
-                       quant_threshold(P.particleRadius + P.particleRadius, gs->frame.scale),
-                       forceOut, slotKeys ? 1 : 0, rows ? *rows : RowHists{});
+                       RowFilter{quant_threshold(P.particleRadius + P.particleRadius,
+                                                 gs->frame.scale),
+                                 gs->frame.scale},
+                       wrap_cut(P, *gs), forceOut, slotKeys ? 1 : 0, rows ? *rows : RowHists{});
   else
     hipLaunchKernelGGL((k_collide_v3<kFuse, kPoly, false>), g, b, 0, s, P, B, d2, newVel,
                        sortedPos, sortedVel, index, cellStart, cellEnd, n, kCollideXcdGroup, pos,
                        dt, keysOut, passes, gHist, counters, devFlags, slotOf, idOfSlot,
-                       inv_cell(P), nullptr, 0u, forceOut, 0, RowHists{});
+                       inv_cell(P), nullptr, RowFilter{}, WrapCut{}, forceOut, 0, RowHists{});
 }
 
 hipError_t launch_collide(hipStream_t s, const fc_sim_params& P, bool poly, uint32_t* devFlags,

@@ -252,8 +252,10 @@ fc_status collide_reference_arrays(fc_context* ctx, float* newVel, float* force,
     }
     gs.sortedQ = ctx->rowsQ;
     gs.frame = quant_frame_for(false);  // integrate's box walls
+    gs.outside = ctx->devFlags + 1;
+    gs.epoch = ++ctx->rowsEpoch;
     FC_HIP_TRY(launch_rows_state(ctx->stream, P, gs.frame, (const float4*)sortedPos, vel, n,
-                                 ctx->rowsVel, ctx->rowsQ));
+                                 ctx->rowsVel, ctx->rowsQ, ctx->devFlags + 1, gs.epoch));
     vel = ctx->rowsVel;
     gathered = &gs;
   }
@@ -303,13 +305,13 @@ fc_status fc_context_create(int device, fc_context** out) {
   ctx->params = default_params(0, fc_uint3{64, 64, 64});
   ctx->paramsSet = true;
   SortScratch& s = ctx->sort;
-  bool ok = hipMalloc(&ctx->devFlags, sizeof(uint32_t)) == hipSuccess &&
+  bool ok = hipMalloc(&ctx->devFlags, 2 * sizeof(uint32_t)) == hipSuccess &&
             hipMalloc(&s.counters, RSC_COUNT * sizeof(uint32_t)) == hipSuccess &&
             hipMalloc(&s.histogram, (size_t)RS_HIST_COPIES * RS_MAX_PASSES * RS_RADIX *
                                         sizeof(uint32_t)) == hipSuccess &&
             hipMemset(s.histogram, 0, (size_t)RS_HIST_COPIES * RS_MAX_PASSES * RS_RADIX *
                                           sizeof(uint32_t)) == hipSuccess &&
-            hipMemset(ctx->devFlags, 0, sizeof(uint32_t)) == hipSuccess &&
+            hipMemset(ctx->devFlags, 0, 2 * sizeof(uint32_t)) == hipSuccess &&
             hipMemset(s.counters, 0, RSC_COUNT * sizeof(uint32_t)) == hipSuccess;
   if (!ok) {
     fc_context_destroy(ctx);

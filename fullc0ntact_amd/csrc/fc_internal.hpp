@@ -252,9 +252,15 @@ hipError_t launch_reorder(hipStream_t s, uint32_t* cellStart, uint32_t* cellEnd,
 // coordinates in `frame`: a system's arrays written by its sort's
 // SortGather, or the ones launch_rows_state builds for the reference-style
 // collide.
+// walled: integrate's box walls, with the parameters' radius, bound every
+// position; else outside (if given) holds `epoch` when launch_rows_state
+// found a sphere whose cell index lies outside the grid.
 struct GatheredState {
   const uint2* sortedQ = nullptr;
   QuantFrame frame;
+  bool walled = false;
+  const uint32_t* outside = nullptr;
+  uint32_t epoch = 0;
 };
 hipError_t launch_collide(hipStream_t s, const fc_sim_params& P, bool poly, uint32_t* devFlags,
                           float4* newVel, const float4* sortedPos, const float4* sortedVel,
@@ -268,7 +274,7 @@ hipError_t launch_collide(hipStream_t s, const fc_sim_params& P, bool poly, uint
 // kSortedPosPad entries) from the reference's sorted arrays.
 hipError_t launch_rows_state(hipStream_t s, const fc_sim_params& P, const QuantFrame& frame,
                              const float4* sortedPos, const float4* sortedVel, uint32_t n,
-                             float4* velOut, uint2* qOut);
+                             float4* velOut, uint2* qOut, uint32_t* outside, uint32_t epoch);
 // Whether the reference-style collide takes the row-range kernel through
 // launch_rows_state (large systems; small ones take the row-split kernel
 // on the reference's arrays as they are).
@@ -278,6 +284,12 @@ float contact_d2_threshold(float R);
 // Exact reciprocals of the cell sizes when all three are powers of two (the
 // multiply then equals the division), else zeros (cell_quotients divides).
 v3f inv_cell(const fc_sim_params& P);
+// Whether spheres of opposite ends of the grid, G - 2 cells apart, are out of
+// contact along every axis.
+bool wraps_out_of_reach(const fc_sim_params& P);
+// Whether the box walls (integrate_box) keep every position inside the grid,
+// so that no cell index wraps.
+bool walls_inside_grid(const fc_sim_params& P);
 // Bound on the squared fixed-point distance (units of 1/scale) of every pair
 // closer than R, for the row-range collide's candidate filter.
 uint32_t quant_threshold(float R, float scale);
@@ -321,7 +333,10 @@ struct fc_context {
   fc_sim_params params{};
   bool paramsSet = false;
   fc::SortScratch sort;
-  uint32_t* devFlags = nullptr;   // device error word
+  // device error word; then the epoch of the last reference-style collide
+  // whose spheres left the grid (GatheredState::outside)
+  uint32_t* devFlags = nullptr;
+  uint32_t rowsEpoch = 0;
   fc::StageTimer timer;
   double* statsScratch = nullptr; // FP64 reduction partials + histogram bins
   // State built for the row-range walk by the reference-style collide
@@ -434,4 +449,6 @@ struct fc_system {
   fc::RowTables rowTables;
   fc::BoundaryArg boundary_arg() const;
   fc::QuantFrame quant_frame() const;
+  // whether integrate's box walls, with one radius, bound every position
+  bool walled() const;
 };

@@ -137,7 +137,7 @@ fc_status enqueue_update(fc_system* sys, float dt, StageTimer* timer) {
     if (e != hipSuccess) return hip_error(e, "cell bounds");
   }
   if (timer) timer->begin(st, "collide");
-  const GatheredState gs{sys->sortedQ, ga.frame};
+  const GatheredState gs{sys->sortedQ, ga.frame, sys->walled()};
   e = launch_collide(st, P, sys->polydisperse != 0, ctx->devFlags, sys->vel, sys->sortedPos,
                      sys->sortedVel, sys->index, sys->cellStart, sys->cellEnd, n, nullptr, &gs);
   if (timer) timer->end(st);
@@ -287,7 +287,7 @@ fc_status enqueue_run_body(fc_system* sys, float dt, bool clearInSort, bool last
     if (e != hipSuccess) return hip_error(e, "cell bounds");
   }
   if (timer) timer->begin(st, last ? "collide" : "collide_integrate");
-  const GatheredState gs{sys->sortedQ, ga.frame};
+  const GatheredState gs{sys->sortedQ, ga.frame, sys->walled()};
   if (last)
     e = launch_collide(st, P, sys->polydisperse != 0, ctx->devFlags, sys->vel, sys->sortedPos,
                        sys->sortedVel, sys->index, sys->cellStart, sys->cellEnd, n,
@@ -378,6 +378,10 @@ using namespace fc;
 // [-1, 10].  One scale for all axes keeps fixed-point distances isotropic.
 fc::QuantFrame fc_system::quant_frame() const {
   return fc::quant_frame_for(boundary == FC_BOUNDARY_DISTMAP && boundaryMap != nullptr);
+}
+
+bool fc_system::walled() const {
+  return !polydisperse && !(boundary == FC_BOUNDARY_DISTMAP && boundaryMap != nullptr);
 }
 
 fc::BoundaryArg fc_system::boundary_arg() const {
