@@ -216,11 +216,13 @@ __global__ __launch_bounds__(BS, kBatchWavesPerSimd) void k_batch_collide_rows(
     const size_t base = (size_t)lead * C;
     const float4 p4 = sortedPos[k];
     const v3f pos = xyz(p4), vel = xyz(v4);
+    bool left;  // (never with one radius)
     const v3f force = add_collider(
         P, pos, vel, P.particleRadius,
         collide_one_rows<false, BS>(P, c.invCell, c.contactD2, k, pos, vel, P.particleRadius,
                                     sortedPos, sortedVel, sortedQ, RowFilter{c.qThreshold, 0.0f},
-                                    c.cutWraps != 0u, cellStart + base, cellEnd + base, n, s_list));
+                                    c.cutWraps != 0u, cellStart + base, cellEnd + base, n, s_list,
+                                    left));
     newVel[index[k]] = make_float4(vel.x + force.x, vel.y + force.y, vel.z + force.z, 0.0f);
   }
 }
@@ -268,11 +270,13 @@ __global__ __launch_bounds__(BS, kBatchWavesPerSimd) void k_batch_collide_run(
     const size_t base = (size_t)lead * C;
     const float4 p4 = sortedPos[k];
     const v3f p0 = xyz(p4), v0 = xyz(v4);
+    bool left;  // (never with one radius)
     const v3f force = add_collider(
         P, p0, v0, P.particleRadius,
         collide_one_rows<false, BS>(P, c.invCell, c.contactD2, k, p0, v0, P.particleRadius,
                                     sortedPos, sortedVel, sortedQ, RowFilter{c.qThreshold, 0.0f},
-                                    c.cutWraps != 0u, cellStart + base, cellEnd + base, n, s_list));
+                                    c.cutWraps != 0u, cellStart + base, cellEnd + base, n, s_list,
+                                    left));
     const uint32_t orig = index[k];
     const v3f nv = make_v3(v0.x + force.x, v0.y + force.y, v0.z + force.z);
     if (kLast) {

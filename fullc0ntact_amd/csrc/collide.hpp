@@ -280,6 +280,11 @@ struct RowFilter {
 // order.  As in collide_one_v3 every dropped or non-touching candidate
 // contributed exactly +0, so the result is bit-identical to the 27-cell
 // loop.  Returns the 27 cells' sum, as collide_one_v3 does.
+//
+// A lane whose list overflows, or with a row of two runs, has a path of its
+// own at the end.  With kPoly it is left to k_collide_piles instead
+// (`left`): log-normal radii pile up in cells of 50 and more, and the wave
+// that held such lanes was the launch's tail.
 template <bool kPoly, int BS>
 __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invCell,
                                                 float contactD2, uint32_t k, v3f pos, v3f vel,
@@ -289,7 +294,7 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
                                                 RowFilter filter, bool cutWraps,
                                                 const uint32_t* __restrict__ cellStart,
                                                 const uint32_t* __restrict__ cellEnd, uint32_t n,
-                                                uint32_t (*s_list)[BS]) {
+                                                uint32_t (*s_list)[BS], bool& left) {
   // Equal radii: the launch's bounds for the contact distance 2 r.  With
   // radii of their own, no neighbour is larger than particleRadius, so this
   // sphere's contacts lie within rA + particleRadius: on a log-normal bed
@@ -356,7 +361,8 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
   // away, out of contact (wraps_out_of_reach).  Cutting them keeps the lanes
   // at a wall out of the direct loop below, which a row of two runs takes:
   // where the grid covers the box exactly, as the class defaults do, most
-  // waves hold such a lane.  500,009 spheres in a 128^3 grid: TIMES_STAGES.
+  // waves hold such a lane (the collide of 500,009 settled spheres in a 128^3
+  // grid: 101 -> 49 us).
   if (cutWraps) {
     const uint32_t yc = (uint32_t)gy & my, zc = (uint32_t)gz & mz;
     lo2 = make_v3(xc == 0u ? INFINITY : lo2.x, yc == 0u ? INFINITY : lo2.y,
@@ -440,6 +446,7 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
   }
 
   v3f force = make_v3(0.0f, 0.0f, 0.0f);
+  left = kPoly && (split || cnt > (uint32_t)kListCap);
   if (!split && cnt <= (uint32_t)kListCap) {
     // ---- phase B ----
     // kPairBatch list entries per iteration (entries past cnt load the
@@ -475,14 +482,12 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
       }
     }
     force = make_v3(force.x + cf.x, force.y + cf.y, force.z + cf.z);
-  } else if (!split) {
-    // The list overflowed (a densely packed bed: up to ~60 contacts; cells
-    // of 50 and more where spheres pile up): walk the nine row ranges again
-    // as one flattened sequence, filling the list and emptying it through
-    // the exact pair force in turns, the lanes of the wave together -- the
-    // list path's terms in the list path's order.  Only what passes the
-    // filter reaches the pair force (a walk that sent every candidate
-    // through it took TIMES_KNOT).
+  } else if (!kPoly && !split) {
+    // The list overflowed (a densely packed bed: up to ~60 contacts): walk
+    // the nine row ranges again as one flattened sequence, filling the list
+    // and emptying it through the exact pair force in turns, the lanes of
+    // the wave together -- the list path's terms in the list path's order.
+    // Only what passes the filter reaches the pair force.
     uint32_t B[9], Q[9];  // slots before row r; slot t of row r is sphere t + Q[r]
     uint32_t total = 0;
 #pragma unroll
@@ -537,7 +542,7 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
               curHash = hu;
             }
             v3f f = collide_spheres_fast(pos, xyz(qp[u]), vel, xyz(qv[u]), rA,
-                                         kPoly ? qp[u].w : rA, P.spring, P.damping, P.shear,
+                                         rA, P.spring, P.damping, P.shear,
                                          P.attraction);
             cf = make_v3(cf.x + f.x, cf.y + f.y, cf.z + f.z);
           }
@@ -545,7 +550,7 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
       }
     }
     force = make_v3(force.x + cf.x, force.y + cf.y, force.z + cf.z);
-  } else {
+  } else if (!kPoly) {
     for (int dz = -1; dz <= 1; ++dz)
       for (int dy = -1; dy <= 1; ++dy)
         for (int dx = -1; dx <= 1; ++dx) {
@@ -558,7 +563,7 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
             if (jj != k) {
               const float4 pj = sortedPos[jj];
               v3f f = collide_spheres(pos, xyz(pj), vel, xyz(sortedVel[jj]), rA,
-                                      kPoly ? pj.w : rA, P.spring, P.damping, P.shear,
+                                      rA, P.spring, P.damping, P.shear,
                                       P.attraction);
               cf = make_v3(cf.x + f.x, cf.y + f.y, cf.z + f.z);
             }

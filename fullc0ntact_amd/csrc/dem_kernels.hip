@@ -317,6 +317,45 @@ __global__ __launch_bounds__(kBlock) void k_collide_v2(
 // against 94.3 us.
 constexpr int kCollideWavesPerSimd = 5;
 
+// What follows the 27 cells' sum for one sphere: the cursor sphere, the new
+// velocity at the sphere's id, and with kFuse the next update's integrate and
+// hash (its key returned).
+template <bool kFuse>
+__device__ __forceinline__ uint32_t collide_finish(
+    const fc_sim_params& P, const BoundaryArg& B, const float4& p4, v3f pos0, v3f vel0, float rA,
+    v3f force, uint32_t k, uint32_t orig, float4* __restrict__ newVel, float4* __restrict__ pos,
+    float dt, v3f invCell, uint32_t oldKey, uint32_t* __restrict__ keysOut,
+    uint32_t* __restrict__ slotOf, uint32_t* __restrict__ idOfSlot, bool slotKeys,
+    float* __restrict__ forceOut) {
+  if (kFuse || forceOut == nullptr) {
+    force = add_collider(P, pos0, vel0, rA, force);
+  } else {  // evalForces: no cursor sphere, the force stored as float3
+    forceOut[3 * (size_t)orig] = force.x;
+    forceOut[3 * (size_t)orig + 1] = force.y;
+    forceOut[3 * (size_t)orig + 2] = force.z;
+  }
+  const v3f nv = make_v3(vel0.x + force.x, vel0.y + force.y, vel0.z + force.z);
+  if (!kFuse) {
+    newVel[orig] = make_float4(nv.x, nv.y, nv.z, 0.0f);
+    if (pos) pos[orig] = p4;
+    return 0u;
+  }
+  v3f p = pos0, v = nv;
+  integrate_with(P, B, p4.w, dt, p, v);
+  pos[k] = make_float4(p.x, p.y, p.z, p4.w);
+  newVel[k] = make_float4(v.x, v.y, v.z, 0.0f);
+  const uint32_t key = hash_of_q(P, cell_quotients(P, invCell, p));
+  if (slotKeys) {
+    // at the slot, with whether the sphere changed cell, for the row resort
+    keysOut[k] = key != oldKey ? (key | kMovedBit) : key;
+  } else {
+    keysOut[orig] = key;
+    slotOf[orig] = k;
+  }
+  idOfSlot[k] = orig;
+  return key;
+}
+
 // Whether the wrapped cells may be cut (collide_one_rows): known by the
 // launch, or unless the arrays' check wrote `epoch` (GatheredState).
 struct WrapCut {
@@ -333,7 +372,7 @@ __global__ __launch_bounds__(kBlock, kCollideWavesPerSimd) void k_collide_v3(
     float dt, uint32_t* __restrict__ keysOut, int passes, uint32_t* gHist, uint32_t* counters,
     uint32_t* devFlags, uint32_t* __restrict__ slotOf, uint32_t* __restrict__ idOfSlot,
     v3f invCell, const uint2* __restrict__ sortedQ, RowFilter filter, WrapCut wraps,
-    float* __restrict__ forceOut, int slotKeys, RowHists rows) {
+    float* __restrict__ forceOut, int slotKeys, RowHists rows, uint32_t* __restrict__ piles) {
   __shared__ uint32_t s_list[kListCap + 1][kBlock];
   const bool cutWraps =
       wraps.cut != 0u && (wraps.outside == nullptr || *wraps.outside != wraps.epoch);
@@ -348,6 +387,7 @@ __global__ __launch_bounds__(kBlock, kCollideWavesPerSimd) void k_collide_v3(
     histogram_producer_prologue(gHist, passes, counters);
   }
   uint32_t key = 0, oldKey = 0;
+  bool left = false;
   if (valid) {
     const float4 p4 = sortedPos[k];
     const float rA = kPoly ? p4.w : P.particleRadius;
@@ -358,44 +398,149 @@ __global__ __launch_bounds__(kBlock, kCollideWavesPerSimd) void k_collide_v3(
     v3f force =
         kRows ? collide_one_rows<kPoly, kBlock>(P, invCell, contactD2, k, pos0, vel0, rA,
                                                 sortedPos, sortedVel, sortedQ, filter, cutWraps,
-                                                cellStart, cellEnd, n, s_list)
+                                                cellStart, cellEnd, n, s_list, left)
               : collide_one_v3<kPoly, kBlock>(P, contactD2, k, pos0, vel0, rA, sortedPos,
                                               sortedVel, cellStart, cellEnd, n, s_list);
-    const uint32_t orig = index[k];
-    if (kFuse || forceOut == nullptr) {
-      force = add_collider(P, pos0, vel0, rA, force);
-    } else {  // evalForces: no cursor sphere, the force stored as float3
-      forceOut[3 * (size_t)orig] = force.x;
-      forceOut[3 * (size_t)orig + 1] = force.y;
-      forceOut[3 * (size_t)orig + 2] = force.z;
-    }
-    const v3f nv = make_v3(vel0.x + force.x, vel0.y + force.y, vel0.z + force.z);
-    if (!kFuse) {
-      newVel[orig] = make_float4(nv.x, nv.y, nv.z, 0.0f);
-      if (pos) pos[orig] = p4;
+    if (kPoly && kRows && left) {
+      piles[2 + atomicAdd(&piles[0], 1u)] = k;
     } else {
-      v3f p = xyz(p4), v = nv;
-      integrate_with(P, B, p4.w, dt, p, v);
-      pos[k] = make_float4(p.x, p.y, p.z, p4.w);
-      newVel[k] = make_float4(v.x, v.y, v.z, 0.0f);
-      key = hash_of_q(P, cell_quotients(P, invCell, p));
-      if (slotKeys) {
-        // at the slot, with whether the sphere changed cell, for the row resort
-        keysOut[k] = key != oldKey ? (key | kMovedBit) : key;
-      } else {
-        keysOut[orig] = key;
-        slotOf[orig] = k;
-      }
-      idOfSlot[k] = orig;
+      key = collide_finish<kFuse>(P, B, p4, pos0, vel0, rA, force, k, index[k], newVel, pos, dt,
+                                  invCell, oldKey, keysOut, slotOf, idOfSlot, slotKeys != 0,
+                                  forceOut);
     }
   }
   if (digitHist) {
     __syncthreads();
-    histogram_add_digit(s_hist, key & (RS_RADIX - 1), valid);
+    histogram_add_digit(s_hist, key & (RS_RADIX - 1), valid && !left);
     __syncthreads();
     histogram_flush(s_hist, gHist, 0);
   } else if (kFuse) {
-    row_histograms(rows, k, key, oldKey, valid);
+    row_histograms(rows, k, key, oldKey, valid && !left);
+  }
+}
+
+// The spheres that a polydisperse k_collide_v3 left (their lists overflowed,
+// or a row of theirs has two runs), one wave each: lanes 0-26 take a
+// neighbour cell each (those out of reach cut, as collide_one_rows does),
+// then the wave takes the cells' spheres 64 at a time through the exact pair
+// force, and each cell's lane adds its own in index order, so the 27
+// partials and their order are the reference's.  A sphere with 300
+// candidates is a chain of about five rounds here and of 90 in a lane of its
+// own, which was the launch's tail: 120,011 log-normal spheres settled on a
+// knot, fused collide 189 us with every candidate through the pair force in
+// the lane, 133 us with lists refilled in the lane, 66 us with this launch.
+// Equal radii keep the lane's own path: their lists overflow only while a
+// bed is compressed, and an empty launch costs about 2 us a step.
+constexpr unsigned kPileBlocks = 512;
+
+template <bool kFuse>
+__global__ __launch_bounds__(kBlock) void k_collide_piles(
+    fc_sim_params P, BoundaryArg B, float contactD2, float4* __restrict__ newVel,
+    const float4* __restrict__ sortedPos, const float4* __restrict__ sortedVel,
+    const uint32_t* __restrict__ index, const uint32_t* __restrict__ cellStart,
+    const uint32_t* __restrict__ cellEnd, uint32_t n, float4* __restrict__ pos, float dt,
+    uint32_t* __restrict__ keysOut, uint32_t* gHist, uint32_t* __restrict__ slotOf,
+    uint32_t* __restrict__ idOfSlot, v3f invCell, int slotKeys, RowHists rows,
+    uint32_t* __restrict__ piles) {
+  __shared__ float s_f[kBlock / 64][3][64];
+  __shared__ uint32_t s_first[kBlock / 64][32], s_end[kBlock / 64][32];
+  const int lane = (int)(threadIdx.x & 63u), w = (int)(threadIdx.x >> 6);
+  const uint32_t count = min(piles[0], n);
+  for (uint32_t i = blockIdx.x * (kBlock / 64) + (uint32_t)w; i < count;
+       i += gridDim.x * (kBlock / 64)) {
+    const uint32_t k = piles[2 + i];
+    const float4 p4 = sortedPos[k], v4 = sortedVel[k];
+    const v3f pos0 = xyz(p4), vel0 = xyz(v4);
+    const float rA = p4.w, reach = rA + P.particleRadius;
+    const v3f q = cell_quotients(P, invCell, pos0);
+    uint32_t first = 0, len = 0;
+    if (lane < 27) {
+      const int d[3] = {lane % 3 - 1, lane / 3 % 3 - 1, lane / 9 - 1};
+      const float qa[3] = {q.x, q.y, q.z};
+      const float cs[3] = {P.cellSize.x, P.cellSize.y, P.cellSize.z};
+      float g = 0.0f;  // lower bound on the squared distance to the cell
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const float f = qa[a] - floorf(qa[a]), u = fmaf(fabsf(qa[a]), 0x1p-20f, 0x1p-20f);
+        const float e = fmaxf((d[a] < 0 ? f : 1.0f - f) - u, 0.0f) * cs[a];
+        g += d[a] == 0 ? 0.0f : e * e;
+      }
+      const float d2 = fminf(contactD2, reach * reach * (1.0f + 0x1p-20f));
+      const float thr = fmaxf(d2 * (1.0f + 0x1p-18f), d2 + 0x1p-140f) * (1.0f + 0x1p-16f);
+      const uint32_t h = grid_hash(cell_of_quotient(q.x) + d[0], cell_of_quotient(q.y) + d[1],
+                                   cell_of_quotient(q.z) + d[2], P.gridSize);
+      const uint32_t s = cellStart[h], e = min(cellEnd[h], n);
+      if (s != CELL_EMPTY && s < e && !(g >= thr)) {
+        first = s;
+        len = e - s;
+      }
+    }
+    uint32_t end = len;  // inclusive sum over the cells
+#pragma unroll
+    for (int off = 1; off < 32; off <<= 1) {
+      const uint32_t t = __shfl_up(end, off);
+      if (lane >= off) end += t;
+    }
+    const uint32_t begin = end - len, total = __shfl(end, 26);
+    if (lane < 27) {
+      s_first[w][lane] = first - begin;  // modulo 2^32: candidate t is sphere t + this
+      s_end[w][lane] = end;
+    }
+    __builtin_amdgcn_wave_barrier();
+    v3f cf = make_v3(0.0f, 0.0f, 0.0f);
+    for (uint32_t t0 = 0; t0 < total; t0 += 64u) {
+      const uint32_t t = t0 + (uint32_t)lane;
+      v3f f = make_v3(0.0f, 0.0f, 0.0f);
+      if (t < total) {
+        int c = 0;  // the first cell that ends past t
+#pragma unroll
+        for (int step = 16; step > 0; step >>= 1)
+          if (c + step <= 26 && s_end[w][c + step - 1] <= t) c += step;
+        const uint32_t j = t + s_first[w][c];
+        if (j != k) {
+          const float4 pj = sortedPos[j];
+          f = collide_spheres_fast(pos0, xyz(pj), vel0, xyz(sortedVel[j]), rA, pj.w, P.spring,
+                                   P.damping, P.shear, P.attraction);
+        }
+      }
+      s_f[w][0][lane] = f.x;
+      s_f[w][1][lane] = f.y;
+      s_f[w][2][lane] = f.z;
+      __builtin_amdgcn_wave_barrier();
+      if (lane < 27) {
+        const uint32_t a = begin > t0 ? begin : t0, b = end < t0 + 64u ? end : t0 + 64u;
+        for (uint32_t u = a; u < b; ++u)
+          cf = make_v3(cf.x + s_f[w][0][u - t0], cf.y + s_f[w][1][u - t0],
+                       cf.z + s_f[w][2][u - t0]);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    v3f force = make_v3(0.0f, 0.0f, 0.0f);
+    for (int c = 0; c < 27; ++c)
+      force = make_v3(force.x + __shfl(cf.x, c), force.y + __shfl(cf.y, c),
+                      force.z + __shfl(cf.z, c));
+    if (lane == 0) {
+      const uint32_t oldKey = __float_as_uint(v4.w);
+      const uint32_t key = collide_finish<kFuse>(
+          P, B, p4, pos0, vel0, rA, force, k, index[k], newVel, pos, dt, invCell, oldKey, keysOut,
+          slotOf, idOfSlot, slotKeys != 0, nullptr);
+      if (kFuse && rows.rowHist != nullptr) {
+        const uint32_t r = key >> rows.shift, at = r * kRowCopies + row_copy(k);
+        atomicAdd(&rows.rowHist[at], 1u);
+        if (r != (oldKey >> rows.shift)) atomicAdd(&rows.chgHist[at], 1u);
+      } else if (kFuse) {
+        atomicAdd(&hist_buffer(gHist, 0)[(blockIdx.x % RS_HIST_COPIES) * RS_RADIX +
+                                         (key & (RS_RADIX - 1))],
+                  1u);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  // every block has read the count before it reports here
+  __syncthreads();
+  if (threadIdx.x == 0 && atomicAdd(&piles[1], 1u) == gridDim.x - 1u) {
+    piles[0] = 0u;
+    piles[1] = 0u;
   }
 }
 
@@ -459,29 +604,8 @@ __global__ __launch_bounds__(kBlock) void k_collide_split(
   const bool owner = valid && r == 0;
   if (owner) {
     if (kPoly && !(rA <= P.particleRadius)) atomicOr(devFlags, DEVERR_RADIUS);
-    const v3f pos0 = xyz(p4);
-    const uint32_t orig = index[k];
-    if (kFuse || forceOut == nullptr) {
-      force = add_collider(P, pos0, vel0, rA, force);
-    } else {  // evalForces: no cursor sphere, the force stored as float3
-      forceOut[3 * (size_t)orig] = force.x;
-      forceOut[3 * (size_t)orig + 1] = force.y;
-      forceOut[3 * (size_t)orig + 2] = force.z;
-    }
-    const v3f nv = make_v3(vel0.x + force.x, vel0.y + force.y, vel0.z + force.z);
-    if (!kFuse) {
-      newVel[orig] = make_float4(nv.x, nv.y, nv.z, 0.0f);
-      if (pos) pos[orig] = p4;
-    } else {
-      v3f p = pos0, v = nv;
-      integrate_with(P, B, p4.w, dt, p, v);
-      pos[k] = make_float4(p.x, p.y, p.z, p4.w);
-      newVel[k] = make_float4(v.x, v.y, v.z, 0.0f);
-      key = hash_of_q(P, cell_quotients(P, invCell, p));
-      keysOut[orig] = key;
-      slotOf[orig] = k;
-      idOfSlot[k] = orig;
-    }
+    key = collide_finish<kFuse>(P, B, p4, xyz(p4), vel0, rA, force, k, index[k], newVel, pos, dt,
+                                invCell, 0u, keysOut, slotOf, idOfSlot, false, forceOut);
   }
   if (kFuse) {
     __syncthreads();
@@ -686,7 +810,7 @@ static void launch_v3(hipStream_t s, const GatheredState* gs, dim3 g, dim3 b,
                        newVel, sortedPos, sortedVel, index, cellStart, cellEnd, n, pos, dt,
                        keysOut, passes, gHist, counters, devFlags, slotOf, idOfSlot, inv_cell(P),
                        forceOut);
-  } else if (gs != nullptr && rows_walk_ok(P))
+  } else if (gs != nullptr && rows_walk_ok(P)) {
     hipLaunchKernelGGL((k_collide_v3<kFuse, kPoly, true>), g, b, 0, s, P, B, d2, newVel,
                        sortedPos, sortedVel, index, cellStart, cellEnd, n, kCollideXcdGroup, pos,
                        dt, keysOut, passes, gHist, counters, devFlags, slotOf, idOfSlot,
@@ -694,12 +818,19 @@ static void launch_v3(hipStream_t s, const GatheredState* gs, dim3 g, dim3 b,
                        RowFilter{quant_threshold(P.particleRadius + P.particleRadius,
                                                  gs->frame.scale),
                                  gs->frame.scale},
-                       wrap_cut(P, *gs), forceOut, slotKeys ? 1 : 0, rows ? *rows : RowHists{});
-  else
+                       wrap_cut(P, *gs), forceOut, slotKeys ? 1 : 0, rows ? *rows : RowHists{},
+                       gs->piles);
+    if (kPoly)
+      hipLaunchKernelGGL(k_collide_piles<kFuse>, dim3(kPileBlocks), b, 0, s, P, B, d2, newVel,
+                         sortedPos, sortedVel, index, cellStart, cellEnd, n, pos, dt, keysOut,
+                         gHist, slotOf, idOfSlot, inv_cell(P), slotKeys ? 1 : 0,
+                         rows ? *rows : RowHists{}, gs->piles);
+  } else
     hipLaunchKernelGGL((k_collide_v3<kFuse, kPoly, false>), g, b, 0, s, P, B, d2, newVel,
                        sortedPos, sortedVel, index, cellStart, cellEnd, n, kCollideXcdGroup, pos,
                        dt, keysOut, passes, gHist, counters, devFlags, slotOf, idOfSlot,
-                       inv_cell(P), nullptr, RowFilter{}, WrapCut{}, forceOut, 0, RowHists{});
+                       inv_cell(P), nullptr, RowFilter{}, WrapCut{}, forceOut, 0, RowHists{},
+                       nullptr);
 }
 
 hipError_t launch_collide(hipStream_t s, const fc_sim_params& P, bool poly, uint32_t* devFlags,

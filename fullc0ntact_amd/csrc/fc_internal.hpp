@@ -255,12 +255,16 @@ hipError_t launch_reorder(hipStream_t s, uint32_t* cellStart, uint32_t* cellEnd,
 // walled: integrate's box walls, with the parameters' radius, bound every
 // position; else outside (if given) holds `epoch` when launch_rows_state
 // found a sphere whose cell index lies outside the grid.
+// piles: [0] the number of spheres that a polydisperse collide left to
+// k_collide_piles, [1] its finished blocks (both zero between launches),
+// then their sorted indices (n words).
 struct GatheredState {
   const uint2* sortedQ = nullptr;
   QuantFrame frame;
   bool walled = false;
   const uint32_t* outside = nullptr;
   uint32_t epoch = 0;
+  uint32_t* piles = nullptr;
 };
 hipError_t launch_collide(hipStream_t s, const fc_sim_params& P, bool poly, uint32_t* devFlags,
                           float4* newVel, const float4* sortedPos, const float4* sortedVel,
@@ -444,6 +448,7 @@ struct fc_system {
   int boundaryBx = 0, boundaryBy = 0;
   // Radii from pos.w (set by fc_system_set_polydisperse).
   int polydisperse = 0;
+  uint32_t* piles = nullptr;  // GatheredState::piles, once polydisperse
   // Row resort tables of multi-step runs (allocated by the first run that
   // uses them).
   fc::RowTables rowTables;

@@ -55,6 +55,8 @@ void free_system_buffers(fc_system* sys) {
   hipFree(sys->idOfSlot);
   hipFree(sys->cellStart);
   hipFree(sys->cellEnd);
+  hipFree(sys->piles);
+  sys->piles = nullptr;
   sys->pos = sys->vel = sys->sortedPos = sys->sortedVel = nullptr;
   sys->sortedQ = nullptr;
   sys->hash = sys->index = sys->keys = sys->slotOf = sys->idOfSlot = nullptr;
@@ -137,7 +139,11 @@ fc_status enqueue_update(fc_system* sys, float dt, StageTimer* timer) {
     if (e != hipSuccess) return hip_error(e, "cell bounds");
   }
   if (timer) timer->begin(st, "collide");
-  const GatheredState gs{sys->sortedQ, ga.frame, sys->walled()};
+  GatheredState gs;
+  gs.sortedQ = sys->sortedQ;
+  gs.frame = ga.frame;
+  gs.walled = sys->walled();
+  gs.piles = sys->piles;
   e = launch_collide(st, P, sys->polydisperse != 0, ctx->devFlags, sys->vel, sys->sortedPos,
                      sys->sortedVel, sys->index, sys->cellStart, sys->cellEnd, n, nullptr, &gs);
   if (timer) timer->end(st);
@@ -287,7 +293,11 @@ fc_status enqueue_run_body(fc_system* sys, float dt, bool clearInSort, bool last
     if (e != hipSuccess) return hip_error(e, "cell bounds");
   }
   if (timer) timer->begin(st, last ? "collide" : "collide_integrate");
-  const GatheredState gs{sys->sortedQ, ga.frame, sys->walled()};
+  GatheredState gs;
+  gs.sortedQ = sys->sortedQ;
+  gs.frame = ga.frame;
+  gs.walled = sys->walled();
+  gs.piles = sys->piles;
   if (last)
     e = launch_collide(st, P, sys->polydisperse != 0, ctx->devFlags, sys->vel, sys->sortedPos,
                        sys->sortedVel, sys->index, sys->cellStart, sys->cellEnd, n,
@@ -423,6 +433,11 @@ fc_status fc_system_set_boundary(fc_system* sys, fc_boundary mode, const fc_dist
 fc_status fc_system_set_polydisperse(fc_system* sys, int enable) {
   if (!sys) return set_error(FC_ERROR_INVALID_VALUE, "sys is NULL");
   FC_HIP_TRY(hipStreamSynchronize(sys->ctx->stream));
+  if (enable && !sys->piles) {
+    const size_t words = (size_t)sys->n + 2;
+    FC_HIP_TRY(hipMalloc(&sys->piles, words * sizeof(uint32_t)));
+    FC_HIP_TRY(hipMemset(sys->piles, 0, 2 * sizeof(uint32_t)));
+  }
   sys->polydisperse = enable ? 1 : 0;
   drop_graph(sys);  // the captured step carries the radius mode in its kernels
   return FC_SUCCESS;

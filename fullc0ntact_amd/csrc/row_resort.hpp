@@ -49,7 +49,7 @@ __device__ __forceinline__ uint32_t lowest_lane(uint64_t m) {
 __device__ __forceinline__ void row_histograms(const RowHists& rh, uint32_t slot, uint32_t key,
                                                uint32_t oldKey, bool valid) {
   const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t r = key >> rh.shift;
+  const uint32_t r = valid ? key >> rh.shift : 0xffffffffu;  // no valid lane's row
   const uint32_t at = r * kRowCopies + row_copy(slot);
   const uint32_t rPrev = __shfl_up(r, 1);
   const bool head = valid && (lane == 0u || r != rPrev);
