@@ -88,9 +88,7 @@ __device__ __forceinline__ bf16x8 pack8(float a0, float a1, float a2, float a3, 
 }
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int kTile = 64;  // samples per training tile
-constexpr int kTB = 256;   // training / inference block
-constexpr int kWPad = 10500;
+constexpr int kTB = 256;  // inference block
 
 __device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + __expf(-z)); }
 // SiLU of the inference path: the hardware exp2 and reciprocal (about 1 ulp
@@ -99,10 +97,6 @@ __device__ __forceinline__ float silu_fast(float z) {
   return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.4426950408889634f));
 }
 __device__ __forceinline__ float silu(float z) { return z * sigmoidf_(z); }
-__device__ __forceinline__ float silu_grad(float z) {
-  const float s = sigmoidf_(z);
-  return s * (1.0f + z * (1.0f - s));
-}
 
 // sin(2 pi t) and cos(2 pi t) with the hardware's revolution-based
 // instructions after reducing t to [-1/2, 1/2].
@@ -174,221 +168,284 @@ __global__ __launch_bounds__(kTB) void k_sdf_eval_f32(const float* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// Training: forward + backward of 64-sample tiles of one body's minibatch.
-// Block (blk, body) handles tiles blk*tilesPerBlock .. +tilesPerBlock-1 and
-// writes the sum of their weight gradients (dL/dp of L = 1/M sum (y - t)^2,
-// M = minibatch size) and of their squared errors.  Thread t owns the 4x4
-// output tile (t / 16, t % 16) of every 64x64 product and the matching
-// gradient entries, accumulated in registers over the block's tiles.
+// Training: forward + backward of 128-sample tiles of one body's minibatch, on
+// the 16x16x4 FP32 MFMA (products and sums in binary32).  Block (blk, body)
+// handles tiles blk*tilesPerBlock .. +tilesPerBlock-1 and writes the sum of
+// their weight gradients (dL/dp of L = 1/M sum (y - t)^2, M = minibatch size)
+// and of their squared errors.
+//
+// A wave takes 16 samples, the columns of its products; a lane (g = lane / 16,
+// c = lane % 16) holds features 16 ob + 4 g + r (r = 0..3) of sample c after
+// a layer.  With step (ob, r) of the next contraction over those features,
+// that register is the B operand as it stands, forward (W, rows = outputs) and
+// backward (W transposed, rows = inputs), so the activations need no
+// transpose between layers.  The weight gradients contract over the samples
+// of all waves: activations and output gradients go through LDS once
+// (train_put / train_get, a swizzle without bank conflicts either way), and
+// each wave owns two 16x16 blocks of a 64x64 gradient, so its accumulators
+// are few and live in registers over the block's tiles.
+//
+// Bound by the FP32 matrix rate: 448 MFMAs of 32 cycles a wave and tile.  One
+// gradient of 8 bodies x 16384 samples, copied to the host: 605 us with 4x4
+// register tiles on the vector units (one wave per SIMD, 16-way bank
+// conflicts in the transposed products), 163 us with this.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kTB) void k_sdf_grad_tiles(
+constexpr int kTrainTile = 128;             // samples per tile: 16 per wave
+constexpr int kTrainThreads = 512;          // 8 waves, two per SIMD
+constexpr int kTrainWaves = kTrainThreads / 64;
+// A weight block's 64 words, one per lane of its operand; the odd stride puts
+// the transposed read of the backward pass on 64 distinct banks as well.
+constexpr int kFragStride = 65;
+constexpr int kRowsW1 = 0, kRowsW2 = 32, kRowsW3 = 96, kRowsW = 160;
+
+// Registers d[4 ob + r] (features 16 ob + 4 g + r of sample c) to LDS.
+template <int kBlocks>
+__device__ __forceinline__ void train_put(float* buf, const float* d, int g, int c) {
+#pragma unroll
+  for (int ob = 0; ob < kBlocks; ++ob)
+    *reinterpret_cast<float4*>(buf + (4 * ob + g) * 64 + ((c ^ (g << 2)) << 2)) =
+        make_float4(d[4 * ob], d[4 * ob + 1], d[4 * ob + 2], d[4 * ob + 3]);
+}
+
+// Where feature 16 ob + i of sample 4 step + g of a wave's tile lies (without
+// the 256 ob): an operand of the contraction over samples.
+__device__ __forceinline__ int train_get(int step, int g, int i) {
+  return (i >> 2) * 64 + ((step ^ (i >> 2)) << 4) + (g << 2) + (i & 3);
+}
+
+__global__ __launch_bounds__(kTrainThreads) void k_sdf_grad_tiles(
     const float* __restrict__ params, const float* __restrict__ freq,
     const float* __restrict__ frame, const float* __restrict__ pts,
     const float* __restrict__ labels, uint32_t samplesPerBody, uint32_t batchStart,
     uint32_t batchSize, uint32_t tilesPerBlock, float invM, float* __restrict__ partial,
     float* __restrict__ lossPartial) {
-  __shared__ float W[kWPad];
-  __shared__ float X0[kTile * kSdfIn];
-  __shared__ float Z1[kTile * kSdfHidden], A1[kTile * kSdfHidden];
-  __shared__ float Z2[kTile * kSdfHidden], A2[kTile * kSdfHidden];
-  __shared__ float Z3[kTile * kSdfHidden], A3[kTile * kSdfHidden];
-  __shared__ float Y[kTile];
-  __shared__ float FR[kSdfFreqs * 3 + 4];
-  __shared__ float red[kTB / 64];
+  __shared__ float s_w[kRowsW * kFragStride];
+  __shared__ float s_bias[4 * kSdfHidden];  // b1, b2, b3, w4
+  __shared__ float s_fr[kSdfFreqs * 3 + 4];
+  __shared__ float s_x0[kTrainWaves][16 * kSdfIn];
+  __shared__ float s_a1[kTrainWaves][16 * kSdfHidden];
+  __shared__ float s_a2[kTrainWaves][16 * kSdfHidden];  // then dZ2
+  __shared__ float s_dz[kTrainWaves][16 * kSdfHidden];  // dZ3, then dZ1
 
   const uint32_t body = blockIdx.y, blk = blockIdx.x, nblk = gridDim.x;
-  const int t = threadIdx.x, rb = t >> 4, cb = t & 15;
+  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6, g = lane >> 4, c = lane & 15;
   const float* P = params + (size_t)body * kSdfStride;
-  for (int i = t; i < kSdfParams; i += kTB) W[i] = P[i];
-  if (t < kSdfFreqs * 3) FR[t] = freq[(size_t)body * kSdfFreqs * 3 + t];
-  if (t < 4) FR[kSdfFreqs * 3 + t] = frame[(size_t)body * 4 + t];
+  // row ob2 * steps + (4 ob + r) of a layer: W[16 ob + 4 g + r][16 ob2 + c]
+  for (int e = t; e < kRowsW * 64; e += kTrainThreads) {
+    const int row = e >> 6, l = e & 63;
+    const int off = row < kRowsW2 ? kSdfOffW1 : (row < kRowsW3 ? kSdfOffW2 : kSdfOffW3);
+    const int rr = row - (row < kRowsW2 ? kRowsW1 : (row < kRowsW3 ? kRowsW2 : kRowsW3));
+    const int steps = row < kRowsW2 ? 8 : 16;
+    const int ob2 = rr / steps, st = rr % steps;
+    const int in = 16 * (st >> 2) + 4 * (l >> 4) + (st & 3), out = 16 * ob2 + (l & 15);
+    s_w[row * kFragStride + l] = P[off + in * kSdfHidden + out];
+  }
+  for (int e = t; e < 4 * kSdfHidden; e += kTrainThreads) {
+    const int which = e / kSdfHidden, o = e % kSdfHidden;
+    const int off = which == 0 ? kSdfOffB1
+                               : (which == 1 ? kSdfOffB2 : (which == 2 ? kSdfOffB3 : kSdfOffW4));
+    s_bias[e] = P[off + o];
+  }
+  if (t < kSdfFreqs * 3) s_fr[t] = freq[(size_t)body * kSdfFreqs * 3 + t];
+  if (t < 4) s_fr[kSdfFreqs * 3 + t] = frame[(size_t)body * 4 + t];
+  const float b4 = P[kSdfOffB4];
 
-  float gW1[2][4] = {}, gW2[4][4] = {}, gW3[4][4] = {};
-  float gW4 = 0.0f, gb1 = 0.0f, gb2 = 0.0f, gb3 = 0.0f, gb4 = 0.0f, lossAcc = 0.0f;
+  // this wave's gradient blocks: inputs 16 (w / 2), outputs 32 (w % 2) + 0, 16
+  // (layers 3 and 2); inputs 16 (w / 4), outputs 16 (w % 4) (layer 1)
+  floatx4 gW3[2] = {}, gW2[2] = {}, gW1 = {};
+  float gb3[2] = {}, gb2[2] = {}, gb1 = 0.0f;
+  float gW4[16] = {}, gb4 = 0.0f, lossAcc = 0.0f;
+  const int ib = w >> 1, jb = 2 * (w & 1), ib1 = w >> 2, jb1 = w & 3;
+  int at[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) at[s] = train_get(s, g, c);
+  const int back = (c & 3) * kFragStride + (c >> 2) * 16 + 4 * g;
   const uint32_t batchEnd = batchStart + batchSize;
 
   for (uint32_t u = 0; u < tilesPerBlock; ++u) {
-    const uint32_t tile = blk * tilesPerBlock + u;
-    const uint32_t s0 = batchStart + tile * kTile;
-    __syncthreads();
-    // features
-    for (int idx = t; idx < kTile * kSdfFreqs; idx += kTB) {
-      const int s = idx / kSdfFreqs, k = idx % kSdfFreqs;
-      const uint32_t gs = s0 + s;
-      float sv = 0.0f, cv = 0.0f;
-      if (gs < batchEnd && gs < samplesPerBody) {
-        const float* q = pts + ((size_t)body * samplesPerBody + gs) * 3;
-        float x, y, z;
-        sdf_norm(FR + kSdfFreqs * 3, q[0], q[1], q[2], x, y, z);
-        sincos_rev(FR[3 * k] * x + FR[3 * k + 1] * y + FR[3 * k + 2] * z, sv, cv);
+    const uint32_t s0 = batchStart + (blk * tilesPerBlock + u) * (uint32_t)kTrainTile;
+    if (s0 >= batchEnd) break;  // (the same for the block)
+    __syncthreads();            // the weights; the last tile's readers of X0 and dZ1
+    const uint32_t gs = s0 + 16u * (uint32_t)w + (uint32_t)c;
+    const bool live = gs < batchEnd && gs < samplesPerBody;
+    // ---- features: sines 4 g + j, cosines 16 + 4 g + j
+    float x0[8] = {};
+    if (live) {
+      const float* q = pts + ((size_t)body * samplesPerBody + gs) * 3;
+      float x, y, z;
+      sdf_norm(s_fr + kSdfFreqs * 3, q[0], q[1], q[2], x, y, z);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int k = 4 * g + j;
+        sincos_rev(s_fr[3 * k] * x + s_fr[3 * k + 1] * y + s_fr[3 * k + 2] * z, x0[j], x0[4 + j]);
       }
-      X0[s * kSdfIn + k] = sv;
-      X0[s * kSdfIn + kSdfFreqs + k] = cv;
     }
-    __syncthreads();
-    // ---- forward: Z = A W + b, A' = SiLU(Z), 4x4 tile per thread
-    {
-      float acc[4][4];
-      for (int a = 0; a < 4; ++a)
-        for (int c = 0; c < 4; ++c) acc[a][c] = W[kSdfOffB1 + 4 * cb + c];
-      for (int i = 0; i < kSdfIn; ++i) {
-        float w[4], x[4];
-        for (int c = 0; c < 4; ++c) w[c] = W[kSdfOffW1 + i * kSdfHidden + 4 * cb + c];
-        for (int a = 0; a < 4; ++a) x[a] = X0[(4 * rb + a) * kSdfIn + i];
-        for (int a = 0; a < 4; ++a)
-          for (int c = 0; c < 4; ++c) acc[a][c] += x[a] * w[c];
-      }
-      for (int a = 0; a < 4; ++a)
-        for (int c = 0; c < 4; ++c) {
-          const int e = (4 * rb + a) * kSdfHidden + 4 * cb + c;
-          Z1[e] = acc[a][c];
-          A1[e] = silu(acc[a][c]);
-        }
+    train_put<2>(s_x0[w], x0, g, c);
+    // ---- forward: Z = A W + b, A' = SiLU(Z), and SiLU'(Z) for the way back
+    float act[16], d1[16], d2[16], d3[16];
+    floatx4 z[4];
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) z[ob][r] = s_bias[16 * ob + 4 * g + r];
+#pragma unroll
+    for (int st = 0; st < 8; ++st)
+#pragma unroll
+      for (int ob = 0; ob < 4; ++ob)
+        z[ob] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+            s_w[(kRowsW1 + ob * 8 + st) * kFragStride + lane], x0[st], z[ob], 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float v = z[e >> 2][e & 3], s = sigmoidf_(v);
+      act[e] = v * s;
+      d1[e] = s * (1.0f + v * (1.0f - s));
     }
-    __syncthreads();
-    const float* Ain[2] = {A1, A2};
-    float* Zout[2] = {Z2, Z3};
-    float* Aout[2] = {A2, A3};
+    train_put<4>(s_a1[w], act, g, c);
 #pragma unroll
     for (int L = 0; L < 2; ++L) {
-      const int offW = L == 0 ? kSdfOffW2 : kSdfOffW3, offB = L == 0 ? kSdfOffB2 : kSdfOffB3;
-      float acc[4][4];
-      for (int a = 0; a < 4; ++a)
-        for (int c = 0; c < 4; ++c) acc[a][c] = W[offB + 4 * cb + c];
-      for (int i = 0; i < kSdfHidden; ++i) {
-        float w[4], x[4];
-        for (int c = 0; c < 4; ++c) w[c] = W[offW + i * kSdfHidden + 4 * cb + c];
-        for (int a = 0; a < 4; ++a) x[a] = Ain[L][(4 * rb + a) * kSdfHidden + i];
-        for (int a = 0; a < 4; ++a)
-          for (int c = 0; c < 4; ++c) acc[a][c] += x[a] * w[c];
+      const int rows = L == 0 ? kRowsW2 : kRowsW3;
+#pragma unroll
+      for (int ob = 0; ob < 4; ++ob)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z[ob][r] = s_bias[(L + 1) * kSdfHidden + 16 * ob + 4 * g + r];
+#pragma unroll
+      for (int st = 0; st < 16; ++st)
+#pragma unroll
+        for (int ob = 0; ob < 4; ++ob)
+          z[ob] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              s_w[(rows + ob * 16 + st) * kFragStride + lane], act[st], z[ob], 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float v = z[e >> 2][e & 3], s = sigmoidf_(v);
+        act[e] = v * s;
+        (L == 0 ? d2 : d3)[e] = s * (1.0f + v * (1.0f - s));
       }
-      for (int a = 0; a < 4; ++a)
-        for (int c = 0; c < 4; ++c) {
-          const int e = (4 * rb + a) * kSdfHidden + 4 * cb + c;
-          Zout[L][e] = acc[a][c];
-          Aout[L][e] = silu(acc[a][c]);
-        }
-      __syncthreads();
+      if (L == 0) train_put<4>(s_a2[w], act, g, c);
     }
-    // ---- output and loss: sample s = t / 4, quarter t % 4 of the 64 terms
-    {
-      const int s = t >> 2, part = t & 3;
-      float yv = 0.0f;
-      for (int i = 16 * part; i < 16 * part + 16; ++i) yv += A3[s * kSdfHidden + i] * W[kSdfOffW4 + i];
-      yv += __shfl_xor(yv, 1);
-      yv += __shfl_xor(yv, 2);
-      if (part == 0) {
-        const uint32_t gs = s0 + s;
-        float dy = 0.0f;
-        if (gs < batchEnd && gs < samplesPerBody) {
-          const float target = labels[(size_t)body * samplesPerBody + gs] / FR[kSdfFreqs * 3 + 3];
-          const float err = (yv + W[kSdfOffB4]) - target;
-          lossAcc += err * err;
-          dy = 2.0f * err * invM;
-        }
-        Y[s] = dy;
-      }
+    // ---- output, loss, and the output layer's gradient
+    float y = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      y += act[e] * s_bias[3 * kSdfHidden + 16 * (e >> 2) + 4 * g + (e & 3)];
+    y += __shfl_xor(y, 16);
+    y += __shfl_xor(y, 32);
+    float dy = 0.0f;
+    if (live) {
+      const float target = labels[(size_t)body * samplesPerBody + gs] / s_fr[kSdfFreqs * 3 + 3];
+      const float err = (y + b4) - target;
+      if (g == 0) lossAcc += err * err;
+      dy = 2.0f * err * invM;
     }
+    if (g == 0) gb4 += dy;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      gW4[e] += act[e] * dy;
+      act[e] = dy * s_bias[3 * kSdfHidden + 16 * (e >> 2) + 4 * g + (e & 3)] * d3[e];  // dZ3
+    }
+    train_put<4>(s_dz[w], act, g, c);
     __syncthreads();
-    // ---- backward
-    // dW4, db4 (from A3, Y) before A3 is overwritten
-    if (t < kSdfHidden) {
-      float a = 0.0f;
-      for (int s = 0; s < kTile; ++s) a += A3[s * kSdfHidden + t] * Y[s];
-      gW4 += a;
-    }
-    if (t == 0) {
-      float a = 0.0f;
-      for (int s = 0; s < kTile; ++s) a += Y[s];
-      gb4 += a;
-    }
-    // dZ3 = dy w4 SiLU'(Z3), in place in Z3
-    for (int a = 0; a < 4; ++a)
-      for (int c = 0; c < 4; ++c) {
-        const int s = 4 * rb + a, o = 4 * cb + c;
-        const int e = s * kSdfHidden + o;
-        Z3[e] = Y[s] * W[kSdfOffW4 + o] * silu_grad(Z3[e]);
-      }
-    __syncthreads();
-    // layers 3 and 2: dW += A_in^T dZ, db += sum dZ, dZ_in = (dZ W^T) SiLU'(Z_in)
-    float* dZ = Z3;
+    // ---- layers 3 and 2: dW += A_in^T dZ over the block's samples, and
+    // dZ_in = (W dZ) SiLU'(Z_in) of the wave's own
 #pragma unroll
     for (int L = 1; L >= 0; --L) {
-      const float* Aprev = L == 1 ? A2 : A1;
-      const float* Zprev = L == 1 ? Z2 : Z1;
-      const int offW = L == 1 ? kSdfOffW3 : kSdfOffW2;
-      float(*gW)[4] = L == 1 ? gW3 : gW2;
-      for (int s = 0; s < kTile; ++s) {
-        float x[4], d[4];
-        for (int a = 0; a < 4; ++a) x[a] = Aprev[s * kSdfHidden + 4 * rb + a];
-        for (int c = 0; c < 4; ++c) d[c] = dZ[s * kSdfHidden + 4 * cb + c];
-        for (int a = 0; a < 4; ++a)
-          for (int c = 0; c < 4; ++c) gW[a][c] += x[a] * d[c];
-      }
-      if (t < kSdfHidden) {
-        float a = 0.0f;
-        for (int s = 0; s < kTile; ++s) a += dZ[s * kSdfHidden + t];
-        if (L == 1) gb3 += a;
-        else gb2 += a;
-      }
-      // dA_prev[s][i] = sum_o dZ[s][o] W[i][o]; tile (s-block rb, i-block cb)
-      float acc[4][4] = {};
-      for (int o = 0; o < kSdfHidden; ++o) {
-        float d[4], w[4];
-        for (int a = 0; a < 4; ++a) d[a] = dZ[(4 * rb + a) * kSdfHidden + o];
-        for (int c = 0; c < 4; ++c) w[c] = W[offW + (4 * cb + c) * kSdfHidden + o];
-        for (int a = 0; a < 4; ++a)
-          for (int c = 0; c < 4; ++c) acc[a][c] += d[a] * w[c];
-      }
-      float* dst = L == 1 ? A3 : Z3;  // A3 is dead after dW4; Z3 (dZ3) after this layer
-      __syncthreads();
-      for (int a = 0; a < 4; ++a)
-        for (int c = 0; c < 4; ++c) {
-          const int e = (4 * rb + a) * kSdfHidden + 4 * cb + c;
-          dst[e] = acc[a][c] * silu_grad(Zprev[e]);
+      const float(*aIn)[16 * kSdfHidden] = L == 1 ? s_a2 : s_a1;
+      const float(*dOut)[16 * kSdfHidden] = L == 1 ? s_dz : s_a2;
+      floatx4* gW = L == 1 ? gW3 : gW2;
+      float* gb = L == 1 ? gb3 : gb2;
+      const int rows = L == 1 ? kRowsW3 : kRowsW2;
+#pragma unroll 2
+      for (int v = 0; v < kTrainWaves; ++v)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const float a = aIn[v][256 * ib + at[s]];
+          const float o0 = dOut[v][256 * jb + at[s]], o1 = dOut[v][256 * (jb + 1) + at[s]];
+          gW[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, o0, gW[0], 0, 0, 0);
+          gW[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, o1, gW[1], 0, 0, 0);
+          gb[0] += o0;
+          gb[1] += o1;
         }
+#pragma unroll
+      for (int ob = 0; ob < 4; ++ob) z[ob] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int st = 0; st < 16; ++st)
+#pragma unroll
+        for (int ob = 0; ob < 4; ++ob)
+          z[ob] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              s_w[(rows + 16 * (st >> 2) + 4 * ob) * kFragStride + back + (st & 3)], act[st],
+              z[ob], 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) act[e] = z[e >> 2][e & 3] * (L == 1 ? d2 : d1)[e];
+      if (L == 1) __syncthreads();  // the readers of A2, whose place dZ2 takes
+      train_put<4>(L == 1 ? s_a2[w] : s_dz[w], act, g, c);
       __syncthreads();
-      dZ = dst;
     }
-    // layer 1: dW1 += X0^T dZ1 (inputs 2rb, 2rb+1), db1
-    for (int s = 0; s < kTile; ++s) {
-      float x[2], d[4];
-      for (int a = 0; a < 2; ++a) x[a] = X0[s * kSdfIn + 2 * rb + a];
-      for (int c = 0; c < 4; ++c) d[c] = dZ[s * kSdfHidden + 4 * cb + c];
-      for (int a = 0; a < 2; ++a)
-        for (int c = 0; c < 4; ++c) gW1[a][c] += x[a] * d[c];
-    }
-    if (t < kSdfHidden) {
-      float a = 0.0f;
-      for (int s = 0; s < kTile; ++s) a += dZ[s * kSdfHidden + t];
-      gb1 += a;
-    }
+    // ---- layer 1: dW1 += X0^T dZ1
+#pragma unroll 2
+    for (int v = 0; v < kTrainWaves; ++v)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const float o = s_dz[v][256 * jb1 + at[s]];
+        gW1 = __builtin_amdgcn_mfma_f32_16x16x4f32(s_x0[v][256 * ib1 + at[s]], o, gW1, 0, 0, 0);
+        gb1 += o;
+      }
   }
-  // write this block's sums
+  // ---- this block's sums: row 4 g + r, column c of each gradient block
   float* G = partial + ((size_t)body * nblk + blk) * kSdfStride;
-  for (int a = 0; a < 2; ++a)
-    for (int c = 0; c < 4; ++c) G[kSdfOffW1 + (2 * rb + a) * kSdfHidden + 4 * cb + c] = gW1[a][c];
-  for (int a = 0; a < 4; ++a)
-    for (int c = 0; c < 4; ++c) {
-      G[kSdfOffW2 + (4 * rb + a) * kSdfHidden + 4 * cb + c] = gW2[a][c];
-      G[kSdfOffW3 + (4 * rb + a) * kSdfHidden + 4 * cb + c] = gW3[a][c];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int in = 16 * ib + 4 * g + r, in1 = 16 * ib1 + 4 * g + r;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      G[kSdfOffW3 + in * kSdfHidden + 16 * (jb + b) + c] = gW3[b][r];
+      G[kSdfOffW2 + in * kSdfHidden + 16 * (jb + b) + c] = gW2[b][r];
     }
-  if (t < kSdfHidden) {
-    G[kSdfOffB1 + t] = gb1;
-    G[kSdfOffB2 + t] = gb2;
-    G[kSdfOffB3 + t] = gb3;
-    G[kSdfOffW4 + t] = gW4;
+    G[kSdfOffW1 + in1 * kSdfHidden + 16 * jb1 + c] = gW1[r];
   }
-  if (t == 0) G[kSdfOffB4] = gb4;
-  // block sum of squared errors (lanes 4s hold the sample terms)
-  float l = lossAcc;
-  for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
-  if ((t & 63) == 0) red[t >> 6] = l;
+  // biases: the lanes of a column hold its samples' shares
+  auto over_g = [](float v) {
+    v += __shfl_xor(v, 16);
+    return v + __shfl_xor(v, 32);
+  };
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const float v3 = over_g(gb3[b]), v2 = over_g(gb2[b]);
+    if (ib == 0 && g == 0) {
+      G[kSdfOffB3 + 16 * (jb + b) + c] = v3;
+      G[kSdfOffB2 + 16 * (jb + b) + c] = v2;
+    }
+  }
+  const float v1 = over_g(gb1);
+  if (ib1 == 0 && g == 0) G[kSdfOffB1 + 16 * jb1 + c] = v1;
+  // output layer and loss: over the samples (lanes of a group), then the waves
+  float* red = &s_a1[0][0];  // [waves][64 + 2]
   __syncthreads();
-  if (t == 0) {
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    float v = gW4[e];
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    if (c == 0) red[w * 66 + 16 * (e >> 2) + 4 * g + (e & 3)] = v;
+  }
+  float l = lossAcc;
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) {
+    gb4 += __shfl_xor(gb4, off);
+    l += __shfl_xor(l, off);
+  }
+  if (lane == 0) {
+    red[w * 66 + 64] = gb4;
+    red[w * 66 + 65] = l;
+  }
+  __syncthreads();
+  if (t < 66) {
     float s = 0.0f;
-    for (int w = 0; w < kTB / 64; ++w) s += red[w];
-    lossPartial[(size_t)body * nblk + blk] = s;
+    for (int v = 0; v < kTrainWaves; ++v) s += red[v * 66 + t];
+    if (t < 64)
+      G[kSdfOffW4 + t] = s;
+    else if (t == 64)
+      G[kSdfOffB4] = s;
+    else
+      lossPartial[(size_t)body * nblk + blk] = s;
   }
 }
 
@@ -405,10 +462,19 @@ __global__ __launch_bounds__(kTB) void k_sdf_reduce_step(
   const uint32_t p = (uint32_t)(idx % kSdfStride);
   if (p >= (uint32_t)kSdfParams) return;  // padding
   float g = 0.0f;
-  for (uint32_t k = 0; k < nblk; ++k) g += partial[((size_t)b * nblk + k) * kSdfStride + p];
+  const float* at = partial + (size_t)b * nblk * kSdfStride + p;
+  uint32_t k = 0;
+  for (; k + 8 <= nblk; k += 8) {  // eight loads in flight, added in order
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = at[(size_t)(k + u) * kSdfStride];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) g += v[u];
+  }
+  for (; k < nblk; ++k) g += at[(size_t)k * kSdfStride];
   if (p == 0) {
     float l = 0.0f;
-    for (uint32_t k = 0; k < nblk; ++k) l += lossPartial[(size_t)b * nblk + k];
+    for (uint32_t q = 0; q < nblk; ++q) l += lossPartial[(size_t)b * nblk + q];
     loss[b] += l * invM;
   }
   if (!adam) {
@@ -1066,7 +1132,8 @@ void free_sdf(fc_sdf* m) {
   hipFree(m->lossOut);
 }
 
-constexpr uint32_t kTilesPerBlock = 8;
+// Training blocks resident at once: one per CU (154 KB of LDS each).
+constexpr uint32_t kTrainBlocks = 256;
 // Waves of the inference kernel (the 20 weight fragments in registers,
 // 170 VGPRs: two waves per SIMD of the 256 CUs) and of the cull (fragments
 // loaded where used, under 100 VGPRs: four waves per SIMD).
@@ -1092,13 +1159,18 @@ uint32_t mfma_blocks(uint32_t n, uint32_t maxWaves = kMaxInferWaves) {
 fc_status sdf_step(fc_sdf* m, const float* pts, const float* labels, uint32_t samplesPerBody,
                    uint32_t batchStart, uint32_t batchSize, int adam, float lr) {
   hipStream_t st = m->ctx->stream;
-  const uint32_t tiles = (batchSize + kTile - 1) / kTile;
-  const uint32_t nblk = (tiles + kTilesPerBlock - 1) / kTilesPerBlock;
+  // One round of resident blocks where that leaves each a few tiles; a body
+  // keeps at least one block, and a block takes at most 8 tiles, so that the
+  // sums' order does not grow with the card.
+  const uint32_t tiles = (uint32_t)(((uint64_t)batchSize + kTrainTile - 1) / kTrainTile);
+  uint64_t perBlock = ((uint64_t)tiles * m->B + kTrainBlocks - 1) / kTrainBlocks;
+  if (perBlock > 8) perBlock = 8;
+  const uint32_t nblk = (uint32_t)((tiles + perBlock - 1) / perBlock);
   FC_TRY(ensure_partials(m, (size_t)m->B * nblk * kSdfStride, (size_t)m->B * nblk));
   const float invM = 1.0f / (float)batchSize;
-  hipLaunchKernelGGL(k_sdf_grad_tiles, dim3(nblk, m->B), dim3(kTB), 0, st, m->params, m->freq,
-                     m->frame, pts, labels, samplesPerBody, batchStart, batchSize,
-                     kTilesPerBlock, invM, m->partial, m->lossPartial);
+  hipLaunchKernelGGL(k_sdf_grad_tiles, dim3(nblk, m->B), dim3(kTrainThreads), 0, st,
+                     m->params, m->freq, m->frame, pts, labels, samplesPerBody, batchStart,
+                     batchSize, (uint32_t)perBlock, invM, m->partial, m->lossPartial);
   FC_HIP_TRY(hipGetLastError());
   float c1 = 1.0f, c2 = 1.0f;
   if (adam) {

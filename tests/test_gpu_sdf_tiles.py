@@ -1,0 +1,37 @@
+"""The training kernel's gradient at the edges of its 128-sample tiles and of
+its blocks (one sample, a tile less and more by one, several tiles per block,
+many bodies) against the oracle's binary64 gradient."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bodies,samples", [(1, 1), (1, 127), (2, 128), (1, 129), (3, 1000),
+                                            (40, 1025)])
+def test_gradient_tiles(gpu_ctx, bodies, samples):
+    from fullc0ntact_amd import _lib
+    from fullc0ntact_amd.sdf import SdfSurrogate
+    print(bodies, samples, flush=True)
+    rng = np.random.default_rng(samples)
+    s = SdfSurrogate(gpu_ctx, rng.uniform(-0.1, 0.1, (bodies, 3)),
+                     rng.uniform(0.8, 1.2, bodies), seed=7)
+    p, f, fr = s.params()
+    p = p + rng.normal(0.0, 0.03, p.shape).astype(np.float32)
+    s.set_params(p)
+    pts = rng.uniform(-0.7, 0.7, (bodies, samples, 3)).astype(np.float32)
+    lab = rng.uniform(-0.3, 0.3, (bodies, samples)).astype(np.float32)
+    dp = _lib.DeviceArray.from_host(gpu_ctx, pts)
+    dl = _lib.DeviceArray.from_host(gpu_ctx, lab)
+    g, loss = s.loss_grad(dp, dl, samples)
+    for b in {0, bodies // 2, bodies - 1}:
+        ref, L = orc.sdf_loss_grad(p[b], f[b], fr[b], pts[b], lab[b])
+        # binary32 sums of a few hundred terms; the hardware sine and cosine
+        assert abs(loss[b] - L) <= 1e-5 * L
+        gb = g[b, :s.nparams].astype(np.float64)
+        assert np.max(np.abs(gb - ref)) <= 1e-4 * np.max(np.abs(ref))
+    s.close()
