@@ -297,14 +297,14 @@ unsigned sdf_blocks(uint64_t npts) {
 }
 
 // The tree's scratch, grown to the largest mesh the context has seen (about
-// 130 bytes a triangle); false when there is no memory for it, or inside a
+// 130 bytes a triangle, 8 more per point up to 2^22); false when there is no memory for it, or inside a
 // graph capture, where it could not grow.  The callers then take the brute
 // force alone.
-bool tree_scratch(fc_context* ctx, uint32_t nt, size_t extra) {
+bool tree_scratch(fc_context* ctx, uint32_t nt, uint32_t sorted, size_t extra) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
     return false;
-  if (ensure_sort_capacity(ctx, nt) != FC_SUCCESS) {
+  if (ensure_sort_capacity(ctx, sorted) != FC_SUCCESS) {
     (void)hipGetLastError();
     return false;
   }
@@ -339,9 +339,12 @@ hipError_t launch_mesh_sdf_points(fc_context* ctx, const double* verts, uint32_t
   if (np == 0) return hipSuccess;
   hipStream_t s = ctx->stream;
   MeshTree T;
-  if (mesh_tree_pays(nt, np) && tree_scratch(ctx, nt, 0)) {
+  if (mesh_tree_pays(nt, np) &&
+      tree_scratch(ctx, nt, tree_sort_pairs(nt, np), tree_points_bytes(np))) {
     hipError_t e = launch_mesh_tree(ctx, verts, nv, tris, nt, ctx->meshScratch, &T);
-    if (e == hipSuccess) e = launch_tree_points(s, T, verts, nv, tris, nt, pts, np, sdf, cp);
+    if (e == hipSuccess)
+      e = launch_tree_points(ctx, T, verts, nv, tris, nt, pts, np,
+                             static_cast<char*>(ctx->meshScratch) + mesh_tree_bytes(nt), sdf, cp);
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(k_mesh_sdf<false>, dim3(sdf_blocks(np)), dim3(kBlock), 0, s, T.info, verts,
@@ -791,8 +794,8 @@ fc_status fc_distmap_build(fc_context* ctx, const double* vertices, uint32_t num
   if (e == hipSuccess) e = hipMemcpyAsync(m->ys, ax[1].data(), ax[1].size() * 4, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipMemcpyAsync(m->zs, ax[2].data(), ax[2].size() * 4, hipMemcpyHostToDevice, st);
   MeshTree T;
-  if (e == hipSuccess && mesh_tree_pays(numTriangles, m->V) && tree_lattice_fits(cells) &&
-      tree_scratch(ctx, numTriangles, 0)) {
+  if (e == hipSuccess && mesh_tree_pays(numTriangles, m->V) && tree_lattice_fits(cells, b, cs) &&
+      tree_scratch(ctx, numTriangles, numTriangles, 0)) {
     e = launch_mesh_tree(ctx, dv, numVertices, dt, numTriangles, ctx->meshScratch, &T);
     if (e == hipSuccess)
       e = launch_tree_lattice(st, T, dv, numVertices, dt, numTriangles, m->cells, b, cs, m->cpd,

@@ -29,64 +29,40 @@ __host__ __device__ __forceinline__ double point_triangle_dist2(const double q[3
   const double e = E1[0] * D[0] + E1[1] * D[1] + E1[2] * D[2];
   const double det = a * c - b * b;
   double s = b * e - c * d, t = b * d - a * e;
-  if (s + t <= det) {
-    if (s < 0.0) {
-      if (t < 0.0) {  // region 4
-        if (d < 0.0) {
-          t = 0.0;
-          s = (-d >= a) ? 1.0 : -d / a;
-        } else {
-          s = 0.0;
-          t = (e >= 0.0) ? 0.0 : ((-e >= c) ? 1.0 : -e / c);
-        }
-      } else {  // region 3
-        s = 0.0;
-        t = (e >= 0.0) ? 0.0 : ((-e >= c) ? 1.0 : -e / c);
-      }
-    } else if (t < 0.0) {  // region 5
-      t = 0.0;
-      s = (d >= 0.0) ? 0.0 : ((-d >= a) ? 1.0 : -d / a);
-    } else {  // region 0
-      const double inv = 1.0 / det;
-      s *= inv;
-      t *= inv;
-    }
+  // The regions differ in the edge they clamp to, all with one quotient: on
+  // E0 (t = 0) -d / a, on E1 (s = 0) -e / c, on the third edge s or t =
+  // (difference of its ends' slopes) / |E1 - E0|^2, each within [0, 1]; inside,
+  // 1 / det.  The operands are picked first, so that a wave whose lanes lie in
+  // different regions divides once.
+  const bool inner = s + t <= det, sNeg = s < 0.0, tNeg = t < 0.0;
+  const double ce = c + e, bd = b + d, ad = a + d, be = b + e;
+  const bool inside = inner && !sNeg && !tNeg;                      // region 0
+  const bool third2 = !inner && sNeg && ce > bd;                    // region 2
+  const bool third6 = !inner && !sNeg && tNeg && ad > be;           // region 6
+  const bool third = third2 || third6 || (!inner && !sNeg && !tNeg);  // region 1
+  // regions 4 (one side), 5 and 6 (rest); else 4 (other side), 3 and 2 (rest)
+  const bool first = inner ? (sNeg ? tNeg && d < 0.0 : tNeg) : !sNeg && tNeg && !third6;
+  const double num = inside ? 1.0 : (third6 ? ad - be : (third ? ce - bd : (first ? -d : -e)));
+  const double den = inside ? det : (third ? a - 2.0 * b + c : (first ? a : c));
+  double x = num / den;
+  if (num >= den) x = 1.0;
+  if (num <= 0.0) x = 0.0;
+  if (inside) {
+    const double inv = num / den;
+    s *= inv;
+    t *= inv;
+  } else if (third) {
+    s = third6 ? 1.0 - x : x;
+    t = third6 ? x : 1.0 - x;
   } else {
-    if (s < 0.0) {  // region 2
-      const double tmp0 = b + d, tmp1 = c + e;
-      if (tmp1 > tmp0) {
-        const double numer = tmp1 - tmp0, denom = a - 2.0 * b + c;
-        s = (numer >= denom) ? 1.0 : numer / denom;
-        t = 1.0 - s;
-      } else {
-        s = 0.0;
-        t = (tmp1 <= 0.0) ? 1.0 : ((e >= 0.0) ? 0.0 : -e / c);
-      }
-    } else if (t < 0.0) {  // region 6
-      const double tmp0 = b + e, tmp1 = a + d;
-      if (tmp1 > tmp0) {
-        const double numer = tmp1 - tmp0, denom = a - 2.0 * b + c;
-        t = (numer >= denom) ? 1.0 : numer / denom;
-        s = 1.0 - t;
-      } else {
-        t = 0.0;
-        s = (tmp1 <= 0.0) ? 1.0 : ((d >= 0.0) ? 0.0 : -d / a);
-      }
-    } else {  // region 1
-      const double numer = (c + e) - (b + d);
-      if (numer <= 0.0) {
-        s = 0.0;
-      } else {
-        const double denom = a - 2.0 * b + c;
-        s = (numer >= denom) ? 1.0 : numer / denom;
-      }
-      t = 1.0 - s;
-    }
+    s = first ? x : 0.0;
+    t = first ? 0.0 : x;
   }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) cp[k] = (B[k] + s * E0[k]) + t * E1[k];
   double r2 = 0.0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    cp[k] = (B[k] + s * E0[k]) + t * E1[k];
     const double diff = cp[k] - q[k];
     r2 += diff * diff;
   }

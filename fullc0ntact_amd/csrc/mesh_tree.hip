@@ -37,6 +37,12 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr uint32_t kInfoBlocks = 64;
+// Free points are sorted and taken this many at a time (bounds the scratch).
+constexpr uint64_t kPointChunk = 1ull << 22;
+// Fewer points share a wave (down to 8) until there are this many waves, four
+// per SIMD: a wave's walk is a chain of dependent steps, longer the further
+// apart its points lie.
+constexpr uint32_t kPointWaves = 4096;
 
 __device__ __forceinline__ unsigned long long mesh_key(double d) {
   const unsigned long long u = (unsigned long long)__double_as_longlong(d);
@@ -231,6 +237,15 @@ __global__ __launch_bounds__(1024) void k_tree_levels(TreeBuild B) {
   }
 }
 
+// Read-only memory at a wave-uniform address, through the scalar cache into
+// scalar registers (the tree is written by earlier launches only).
+template <typename E>
+using Uniform = const E __attribute__((address_space(4)))*;
+template <typename E>
+__device__ __forceinline__ Uniform<E> uniform(const E* p) {
+  return reinterpret_cast<Uniform<E>>(reinterpret_cast<uintptr_t>(p));
+}
+
 // The brute force's winding sum, in its order, for the lanes that `need` it,
 // one such lane's point at a time: the wave takes 64 triangles' solid angles
 // together and adds them one by one.
@@ -265,110 +280,290 @@ __device__ __forceinline__ double winding_sum(bool need, const double q[3],
 
 __device__ __forceinline__ bool winds(double w) { return w / (4.0 * 3.14159265358979323846) > 0.5; }
 
-// The smallest (squared distance, triangle number) of q.  s_lb: this lane's
-// column of the block's [levels][8][lanes] child distances.
-struct Nearest {
-  double d2;
-  uint32_t id;
-  double cp[3];
+// The closest triangles of a wave's 64 points, one per lane, found together.
+// The points are neighbours, so the wave walks the tree once for all of them:
+// a box is entered when any lane has to look into it, nearest first as seen
+// from one lane, and its eight children's bounds are read once (uniform
+// loads).  What a lane still has to test exactly, the triangles whose box is
+// within its best distance and of which some corner lies in front of the
+// plane through its best point (every point closer than that is), goes to a
+// list of (lane, triangle) pairs that the wave takes 64 at a time, so that
+// point_triangle_dist2, 300 instructions of binary64, runs with all lanes.
+//
+// Bound by issue: a wave takes about 65 boxes of eight, 74 triangles and 25
+// rounds of pairs.  274,625 lattice points against 6,144 triangles: a search
+// per lane, diverging at every step, took 1.02 ms; this 0.36 ms.
+constexpr int kLanes = 64;  // one wave per block
+
+// (4 waves per SIMD at 108 VGPRs: 598 us a build against 578)
+constexpr int kTreeWavesPerSimd = 5;
+
+struct TreeShared {
+  double q[3][kLanes];
+  double cp[3][kLanes];
+  unsigned long long d2[kLanes];
+  uint32_t id[kLanes];
+  uint32_t pair[2 * kLanes];  // lane << 26 | triangle in tree order
+  float lb[8][kLanes];
 };
 
-constexpr int kLanes = 64;  // one wave per block: no barriers, any balance
+struct Nearest {
+  double d2 = DBL_MAX;
+  uint32_t id = 0xffffffffu;
+  double cp[3] = {0.0, 0.0, 0.0};
+};
 
-__device__ __forceinline__ Nearest tree_nearest(const MeshTree& T, const double q[3],
-                                                double delta, float (*s_lb)[8][kLanes]) {
-  Nearest best;
-  best.d2 = DBL_MAX;
-  best.id = 0xffffffffu;
-  best.cp[0] = best.cp[1] = best.cp[2] = 0.0;
-  float qlo[3], qhi[3];
+__device__ __forceinline__ void tree_nearest(const MeshTree& T, const double q[3], double delta,
+                                             bool active, int centre, uint32_t lanes,
+                                             TreeShared& S, Nearest& best) {
+  const int lane = (int)(threadIdx.x & 63u);
+  float qf[3];
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    qlo[a] = __double2float_rd(q[a]);
-    qhi[a] = __double2float_ru(q[a]);
+    qf[a] = (float)q[a];
+    S.q[a][lane] = q[a];
   }
-  const int lane = (int)(threadIdx.x & 63u);
-  // (sqrt(d2) + delta)^2, rounded up: a box at least this far holds no winner
-  float limit = INFINITY;
-  uint64_t todo = 0;  // a byte per level: the children still to be taken
-  int level = T.levels - 1;
-  uint32_t group = 0;
-  bool enter = true;
-  while (true) {
-    if (enter) {
-      const float4* b = reinterpret_cast<const float4*>(T.box[level] + (size_t)group * 48u);
-      float lb[8] = {};
+  S.d2[lane] = (unsigned long long)__double_as_longlong(best.d2);
+  // (sqrt(d2) + delta)^2, with room for the float rounding of the boxes'
+  // distances (2^-20 of the largest coordinate: delta is 2^-44 of it): a box
+  // at least this far holds no winner
+  const double deltaF = delta * 0x1p24;
+  float limit = active ? FLT_MAX : -1.0f;
+  // unit vector to the best point (0 before there is one), and where the
+  // plane with this normal is too far: u . q + sqrt(d2) + delta
+  double u[3] = {0.0, 0.0, 0.0}, front = INFINITY;
+  uint32_t pairs = 0;
+  // (fewer lanes test sooner, so that their bounds do not lag)
+  const uint32_t full = min(2u * lanes, 64u);
+
+  // Takes up to 64 pairs from the front of the list.
+  auto test_pairs = [&]() {
+    __syncthreads();
+    const uint32_t cnt = pairs < 64u ? pairs : 64u;
+    const bool on = (uint32_t)lane < cnt;
+    const uint32_t e = S.pair[lane], l = on ? e >> 26 : 0u, at = on ? e & 0x03ffffffu : 0u;
+    double p[3], c[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) p[a] = S.q[a][l];
+    const TreeTri& R = T.tri[at];
+    const uint32_t id = (uint32_t)R.id;
+    const double d2 = point_triangle_dist2(p, R.v, R.v + 3, R.v + 6, c);
+    // squared distances are not negative: their bits order as they do (a
+    // NaN's above all of them)
+    const unsigned long long key = (unsigned long long)__double_as_longlong(d2);
+    if (on) atomicMin(&S.d2[l], key);
+    __syncthreads();
+    const unsigned long long mine = S.d2[lane];
+    const bool closer = mine < (unsigned long long)__double_as_longlong(best.d2);
+    S.id[lane] = closer ? 0xffffffffu : best.id;
+    __syncthreads();
+    const bool least = on && key == S.d2[l];
+    if (least) atomicMin(&S.id[l], id);
+    __syncthreads();
+    if (least && S.id[l] == id) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) S.cp[a][l] = c[a];
+    }
+    __syncthreads();
+    if (closer || S.id[lane] != best.id) {
+      best.d2 = __longlong_as_double((long long)mine);
+      best.id = S.id[lane];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) best.cp[a] = S.cp[a][lane];
+      const double dist = sqrt(best.d2), r = dist + delta, rf = dist + deltaF;
+      limit = __double2float_ru(rf * rf * (1.0 + 0x1p-20));
+      // (a little short of one, so that no rounding makes it longer)
+      const double inv = dist > 0.0 ? (1.0 - 1e-12) / dist : 0.0;
+      front = r;
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        const float4 l0 = b[2 * a], l1 = b[2 * a + 1], h0 = b[6 + 2 * a], h1 = b[7 + 2 * a];
-        const float lo[8] = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
-        const float hi[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const float d = fmaxf(fmaxf(lo[u] - qhi[a], qlo[a] - hi[u]), 0.0f);
-          lb[u] += d * d;
-        }
-      }
-      uint32_t m = 0;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        // below the exact box distance by more than its few roundings
-        const float x = lb[u] * (1.0f - 0x1p-20f);
-        s_lb[level][u][lane] = x;
-        if (!(x > limit) && group * 8u + (uint32_t)u < T.count[level]) m |= 1u << u;
-      }
-      todo = (todo & ~(0xffull << (8 * level))) | ((uint64_t)m << (8 * level));
-      enter = false;
-    }
-    // the nearest child still to be taken
-    uint32_t m = (uint32_t)(todo >> (8 * level)) & 0xffu;
-    float near = INFINITY;
-    int pick = -1;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      if ((m >> u) & 1u) {
-        const float x = s_lb[level][u][lane];
-        if (!(x > limit) && (pick < 0 || x < near)) {
-          near = x;
-          pick = u;
-        }
+        u[a] = (best.cp[a] - q[a]) * inv;
+        front += u[a] * q[a];
       }
     }
-    if (pick < 0) {  // none left within reach
-      if (++level == T.levels) break;
+    // what is left moves to the front
+    const uint32_t rest = pairs - cnt;
+    const uint32_t next = (uint32_t)lane < rest ? S.pair[64 + lane] : 0u;
+    __syncthreads();
+    if ((uint32_t)lane < rest) S.pair[lane] = next;
+    pairs = rest;
+  };
+
+  // Lane L keeps level L's boxes still to be entered: three bits each, the
+  // nearest lowest, and their number from bit 24 on.
+  uint32_t todo = 0;
+  int level = T.levels - 1;
+  uint32_t group = 0;
+  while (true) {
+    // ---- the eight boxes of a group
+    const Uniform<float> b = uniform(T.box[level] + (size_t)group * 48u);
+    float lb[8] = {};
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const float d = fmaxf(fmaxf(b[8 * a + c] - qf[a], qf[a] - b[24 + 8 * a + c]), 0.0f);
+        lb[c] = fmaf(d, d, lb[c]);
+      }
+    // the boxes some lane has to look into (a group's spare boxes are inside
+    // out, infinitely far), and their distances from the centre lane
+    uint32_t open = 0, key[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const uint32_t any = __ballot(!(lb[c] > limit)) != 0ull ? 1u : 0u;
+      open |= any << c;
+      // (the distance's sign bit is clear: its bits order as it does)
+      const uint32_t at =
+          ((uint32_t)__builtin_amdgcn_readlane(__float_as_int(lb[c]), centre) & ~7u) | (uint32_t)c;
+      key[c] = any ? at : 0xffffffffu;
+    }
+    if (level == 0) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) S.lb[c][lane] = lb[c];
+#pragma unroll 1
+      for (uint32_t left = open; left != 0u; left &= left - 1u) {
+        const uint32_t c = (uint32_t)__ffs((int)left) - 1u;
+        const float x = S.lb[c][lane];
+        if (__ballot(!(x > limit)) == 0ull) continue;
+        const uint32_t at = group * 8u + c;
+        const Uniform<double> v = uniform(T.tri[at].v);
+        double s[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          s[k] = fma(u[2], v[3 * k + 2], fma(u[1], v[3 * k + 1], u[0] * v[3 * k]));
+        const bool test = !(x > limit) && !(fmin(s[0], fmin(s[1], s[2])) > front);
+        const uint64_t m = __ballot(test);
+        if (test)
+          S.pair[pairs + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] =
+              ((uint32_t)lane << 26) | at;
+        pairs += (uint32_t)__popcll(m);
+        if (pairs >= full) test_pairs();
+      }
+    } else {
+      // nearest first (a network of 19 exchanges)
+      constexpr int kNet[19][2] = {{0, 1}, {2, 3}, {4, 5}, {6, 7}, {0, 2}, {1, 3}, {4, 6},
+                                   {5, 7}, {1, 2}, {5, 6}, {0, 4}, {3, 7}, {1, 5}, {2, 6},
+                                   {1, 4}, {3, 6}, {2, 4}, {3, 5}, {3, 4}};
+#pragma unroll
+      for (int x = 0; x < 19; ++x) {
+        const uint32_t lo = min(key[kNet[x][0]], key[kNet[x][1]]);
+        const uint32_t hi = max(key[kNet[x][0]], key[kNet[x][1]]);
+        key[kNet[x][0]] = lo;
+        key[kNet[x][1]] = hi;
+      }
+      uint32_t word = (uint32_t)__popc(open) << 24;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) word |= (key[c] & 7u) << (3 * c);
+      if (lane == level) todo = word;
+    }
+    // ---- the next group: a box still to be entered, on this level or above
+    uint32_t word = level == 0 ? 0u : (uint32_t)__builtin_amdgcn_readlane((int)todo, level);
+    while ((word >> 24) == 0u) {
       group >>= 3;
-      continue;
+      if (++level >= T.levels) break;
+      word = (uint32_t)__builtin_amdgcn_readlane((int)todo, level);
     }
-    todo &= ~(1ull << (8 * level + pick));
-    const uint32_t child = group * 8u + (uint32_t)pick;
-    if (level > 0) {
-      group = child;
-      --level;
-      enter = true;
-      continue;
-    }
-    const TreeTri& R = T.tri[child];
-    double v[9], c[3];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) v[k] = R.v[k];
-    const uint32_t id = (uint32_t)R.id;
-    const double d2 = point_triangle_dist2(q, v, v + 3, v + 6, c);
-    if (d2 < best.d2 || (d2 == best.d2 && id < best.id)) {
-      best.d2 = d2;
-      best.id = id;
-      best.cp[0] = c[0];
-      best.cp[1] = c[1];
-      best.cp[2] = c[2];
-      const double r = sqrt(d2) + delta;
-      limit = __double2float_ru(r * r * (1.0 + 1e-12));
-    }
+    if (level >= T.levels) break;
+    if (lane == level) todo = (((word >> 24) - 1u) << 24) | ((word & 0xffffffu) >> 3);
+    group = group * 8u + (word & 7u);
+    --level;
   }
-  return best;
+  while (pairs > 0u) test_pairs();
+}
+
+// The brute force's search for the lanes that `need` it (points beyond the
+// float range that the tree's boxes are compared in), one such lane's point
+// at a time, the wave over the triangles.
+__device__ __forceinline__ void brute_nearest(bool need, const double q[3],
+                                              const double* __restrict__ verts, uint32_t nv,
+                                              const uint32_t* __restrict__ tris, uint32_t nt,
+                                              Nearest& best) {
+  const uint32_t lane = threadIdx.x & 63u;
+  for (uint64_t todo = __ballot(need); todo != 0ull; todo &= todo - 1ull) {
+    const int who = __ffsll((unsigned long long)todo) - 1;
+    const double p[3] = {__shfl(q[0], who), __shfl(q[1], who), __shfl(q[2], who)};
+    Nearest r;
+    for (uint32_t t = lane; t < nt; t += 64u) {
+      double v[9], c[3];
+      uint32_t vi[3];
+      load_corners(verts, nv, tris, t, v, vi);
+      const double d2 = point_triangle_dist2(p, v, v + 3, v + 6, c);
+      if (d2 < r.d2) {
+        r.d2 = d2;
+        r.id = t;
+        r.cp[0] = c[0];
+        r.cp[1] = c[1];
+        r.cp[2] = c[2];
+      }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      const double d2 = __shfl_xor(r.d2, off);
+      const uint32_t id = (uint32_t)__shfl_xor((int)r.id, off);
+      const double c[3] = {__shfl_xor(r.cp[0], off), __shfl_xor(r.cp[1], off),
+                           __shfl_xor(r.cp[2], off)};
+      if (d2 < r.d2 || (d2 == r.d2 && id < r.id)) {
+        r.d2 = d2;
+        r.id = id;
+        r.cp[0] = c[0];
+        r.cp[1] = c[1];
+        r.cp[2] = c[2];
+      }
+    }
+    if ((int)lane == who) best = r;
+  }
 }
 
 __device__ __forceinline__ double rounding_margin(const MeshInfo& I, const double q[3]) {
   const double m = mesh_magnitude(I) + fmax(fabs(q[0]), fmax(fabs(q[1]), fabs(q[2])));
   return 256.0 * 2.220446049250313e-16 * m;
+}
+
+// The triangles whose boxes a ray from (x, y, z) along +x meets, 64 boxes (two
+// levels of the tree) a step, one per lane: leaf(in, t) is called by the whole
+// wave with up to 64 of them, lane by lane (`in`: the lane has one, number t
+// in tree order).
+template <class Leaf>
+__device__ __forceinline__ void ray_boxes(const MeshTree& T, float x, float yLo, float yHi,
+                                          float zLo, float zHi, Leaf leaf) {
+  const int lane = (int)(threadIdx.x & 63u);
+  // the top levels hold at most 8 and 64 boxes: start on an even one
+  int level = (T.levels - 1) & ~1;
+  const int top = level;
+  uint32_t first = 0;  // of the 64 boxes
+  // lane `level` keeps that level's boxes still to be opened, and their first
+  uint32_t todoLo = 0, todoHi = 0, firstOf = 0;
+  while (true) {
+    const uint32_t i = first + (uint32_t)lane;
+    bool in = i < T.count[level];
+    if (in) {
+      const float* b = T.box[level] + box_at(i);
+      in = b[24] >= x && b[8] <= yHi && b[32] >= yLo && b[16] <= zHi && b[40] >= zLo;
+    }
+    const uint64_t m = __ballot(in);
+    if (level == 0) {
+      if (m != 0ull) leaf(in, i);
+    } else if (lane == level) {
+      todoLo = (uint32_t)m;
+      todoHi = (uint32_t)(m >> 32);
+      firstOf = first;
+    }
+    // the next box to open, on this level or above
+    uint64_t left = level == 0 ? 0ull : m;
+    while (left == 0ull) {
+      level += 2;
+      if (level > top) return;
+      left = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)todoHi, level) << 32 |
+             (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)todoLo, level);
+    }
+    const uint32_t bit = (uint32_t)__ffsll((unsigned long long)left) - 1u;
+    left &= left - 1ull;
+    first = ((uint32_t)__builtin_amdgcn_readlane((int)firstOf, level) + bit) * 64u;
+    if (lane == level) {
+      todoLo = (uint32_t)left;
+      todoHi = (uint32_t)(left >> 32);
+    }
+    level -= 2;
+  }
 }
 
 // One wave per lattice line along x (all its vertices share the ray's y and
@@ -385,153 +580,114 @@ __global__ __launch_bounds__(kLanes) void k_tree_lines(MeshTree T, int nx, int n
   const int x0 = (int)blockIdx.y * (kLanes * kLineChunks);
   const uint32_t iy = blockIdx.x % (uint32_t)ny, iz = blockIdx.x / (uint32_t)ny;
   const double qy = by + (double)iy * cs, qz = bz + (double)iz * cs;
-  const float qyLo = __double2float_rd(qy), qyHi = __double2float_ru(qy);
-  const float qzLo = __double2float_rd(qz), qzHi = __double2float_ru(qz);
   int wind[kLineChunks] = {};
   bool unsure[kLineChunks] = {};
-  uint64_t todo = 0;
-  int level = T.levels - 1;
-  uint32_t group = 0;
-  bool enter = true;
-  while (true) {
-    if (enter) {
-      // lanes 0-7 take a child each
-      const int u = lane & 7;
-      const float* b = T.box[level] + (size_t)group * 48u + u;
-      const bool in = lane < 8 && group * 8u + (uint32_t)u < T.count[level] && b[8] <= qyHi &&
-                      b[32] >= qyLo && b[16] <= qzHi && b[40] >= qzLo;
-      const uint64_t m = __ballot(in);
-      todo = (todo & ~(0xffull << (8 * level))) | (m << (8 * level));
-      enter = false;
-    }
-    const uint32_t m = (uint32_t)(todo >> (8 * level)) & 0xffu;
-    if (m == 0u) {
-      if (++level == T.levels) break;
-      group >>= 3;
-      continue;
-    }
-    const uint32_t child = group * 8u + (uint32_t)(__ffs((int)m) - 1);
-    todo &= ~(1ull << (8 * level + (__ffs((int)m) - 1)));
-    if (level > 0) {
-      group = child;
-      --level;
-      enter = true;
-      continue;
-    }
-    const TreeTri& R = T.tri[child];
-    double v[9];
+  ray_boxes(T, -INFINITY, __double2float_rd(qy), __double2float_ru(qy), __double2float_rd(qz),
+            __double2float_ru(qz), [&](bool in, uint32_t t) {
+              double v[9] = {};
+              int cover = 0;
+              if (in) {
 #pragma unroll
-    for (int k = 0; k < 9; ++k) v[k] = R.v[k];
-    const int cover = ray_cover(qy, qz, v, v + 3, v + 6);
-    if (cover == 0) continue;
+                for (int k = 0; k < 9; ++k) v[k] = T.tri[t].v[k];
+                cover = ray_cover(qy, qz, v, v + 3, v + 6);
+              }
+              // each covering triangle in turn, for all the line's vertices
+              for (uint64_t m = __ballot(cover != 0); m != 0ull; m &= m - 1ull) {
+                const int who = __ffsll((unsigned long long)m) - 1;
+                double c[9];
 #pragma unroll
-    for (int c = 0; c < kLineChunks; ++c) {
-      if (x0 + c * kLanes < nx) {
-        const double q[3] = {bx + (double)(x0 + c * kLanes + lane) * cs, qy, qz};
-        const int side = plane_side(q, v, v + 3, v + 6);
-        if (side == cover) wind[c] += cover;
-        unsure[c] = unsure[c] || side == 0;
-      }
-    }
-  }
+                for (int k = 0; k < 9; ++k) c[k] = __shfl(v[k], who);
+                const int up = __builtin_amdgcn_readlane(cover, who);
 #pragma unroll
-  for (int c = 0; c < kLineChunks; ++c) {
-    const int x = x0 + c * kLanes + lane;
+                for (int h = 0; h < kLineChunks; ++h) {
+                  if (x0 + h * kLanes < nx) {
+                    const double q[3] = {bx + (double)(x0 + h * kLanes + lane) * cs, qy, qz};
+                    const int side = plane_side(q, c, c + 3, c + 6);
+                    if (side == up) wind[h] += up;
+                    unsure[h] = unsure[h] || side == 0;
+                  }
+                }
+              }
+            });
+#pragma unroll
+  for (int h = 0; h < kLineChunks; ++h) {
+    const int x = x0 + h * kLanes + lane;
     if (x < nx)
-      nrm[((size_t)iz * ny + iy) * nx + x].w = unsure[c] ? 2.0f : (wind[c] > 0 ? 1.0f : 0.0f);
+      nrm[((size_t)iz * ny + iy) * nx + x].w = unsure[h] ? 2.0f : (wind[h] > 0 ? 1.0f : 0.0f);
   }
 }
 
-// The same for one point per lane.
-__device__ __forceinline__ int tree_inside(const MeshTree& T, const double q[3]) {
-  float qlo[3], qhi[3];
+// The same for free points, kRaysPerWave of them one after the other (those
+// whose ray misses the mesh's box need none): sdf[v] receives what
+// k_tree_lines leaves in nrm[v].w.
+constexpr uint32_t kRaysPerWave = 4;
+
+__global__ __launch_bounds__(kLanes) void k_tree_signs(MeshTree T,
+                                                       const double* __restrict__ pts, uint32_t n,
+                                                       const uint32_t* __restrict__ order,
+                                                       double* __restrict__ sdf) {
+  const MeshInfo I = *T.info;
+  if (!mesh_closed(I)) return;
+  const int lane = (int)threadIdx.x;
+  const uint32_t k = blockIdx.x * kRaysPerWave + (uint32_t)lane;
+  const bool valid = (uint32_t)lane < kRaysPerWave && k < n;
+  const size_t v = valid ? order[k] : 0;
+  double q[3] = {0.0, 0.0, 0.0};
+  bool meets = valid;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    qlo[a] = __double2float_rd(q[a]);
-    qhi[a] = __double2float_ru(q[a]);
+    if (valid) q[a] = pts[3 * v + a];
+    // (false for a NaN, whose sums of solid angles are NaN: outside)
+    meets = meets && q[a] <= mesh_key_value(I.hi[a]) && (a == 0 || q[a] >= mesh_key_value(I.lo[a]));
   }
-  int wind = 0;
-  bool unsure = false;
-  uint64_t todo = 0;
-  int level = T.levels - 1;
-  uint32_t group = 0;
-  bool enter = true;
-  while (true) {
-    if (enter) {
-      const float4* b = reinterpret_cast<const float4*>(T.box[level] + (size_t)group * 48u);
-      uint32_t m = 0;
-      float lo[3][8], hi[3][8];
+  double where = 0.0;
+  for (uint64_t m = __ballot(meets); m != 0ull; m &= m - 1ull) {
+    const int who = __ffsll((unsigned long long)m) - 1;
+    const double p[3] = {__shfl(q[0], who), __shfl(q[1], who), __shfl(q[2], who)};
+    int wind = 0;
+    bool unsure = false;
+    ray_boxes(T, __double2float_rd(p[0]), __double2float_rd(p[1]), __double2float_ru(p[1]),
+              __double2float_rd(p[2]), __double2float_ru(p[2]), [&](bool in, uint32_t t) {
+                int cover = 0, side = 0;
+                if (in) {
+                  double c[9];
 #pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        const float4 l0 = b[2 * a], l1 = b[2 * a + 1], h0 = b[6 + 2 * a], h1 = b[7 + 2 * a];
-        const float l[8] = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
-        const float h[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          lo[a][u] = l[u];
-          hi[a][u] = h[u];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (hi[0][u] >= qlo[0] && lo[1][u] <= qhi[1] && hi[1][u] >= qlo[1] &&
-            lo[2][u] <= qhi[2] && hi[2][u] >= qlo[2] && group * 8u + (uint32_t)u < T.count[level])
-          m |= 1u << u;
-      todo = (todo & ~(0xffull << (8 * level))) | ((uint64_t)m << (8 * level));
-      enter = false;
-    }
-    const uint32_t m = (uint32_t)(todo >> (8 * level)) & 0xffu;
-    if (m == 0u) {
-      if (++level == T.levels) break;
-      group >>= 3;
-      continue;
-    }
-    const uint32_t child = group * 8u + (uint32_t)(__ffs((int)m) - 1);
-    todo &= ~(1ull << (8 * level + (__ffs((int)m) - 1)));
-    if (level > 0) {
-      group = child;
-      --level;
-      enter = true;
-      continue;
-    }
-    const TreeTri& R = T.tri[child];
-    double v[9];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) v[k] = R.v[k];
-    const int cover = ray_cover(q[1], q[2], v, v + 3, v + 6);
-    if (cover != 0) {
-      const int side = plane_side(q, v, v + 3, v + 6);
-      if (side == cover) wind += cover;
-      unsure = unsure || side == 0;
-    }
+                  for (int j = 0; j < 9; ++j) c[j] = T.tri[t].v[j];
+                  cover = ray_cover(p[1], p[2], c, c + 3, c + 6);
+                  if (cover != 0) side = plane_side(p, c, c + 3, c + 6);
+                }
+                wind += (int)__popcll(__ballot(cover == 1 && side == 1)) -
+                        (int)__popcll(__ballot(cover == -1 && side == -1));
+                unsure = unsure || __ballot(cover != 0 && side == 0) != 0ull;
+              });
+    if (lane == who) where = unsure ? 2.0 : (wind > 0 ? 1.0 : 0.0);
   }
-  return unsure ? 2 : (wind > 0 ? 1 : 0);
+  if (valid) sdf[v] = where;
 }
 
-// A wave takes a 4 x 4 x 4 block of lattice vertices, whose searches visit
-// mostly the same boxes.
-__global__ __launch_bounds__(kLanes) void k_tree_lattice(
+// A wave takes a 4 x 4 x 4 block of lattice vertices (4 x 4 x 2 and 4 x 4 x 1:
+// 664 and 899 us a build against 626).
+__global__ __launch_bounds__(kLanes, kTreeWavesPerSimd) void k_tree_lattice(
     MeshTree T, const double* __restrict__ verts, uint32_t nv, const uint32_t* __restrict__ tris,
     uint32_t nt, int nx, int ny, int nz, int kx, int ky, double bx, double by, double bz,
     double cs, float4* __restrict__ cpd, float4* __restrict__ nrm) {
-  extern __shared__ float s_mem[];
+  __shared__ TreeShared S;
   const MeshInfo I = *T.info;
   if (!mesh_closed(I)) return;
   const uint32_t b = blockIdx.x;
   const int ix = (int)(b % (uint32_t)kx) * 4 + (int)(threadIdx.x & 3u);
   const int iy = (int)(b / (uint32_t)kx % (uint32_t)ky) * 4 + (int)((threadIdx.x >> 2) & 3u);
-  const int iz = (int)(b / ((uint32_t)kx * (uint32_t)ky)) * 4 + (int)(threadIdx.x >> 4);
+  const int iz =
+      (int)(b / ((uint32_t)kx * (uint32_t)ky)) * 4 + (int)(threadIdx.x >> 4);
   const bool valid = ix < nx && iy < ny && iz < nz;
   const size_t v = valid ? ((size_t)iz * ny + iy) * nx + ix : 0;
   const double q[3] = {bx + (double)ix * cs, by + (double)iy * cs, bz + (double)iz * cs};
   const double delta = rounding_margin(I, q);
+  // lane 21 is the block's vertex (1, 1, 1); lane 0 is always a vertex
+  const int centre = ((__ballot(valid) >> 21) & 1ull) != 0ull ? 21 : 0;
   Nearest r;
-  r.d2 = DBL_MAX;
-  float where = 0.0f;
-  if (valid) {
-    where = nrm[v].w;
-    r = tree_nearest(T, q, delta, reinterpret_cast<float(*)[8][kLanes]>(s_mem));
-  }
+  tree_nearest(T, q, delta, valid, centre, kLanes, S, r);
+  const float where = valid ? nrm[v].w : 0.0f;
   const double dist = sqrt(r.d2);
   bool inside = where == 1.0f;
   const bool need = valid && (where == 2.0f || dist <= delta);
@@ -544,31 +700,56 @@ __global__ __launch_bounds__(kLanes) void k_tree_lattice(
                        0.0f);
 }
 
-__global__ __launch_bounds__(kLanes) void k_tree_points(
+// Free points are taken in the Morton order of their places in three times
+// the mesh's box (any order gives the same results; a wave's points should
+// be neighbours).
+__global__ __launch_bounds__(kBlock) void k_point_morton(const double* __restrict__ pts,
+                                                         uint32_t n,
+                                                         const MeshInfo* __restrict__ I,
+                                                         uint32_t* __restrict__ keys) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  uint32_t key = 0;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const double lo = mesh_key_value(I->lo[a]), hi = mesh_key_value(I->hi[a]), ext = hi - lo;
+    const double u = (pts[3 * (size_t)i + a] - (lo - ext)) / (3.0 * ext) * 256.0;
+    key |= spread3((uint32_t)fmin(fmax(u, 0.0), 255.0)) << a;  // (a NaN reads 0)
+  }
+  keys[i] = key;
+}
+
+__global__ __launch_bounds__(kLanes, kTreeWavesPerSimd) void k_tree_points(
     MeshTree T, const double* __restrict__ verts, uint32_t nv, const uint32_t* __restrict__ tris,
-    uint32_t nt, const double* __restrict__ pts, uint64_t np, double* __restrict__ sdf,
-    double* __restrict__ cp) {
-  extern __shared__ float s_mem[];
+    uint32_t nt, const double* __restrict__ pts, uint32_t n, const uint32_t* __restrict__ order,
+    uint32_t perWave, double* __restrict__ sdf, double* __restrict__ cp) {
+  __shared__ TreeShared S;
   const MeshInfo I = *T.info;
   if (!mesh_closed(I)) return;
-  const uint64_t v = (uint64_t)blockIdx.x * kLanes + threadIdx.x;
-  const bool valid = v < np;
+  const uint32_t k = blockIdx.x * perWave + threadIdx.x;
+  const bool valid = threadIdx.x < perWave && k < n;
+  const size_t v = valid ? order[k] : 0;
   double q[3] = {0.0, 0.0, 0.0};
-  Nearest r;
-  r.d2 = DBL_MAX;
-  int where = 0;
+  bool finite = valid;
   if (valid) {
 #pragma unroll
-    for (int a = 0; a < 3; ++a) q[a] = pts[3 * v + a];
+    for (int a = 0; a < 3; ++a) {
+      q[a] = pts[3 * v + a];
+      finite = finite && fabs(q[a]) <= kTreeRange;
+    }
   }
   const double delta = rounding_margin(I, q);
-  if (valid) {
-    r = tree_nearest(T, q, delta, reinterpret_cast<float(*)[8][kLanes]>(s_mem));
-    where = tree_inside(T, q);
-  }
+  const uint64_t on = __ballot(finite);
+  const int mid = (int)(perWave / 2);
+  const int centre =
+      ((on >> mid) & 1ull) != 0ull || on == 0ull ? mid : __ffsll((unsigned long long)on) - 1;
+  Nearest r;
+  if (on != 0ull) tree_nearest(T, q, delta, finite, centre, perWave, S, r);
+  brute_nearest(valid && !finite, q, verts, nv, tris, nt, r);
+  const double where = valid ? sdf[v] : 0.0;
   const double dist = sqrt(r.d2);
-  bool inside = where == 1;
-  const bool need = valid && (where == 2 || dist <= delta);
+  bool inside = where == 1.0;
+  const bool need = valid && (where == 2.0 || dist <= delta);
   const double w = winding_sum(need, q, verts, nv, tris, nt);
   if (need) inside = winds(w);
   if (!valid) return;
@@ -598,15 +779,18 @@ size_t tree_levels(uint32_t nt, uint32_t count[kTreeMaxLevels], int* levels) {
 
 }  // namespace
 
-// The brute force costs about 7.7 ps per point-triangle pair at full load;
-// the tree's build and its searches' fixed cost are about 100 us.  Below
-// 256 triangles the tree has two levels and saves little.
+// The brute force costs 1.1 us a triangle however few the points (a wave
+// walks all of them) and 7.7 ps a pair at full load; the tree's build and its
+// searches' fixed cost are about 110 us.
 bool mesh_tree_pays(uint32_t nt, uint64_t npts) {
-  return nt >= 256u && nt <= (1u << 22) && npts < (1ull << 31) &&
-         npts * (uint64_t)nt >= (1ull << 24);
+  return nt >= 128u && nt <= (1u << 22) && npts < (1ull << 31);
 }
 
-bool tree_lattice_fits(const int cells[3]) {
+bool tree_lattice_fits(const int cells[3], const double bmin[3], double cs) {
+  for (int a = 0; a < 3; ++a) {
+    const double lo = bmin[a], hi = bmin[a] + (double)cells[a] * cs;
+    if (!(lo >= -kTreeRange && lo <= kTreeRange && hi <= kTreeRange)) return false;
+  }
   const uint64_t nx = (uint64_t)cells[0] + 1, ny = (uint64_t)cells[1] + 1,
                  nz = (uint64_t)cells[2] + 1;
   // threads of one launch dimension stay below 2^32
@@ -677,18 +861,50 @@ hipError_t launch_tree_lattice(hipStream_t s, const MeshTree& T, const double* v
                      dim3(kLanes), 0, s, T, nx, ny, bmin[0], bmin[1], bmin[2], cs, nrm);
   const int kx = (nx + 3) / 4, ky = (ny + 3) / 4, kz = (nz + 3) / 4;
   hipLaunchKernelGGL(k_tree_lattice, dim3((unsigned)kx * (unsigned)ky * (unsigned)kz),
-                     dim3(kLanes), (size_t)T.levels * 8 * kLanes * sizeof(float), s, T, verts, nv,
-                     tris, nt, nx, ny, nz, kx, ky, bmin[0], bmin[1], bmin[2], cs, cpd, nrm);
+                     dim3(kLanes), 0, s, T, verts, nv, tris, nt, nx, ny, nz, kx, ky, bmin[0],
+                     bmin[1], bmin[2], cs, cpd, nrm);
   return hipGetLastError();
 }
 
-hipError_t launch_tree_points(hipStream_t s, const MeshTree& T, const double* verts, uint32_t nv,
-                              const uint32_t* tris, uint32_t nt, const double* pts, uint64_t np,
-                              double* sdf, double* cp) {
-  hipLaunchKernelGGL(k_tree_points, dim3((unsigned)((np + kLanes - 1) / kLanes)), dim3(kLanes),
-                     (size_t)T.levels * 8 * kLanes * sizeof(float), s, T, verts, nv, tris, nt, pts,
-                     np, sdf, cp);
-  return hipGetLastError();
+size_t tree_points_bytes(uint64_t np) {
+  const uint64_t chunk = np < kPointChunk ? np : kPointChunk;
+  return 2 * align256((size_t)chunk * sizeof(uint32_t));
+}
+
+uint32_t tree_sort_pairs(uint32_t nt, uint64_t np) {
+  const uint64_t chunk = np < kPointChunk ? np : kPointChunk;
+  return chunk > nt ? (uint32_t)chunk : nt;
+}
+
+hipError_t launch_tree_points(fc_context* ctx, const MeshTree& T, const double* verts,
+                              uint32_t nv, const uint32_t* tris, uint32_t nt, const double* pts,
+                              uint64_t np, void* block, double* sdf, double* cp) {
+  hipStream_t s = ctx->stream;
+  const uint64_t chunk = np < kPointChunk ? np : kPointChunk;
+  uint32_t* keys = static_cast<uint32_t*>(block);
+  uint32_t* order =
+      reinterpret_cast<uint32_t*>(static_cast<char*>(block) + align256((size_t)chunk * 4));
+  for (uint64_t at = 0; at < np; at += chunk) {
+    const uint32_t n = (uint32_t)(np - at < chunk ? np - at : chunk);
+    const double* p = pts + 3 * at;
+    hipLaunchKernelGGL(k_point_morton, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, p, n,
+                       T.info, keys);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess)
+      e = radix_sort_pairs(s, ctx->sort, ctx->devFlags, keys, nullptr, keys, order, n,
+                           kMortonBits, nullptr);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_tree_signs, dim3((n + kRaysPerWave - 1) / kRaysPerWave), dim3(kLanes), 0,
+                       s, T, p, n, order, sdf + at);
+    uint32_t perWave = 8;
+    while (perWave < (uint32_t)kLanes && n / perWave > kPointWaves) perWave *= 2;
+    hipLaunchKernelGGL(k_tree_points, dim3((n + perWave - 1) / perWave), dim3(kLanes), 0, s, T,
+                       verts, nv, tris, nt, p, n, order, perWave, sdf + at,
+                       cp ? cp + 3 * at : nullptr);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace fc

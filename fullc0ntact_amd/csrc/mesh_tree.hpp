@@ -42,6 +42,10 @@ __device__ __forceinline__ double mesh_key_value(unsigned long long k) {
   return __longlong_as_double((long long)u);
 }
 
+// The tree's boxes are compared in binary32: squared distances of points and
+// meshes within this range stay in its range.
+constexpr double kTreeRange = 1e15;
+
 // Largest corner coordinate by magnitude.
 __device__ __forceinline__ double mesh_magnitude(const MeshInfo& I) {
   double m = 0.0;
@@ -53,18 +57,19 @@ __device__ __forceinline__ double mesh_magnitude(const MeshInfo& I) {
 
 // Whether the tree's signs hold: the mesh is closed and consistently
 // oriented (every directed edge matched by its opposite, by two 64-bit
-// sums), finite, and of a magnitude whose products stay in range.  The
+// sums), finite, and of a magnitude whose squares stay in range.  The
 // brute-force kernel takes the meshes for which it is false.
 __device__ __forceinline__ bool mesh_closed(const MeshInfo& I) {
   const double m = mesh_magnitude(I);
-  return I.bad == 0u && I.edges[0] == 0ull && I.edges[1] == 0ull && m < 1e60 && m > 1e-60;
+  return I.bad == 0u && I.edges[0] == 0ull && I.edges[1] == 0ull && m < kTreeRange &&
+         m > 1.0 / kTreeRange;
 }
 
-// Meshes of fewer triangles, and fewer point-triangle pairs, take the brute
-// force: see mesh_tree.hip.
+// Meshes of fewer triangles take the brute force: see mesh_tree.hip.
 bool mesh_tree_pays(uint32_t nt, uint64_t npts);
-// Whether the lattice's launches stay within the grid limits.
-bool tree_lattice_fits(const int cells[3]);
+// Whether the lattice's launches stay within the grid limits, and its
+// coordinates within kTreeRange.
+bool tree_lattice_fits(const int cells[3], const double bmin[3], double cs);
 // Device bytes the tree of nt triangles needs.
 size_t mesh_tree_bytes(uint32_t nt);
 // Builds the tree of the mesh (device arrays; triangle indices are clamped
@@ -77,8 +82,12 @@ hipError_t launch_mesh_tree(fc_context* ctx, const double* verts, uint32_t nv,
 hipError_t launch_tree_lattice(hipStream_t s, const MeshTree& T, const double* verts, uint32_t nv,
                                const uint32_t* tris, uint32_t nt, const int cells[3],
                                const double bmin[3], double cs, float4* cpd, float4* nrm);
-hipError_t launch_tree_points(hipStream_t s, const MeshTree& T, const double* verts, uint32_t nv,
-                              const uint32_t* tris, uint32_t nt, const double* pts, uint64_t np,
-                              double* sdf, double* cp);
+hipError_t launch_tree_points(fc_context* ctx, const MeshTree& T, const double* verts,
+                              uint32_t nv, const uint32_t* tris, uint32_t nt, const double* pts,
+                              uint64_t np, void* block, double* sdf, double* cp);
+// Device bytes the free points' order needs in `block`, and the pairs the
+// context's sort scratch must hold for a mesh and its points.
+size_t tree_points_bytes(uint64_t np);
+uint32_t tree_sort_pairs(uint32_t nt, uint64_t np);
 
 }  // namespace fc
