@@ -296,19 +296,19 @@ unsigned sdf_blocks(uint64_t npts) {
   return g < kSdfMaxBlocks ? g : kSdfMaxBlocks;
 }
 
-// The tree's scratch, grown to the largest mesh the context has seen (about
-// 130 bytes a triangle, 8 more per point up to 2^22); false when there is no memory for it, or inside a
-// graph capture, where it could not grow.  The callers then take the brute
-// force alone.
-bool tree_scratch(fc_context* ctx, uint32_t nt, uint32_t sorted, size_t extra) {
+// Grows the context's mesh scratch to `need` bytes (the tree: about 130 a
+// triangle, 8 more per free point up to 2^22; a builder's copy of its mesh)
+// and its sort scratch to `sorted` pairs.  False when there is no memory, or
+// inside a graph capture, where they could not grow.  The callers then take
+// the brute force alone.
+bool tree_scratch(fc_context* ctx, uint32_t sorted, size_t need) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
     return false;
-  if (ensure_sort_capacity(ctx, sorted) != FC_SUCCESS) {
+  if (sorted > 0 && ensure_sort_capacity(ctx, sorted) != FC_SUCCESS) {
     (void)hipGetLastError();
     return false;
   }
-  const size_t need = mesh_tree_bytes(nt) + extra;
   if (ctx->meshCapacity >= need) return true;
   if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
   (void)hipFree(ctx->meshScratch);
@@ -340,7 +340,7 @@ hipError_t launch_mesh_sdf_points(fc_context* ctx, const double* verts, uint32_t
   hipStream_t s = ctx->stream;
   MeshTree T;
   if (mesh_tree_pays(nt, np) &&
-      tree_scratch(ctx, nt, tree_sort_pairs(nt, np), tree_points_bytes(np))) {
+      tree_scratch(ctx, tree_sort_pairs(nt, np), mesh_tree_bytes(nt) + tree_points_bytes(np))) {
     hipError_t e = launch_mesh_tree(ctx, verts, nv, tris, nt, ctx->meshScratch, &T);
     if (e == hipSuccess)
       e = launch_tree_points(ctx, T, verts, nv, tris, nt, pts, np,
@@ -362,6 +362,7 @@ struct fc_distmap {
   float cellSize = 0.0f;
   float bmin[3] = {0, 0, 0};
   float bmax[3] = {0, 0, 0};
+  void* block = nullptr;  // the allocation that the arrays below lie in
   float* xs = nullptr;
   float* ys = nullptr;
   float* zs = nullptr;
@@ -460,6 +461,23 @@ DistMapView distmap_view(const fc_distmap* m) {
 
 namespace {
 
+// Where the coordinates of axis a start in the map's allocation, in floats
+// (a = 3: their end).
+size_t axis_offset(const fc_distmap* m, int a) {
+  size_t at = 0;
+  for (int k = 0; k < a; ++k) at += ((size_t)m->cells[k] + 1 + 63) / 64 * 64;
+  return at;
+}
+
+// Uploads the lattice coordinates of the three axes in one copy.
+hipError_t upload_axes(fc_distmap* m, const std::vector<float> ax[3], hipStream_t s) {
+  std::vector<float> host(axis_offset(m, 3), 0.0f);
+  for (int a = 0; a < 3; ++a) std::copy(ax[a].begin(), ax[a].end(), host.begin() + axis_offset(m, a));
+  hipError_t e = hipMemcpyAsync(m->block, host.data(), host.size() * sizeof(float),
+                                hipMemcpyHostToDevice, s);
+  return e == hipSuccess ? hipStreamSynchronize(s) : e;
+}
+
 fc_status alloc_map(fc_context* ctx, const int32_t cells[3], fc_distmap** out) {
   for (int a = 0; a < 3; ++a)
     if (cells[a] < 1) return set_error(FC_ERROR_INVALID_VALUE, "cells must be >= 1 per axis");
@@ -469,11 +487,17 @@ fc_status alloc_map(fc_context* ctx, const int32_t cells[3], fc_distmap** out) {
   m->ctx = ctx;
   for (int a = 0; a < 3; ++a) m->cells[a] = cells[a];
   m->V = V;
-  hipError_t e = hipMalloc(&m->xs, (cells[0] + 1) * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&m->ys, (cells[1] + 1) * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&m->zs, (cells[2] + 1) * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&m->cpd, V * sizeof(float4));
-  if (e == hipSuccess) e = hipMalloc(&m->nrm, V * sizeof(float4));
+  // one allocation: the axes (map_axes' layout), then the vertices' arrays
+  const size_t axes = axis_offset(m, 3);
+  const hipError_t e = hipMalloc(&m->block, axes * sizeof(float) + 2 * V * sizeof(float4));
+  if (e == hipSuccess) {
+    float* at = static_cast<float*>(m->block);
+    m->xs = at;
+    m->ys = at + axis_offset(m, 1);
+    m->zs = at + axis_offset(m, 2);
+    m->cpd = reinterpret_cast<float4*>(at + axes);
+    m->nrm = m->cpd + V;
+  }
   if (e != hipSuccess) {
     fc_distmap_destroy(m);
     return hip_error(e, "distance map allocation");
@@ -720,7 +744,9 @@ fc_status fc_distmap_create(fc_context* ctx, const int32_t cells[3], float cellS
   FC_TRY(alloc_map(ctx, cells, &m));
   const int cx = cells[0], cy = cells[1], cz = cells[2];
   const size_t ix = cx + 1, islice = ix * (cy + 1), V = m->V;
-  std::vector<float> xs(cx + 1), ys(cy + 1), zs(cz + 1);
+  std::vector<float> ax[3] = {std::vector<float>(cx + 1), std::vector<float>(cy + 1),
+                              std::vector<float>(cz + 1)};
+  std::vector<float>&xs = ax[0], &ys = ax[1], &zs = ax[2];
   for (int i = 0; i <= cx; ++i) xs[i] = vertexCoords[3 * i];
   for (int i = 0; i <= cy; ++i) ys[i] = vertexCoords[3 * (i * ix) + 1];
   for (int i = 0; i <= cz; ++i) zs[i] = vertexCoords[3 * (i * islice) + 2];
@@ -743,9 +769,7 @@ fc_status fc_distmap_create(fc_context* ctx, const int32_t cells[3], float cellS
     m->bmax[a] = bmax[a];
   }
   hipStream_t st = ctx->stream;
-  hipError_t e = hipMemcpyAsync(m->xs, xs.data(), xs.size() * 4, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(m->ys, ys.data(), ys.size() * 4, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(m->zs, zs.data(), zs.size() * 4, hipMemcpyHostToDevice, st);
+  hipError_t e = upload_axes(m, ax, st);
   if (e == hipSuccess) e = hipMemcpyAsync(m->cpd, cpd.data(), V * 16, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipMemcpyAsync(m->nrm, nrm.data(), V * 16, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -782,20 +806,23 @@ fc_status fc_distmap_build(fc_context* ctx, const double* vertices, uint32_t num
   }
   m->cellSize = cellSize;
   hipStream_t st = ctx->stream;
-  double* dv = nullptr;
-  uint32_t* dt = nullptr;
-  hipError_t e = hipMalloc(&dv, (size_t)numVertices * 3 * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&dt, (size_t)numTriangles * 3 * sizeof(uint32_t));
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(dv, vertices, (size_t)numVertices * 24, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(dt, triangles, (size_t)numTriangles * 12, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(m->xs, ax[0].data(), ax[0].size() * 4, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(m->ys, ax[1].data(), ax[1].size() * 4, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(m->zs, ax[2].data(), ax[2].size() * 4, hipMemcpyHostToDevice, st);
+  // the mesh's copy lies in the context's scratch, after the tree
+  const size_t vb = (size_t)numVertices * 3 * sizeof(double),
+               tb = (size_t)numTriangles * 3 * sizeof(uint32_t);
+  const bool tree = mesh_tree_pays(numTriangles, m->V) && tree_lattice_fits(cells, b, cs);
+  const size_t at = tree ? mesh_tree_bytes(numTriangles) : 0;
+  hipError_t e = hipSuccess;
+  void* own = nullptr;
+  const bool kept = tree_scratch(ctx, tree ? numTriangles : 0, at + vb + tb);
+  if (!kept) e = hipMalloc(&own, vb + tb);
+  double* dv = reinterpret_cast<double*>(kept ? static_cast<char*>(ctx->meshScratch) + at
+                                              : static_cast<char*>(own));
+  uint32_t* dt = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(dv) + vb);
+  if (e == hipSuccess) e = hipMemcpyAsync(dv, vertices, vb, hipMemcpyHostToDevice, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(dt, triangles, tb, hipMemcpyHostToDevice, st);
+  if (e == hipSuccess) e = upload_axes(m, ax, st);
   MeshTree T;
-  if (e == hipSuccess && mesh_tree_pays(numTriangles, m->V) && tree_lattice_fits(cells, b, cs) &&
-      tree_scratch(ctx, numTriangles, numTriangles, 0)) {
+  if (e == hipSuccess && tree && kept) {
     e = launch_mesh_tree(ctx, dv, numVertices, dt, numTriangles, ctx->meshScratch, &T);
     if (e == hipSuccess)
       e = launch_tree_lattice(st, T, dv, numVertices, dt, numTriangles, m->cells, b, cs, m->cpd,
@@ -808,8 +835,7 @@ fc_status fc_distmap_build(fc_context* ctx, const double* vertices, uint32_t num
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);
-  hipFree(dv);
-  hipFree(dt);
+  hipFree(own);
   if (e != hipSuccess) {
     fc_distmap_destroy(m);
     return hip_error(e, "distance map build");
@@ -822,11 +848,7 @@ fc_status fc_distmap_destroy(fc_distmap* m) {
   if (!m) return FC_SUCCESS;
   // No use of m->ctx: the context may already be gone; hipFree waits for
   // the device.
-  hipFree(m->xs);
-  hipFree(m->ys);
-  hipFree(m->zs);
-  hipFree(m->cpd);
-  hipFree(m->nrm);
+  hipFree(m->block);
   delete m;
   return FC_SUCCESS;
 }
