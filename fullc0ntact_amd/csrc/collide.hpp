@@ -573,14 +573,20 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
   return force;
 }
 
+// Candidates per round of collide_row_cells.
+#ifndef FC_ROW_BATCH
+#define FC_ROW_BATCH 4
+#endif
+constexpr int kRowBatch = FC_ROW_BATCH;
+
 // One neighbour row of collide_one_rows for the row-split collide of small
 // systems, where nine lanes share a sphere (row r = 3 (dz + 1) + (dy + 1)):
 // the partial force sums of the row's three cells (dx = -1, 0, 1), each in
 // index order from +0, with every candidate through the exact pair force
 // (non-touching ones add +0).  Cells out of contact reach are cut as in
 // collide_one_rows (their partials stay +0, which is what the reference
-// adds for them); the cells are walked one by one, so a row that wraps in x
-// needs no special case.  Requires every grid dimension >= 4.
+// adds for them); each cell has its own range, so a row that wraps in x needs
+// no special case.  Requires every grid dimension >= 4.
 template <bool kPoly>
 __device__ __forceinline__ void collide_row_cells(const fc_sim_params& P, v3f invCell,
                                                   float contactD2, uint32_t k, v3f pos, v3f vel,
@@ -618,25 +624,42 @@ __device__ __forceinline__ void collide_row_cells(const fc_sim_params& P, v3f in
   const float gyz = (dy < 0 ? ly * ly : (dy > 0 ? hy * hy : 0.0f)) +
                     (dz < 0 ? lz * lz : (dz > 0 ? hz * hz : 0.0f));
   const bool keep[3] = {!(gyz + lx * lx >= thrCut), !(gyz >= thrCut), !(gyz + hx * hx >= thrCut)};
+  // The three cells as one sequence, kRowBatch candidates a round with their
+  // loads in flight together: a row of three cells holds three to seven
+  // spheres, and walked cell by cell, two at a time, it took up to six
+  // dependent rounds where this takes one or two.
+  uint32_t len[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    cf[c] = make_v3(0.0f, 0.0f, 0.0f);
-    if (st[c] == CELL_EMPTY || !keep[c]) continue;
     const uint32_t e = en[c] > n ? n : en[c];
+    len[c] = st[c] == CELL_EMPTY || !keep[c] || e < st[c] ? 0u : e - st[c];
+    cf[c] = make_v3(0.0f, 0.0f, 0.0f);
+  }
+  const uint32_t b1 = len[0], b2 = b1 + len[1], total = b2 + len[2];
+  const uint32_t q1 = st[1] - b1, q2 = st[2] - b2;  // modulo 2^32
 #pragma unroll 1
-    for (uint32_t j0 = st[c]; j0 < e; j0 += 2) {
-      const uint32_t j1 = j0 + 1u < e ? j0 + 1u : j0;
-      const float4 p0 = sortedPos[j0], p1 = sortedPos[j1];
-      const float4 v0 = sortedVel[j0], v1 = sortedVel[j1];
-      if (j0 != k) {
-        const v3f f = collide_spheres_fast(pos, xyz(p0), vel, xyz(v0), rA, kPoly ? p0.w : rA,
-                                           P.spring, P.damping, P.shear, P.attraction);
-        cf[c] = make_v3(cf[c].x + f.x, cf[c].y + f.y, cf[c].z + f.z);
-      }
-      if (j0 + 1u < e && j1 != k) {
-        const v3f f = collide_spheres_fast(pos, xyz(p1), vel, xyz(v1), rA, kPoly ? p1.w : rA,
-                                           P.spring, P.damping, P.shear, P.attraction);
-        cf[c] = make_v3(cf[c].x + f.x, cf[c].y + f.y, cf[c].z + f.z);
+  for (uint32_t t = 0; t < total; t += kRowBatch) {
+    float4 pj[kRowBatch], vj[kRowBatch];
+    uint32_t jj[kRowBatch];
+#pragma unroll
+    for (int u = 0; u < kRowBatch; ++u) {
+      // (slots past the end read the sphere itself, which is left out)
+      const uint32_t tu = t + (uint32_t)u;
+      jj[u] = tu >= total ? k : tu + (tu < b1 ? st[0] : (tu < b2 ? q1 : q2));
+      pj[u] = sortedPos[jj[u]];
+      vj[u] = sortedVel[jj[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < kRowBatch; ++u) {
+      if (jj[u] != k) {
+        const uint32_t tu = t + (uint32_t)u;
+        const v3f f = collide_spheres_fast(pos, xyz(pj[u]), vel, xyz(vj[u]), rA,
+                                           kPoly ? pj[u].w : rA, P.spring, P.damping, P.shear,
+                                           P.attraction);
+        const int c = tu < b1 ? 0 : (tu < b2 ? 1 : 2);
+#pragma unroll
+        for (int x = 0; x < 3; ++x)
+          if (c == x) cf[x] = make_v3(cf[x].x + f.x, cf[x].y + f.y, cf[x].z + f.z);
       }
     }
   }

@@ -152,6 +152,33 @@ __global__ __launch_bounds__(kBlock) void k_integrate_hash(
   histogram_flush(s_hist, gHist, 0);
 }
 
+// k_integrate_hash for systems whose sort counts ranks (launch_sort_small) and
+// reads no digit histogram: one sphere per thread over many small blocks, no
+// LDS, no atomics.  Bound by one round of loads; with the histogram (whose
+// first block also clears 48 KB of it) 1331 spheres took 8.3 us, this 2.9.
+constexpr int kSmallBlock = 64;
+
+__global__ __launch_bounds__(kSmallBlock) void k_integrate_hash_small(
+    fc_sim_params P, BoundaryArg B, float4* __restrict__ pos, float4* __restrict__ vel, float dt,
+    uint32_t* __restrict__ keysOut, const uint32_t* __restrict__ prevSortedHash,
+    uint32_t* __restrict__ cellStart, uint32_t* __restrict__ cellEnd, uint32_t n) {
+  const uint32_t i = blockIdx.x * kSmallBlock + threadIdx.x;
+  if (i >= n) return;
+  const float4 p4 = pos[i], v4 = vel[i];
+  if (prevSortedHash != nullptr) {
+    const uint32_t h = prevSortedHash[i];
+    if (i == 0 || prevSortedHash[i - 1] != h) {
+      cellStart[h] = CELL_EMPTY;
+      cellEnd[h] = CELL_EMPTY;
+    }
+  }
+  v3f p = xyz(p4), v = xyz(v4);
+  integrate_with(P, B, p4.w, dt, p, v);
+  pos[i] = make_float4(p.x, p.y, p.z, p4.w);
+  vel[i] = make_float4(v.x, v.y, v.z, v4.w);
+  keysOut[i] = hash_of(P, p.x, p.y, p.z);
+}
+
 // reorderDataAndFindCellStartD (particles_kernel.cu:119-182).  The
 // neighbour's hash comes from the previous lane through a cross-lane
 // shuffle; lane 0 of each wave reads it from memory.
@@ -380,8 +407,9 @@ __global__ __launch_bounds__(kBlock, kCollideWavesPerSimd) void k_collide_v3(
   const uint32_t k = xcd_grouped_block(blockIdx.x, gridDim.x, xcdGroup) * kBlock + threadIdx.x;
   const bool valid = k < n;
   // rows.rowHist: the next sort is a row resort, which takes per-row counts
-  // instead of the radix digit histogram (the same for every block)
-  const bool digitHist = kFuse && rows.rowHist == nullptr;
+  // instead of the radix digit histogram; without either, it counts ranks
+  // (up to RS_TILE spheres); the same for every block
+  const bool digitHist = kFuse && rows.rowHist == nullptr && gHist != nullptr;
   if (digitHist) {
     for (int i = threadIdx.x; i < RS_RADIX; i += kBlock) s_hist[i] = 0u;
     histogram_producer_prologue(gHist, passes, counters);
@@ -414,7 +442,7 @@ __global__ __launch_bounds__(kBlock, kCollideWavesPerSimd) void k_collide_v3(
     histogram_add_digit(s_hist, key & (RS_RADIX - 1), valid && !left);
     __syncthreads();
     histogram_flush(s_hist, gHist, 0);
-  } else if (kFuse) {
+  } else if (kFuse && rows.rowHist != nullptr) {
     row_histograms(rows, k, key, oldKey, valid && !left);
   }
 }
@@ -528,7 +556,7 @@ __global__ __launch_bounds__(kBlock) void k_collide_piles(
         const uint32_t r = key >> rows.shift, at = r * kRowCopies + row_copy(k);
         atomicAdd(&rows.rowHist[at], 1u);
         if (r != (oldKey >> rows.shift)) atomicAdd(&rows.chgHist[at], 1u);
-      } else if (kFuse) {
+      } else if (kFuse && gHist != nullptr) {
         atomicAdd(&hist_buffer(gHist, 0)[(blockIdx.x % RS_HIST_COPIES) * RS_RADIX +
                                          (key & (RS_RADIX - 1))],
                   1u);
@@ -548,9 +576,9 @@ __global__ __launch_bounds__(kBlock) void k_collide_piles(
 // k_collide_v3 is then bound by the latency of its chain of dependent
 // loads, not by throughput), with each sphere's nine neighbour rows on nine
 // lanes of a wave (collide_row_cells: seven spheres per wave, lane 63
-// idle).  The row-0 lane gathers the other rows' cell partials by lane
-// shuffles and adds the 27 in the reference order (z, then y, then x), then
-// the cursor sphere; the rest is k_collide_v3's tail (the scatter, or with
+// idle).  Three of its lanes add the rows' 27 cell partials in the reference
+// order (z, then y, then x), a component each, then the row-0 lane the cursor
+// sphere; the rest is k_collide_v3's tail (the scatter, or with
 // kFuse the next update's integrate, hash and histogram), with the same
 // arguments and results.
 constexpr int kSplitSpheresPerWave = 7;
@@ -565,12 +593,13 @@ __global__ __launch_bounds__(kBlock) void k_collide_split(
     uint32_t* devFlags, uint32_t* __restrict__ slotOf, uint32_t* __restrict__ idOfSlot,
     v3f invCell, float* __restrict__ forceOut) {
   __shared__ uint32_t s_hist[kFuse ? RS_RADIX : 1];
+  __shared__ float s_cells[kBlock / 64][9 * 64];
   const int lane = (int)(threadIdx.x & 63u);
   const uint32_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
   const int sl = lane / 9, r = lane - 9 * (lane / 9);
   const uint32_t k = wave * kSplitSpheresPerWave + (uint32_t)sl;
   const bool valid = lane < 9 * kSplitSpheresPerWave && k < n;
-  if (kFuse) {
+  if (kFuse && gHist != nullptr) {
     for (int i = threadIdx.x; i < RS_RADIX; i += kBlock) s_hist[i] = 0u;
     histogram_producer_prologue(gHist, passes, counters);
   }
@@ -578,8 +607,10 @@ __global__ __launch_bounds__(kBlock) void k_collide_split(
   float4 p4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   v3f vel0 = make_v3(0.0f, 0.0f, 0.0f);
   float rA = P.particleRadius;
+  uint32_t orig = 0;  // (read with the state: a round trip less at the end)
   if (valid) {
     p4 = sortedPos[k];
+    orig = index[k];
     vel0 = xyz(sortedVel[k]);
     rA = kPoly ? p4.w : P.particleRadius;
     collide_row_cells<kPoly>(P, invCell, contactD2, k, xyz(p4), vel0, rA, r, sortedPos,
@@ -588,26 +619,32 @@ __global__ __launch_bounds__(kBlock) void k_collide_split(
 #pragma unroll
     for (int c = 0; c < 3; ++c) cf[c] = make_v3(0.0f, 0.0f, 0.0f);
   }
-  // the row-0 lane of each sphere adds the 27 cell partials in order
+  // lanes 0-2 of each sphere add the 27 cell partials in order, a component
+  // each (through LDS: lane shuffles would take 81 and as many adds)
   const int base = 9 * sl;
-  v3f force = make_v3(0.0f, 0.0f, 0.0f);
+  float* cells = s_cells[threadIdx.x >> 6];
 #pragma unroll
-  for (int rr = 0; rr < 9; ++rr) {
-    const int src = base + rr < 64 ? base + rr : 63;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const float x = __shfl(cf[c].x, src), y = __shfl(cf[c].y, src), z = __shfl(cf[c].z, src);
-      force = make_v3(force.x + x, force.y + y, force.z + z);
-    }
+  for (int c = 0; c < 3; ++c) {
+    cells[9 * lane + 3 * c] = cf[c].x;
+    cells[9 * lane + 3 * c + 1] = cf[c].y;
+    cells[9 * lane + 3 * c + 2] = cf[c].z;
   }
+  __builtin_amdgcn_wave_barrier();
+  float sum = 0.0f;
+  if (r < 3 && lane < 9 * kSplitSpheresPerWave) {
+#pragma unroll
+    for (int c = 0; c < 27; ++c) sum += cells[9 * base + 3 * c + r];
+  }
+  const v3f force = make_v3(sum, __shfl(sum, base + 1 < 64 ? base + 1 : 63),
+                            __shfl(sum, base + 2 < 64 ? base + 2 : 63));
   uint32_t key = 0;
   const bool owner = valid && r == 0;
   if (owner) {
     if (kPoly && !(rA <= P.particleRadius)) atomicOr(devFlags, DEVERR_RADIUS);
-    key = collide_finish<kFuse>(P, B, p4, xyz(p4), vel0, rA, force, k, index[k], newVel, pos, dt,
+    key = collide_finish<kFuse>(P, B, p4, xyz(p4), vel0, rA, force, k, orig, newVel, pos, dt,
                                 invCell, 0u, keysOut, slotOf, idOfSlot, false, forceOut);
   }
-  if (kFuse) {
+  if (kFuse && gHist != nullptr) {
     __syncthreads();
     histogram_add_digit(s_hist, key & (RS_RADIX - 1), owner);
     __syncthreads();
@@ -669,6 +706,11 @@ hipError_t launch_integrate_hash(hipStream_t s, const fc_sim_params& P, const Bo
                                  uint32_t* devFlags) {
   (void)devFlags;
   if (n == 0) return hipSuccess;
+  if (n <= (uint32_t)RS_TILE) {
+    hipLaunchKernelGGL(k_integrate_hash_small, dim3(grid_for(n, kSmallBlock)), dim3(kSmallBlock),
+                       0, s, P, B, pos, vel, dt, keysOut, prevSortedHash, cellStart, cellEnd, n);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_integrate_hash, dim3(grid_for(n, kBlock * kIhPer)), dim3(kBlock), 0, s, P, B,
                      pos, vel, dt, keysOut, prevSortedHash, cellStart, cellEnd, n, passes,
                      sort.histogram, sort.counters);
@@ -803,6 +845,8 @@ static void launch_v3(hipStream_t s, const GatheredState* gs, dim3 g, dim3 b,
                       uint32_t* devFlags, uint32_t* slotOf, uint32_t* idOfSlot,
                       float* forceOut = nullptr, bool slotKeys = false,
                       const RowHists* rows = nullptr) {
+  // up to RS_TILE spheres the next sort counts ranks: no digit histogram
+  if (n <= (uint32_t)RS_TILE) gHist = nullptr;
   // (the split kernel reads the reference layout only: no gathered arrays)
   if (rows_walk_ok(P) && n <= kSplitMaxSpheres) {
     const uint32_t waves = (n + kSplitSpheresPerWave - 1) / kSplitSpheresPerWave;

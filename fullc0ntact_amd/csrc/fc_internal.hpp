@@ -169,8 +169,9 @@ hipError_t radix_sort_pairs(hipStream_t stream, SortScratch& s, uint32_t* devFla
 // keys.  Bit-identical to radix_sort_pairs (with the same clearHash and
 // gather) followed by launch_cell_bounds, for keys below numCells (the
 // cells of a system, at most 8 * passes bits wide); inputs and outputs may
-// alias.  The digit-0 histogram of keysIn is not read; H[0] is zeroed for
-// the next sort.
+// alias.  There is no digit histogram: the kernels that write the keys of
+// such a sort (launch_integrate_hash and the fused collide of up to RS_TILE
+// spheres) leave the sort's histograms and epoch alone.
 hipError_t launch_sort_small(hipStream_t stream, SortScratch& s, const uint32_t* keysIn,
                              const uint32_t* valsIn, uint32_t* keysOut, uint32_t* valsOut,
                              uint32_t n, int passes, const uint32_t* clearHash,

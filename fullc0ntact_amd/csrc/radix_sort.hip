@@ -386,8 +386,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
 // a wave reads 64 consecutive words), with no exchange between blocks.  C packs (key << 12) | index, 32 bits wide when the keys' width
 // leaves 12 bits for the index, else 64.  The block also resets the cells
 // of its 16 entries of the previous sorted hashes (clearHash), which no
-// later write of this launch touches, and block 0 zeroes H[0] for the next
-// sort.  The sorted pairs go to keysStage/valsStage; k_small_emit writes
+// later write of this launch touches.  The sorted pairs go to keysStage/valsStage; k_small_emit writes
 // the outputs in a second launch, so that inputs and outputs may alias.
 constexpr uint32_t kRankLanes = 64;                  // lanes per key: one wave
 constexpr uint32_t kRankThreads = 1024;
@@ -399,13 +398,9 @@ __global__ __launch_bounds__(kRankThreads) void k_small_rank(
     const uint32_t* __restrict__ keysIn, const uint32_t* __restrict__ valsIn, uint32_t n,
     const uint32_t* __restrict__ clearHash, uint32_t* __restrict__ cellStart,
     uint32_t* __restrict__ cellEnd, uint32_t* __restrict__ keysStage,
-    uint32_t* __restrict__ valsStage, uint32_t* gHist) {
+    uint32_t* __restrict__ valsStage) {
   __shared__ C s_pair[RS_TILE];
   const uint32_t tid = threadIdx.x;
-  if (blockIdx.x == 0) {
-    uint32_t* h0 = hist_buffer(gHist, 0);
-    for (uint32_t i = tid; i < RS_HIST_COPIES * RS_RADIX; i += kRankThreads) h0[i] = 0u;
-  }
   if (clearHash != nullptr && tid < kRankKeys) {
     const uint32_t idx = blockIdx.x * kRankKeys + tid;
     if (idx < n) {
@@ -485,10 +480,10 @@ hipError_t launch_sort_small(hipStream_t stream, SortScratch& s, const uint32_t*
   const dim3 rankGrid((n + kRankKeys - 1) / kRankKeys);
   if (bits <= 20)
     hipLaunchKernelGGL(k_small_rank<uint32_t>, rankGrid, dim3(kRankThreads), 0, stream, keysIn,
-                       valsIn, n, clearHash, cellStart, cellEnd, s.keysA, s.valsA, s.histogram);
+                       valsIn, n, clearHash, cellStart, cellEnd, s.keysA, s.valsA);
   else
     hipLaunchKernelGGL(k_small_rank<uint64_t>, rankGrid, dim3(kRankThreads), 0, stream, keysIn,
-                       valsIn, n, clearHash, cellStart, cellEnd, s.keysA, s.valsA, s.histogram);
+                       valsIn, n, clearHash, cellStart, cellEnd, s.keysA, s.valsA);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_small_emit, dim3((n + 63) / 64), dim3(64), 0, stream, s.keysA, s.valsA,
