@@ -19,10 +19,10 @@
 //    plane, the brute force's own sum of solid angles is taken, in its
 //    order.  Other meshes stay with the brute force (mesh_closed).
 //
-// Layout: triangles sorted by the Morton code of their centroids, eight
-// consecutive ones to a group, groups of groups above; no topology to build
-// and no pointers, and a node's eight child boxes are 192 consecutive bytes,
-// so one visit is twelve 16-byte loads in flight together (the traversal is
+// Layout: triangles sorted along a Hilbert curve through their centroids,
+// eight consecutive ones to a group, groups of groups above; no topology to
+// build and no pointers, and a node's eight child boxes are 192 consecutive
+// bytes, so one visit is twelve 16-byte loads in flight together (the traversal is
 // a chain of dependent loads; wide nodes make it short).
 #include "mesh_tree.hpp"
 
@@ -135,17 +135,42 @@ __global__ __launch_bounds__(kBlock) void k_mesh_info(const double* __restrict__
   }
 }
 
-// The low 8 bits of x, spread to every third bit.
-__device__ __forceinline__ uint32_t spread3(uint32_t x) {
-  x &= 0xffu;
-  x = (x | (x << 8)) & 0x00f00fu;
-  x = (x | (x << 4)) & 0x0c30c3u;
-  return (x | (x << 2)) & 0x249249u;
+// Place of a cell of a 256^3 grid along a Hilbert curve, by the coordinate
+// transform of J. Skilling, "Programming the Hilbert curve" (AIP Conference
+// Proceedings 707, 2004).  Neighbours along the curve are neighbours in space;
+// in Morton order a group of eight may straddle one of its jumps, and a wave
+// of the search below then visits a quarter more of them (64 against 52 nodes
+// for 6,144 triangles; the lattice's search 354 against 287 us, that of
+// 65,536 free points 353 against 236 us).
+__device__ __forceinline__ uint32_t hilbert_key(uint32_t x, uint32_t y, uint32_t z) {
+  uint32_t v[3] = {x, y, z};
+#pragma unroll
+  for (uint32_t bit = 128u; bit > 1u; bit >>= 1) {
+    const uint32_t low = bit - 1u;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const uint32_t swap = (v[0] ^ v[a]) & low;
+      const bool set = (v[a] & bit) != 0u;
+      v[0] ^= set ? low : swap;  // (for a = 0 the swap is of nothing)
+      if (a > 0) v[a] ^= set ? 0u : swap;
+    }
+  }
+  v[1] ^= v[0];
+  v[2] ^= v[1];
+  uint32_t t = 0;
+#pragma unroll
+  for (uint32_t bit = 128u; bit > 1u; bit >>= 1) t ^= (v[2] & bit) ? bit - 1u : 0u;
+  uint32_t key = 0;
+#pragma unroll
+  for (int k = 7; k >= 0; --k)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) key = key << 1 | (((v[a] ^ t) >> k) & 1u);
+  return key;
 }
 
-constexpr int kMortonBits = 24;
+constexpr int kOrderBits = 24;
 
-__global__ __launch_bounds__(kBlock) void k_mesh_morton(const double* __restrict__ verts,
+__global__ __launch_bounds__(kBlock) void k_mesh_order(const double* __restrict__ verts,
                                                         uint32_t nv,
                                                         const uint32_t* __restrict__ tris,
                                                         uint32_t nt,
@@ -156,16 +181,15 @@ __global__ __launch_bounds__(kBlock) void k_mesh_morton(const double* __restrict
   double v[9];
   uint32_t vi[3];
   load_corners(verts, nv, tris, t, v, vi);
-  uint32_t key = 0;
+  uint32_t at[3];
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
     const double lo = mesh_key_value(I->lo[a]), hi = mesh_key_value(I->hi[a]);
     const double c = (v[a] + v[3 + a] + v[6 + a]) * (1.0 / 3.0);
     // any value orders the triangles (a NaN reads 0)
-    const double u = fmin(fmax((c - lo) / (hi - lo) * 256.0, 0.0), 255.0);
-    key |= spread3((uint32_t)u) << a;
+    at[a] = (uint32_t)fmin(fmax((c - lo) / (hi - lo) * 256.0, 0.0), 255.0);
   }
-  keys[t] = key;
+  keys[t] = hilbert_key(at[0], at[1], at[2]);
 }
 
 __device__ __forceinline__ uint32_t box_at(uint32_t node) {
@@ -290,12 +314,12 @@ __device__ __forceinline__ bool winds(double w) { return w / (4.0 * 3.1415926535
 // list of (lane, triangle) pairs that the wave takes 64 at a time, so that
 // point_triangle_dist2, 300 instructions of binary64, runs with all lanes.
 //
-// Bound by issue: a wave takes about 65 boxes of eight, 74 triangles and 25
+// Bound by issue: a wave takes about 52 boxes of eight, 60 triangles and 20
 // rounds of pairs.  274,625 lattice points against 6,144 triangles: a search
-// per lane, diverging at every step, took 1.02 ms; this 0.36 ms.
+// per lane, diverging at every step, took 1.02 ms; this 0.29 ms.
 constexpr int kLanes = 64;  // one wave per block
 
-// (4 waves per SIMD at 108 VGPRs: 598 us a build against 578)
+// (4 waves per SIMD at 108 VGPRs: 598 us a build against 578, in Morton order)
 constexpr int kTreeWavesPerSimd = 5;
 
 struct TreeShared {
@@ -666,7 +690,7 @@ __global__ __launch_bounds__(kLanes) void k_tree_signs(MeshTree T,
 }
 
 // A wave takes a 4 x 4 x 4 block of lattice vertices (4 x 4 x 2 and 4 x 4 x 1:
-// 664 and 899 us a build against 626).
+// 664 and 899 us a build against 626, in Morton order).
 __global__ __launch_bounds__(kLanes, kTreeWavesPerSimd) void k_tree_lattice(
     MeshTree T, const double* __restrict__ verts, uint32_t nv, const uint32_t* __restrict__ tris,
     uint32_t nt, int nx, int ny, int nz, int kx, int ky, double bx, double by, double bz,
@@ -700,23 +724,23 @@ __global__ __launch_bounds__(kLanes, kTreeWavesPerSimd) void k_tree_lattice(
                        0.0f);
 }
 
-// Free points are taken in the Morton order of their places in three times
+// Free points are taken along the Hilbert curve through their places in three times
 // the mesh's box (any order gives the same results; a wave's points should
 // be neighbours).
-__global__ __launch_bounds__(kBlock) void k_point_morton(const double* __restrict__ pts,
+__global__ __launch_bounds__(kBlock) void k_point_order(const double* __restrict__ pts,
                                                          uint32_t n,
                                                          const MeshInfo* __restrict__ I,
                                                          uint32_t* __restrict__ keys) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  uint32_t key = 0;
+  uint32_t at[3];
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
     const double lo = mesh_key_value(I->lo[a]), hi = mesh_key_value(I->hi[a]), ext = hi - lo;
     const double u = (pts[3 * (size_t)i + a] - (lo - ext)) / (3.0 * ext) * 256.0;
-    key |= spread3((uint32_t)fmin(fmax(u, 0.0), 255.0)) << a;  // (a NaN reads 0)
+    at[a] = (uint32_t)fmin(fmax(u, 0.0), 255.0);  // (a NaN reads 0)
   }
-  keys[i] = key;
+  keys[i] = hilbert_key(at[0], at[1], at[2]);
 }
 
 __global__ __launch_bounds__(kLanes, kTreeWavesPerSimd) void k_tree_points(
@@ -829,11 +853,11 @@ hipError_t launch_mesh_tree(fc_context* ctx, const double* verts, uint32_t nv,
   hipLaunchKernelGGL(k_mesh_info_init, dim3(1), dim3(64), 0, s, info);
   hipLaunchKernelGGL(k_mesh_info, dim3(blocks < kInfoBlocks ? blocks : kInfoBlocks), dim3(kBlock),
                      0, s, verts, nv, tris, nt, info);
-  hipLaunchKernelGGL(k_mesh_morton, dim3(blocks), dim3(kBlock), 0, s, verts, nv, tris, nt, info,
+  hipLaunchKernelGGL(k_mesh_order, dim3(blocks), dim3(kBlock), 0, s, verts, nv, tris, nt, info,
                      keys);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess)
-    e = radix_sort_pairs(s, ctx->sort, ctx->devFlags, keys, nullptr, keys, order, nt, kMortonBits,
+    e = radix_sort_pairs(s, ctx->sort, ctx->devFlags, keys, nullptr, keys, order, nt, kOrderBits,
                          nullptr);
   if (e != hipSuccess) return e;
   const uint32_t padded = (nt + 7u) & ~7u;
@@ -887,12 +911,12 @@ hipError_t launch_tree_points(fc_context* ctx, const MeshTree& T, const double* 
   for (uint64_t at = 0; at < np; at += chunk) {
     const uint32_t n = (uint32_t)(np - at < chunk ? np - at : chunk);
     const double* p = pts + 3 * at;
-    hipLaunchKernelGGL(k_point_morton, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, p, n,
+    hipLaunchKernelGGL(k_point_order, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, p, n,
                        T.info, keys);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
       e = radix_sort_pairs(s, ctx->sort, ctx->devFlags, keys, nullptr, keys, order, n,
-                           kMortonBits, nullptr);
+                           kOrderBits, nullptr);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_tree_signs, dim3((n + kRaysPerWave - 1) / kRaysPerWave), dim3(kLanes), 0,
                        s, T, p, n, order, sdf + at);
