@@ -89,6 +89,8 @@ __device__ __forceinline__ bf16x8 pack8(float a0, float a1, float a2, float a3, 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kTB = 256;  // inference block
+// The network in registers: under 256 of them.
+constexpr int kInferWavesPerSimd = 2;
 
 __device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + __expf(-z)); }
 // SiLU of the inference path: the hardware exp2 and reciprocal (about 1 ulp
@@ -543,21 +545,107 @@ __device__ __forceinline__ bf16x8 act_operand(const floatx4& lo, const floatx4& 
 
 __device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 
+// sin and cos features of one query for the lane's four frequencies (f: the
+// 12 coefficients), as the first layer's B operand.
+__device__ __forceinline__ bf16x8 feature_operand(const float* f, float x, float y, float z) {
+  float sv[4], cv[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    sincos_rev(f[3 * j] * x + f[3 * j + 1] * y + f[3 * j + 2] * z, sv[j], cv[j]);
+  return pack8(sv[0], sv[1], sv[2], sv[3], cv[0], cv[1], cv[2], cv[3]);
+}
+
 // One 16-query tile through the network with 16x16x32 BF16 MFMAs: the
 // queries are the columns, the layer outputs the rows, so every lane group
 // g = lane/16 holds rows 4g..4g+3 of each 16-row block for its query column
-// lane%16.  Returns the network output y for the lane's column.
-template <class Frags>
-__device__ __forceinline__ float sdf_tile_mfma_f(const Frags& frag, const float* __restrict__ P,
-                                                 const float* __restrict__ F, float x, float y,
-                                                 float z, int g) {
-  float sv[4], cv[4];
+// lane%16.  Returns the network output y for the lane's column.  The network
+// is held in registers.
+//
+// Bound by vector issue: a tile's 3,072 activations are 48 to a lane, each
+// one exp2 and one reciprocal (16 cycles a wave) and five products and sums
+// (4 cycles): 2,500 of the tile's 3,000 cycles; the matrix cores are busy for
+// 320.  Everything else is kept out of the tile: biases, last layer and
+// frequencies stay in registers with the fragments (207, two waves per SIMD;
+// 36 loads a tile before), and with the register budget of two waves
+// the accumulators need no copies.  500,003 queries of 8 networks: 50.8 us
+// before, 37.9 with this (42.0 with the biases added by FP32 MFMAs, 39.9 with
+// those and three waves per SIMD: their latency is longer than what they
+// save).
+struct SdfNet {
+  bf16x8 frag[kSdfFrags];
+  floatx4 bias[3][4], w4[4];  // of rows 16 ob + 4g .. + 3
+  float f[12];                // of frequencies 4g .. 4g + 3
+  float b4;
+
+  __device__ __forceinline__ void load(const uint16_t* __restrict__ packed,
+                                       const float* __restrict__ params,
+                                       const float* __restrict__ freq, uint32_t net, int lane) {
+    const int g = lane >> 4;
+    const float* P = params + (size_t)net * kSdfStride;
+    const float* F = freq + (size_t)net * kSdfFreqs * 3 + 12 * g;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int k = 4 * g + j;
-    sincos_rev(F[3 * k] * x + F[3 * k + 1] * y + F[3 * k + 2] * z, sv[j], cv[j]);
+    for (int i = 0; i < kSdfFrags; ++i) frag[i] = load_frag(packed, net, i, lane);
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob) {
+      bias[0][ob] = *reinterpret_cast<const floatx4*>(P + kSdfOffB1 + 16 * ob + 4 * g);
+      bias[1][ob] = *reinterpret_cast<const floatx4*>(P + kSdfOffB2 + 16 * ob + 4 * g);
+      bias[2][ob] = *reinterpret_cast<const floatx4*>(P + kSdfOffB3 + 16 * ob + 4 * g);
+      w4[ob] = *reinterpret_cast<const floatx4*>(P + kSdfOffW4 + 16 * ob + 4 * g);
+    }
+#pragma unroll
+    for (int j = 0; j < 12; ++j) f[j] = F[j];
+    b4 = P[kSdfOffB4];
   }
-  const bf16x8 bop = pack8(sv[0], sv[1], sv[2], sv[3], cv[0], cv[1], cv[2], cv[3]);
+
+  __device__ __forceinline__ float eval(float x, float y, float z) const {
+    const bf16x8 in = feature_operand(f, x, y, z);
+    floatx4 d[4];
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob)
+      d[ob] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag[ob], in, floatx4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+    for (int L = 0; L < 2; ++L) {
+      const bf16x8* w = frag + 4 + 8 * L;
+      const bf16x8 in0 = act(d[0], d[1], bias[L][0], bias[L][1]);
+      const bf16x8 in1 = act(d[2], d[3], bias[L][2], bias[L][3]);
+#pragma unroll
+      for (int ob = 0; ob < 4; ++ob) {
+        const floatx4 acc =
+            __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[2 * ob], in0, floatx4{0, 0, 0, 0}, 0, 0, 0);
+        d[ob] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[2 * ob + 1], in1, acc, 0, 0, 0);
+      }
+    }
+    float yv = 0.0f;
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob) {
+      const floatx4 h = d[ob] + bias[2][ob];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) yv += silu_fast(h[r]) * w4[ob][r];
+    }
+    yv += __shfl_xor(yv, 16);
+    yv += __shfl_xor(yv, 32);
+    return yv + b4;
+  }
+
+ private:
+  static __device__ __forceinline__ bf16x8 act(const floatx4& lo, const floatx4& hi,
+                                               const floatx4& blo, const floatx4& bhi) {
+    const floatx4 a = lo + blo, b = hi + bhi;
+    return pack8(silu_fast(a[0]), silu_fast(a[1]), silu_fast(a[2]), silu_fast(a[3]),
+                 silu_fast(b[0]), silu_fast(b[1]), silu_fast(b[2]), silu_fast(b[3]));
+  }
+};
+
+// The tile with each fragment loaded where it is used (the network's 20 KB
+// of packed weights stay in the L1/L2 caches across the tiles of a wave),
+// which frees the registers that hold them.
+__device__ __forceinline__ float sdf_tile_mfma_loaded(const uint16_t* __restrict__ packed,
+                                                      uint32_t net, int lane,
+                                                      const float* __restrict__ P,
+                                                      const float* __restrict__ F, float x,
+                                                      float y, float z, int g) {
+  const auto frag = [&](int f) { return load_frag(packed, net, f, lane); };
+  const bf16x8 bop = feature_operand(F + 12 * g, x, y, z);
   floatx4 d[4];
 #pragma unroll
   for (int ob = 0; ob < 4; ++ob)
@@ -590,82 +678,60 @@ __device__ __forceinline__ float sdf_tile_mfma_f(const Frags& frag, const float*
   return yv + P[kSdfOffB4];
 }
 
-// The tile with the network's fragments held in registers.
-__device__ __forceinline__ float sdf_tile_mfma(const bf16x8 (&frag)[kSdfFrags],
-                                               const float* __restrict__ P,
-                                               const float* __restrict__ F, float x, float y,
-                                               float z, int g) {
-  return sdf_tile_mfma_f([&](int f) { return frag[f]; }, P, F, x, y, z, g);
-}
-
-// The tile with each fragment loaded where it is used (the network's 20 KB
-// of packed weights stay in the L1/L2 caches across the tiles of a wave),
-// which frees the registers that hold them.
-__device__ __forceinline__ float sdf_tile_mfma_loaded(const uint16_t* __restrict__ packed,
-                                                      uint32_t net, int lane,
-                                                      const float* __restrict__ P,
-                                                      const float* __restrict__ F, float x,
-                                                      float y, float z, int g) {
-  return sdf_tile_mfma_f([&](int f) { return load_frag(packed, net, f, lane); }, P, F, x, y, z,
-                         g);
-}
-
-// Wave-level inference over 16-query tiles (grid-stride).  Queries of one
-// tile that belong to different bodies are run once per distinct body with
-// that body's fragments; out = y * halfExtent (NaN for a body id out of
+// Wave-level inference.  A wave takes a run of 16-query tiles, four at a
+// time: lane l reads and normalises query l of the 64, so each is divided once
+// and not once per lane group, and writes its distance.  Queries of one tile
+// that belong to different bodies are run once per distinct body; the network
+// is read where it changes.  out = y * halfExtent (NaN for a body id out of
 // range).
-__global__ __launch_bounds__(kTB) void k_sdf_infer(const uint16_t* __restrict__ packed,
-                                                   const float* __restrict__ params,
-                                                   const float* __restrict__ freq,
-                                                   const float* __restrict__ frame,
-                                                   const uint32_t* __restrict__ bodies,
-                                                   uint32_t numBodies,
-                                                   const float* __restrict__ pts, uint32_t n,
-                                                   float* __restrict__ out) {
+__global__ __launch_bounds__(kTB, kInferWavesPerSimd) void k_sdf_infer(
+    const uint16_t* __restrict__ packed, const float* __restrict__ params,
+    const float* __restrict__ freq, const float* __restrict__ frame,
+    const uint32_t* __restrict__ bodies, uint32_t numBodies, const float* __restrict__ pts,
+    uint32_t n, float* __restrict__ out) {
   const int lane = threadIdx.x & 63, g = lane >> 4, col = lane & 15;
-  const uint32_t wave = (blockIdx.x * kTB + threadIdx.x) >> 6;
   const uint32_t nWaves = (gridDim.x * kTB) >> 6;
-  const uint32_t tiles = (n + 15) / 16;
-  // contiguous runs of tiles per wave: consecutive tiles share a network,
-  // so the weight fragments are reloaded only where the network changes
-  const uint32_t per = (tiles + nWaves - 1) / nWaves;
-  const uint32_t t0 = wave * per, t1 = t0 + per < tiles ? t0 + per : tiles;
-  bf16x8 frag[kSdfFrags];
-  int cur = -1;
-  for (uint32_t tile = t0; tile < t1; ++tile) {
-    const uint32_t q = tile * 16 + col;
-    const bool valid = q < n;
-    uint32_t body = valid ? (bodies ? bodies[q] : 0u) : 0u;
-    float qx = 0.0f, qy = 0.0f, qz = 0.0f;
-    if (valid) {
-      qx = pts[3 * q];
-      qy = pts[3 * q + 1];
-      qz = pts[3 * q + 2];
-      if (body >= numBodies) {
-        if (g == 0) out[q] = __int_as_float(0x7fc00000);
+  const uint32_t wave = (blockIdx.x * kTB + threadIdx.x) >> 6;
+  const uint32_t tiles = n / 16 + (n % 16 != 0 ? 1u : 0u);
+  // contiguous runs of tiles per wave: consecutive tiles share a network
+  const uint32_t t0 = (uint32_t)((uint64_t)tiles * wave / nWaves),
+                 t1 = (uint32_t)((uint64_t)tiles * (wave + 1) / nWaves);
+  SdfNet net;
+  uint32_t cur = 0xffffffffu;
+  for (uint32_t t = t0; t < t1; t += 4) {
+    const size_t q = (size_t)t * 16 + lane;
+    const bool valid = q < n && t + g < t1;
+    float x = 0.0f, y = 0.0f, z = 0.0f, scale = 0.0f;
+    uint32_t body = numBodies;
+    if (valid) body = bodies ? bodies[q] : 0u;
+    const bool known = body < numBodies;
+    if (known) {
+      const float4 fr = *reinterpret_cast<const float4*>(frame + (size_t)body * 4);
+      sdf_norm(&fr.x, pts[3 * q], pts[3 * q + 1], pts[3 * q + 2], x, y, z);
+      scale = fr.w;
+    }
+    float res = __int_as_float(0x7fc00000);
+    for (int u = 0; u < 4; ++u) {
+      bool remaining = known && g == u;
+      uint64_t mask = __ballot(remaining);
+      if (mask == 0ull) continue;
+      const int from = 16 * u + col;
+      const float tx = __shfl(x, from), ty = __shfl(y, from), tz = __shfl(z, from);
+      while (mask != 0ull) {
+        const uint32_t lead =
+            (uint32_t)__builtin_amdgcn_readlane((int)body, __ffsll((unsigned long long)mask) - 1);
+        if (lead != cur) {
+          net.load(packed, params, freq, lead, lane);
+          cur = lead;
+        }
+        const float yv = net.eval(tx, ty, tz);
+        const bool mine = remaining && body == lead;
+        if (mine) res = yv * scale;
+        remaining = remaining && !mine;
+        mask = __ballot(remaining);
       }
     }
-    bool remaining = valid && body < numBodies;
-    while (true) {
-      const uint64_t mask = __ballot(remaining);
-      if (mask == 0) break;
-      const int leadLane = __ffsll((unsigned long long)mask) - 1;
-      const uint32_t lead = (uint32_t)__shfl((int)body, leadLane);
-      if ((int)lead != cur) {
-#pragma unroll
-        for (int f = 0; f < kSdfFrags; ++f) frag[f] = load_frag(packed, lead, f, lane);
-        cur = (int)lead;
-      }
-      const float* P = params + (size_t)lead * kSdfStride;
-      const float* F = freq + (size_t)lead * kSdfFreqs * 3;
-      const float* fr = frame + (size_t)lead * 4;
-      float x, y, z;
-      sdf_norm(fr, qx, qy, qz, x, y, z);
-      const float yv = sdf_tile_mfma(frag, P, F, x, y, z, g);
-      const bool mine = remaining && body == lead;
-      if (mine && g == 0) out[q] = yv * fr[3];
-      remaining = remaining && !mine;
-    }
+    if (valid) out[q] = res;
   }
 }
 
@@ -850,13 +916,6 @@ __global__ __launch_bounds__(kBT) void k_bucket_scatter(const uint16_t* __restri
   }
 }
 
-// Whether the cull loads each weight fragment where it is used (fewer
-// registers, more waves per SIMD) instead of holding all 20 per wave.
-#ifndef FC_CULL_LOADED_FRAGS
-#define FC_CULL_LOADED_FRAGS 1
-#endif
-constexpr bool kCullLoadedFrags = FC_CULL_LOADED_FRAGS != 0;
-
 // Surrogate cull over the bucketed spheres: the BF16 network predicts each
 // in-box sphere's distance, and those within radius + margin[body] are
 // listed for the exact query: wave w lists its candidates from band[16 t0]
@@ -875,12 +934,9 @@ __global__ __launch_bounds__(kTB) void k_boundary_cull(
   // were cleared by the bucketing), shared evenly among the waves
   const uint32_t n = *inBoxCount;
   const uint32_t tiles = (n + 15) / 16;
-  // contiguous runs of tiles per wave: consecutive tiles share a network,
-  // so the weight fragments are reloaded only where the network changes
+  // contiguous runs of tiles per wave: consecutive tiles share a network
   const uint32_t per = (tiles + nWaves - 1) / nWaves;
   const uint32_t t0 = wave * per, t1 = t0 + per < tiles ? t0 + per : tiles;
-  bf16x8 frag[kSdfFrags];
-  int cur = -1;
   // the wave's candidates are listed from band[16 t0] on (its slots' range)
   uint32_t listed = 0;
   for (uint32_t tile = t0; tile < t1; ++tile) {
@@ -902,19 +958,12 @@ __global__ __launch_bounds__(kTB) void k_boundary_cull(
       if (mask == 0) break;
       const int leadLane = __ffsll((unsigned long long)mask) - 1;
       const int lead = __shfl(net, leadLane);
-      if (!kCullLoadedFrags && lead != cur) {
-#pragma unroll
-        for (int f = 0; f < kSdfFrags; ++f) frag[f] = load_frag(packed, (uint32_t)lead, f, lane);
-        cur = lead;
-      }
       const float* P = params + (size_t)lead * kSdfStride;
       const float* F = freq + (size_t)lead * kSdfFreqs * 3;
       const float* fr = frame + (size_t)lead * 4;
       float x, y, z;
       sdf_norm(fr, q.x, q.y, q.z, x, y, z);
-      const float yv = kCullLoadedFrags
-                           ? sdf_tile_mfma_loaded(packed, (uint32_t)lead, lane, P, F, x, y, z, g)
-                           : sdf_tile_mfma(frag, P, F, x, y, z, g);
+      const float yv = sdf_tile_mfma_loaded(packed, (uint32_t)lead, lane, P, F, x, y, z, g);
       const bool mine = remaining && net == lead;
       if (mine) cand = yv * fr[3] <= radius + margins[body];
       remaining = remaining && !mine;
@@ -1015,7 +1064,7 @@ __device__ __forceinline__ uint32_t float_key(float f) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-__global__ __launch_bounds__(kTB) void k_sdf_map_margin(
+__global__ __launch_bounds__(kTB, kInferWavesPerSimd) void k_sdf_map_margin(
     const uint16_t* __restrict__ packed, const float* __restrict__ params,
     const float* __restrict__ freq, const float* __restrict__ frame, uint32_t net,
     DistMapView m, float radius, float band, uint32_t* __restrict__ stats) {
@@ -1026,12 +1075,9 @@ __global__ __launch_bounds__(kTB) void k_sdf_map_margin(
   const uint32_t bx = (nx + 3u) / 4u, by = (ny + 1u) / 2u, bz = (nz + 1u) / 2u;
   const uint64_t blocks = (uint64_t)bx * by * bz;
   const uint32_t dx = (uint32_t)col & 3u, dy = ((uint32_t)col >> 2) & 1u, dz = (uint32_t)col >> 3;
-  const float* P = params + (size_t)net * kSdfStride;
-  const float* F = freq + (size_t)net * kSdfFreqs * 3;
   const float* fr = frame + (size_t)net * 4;
-  bf16x8 frag[kSdfFrags];
-#pragma unroll
-  for (int f = 0; f < kSdfFrags; ++f) frag[f] = load_frag(packed, net, f, lane);
+  SdfNet mlp;
+  mlp.load(packed, params, freq, net, lane);
   float over = -INFINITY, slope = 0.0f, err = 0.0f;
   uint32_t count = 0;
   for (uint64_t blk = wave; blk < blocks; blk += nWaves) {
@@ -1050,7 +1096,7 @@ __global__ __launch_bounds__(kTB) void k_sdf_map_margin(
     if (__ballot(inBand) == 0ull) continue;
     float x, y, z;
     sdf_norm(fr, qx, qy, qz, x, y, z);
-    const float yv = sdf_tile_mfma(frag, P, F, x, y, z, g) * fr[3];
+    const float yv = mlp.eval(x, y, z) * fr[3];
     // neighbours along x (column + 1), y (+ 4) and z (+ 8) inside the block
     const int base = lane & 48;
     const int cX = (col + 1) & 15, cY = (col + 4) & 15, cZ = (col + 8) & 15;
@@ -1134,21 +1180,20 @@ void free_sdf(fc_sdf* m) {
 
 // Training blocks resident at once: one per CU (154 KB of LDS each).
 constexpr uint32_t kTrainBlocks = 256;
-// Waves of the inference kernel (the 20 weight fragments in registers,
-// 170 VGPRs: two waves per SIMD of the 256 CUs) and of the cull (fragments
-// loaded where used, under 100 VGPRs: four waves per SIMD).
-constexpr uint32_t kMaxInferWaves = 2048;
+// Waves resident at once of the inference kernels (the network in registers)
+// and of the cull (fragments loaded where used, under 100 VGPRs: four waves
+// per SIMD), on 1,024 SIMDs.
+constexpr uint32_t kMaxInferWaves = 1024 * kInferWavesPerSimd;
 #ifndef FC_CULL_WAVES
 #define FC_CULL_WAVES 4096
 #endif
 constexpr uint32_t kMaxCullWaves = FC_CULL_WAVES;
 
-// Blocks (of 4 waves) of the MFMA kernels for n queries: at most the waves
-// that are resident at once, each wave taking at least 16 tiles, so no wave
-// waits for a second round.
+// Blocks (of 4 waves) of the MFMA kernels for n queries: a tile a wave up to
+// the waves that are resident at once, so no wave waits for a second round
+// (8,192 queries at 16 tiles a wave: 30 us, at four: 7.9, at one: 4.6).
 uint32_t mfma_blocks(uint32_t n, uint32_t maxWaves = kMaxInferWaves) {
-  const uint32_t tiles = (n + 15) / 16;
-  uint32_t waves = (tiles + 15) / 16;
+  uint32_t waves = n / 16 + (n % 16 != 0 ? 1u : 0u);
   if (waves > maxWaves) waves = maxWaves;
   const uint32_t blocks = (waves + 3) / 4;
   return blocks == 0 ? 1u : blocks;

@@ -35,3 +35,43 @@ def test_gradient_tiles(gpu_ctx, bodies, samples):
         gb = g[b, :s.nparams].astype(np.float64)
         assert np.max(np.abs(gb - ref)) <= 1e-4 * np.max(np.abs(ref))
     s.close()
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 63, 65, 1000, 32769])
+def test_inference_tiles(gpu_ctx, n):
+    """Inference at the edges of its 16-query tiles, of its groups of four
+    tiles and of one tile per wave; runs of one body, mixed tiles and ids out
+    of range."""
+    from fullc0ntact_amd.sdf import BF16, SdfSurrogate
+    print(n, flush=True)
+    rng = np.random.default_rng(n)
+    s = SdfSurrogate(gpu_ctx, rng.uniform(-0.1, 0.1, (3, 3)), rng.uniform(0.8, 1.2, 3), seed=7)
+    p, f, fr = s.params()
+    pts = rng.uniform(-0.8, 0.8, (n, 3)).astype(np.float32)
+    bodies = np.where(np.arange(n) < n // 2, 2, rng.integers(0, 4, n)).astype(np.uint32)
+    y = s.eval(pts, bodies, BF16)
+    assert np.all(np.isnan(y[bodies == 3]))
+    for b in range(3):
+        m = bodies == b
+        if m.any():
+            scale = np.max(np.abs(orc.sdf_forward(p[b], f[b], fr[b], pts[:512])))
+            ref = orc.sdf_forward(p[b], f[b], fr[b], pts[m], bf16=True)
+            # the bound of the whole-network test: BF16 activations that round the other way
+            assert np.max(np.abs(y[m] - ref)) <= 2e-3 * max(scale, 0.1), b
+    s.close()
+
+
+@pytest.mark.parametrize("n", [32769, 150001])
+def test_inference_is_the_same_in_parts(gpu_ctx, n):
+    """A query's distance does not depend on the call it stands in: many tiles
+    per wave and mixed tiles against calls of 1,000 queries, bit for bit."""
+    from fullc0ntact_amd.sdf import BF16, SdfSurrogate
+    print(n, flush=True)
+    rng = np.random.default_rng(n)
+    s = SdfSurrogate(gpu_ctx, rng.uniform(-0.1, 0.1, (3, 3)), rng.uniform(0.8, 1.2, 3), seed=7)
+    pts = rng.uniform(-0.8, 0.8, (n, 3)).astype(np.float32)
+    bodies = np.where(np.arange(n) < n // 2, 2, rng.integers(0, 4, n)).astype(np.uint32)
+    y = s.eval(pts, bodies, BF16)
+    parts = [s.eval(pts[i:i + 1000], bodies[i:i + 1000], BF16) for i in range(0, n, 1000)]
+    assert np.array_equal(y.view(np.uint32), np.concatenate(parts).view(np.uint32))
+    s.close()
