@@ -88,6 +88,8 @@ __device__ __forceinline__ bf16x8 pack8(float a0, float a1, float a2, float a3, 
 }
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
+__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+
 constexpr int kTB = 256;  // inference block
 // The network in registers: under 256 of them.
 constexpr int kInferWavesPerSimd = 2;
@@ -187,10 +189,18 @@ __global__ __launch_bounds__(kTB) void k_sdf_eval_f32(const float* __restrict__ 
 // each wave owns two 16x16 blocks of a 64x64 gradient, so its accumulators
 // are few and live in registers over the block's tiles.
 //
-// Bound by the FP32 matrix rate: 448 MFMAs of 32 cycles a wave and tile.  One
-// gradient of 8 bodies x 16384 samples, copied to the host: 605 us with 4x4
-// register tiles on the vector units (one wave per SIMD, 16-way bank
-// conflicts in the transposed products), 163 us with this.
+// Bound by the FP32 units: 448 MFMAs of 32 cycles a wave and tile, during
+// which the SIMD's other wave cannot issue FP32 vector instructions either
+// (measured: a loop of FMAs and one of these MFMAs on two waves of a SIMD take
+// the sum of their times), so every vector instruction adds to the MFMAs'
+// time.  Hence: reads of LDS with one address register and immediate offsets,
+// a bias gradient summed by the waves in shares, the reciprocal with one
+// Newton step, the weights read in five 16-byte loads a thread and each tile's
+// samples a tile ahead (880 vector instructions a wave and tile, 2,000 before
+// these).  8 bodies x 16384 samples: 550 us with 4x4 register tiles on the
+// vector units (one wave per SIMD, 16-way bank conflicts in the transposed
+// products), 106 us with the MFMAs, 91 us with the vector work cut (the MFMAs
+// alone: 55 us at the clock that they sustain).
 // ---------------------------------------------------------------------------
 constexpr int kTrainTile = 128;             // samples per tile: 16 per wave
 constexpr int kTrainThreads = 512;          // 8 waves, two per SIMD
@@ -199,6 +209,15 @@ constexpr int kTrainWaves = kTrainThreads / 64;
 // the transposed read of the backward pass on 64 distinct banks as well.
 constexpr int kFragStride = 65;
 constexpr int kRowsW1 = 0, kRowsW2 = 32, kRowsW3 = 96, kRowsW = 160;
+// The block's LDS, in words.
+constexpr int kTrainBias = kRowsW * kFragStride;          // b1, b2, b3, w4
+constexpr int kTrainFr = kTrainBias + 4 * kSdfHidden;     // frequencies, frame
+constexpr int kTrainX0 = kTrainFr + 3 * kSdfFreqs + 4;    // per wave: features,
+constexpr int kTrainA1 = kTrainX0 + kTrainWaves * 16 * kSdfIn;      // A1,
+constexpr int kTrainA2 = kTrainA1 + kTrainWaves * 16 * kSdfHidden;  // A2, then dZ2,
+constexpr int kTrainDz = kTrainA2 + kTrainWaves * 16 * kSdfHidden;  // dZ3, then dZ1
+constexpr int kTrainLds = kTrainDz + kTrainWaves * 16 * kSdfHidden;
+static_assert(kTrainX0 % 4 == 0 && kTrainLds * 4 <= 160 * 1024, "");
 
 // Registers d[4 ob + r] (features 16 ob + 4 g + r of sample c) to LDS.
 template <int kBlocks>
@@ -215,45 +234,90 @@ __device__ __forceinline__ int train_get(int step, int g, int i) {
   return (i >> 2) * 64 + ((step ^ (i >> 2)) << 4) + (g << 2) + (i & 3);
 }
 
+// An LDS index that the compiler takes as it stands: the reads around it then
+// share this one register and differ by their immediate offsets (folded into
+// each read's own constant, every read had an addition of its own).
+__device__ __forceinline__ int own_register(int i) {
+  asm("" : "+v"(i));
+  return i;
+}
+
+// SiLU(z) and its derivative s + z s (1 - s), s = 1 / (1 + exp(-z)): the
+// hardware reciprocal with one Newton step (0 for an infinite denominator).
+__device__ __forceinline__ void silu_grad(float z, float& a, float& d) {
+  const float x = 1.0f + __expf(-z);
+  float s = __builtin_amdgcn_rcpf(x);
+  s = __builtin_fmaf(__builtin_fmaf(-x, s, 1.0f), s, s);
+  s = __builtin_amdgcn_div_fixupf(s, x, 1.0f);
+  a = z * s;
+  d = __builtin_fmaf(a, 1.0f - s, s);
+}
+
 __global__ __launch_bounds__(kTrainThreads) void k_sdf_grad_tiles(
     const float* __restrict__ params, const float* __restrict__ freq,
     const float* __restrict__ frame, const float* __restrict__ pts,
     const float* __restrict__ labels, uint32_t samplesPerBody, uint32_t batchStart,
     uint32_t batchSize, uint32_t tilesPerBlock, float invM, float* __restrict__ partial,
     float* __restrict__ lossPartial) {
-  __shared__ float s_w[kRowsW * kFragStride];
-  __shared__ float s_bias[4 * kSdfHidden];  // b1, b2, b3, w4
-  __shared__ float s_fr[kSdfFreqs * 3 + 4];
-  __shared__ float s_x0[kTrainWaves][16 * kSdfIn];
-  __shared__ float s_a1[kTrainWaves][16 * kSdfHidden];
-  __shared__ float s_a2[kTrainWaves][16 * kSdfHidden];  // then dZ2
-  __shared__ float s_dz[kTrainWaves][16 * kSdfHidden];  // dZ3, then dZ1
+  __shared__ __attribute__((aligned(16))) float S[kTrainLds];
 
   const uint32_t body = blockIdx.y, blk = blockIdx.x, nblk = gridDim.x;
-  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6, g = lane >> 4, c = lane & 15;
+  const int t = (int)threadIdx.x, lane = t & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   const float* P = params + (size_t)body * kSdfStride;
+  // the first tile's samples, on their way while the weights are laid out
+  const uint32_t batchEnd = batchStart + batchSize;
+  const float* bodyPts = pts + (size_t)body * samplesPerBody * 3;
+  const float* bodyLab = labels + (size_t)body * samplesPerBody;
+  uint32_t gs = batchStart + blk * tilesPerBlock * (uint32_t)kTrainTile + 16u * (uint32_t)w +
+                (uint32_t)c;
+  bool live = gs < batchEnd && gs < samplesPerBody;
+  float q[3] = {}, label = 0.0f;
+  auto fetch = [&] {
+    if (live) {
+      const float* at = bodyPts + (size_t)gs * 3;
+      q[0] = at[0];
+      q[1] = at[1];
+      q[2] = at[2];
+      label = bodyLab[gs];
+    }
+  };
+  fetch();
   // row ob2 * steps + (4 ob + r) of a layer: W[16 ob + 4 g + r][16 ob2 + c]
-  for (int e = t; e < kRowsW * 64; e += kTrainThreads) {
-    const int row = e >> 6, l = e & 63;
-    const int off = row < kRowsW2 ? kSdfOffW1 : (row < kRowsW3 ? kSdfOffW2 : kSdfOffW3);
-    const int rr = row - (row < kRowsW2 ? kRowsW1 : (row < kRowsW3 ? kRowsW2 : kRowsW3));
-    const int steps = row < kRowsW2 ? 8 : 16;
-    const int ob2 = rr / steps, st = rr % steps;
-    const int in = 16 * (st >> 2) + 4 * (l >> 4) + (st & 3), out = 16 * ob2 + (l & 15);
-    s_w[row * kFragStride + l] = P[off + in * kSdfHidden + out];
+  float4 wq[5];
+#pragma unroll
+  for (int it = 0; it < 5; ++it) {
+    const int off = it == 0 ? kSdfOffW1 : (it < 3 ? kSdfOffW2 : kSdfOffW3);
+    wq[it] = ld4(P + off + 4 * (t + kTrainThreads * (it == 0 ? 0 : (it - 1) % 2)));
   }
-  for (int e = t; e < 4 * kSdfHidden; e += kTrainThreads) {
-    const int which = e / kSdfHidden, o = e % kSdfHidden;
+#pragma unroll
+  for (int it = 0; it < 5; ++it) {
+    const int rows = it == 0 ? kRowsW1 : (it < 3 ? kRowsW2 : kRowsW3);
+    const int steps = it == 0 ? 8 : 16;
+    const int idx = t + kTrainThreads * (it == 0 ? 0 : (it - 1) % 2);
+    const int in = idx >> 4, out = (idx & 15) * 4;
+    const int row = rows + (out >> 4) * steps + 4 * (in >> 4) + (in & 3);
+    float* to = S + row * kFragStride + ((in >> 2) & 3) * 16 + (out & 15);
+    to[0] = wq[it].x;
+    to[1] = wq[it].y;
+    to[2] = wq[it].z;
+    to[3] = wq[it].w;
+  }
+  static_assert(kTrainThreads == 512 && kSdfIn * kSdfHidden == 4 * kTrainThreads, "");
+  if (t < 4 * kSdfHidden) {
+    const int which = t / kSdfHidden;
     const int off = which == 0 ? kSdfOffB1
                                : (which == 1 ? kSdfOffB2 : (which == 2 ? kSdfOffB3 : kSdfOffW4));
-    s_bias[e] = P[off + o];
+    S[kTrainBias + t] = P[off + t % kSdfHidden];
   }
-  if (t < kSdfFreqs * 3) s_fr[t] = freq[(size_t)body * kSdfFreqs * 3 + t];
-  if (t < 4) s_fr[kSdfFreqs * 3 + t] = frame[(size_t)body * 4 + t];
+  if (t < kSdfFreqs * 3) S[kTrainFr + t] = freq[(size_t)body * kSdfFreqs * 3 + t];
+  if (t < 4) S[kTrainFr + kSdfFreqs * 3 + t] = frame[(size_t)body * 4 + t];
   const float b4 = P[kSdfOffB4];
 
   // this wave's gradient blocks: inputs 16 (w / 2), outputs 32 (w % 2) + 0, 16
-  // (layers 3 and 2); inputs 16 (w / 4), outputs 16 (w % 4) (layer 1)
+  // (layers 3 and 2); inputs 16 (w / 4), outputs 16 (w % 4) (layer 1).  Of the
+  // samples' sums for the biases of its outputs a wave takes the share of the
+  // sample waves 2 (w / 2) + 0, 1 (layer 1: 4 (w / 4) + 0 .. 3).
   floatx4 gW3[2] = {}, gW2[2] = {}, gW1 = {};
   float gb3[2] = {}, gb2[2] = {}, gb1 = 0.0f;
   float gW4[16] = {}, gb4 = 0.0f, lossAcc = 0.0f;
@@ -262,78 +326,79 @@ __global__ __launch_bounds__(kTrainThreads) void k_sdf_grad_tiles(
 #pragma unroll
   for (int s = 0; s < 4; ++s) at[s] = train_get(s, g, c);
   const int back = (c & 3) * kFragStride + (c >> 2) * 16 + 4 * g;
-  const uint32_t batchEnd = batchStart + batchSize;
+  const float* fr = S + kTrainFr + kSdfFreqs * 3;
+  float* x0w = S + kTrainX0 + w * 16 * kSdfIn;
+  float* a1w = S + kTrainA1 + w * 16 * kSdfHidden;
+  float* a2w = S + kTrainA2 + w * 16 * kSdfHidden;
+  float* dzw = S + kTrainDz + w * 16 * kSdfHidden;
 
   for (uint32_t u = 0; u < tilesPerBlock; ++u) {
     const uint32_t s0 = batchStart + (blk * tilesPerBlock + u) * (uint32_t)kTrainTile;
     if (s0 >= batchEnd) break;  // (the same for the block)
     __syncthreads();            // the weights; the last tile's readers of X0 and dZ1
-    const uint32_t gs = s0 + 16u * (uint32_t)w + (uint32_t)c;
-    const bool live = gs < batchEnd && gs < samplesPerBody;
     // ---- features: sines 4 g + j, cosines 16 + 4 g + j
-    float x0[8] = {};
+    float x0[8] = {}, target = 0.0f;
+    const bool now = live;
     if (live) {
-      const float* q = pts + ((size_t)body * samplesPerBody + gs) * 3;
       float x, y, z;
-      sdf_norm(s_fr + kSdfFreqs * 3, q[0], q[1], q[2], x, y, z);
+      sdf_norm(fr, q[0], q[1], q[2], x, y, z);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int k = 4 * g + j;
-        sincos_rev(s_fr[3 * k] * x + s_fr[3 * k + 1] * y + s_fr[3 * k + 2] * z, x0[j], x0[4 + j]);
+        const float* f = S + kTrainFr + 3 * (4 * g + j);
+        sincos_rev(f[0] * x + f[1] * y + f[2] * z, x0[j], x0[4 + j]);
       }
+      target = label / fr[3];
     }
-    train_put<2>(s_x0[w], x0, g, c);
+    gs += (uint32_t)kTrainTile;  // the next tile's samples
+    live = u + 1 < tilesPerBlock && gs < batchEnd && gs < samplesPerBody;
+    fetch();
+    train_put<2>(x0w, x0, g, c);
     // ---- forward: Z = A W + b, A' = SiLU(Z), and SiLU'(Z) for the way back
     float act[16], d1[16], d2[16], d3[16];
     floatx4 z[4];
 #pragma unroll
     for (int ob = 0; ob < 4; ++ob)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) z[ob][r] = s_bias[16 * ob + 4 * g + r];
+      for (int r = 0; r < 4; ++r) z[ob][r] = S[kTrainBias + 16 * ob + 4 * g + r];
 #pragma unroll
     for (int st = 0; st < 8; ++st)
 #pragma unroll
       for (int ob = 0; ob < 4; ++ob)
         z[ob] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-            s_w[(kRowsW1 + ob * 8 + st) * kFragStride + lane], x0[st], z[ob], 0, 0, 0);
+            S[(kRowsW1 + ob * 8 + st) * kFragStride + lane], x0[st], z[ob], 0, 0, 0);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const float v = z[e >> 2][e & 3], s = sigmoidf_(v);
-      act[e] = v * s;
-      d1[e] = s * (1.0f + v * (1.0f - s));
-    }
-    train_put<4>(s_a1[w], act, g, c);
+    for (int e = 0; e < 16; ++e) silu_grad(z[e >> 2][e & 3], act[e], d1[e]);
+    train_put<4>(a1w, act, g, c);
 #pragma unroll
     for (int L = 0; L < 2; ++L) {
       const int rows = L == 0 ? kRowsW2 : kRowsW3;
 #pragma unroll
       for (int ob = 0; ob < 4; ++ob)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) z[ob][r] = s_bias[(L + 1) * kSdfHidden + 16 * ob + 4 * g + r];
+        for (int r = 0; r < 4; ++r)
+          z[ob][r] = S[kTrainBias + (L + 1) * kSdfHidden + 16 * ob + 4 * g + r];
 #pragma unroll
       for (int st = 0; st < 16; ++st)
 #pragma unroll
         for (int ob = 0; ob < 4; ++ob)
           z[ob] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-              s_w[(rows + ob * 16 + st) * kFragStride + lane], act[st], z[ob], 0, 0, 0);
+              S[(rows + ob * 16 + st) * kFragStride + lane], act[st], z[ob], 0, 0, 0);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const float v = z[e >> 2][e & 3], s = sigmoidf_(v);
-        act[e] = v * s;
-        (L == 0 ? d2 : d3)[e] = s * (1.0f + v * (1.0f - s));
-      }
-      if (L == 0) train_put<4>(s_a2[w], act, g, c);
+      for (int e = 0; e < 16; ++e)
+        silu_grad(z[e >> 2][e & 3], act[e], (L == 0 ? d2 : d3)[e]);
+      if (L == 0) train_put<4>(a2w, act, g, c);
     }
     // ---- output, loss, and the output layer's gradient
-    float y = 0.0f;
+    float w4[16], y = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
-      y += act[e] * s_bias[3 * kSdfHidden + 16 * (e >> 2) + 4 * g + (e & 3)];
+    for (int e = 0; e < 16; ++e) {
+      w4[e] = S[kTrainBias + 3 * kSdfHidden + 16 * (e >> 2) + 4 * g + (e & 3)];
+      y = __builtin_fmaf(act[e], w4[e], y);
+    }
     y += __shfl_xor(y, 16);
     y += __shfl_xor(y, 32);
     float dy = 0.0f;
-    if (live) {
-      const float target = labels[(size_t)body * samplesPerBody + gs] / s_fr[kSdfFreqs * 3 + 3];
+    if (now) {
       const float err = (y + b4) - target;
       if (g == 0) lossAcc += err * err;
       dy = 2.0f * err * invM;
@@ -341,30 +406,39 @@ __global__ __launch_bounds__(kTrainThreads) void k_sdf_grad_tiles(
     if (g == 0) gb4 += dy;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      gW4[e] += act[e] * dy;
-      act[e] = dy * s_bias[3 * kSdfHidden + 16 * (e >> 2) + 4 * g + (e & 3)] * d3[e];  // dZ3
+      gW4[e] = __builtin_fmaf(act[e], dy, gW4[e]);
+      act[e] = dy * w4[e] * d3[e];  // dZ3
     }
-    train_put<4>(s_dz[w], act, g, c);
+    train_put<4>(dzw, act, g, c);
     __syncthreads();
     // ---- layers 3 and 2: dW += A_in^T dZ over the block's samples, and
     // dZ_in = (W dZ) SiLU'(Z_in) of the wave's own
 #pragma unroll
     for (int L = 1; L >= 0; --L) {
-      const float(*aIn)[16 * kSdfHidden] = L == 1 ? s_a2 : s_a1;
-      const float(*dOut)[16 * kSdfHidden] = L == 1 ? s_dz : s_a2;
       floatx4* gW = L == 1 ? gW3 : gW2;
       float* gb = L == 1 ? gb3 : gb2;
       const int rows = L == 1 ? kRowsW3 : kRowsW2;
-#pragma unroll 2
+      int in[4], out[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        in[s] = own_register((L == 1 ? kTrainA2 : kTrainA1) + 256 * ib + at[s]);
+        out[s] = own_register((L == 1 ? kTrainDz : kTrainA2) + 256 * jb + at[s]);
+      }
+#pragma unroll
       for (int v = 0; v < kTrainWaves; ++v)
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-          const float a = aIn[v][256 * ib + at[s]];
-          const float o0 = dOut[v][256 * jb + at[s]], o1 = dOut[v][256 * (jb + 1) + at[s]];
+          const float a = S[in[s] + 1024 * v];
+          const float o0 = S[out[s] + 1024 * v], o1 = S[out[s] + 1024 * v + 256];
           gW[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, o0, gW[0], 0, 0, 0);
           gW[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, o1, gW[1], 0, 0, 0);
-          gb[0] += o0;
-          gb[1] += o1;
+        }
+#pragma unroll
+      for (int v = 0; v < 2; ++v)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          gb[0] += S[out[s] + 1024 * (2 * ib + v)];
+          gb[1] += S[out[s] + 1024 * (2 * ib + v) + 256];
         }
 #pragma unroll
       for (int ob = 0; ob < 4; ++ob) z[ob] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -373,23 +447,31 @@ __global__ __launch_bounds__(kTrainThreads) void k_sdf_grad_tiles(
 #pragma unroll
         for (int ob = 0; ob < 4; ++ob)
           z[ob] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-              s_w[(rows + 16 * (st >> 2) + 4 * ob) * kFragStride + back + (st & 3)], act[st],
-              z[ob], 0, 0, 0);
+              S[(rows + 16 * (st >> 2) + 4 * ob) * kFragStride + back + (st & 3)], act[st], z[ob],
+              0, 0, 0);
 #pragma unroll
       for (int e = 0; e < 16; ++e) act[e] = z[e >> 2][e & 3] * (L == 1 ? d2 : d1)[e];
       if (L == 1) __syncthreads();  // the readers of A2, whose place dZ2 takes
-      train_put<4>(L == 1 ? s_a2[w] : s_dz[w], act, g, c);
+      train_put<4>(L == 1 ? a2w : dzw, act, g, c);
       __syncthreads();
     }
     // ---- layer 1: dW1 += X0^T dZ1
-#pragma unroll 2
+    int in[4], out[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      in[s] = own_register(kTrainX0 + 256 * ib1 + at[s]);
+      out[s] = own_register(kTrainDz + 256 * jb1 + at[s]);
+    }
+#pragma unroll
     for (int v = 0; v < kTrainWaves; ++v)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const float o = s_dz[v][256 * jb1 + at[s]];
-        gW1 = __builtin_amdgcn_mfma_f32_16x16x4f32(s_x0[v][256 * ib1 + at[s]], o, gW1, 0, 0, 0);
-        gb1 += o;
-      }
+      for (int s = 0; s < 4; ++s)
+        gW1 = __builtin_amdgcn_mfma_f32_16x16x4f32(S[in[s] + 512 * v], S[out[s] + 1024 * v], gW1,
+                                                   0, 0, 0);
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) gb1 += S[out[s] + 1024 * (4 * ib1 + v)];
   }
   // ---- this block's sums: row 4 g + r, column c of each gradient block
   float* G = partial + ((size_t)body * nblk + blk) * kSdfStride;
@@ -403,7 +485,12 @@ __global__ __launch_bounds__(kTrainThreads) void k_sdf_grad_tiles(
     }
     G[kSdfOffW1 + in1 * kSdfHidden + 16 * jb1 + c] = gW1[r];
   }
-  // biases: the lanes of a column hold its samples' shares
+  // biases: the lanes of a column hold its samples' shares, four waves those
+  // of an output (two in layer 1); output layer and loss: over the samples
+  // (lanes of a group), then the waves
+  float* bsum = S + kTrainA1;               // [4 + 4 + 2 shares][64]
+  float* red = bsum + 10 * kSdfHidden;      // [waves][64 + 2]
+  __syncthreads();
   auto over_g = [](float v) {
     v += __shfl_xor(v, 16);
     return v + __shfl_xor(v, 32);
@@ -411,16 +498,13 @@ __global__ __launch_bounds__(kTrainThreads) void k_sdf_grad_tiles(
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
     const float v3 = over_g(gb3[b]), v2 = over_g(gb2[b]);
-    if (ib == 0 && g == 0) {
-      G[kSdfOffB3 + 16 * (jb + b) + c] = v3;
-      G[kSdfOffB2 + 16 * (jb + b) + c] = v2;
+    if (g == 0) {
+      bsum[ib * kSdfHidden + 16 * (jb + b) + c] = v3;
+      bsum[(4 + ib) * kSdfHidden + 16 * (jb + b) + c] = v2;
     }
   }
   const float v1 = over_g(gb1);
-  if (ib1 == 0 && g == 0) G[kSdfOffB1 + 16 * jb1 + c] = v1;
-  // output layer and loss: over the samples (lanes of a group), then the waves
-  float* red = &s_a1[0][0];  // [waves][64 + 2]
-  __syncthreads();
+  if (g == 0) bsum[(8 + ib1) * kSdfHidden + 16 * jb1 + c] = v1;
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
     float v = gW4[e];
@@ -448,6 +532,15 @@ __global__ __launch_bounds__(kTrainThreads) void k_sdf_grad_tiles(
       G[kSdfOffB4] = s;
     else
       lossPartial[(size_t)body * nblk + blk] = s;
+  } else if (t >= 128 && t < 128 + 3 * kSdfHidden) {
+    const int layer = (t - 128) / kSdfHidden, o = t % kSdfHidden;
+    const float* b = bsum + o + 4 * layer * kSdfHidden;
+    const float s = b[0] + b[kSdfHidden];
+    if (layer == 2)
+      G[kSdfOffB1 + o] = s;
+    else
+      G[(layer == 0 ? kSdfOffB3 : kSdfOffB2) + o] =
+          s + (b[2 * kSdfHidden] + b[3 * kSdfHidden]);
   }
 }
 
@@ -542,8 +635,6 @@ __device__ __forceinline__ bf16x8 act_operand(const floatx4& lo, const floatx4& 
                silu_fast(lo[3] + blo.w), silu_fast(hi[0] + bhi.x), silu_fast(hi[1] + bhi.y),
                silu_fast(hi[2] + bhi.z), silu_fast(hi[3] + bhi.w));
 }
-
-__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 
 // sin and cos features of one query for the lane's four frequencies (f: the
 // 12 coefficients), as the first layer's B operand.
