@@ -71,6 +71,11 @@ constexpr int kPairBatch = FC_PAIR_BATCH;
 static_assert(kRowsBatch >= 1 && (uint32_t)kRowsBatch - 1u <= kSortedPosPad, "row padding");
 // Candidates whose loads are issued together in k_collide_v3.
 constexpr int kBatch = 4;
+// Polydisperse: spheres with more candidates than this are left to
+// k_collide_piles unread.  A step of 120,011 / 17,000 spheres on the knot: no
+// bound 87.2 / 70.4 us, 128: 85.0 / 68.8, 96: 111.6 / 65.1, 64: 213 / 63 (a
+// sphere of an ordinary log-normal bed has up to 100).
+constexpr uint32_t kPileCandidates = 128;
 
 // The cursor sphere of collideD (particles_kernel.cu:286-288): its pair
 // force (at rest, no attraction) added to the 27 cells' sum.
@@ -283,8 +288,9 @@ struct RowFilter {
 //
 // A lane whose list overflows, or with a row of two runs, has a path of its
 // own at the end.  With kPoly it is left to k_collide_piles instead
-// (`left`): log-normal radii pile up in cells of 50 and more, and the wave
-// that held such lanes was the launch's tail.
+// (`left`), as is one with more than kPileCandidates: log-normal radii pile
+// up in cells of 50 and more, and the wave that held such lanes was the
+// launch's tail.
 template <bool kPoly, int BS>
 __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invCell,
                                                 float contactD2, uint32_t k, v3f pos, v3f vel,
@@ -393,6 +399,14 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
     len[r] = (n0 || n1 || n2) && b > a ? b - a : 0u;
     split = split || (wrapLo && n0 && (n1 || n2)) || (wrapHi && n2 && (n0 || n1));
   }
+  if (kPoly) {
+    uint32_t total = 0;
+#pragma unroll
+    for (int r = 0; r < 9; ++r) total += len[r];
+    left = split || total > kPileCandidates;
+#pragma unroll
+    for (int r = 0; r < 9; ++r) len[r] = left ? 0u : len[r];
+  }
 
   // ---- phase A: candidates within the contact pre-filter ----
   // The three rows of a z-plane are walked as one flattened sequence of
@@ -446,7 +460,7 @@ __device__ __forceinline__ v3f collide_one_rows(const fc_sim_params& P, v3f invC
   }
 
   v3f force = make_v3(0.0f, 0.0f, 0.0f);
-  left = kPoly && (split || cnt > (uint32_t)kListCap);
+  left = kPoly && (left || cnt > (uint32_t)kListCap);
   if (!split && cnt <= (uint32_t)kListCap) {
     // ---- phase B ----
     // kPairBatch list entries per iteration (entries past cnt load the

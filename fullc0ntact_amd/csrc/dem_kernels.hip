@@ -451,12 +451,15 @@ __global__ __launch_bounds__(kBlock, kCollideWavesPerSimd) void k_collide_v3(
 // or a row of theirs has two runs), one wave each: lanes 0-26 take a
 // neighbour cell each (those out of reach cut, as collide_one_rows does),
 // then the wave takes the cells' spheres 64 at a time through the exact pair
-// force, and each cell's lane adds its own in index order, so the 27
-// partials and their order are the reference's.  A sphere with 300
-// candidates is a chain of about five rounds here and of 90 in a lane of its
-// own, which was the launch's tail: 120,011 log-normal spheres settled on a
-// knot, fused collide 189 us with every candidate through the pair force in
-// the lane, 133 us with lists refilled in the lane, 66 us with this launch.
+// force, and each cell's lane adds its own contacts in index order, so the 27
+// partials and their order are the reference's.  Bound by the latency of the
+// rounds: the next 64 states are loaded while a round is worked on, and only
+// the contacts' forces are added.  A sphere with 300 candidates is a chain of
+// about five rounds here and of 90 in a lane of its own, which was the launch's
+// tail: 120,011 log-normal spheres settled on a knot, fused collide 189 us
+// with every candidate through the pair force in the lane, 133 us with lists
+// refilled in the lane, 61 us with this launch, 54 us with its shorter rounds
+// and the spheres of many candidates left unread.
 // Equal radii keep the lane's own path: their lists overflow only while a
 // bed is compressed, and an empty launch costs about 2 us a step.
 constexpr unsigned kPileBlocks = 512;
@@ -516,30 +519,44 @@ __global__ __launch_bounds__(kBlock) void k_collide_piles(
     }
     __builtin_amdgcn_wave_barrier();
     v3f cf = make_v3(0.0f, 0.0f, 0.0f);
-    for (uint32_t t0 = 0; t0 < total; t0 += 64u) {
-      const uint32_t t = t0 + (uint32_t)lane;
-      v3f f = make_v3(0.0f, 0.0f, 0.0f);
+    float4 pj, vj;
+    bool other = false;
+    auto fetch = [&](uint32_t t) {
+      other = false;
       if (t < total) {
         int c = 0;  // the first cell that ends past t
 #pragma unroll
         for (int step = 16; step > 0; step >>= 1)
           if (c + step <= 26 && s_end[w][c + step - 1] <= t) c += step;
         const uint32_t j = t + s_first[w][c];
-        if (j != k) {
-          const float4 pj = sortedPos[j];
-          f = collide_spheres_fast(pos0, xyz(pj), vel0, xyz(sortedVel[j]), rA, pj.w, P.spring,
-                                   P.damping, P.shear, P.attraction);
-        }
+        other = j != k;
+        pj = sortedPos[j];
+        vj = sortedVel[j];
       }
+    };
+    fetch((uint32_t)lane);
+    for (uint32_t t0 = 0; t0 < total; t0 += 64u) {
+      v3f f = make_v3(0.0f, 0.0f, 0.0f);
+      const float4 pn = pj, vn = vj;
+      const bool pair = other;
+      fetch(t0 + 64u + (uint32_t)lane);  // the next round's, while this one is worked on
+      if (pair)
+        f = collide_spheres_fast(pos0, xyz(pn), vel0, xyz(vn), rA, pn.w, P.spring, P.damping,
+                                 P.shear, P.attraction);
       s_f[w][0][lane] = f.x;
       s_f[w][1][lane] = f.y;
       s_f[w][2][lane] = f.z;
+      // (a zero force adds nothing to a partial, which is never -0)
+      const uint64_t contacts = __ballot(f.x != 0.0f || f.y != 0.0f || f.z != 0.0f);
       __builtin_amdgcn_wave_barrier();
       if (lane < 27) {
         const uint32_t a = begin > t0 ? begin : t0, b = end < t0 + 64u ? end : t0 + 64u;
-        for (uint32_t u = a; u < b; ++u)
-          cf = make_v3(cf.x + s_f[w][0][u - t0], cf.y + s_f[w][1][u - t0],
-                       cf.z + s_f[w][2][u - t0]);
+        uint64_t mine = a < b ? contacts & lanes_from(a - t0) & ~lanes_from(b - t0) : 0ull;
+        while (mine != 0ull) {
+          const uint32_t u = lowest_lane(mine);
+          mine &= mine - 1ull;
+          cf = make_v3(cf.x + s_f[w][0][u], cf.y + s_f[w][1][u], cf.z + s_f[w][2][u]);
+        }
       }
       __builtin_amdgcn_wave_barrier();
     }

@@ -279,18 +279,34 @@ __global__ __launch_bounds__(256) void k_row_changers(RowTables T, const uint32_
     const bool last = valid && (k + 1 == n || oldNext != old[i]);
     const uint64_t lastMask = __ballot(last);
     const uint64_t staysMask = __ballot(valid && (raw[i] & kMovedBit) == 0u);
+    bool clear = false, open = false;
     if (first) {
       const uint64_t ends = lastMask & lanes_from(lane);
       const uint32_t t = ends ? lowest_lane(ends) : 63u;
-      bool stays = (staysMask & lanes_from(lane) & ~lanes_from(t + 1u)) != 0ull;
-      // the cell goes on past the tile's last lane
-      for (uint32_t k2 = k + (64u - lane); !stays && ends == 0ull && k2 < n && hash[k2] == old[i];
-           ++k2)
-        stays = (keys[k2] & kMovedBit) == 0u;
-      if (!stays && old[i] < numCells) {
-        cellStart[old[i]] = CELL_EMPTY;
-        cellEnd[old[i]] = CELL_EMPTY;
+      const bool stays = (staysMask & lanes_from(lane) & ~lanes_from(t + 1u)) != 0ull;
+      clear = !stays && old[i] < numCells;
+      open = clear && ends == 0ull;
+    }
+    // the tile's last cell may go on past it with none of its spheres staying
+    // so far: the wave reads on, 64 at a time (a lane of its own reads one at a
+    // time, and a pile in free fall moves as a whole)
+    const uint64_t openMask = __ballot(open);
+    if (openMask != 0ull) {
+      const uint32_t cell =
+          (uint32_t)__builtin_amdgcn_readlane((int)old[i], (int)lowest_lane(openMask));
+      for (uint32_t base = (tile0 + i + 1u) * 64u;; base += 64u) {
+        const uint32_t k2 = base + lane;
+        const bool in = k2 < n && hash[k2] == cell;
+        if (__ballot(in && (keys[k2] & kMovedBit) == 0u) != 0ull) {
+          if (open) clear = false;
+          break;
+        }
+        if (__ballot(in) != ~0ull) break;  // (a cell's spheres are consecutive)
       }
+    }
+    if (clear) {
+      cellStart[old[i]] = CELL_EMPTY;
+      cellEnd[old[i]] = CELL_EMPTY;
     }
     const uint32_t r = (raw[i] & ~kMovedBit) >> T.shift;
     chg[i] = valid && r != (old[i] >> T.shift);

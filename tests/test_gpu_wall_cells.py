@@ -112,3 +112,33 @@ def test_own_radii_and_piles(gpu_ctx, pile):
         orc.update_ex(st, 0.5, P, None, poly=True)
     _compare_system(ps, st)
     ps.close()
+
+
+@pytest.mark.parametrize("pile", [2, 63, 64, 65, 200, 700])
+def test_piles_that_move_as_a_whole(gpu_ctx, pile):
+    """Cells all of whose spheres leave in one step, beginning anywhere in a
+    64-sphere tile and going on past it: their table entries are cleared (in a
+    run, by the changer pass).  No pair forces, a cell's edge per step."""
+    from fullc0ntact_amd import ParticleSystem, make_params
+    pos, vel = state(4)
+    rng = np.random.default_rng(pile)
+    edge = 2.0 / GRID
+    for c in range(12):
+        k = slice(c * pile, (c + 1) * pile)
+        cell = rng.integers(4, GRID - 12, 3)
+        pos[k, :3] = -1.0 + edge * (cell + 0.5) + rng.uniform(-0.2, 0.2, (pile, 3)) * edge
+        vel[k, :3] = edge / 0.5 * np.array([(c % 3 == a) for a in range(3)], np.float32)
+    if pile > 64:  # one of a pile stays behind
+        vel[11 * pile, :3] = 0.0
+    ps = ParticleSystem(N, (GRID,) * 3, context=gpu_ctx)
+    ps.m_params = make_params(N, GRID, R, spring=0.0, damping=0.0, shear=0.0)
+    ps.setArray(ps.POSITION, pos, 0, N)
+    ps.setArray(ps.VELOCITY, vel, 0, N)
+    st = orc.State(pos, vel, ps.m_params.numCells)
+    P = orc.params_from(ps.m_params)
+    print(pile, flush=True)
+    ps.run(0.5, 5)
+    for _ in range(5):
+        st.update(0.5, P)
+    _compare_system(ps, st)
+    ps.close()
