@@ -597,7 +597,8 @@ __global__ __launch_bounds__(kBlock) void k_collide_piles(
 // order (z, then y, then x), a component each, then the row-0 lane the cursor
 // sphere; the rest is k_collide_v3's tail (the scatter, or with
 // kFuse the next update's integrate, hash and histogram), with the same
-// arguments and results.
+// arguments and results (oldKey, for slotKeys and rows, is the hash that the
+// gather left in sortedVel.w).
 constexpr int kSplitSpheresPerWave = 7;
 
 template <bool kFuse, bool kPoly>
@@ -608,7 +609,7 @@ __global__ __launch_bounds__(kBlock) void k_collide_split(
     const uint32_t* __restrict__ cellEnd, uint32_t n, float4* __restrict__ pos, float dt,
     uint32_t* __restrict__ keysOut, int passes, uint32_t* gHist, uint32_t* counters,
     uint32_t* devFlags, uint32_t* __restrict__ slotOf, uint32_t* __restrict__ idOfSlot,
-    v3f invCell, float* __restrict__ forceOut) {
+    v3f invCell, float* __restrict__ forceOut, int slotKeys, RowHists rows) {
   __shared__ uint32_t s_hist[kFuse ? RS_RADIX : 1];
   __shared__ float s_cells[kBlock / 64][9 * 64];
   const int lane = (int)(threadIdx.x & 63u);
@@ -616,7 +617,8 @@ __global__ __launch_bounds__(kBlock) void k_collide_split(
   const int sl = lane / 9, r = lane - 9 * (lane / 9);
   const uint32_t k = wave * kSplitSpheresPerWave + (uint32_t)sl;
   const bool valid = lane < 9 * kSplitSpheresPerWave && k < n;
-  if (kFuse && gHist != nullptr) {
+  const bool digitHist = kFuse && rows.rowHist == nullptr && gHist != nullptr;
+  if (digitHist) {
     for (int i = threadIdx.x; i < RS_RADIX; i += kBlock) s_hist[i] = 0u;
     histogram_producer_prologue(gHist, passes, counters);
   }
@@ -625,10 +627,13 @@ __global__ __launch_bounds__(kBlock) void k_collide_split(
   v3f vel0 = make_v3(0.0f, 0.0f, 0.0f);
   float rA = P.particleRadius;
   uint32_t orig = 0;  // (read with the state: a round trip less at the end)
+  uint32_t oldKey = 0;
   if (valid) {
     p4 = sortedPos[k];
     orig = index[k];
-    vel0 = xyz(sortedVel[k]);
+    const float4 v4 = sortedVel[k];
+    vel0 = xyz(v4);
+    oldKey = __float_as_uint(v4.w);
     rA = kPoly ? p4.w : P.particleRadius;
     collide_row_cells<kPoly>(P, invCell, contactD2, k, xyz(p4), vel0, rA, r, sortedPos,
                              sortedVel, cellStart, cellEnd, n, cf);
@@ -659,13 +664,21 @@ __global__ __launch_bounds__(kBlock) void k_collide_split(
   if (owner) {
     if (kPoly && !(rA <= P.particleRadius)) atomicOr(devFlags, DEVERR_RADIUS);
     key = collide_finish<kFuse>(P, B, p4, xyz(p4), vel0, rA, force, k, orig, newVel, pos, dt,
-                                invCell, 0u, keysOut, slotOf, idOfSlot, false, forceOut);
+                                invCell, oldKey, keysOut, slotOf, idOfSlot, slotKeys != 0,
+                                forceOut);
   }
-  if (kFuse && gHist != nullptr) {
+  if (digitHist) {
     __syncthreads();
     histogram_add_digit(s_hist, key & (RS_RADIX - 1), owner);
     __syncthreads();
     histogram_flush(s_hist, gHist, 0);
+  } else if (kFuse && rows.rowHist != nullptr) {
+    // the wave's spheres side by side, so that a row's run is counted at once
+    const int from = lane < kSplitSpheresPerWave ? 9 * lane : 0;
+    const uint32_t keyL = (uint32_t)__shfl((int)key, from),
+                   oldL = (uint32_t)__shfl((int)oldKey, from);
+    const bool mine = __shfl(owner ? 1 : 0, from) != 0 && lane < kSplitSpheresPerWave;
+    row_histograms(rows, wave * kSplitSpheresPerWave + (uint32_t)lane, keyL, oldL, mine);
   }
 }
 
@@ -864,13 +877,12 @@ static void launch_v3(hipStream_t s, const GatheredState* gs, dim3 g, dim3 b,
                       const RowHists* rows = nullptr) {
   // up to RS_TILE spheres the next sort counts ranks: no digit histogram
   if (n <= (uint32_t)RS_TILE) gHist = nullptr;
-  // (the split kernel reads the reference layout only: no gathered arrays)
   if (rows_walk_ok(P) && n <= kSplitMaxSpheres) {
     const uint32_t waves = (n + kSplitSpheresPerWave - 1) / kSplitSpheresPerWave;
     hipLaunchKernelGGL((k_collide_split<kFuse, kPoly>), dim3((waves + 3) / 4), b, 0, s, P, B, d2,
                        newVel, sortedPos, sortedVel, index, cellStart, cellEnd, n, pos, dt,
                        keysOut, passes, gHist, counters, devFlags, slotOf, idOfSlot, inv_cell(P),
-                       forceOut);
+                       forceOut, slotKeys ? 1 : 0, rows ? *rows : RowHists{});
   } else if (gs != nullptr && rows_walk_ok(P)) {
     hipLaunchKernelGGL((k_collide_v3<kFuse, kPoly, true>), g, b, 0, s, P, B, d2, newVel,
                        sortedPos, sortedVel, index, cellStart, cellEnd, n, kCollideXcdGroup, pos,
@@ -921,12 +933,20 @@ hipError_t launch_collide(hipStream_t s, const fc_sim_params& P, bool poly, uint
   return hipGetLastError();
 }
 
-// Whether a run's fused collide stores the next key at the sorted slot for
-// a row resort (the row-range kernel on a grid whose row tables fit; the
-// row-split kernel of small systems keeps the key at the id and the slot
-// map, for the radix sort).
+// Whether a run's fused collide stores the next key at the sorted slot for a
+// row resort, on a grid whose row tables fit; up to RS_TILE spheres a step
+// sorts by counting ranks.  Small systems leave grids of many rows (the scan
+// reads every row) and of few (a row beyond the resort's LDS is ranked by
+// counting) to the radix sort, which carries the key at the id and the slot
+// map.  A step of 8,000 / 16,000 spheres with the resort against the radix
+// sort: 64^3 grid 27 / 29 us against 45 / 47, 256^3 30 / 34 against 45 / 48,
+// 64 x 512 x 512 37 / 39 against 45 / 47, 64 x 1024 x 1024 69 / 70 against
+// 53 / 56, 8^3 46 / 74 against 58 / 85, 4^3 143 / 1382 against 150 / 371.
 bool collide_slot_keys(const fc_sim_params& P, uint32_t n) {
-  return n > kSplitMaxSpheres && rows_walk_ok(P) && row_resort_grid_ok(P);
+  if (!rows_walk_ok(P) || !row_resort_grid_ok(P)) return false;
+  if (n > kSplitMaxSpheres) return true;
+  const uint64_t rows = (uint64_t)P.gridSize.y * P.gridSize.z;
+  return n > (uint32_t)RS_TILE && rows <= (1u << 18) && n <= 256u * rows;
 }
 
 bool collide_rows_state_pays(const fc_sim_params& P, uint32_t n) {

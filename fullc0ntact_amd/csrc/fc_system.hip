@@ -162,7 +162,7 @@ fc_status enqueue_update(fc_system* sys, float dt, StageTimer* timer) {
 // which computes exactly what `steps` separate updates compute.
 // Between the fused steps the particle state stays in the previous sort's
 // order: the fused collide writes pos/vel at each particle's sorted slot k
-// (coalesced) and idOfSlot[k] = id.  For large systems (run_row_mode) it
+// (coalesced) and idOfSlot[k] = id.  Over RS_TILE spheres (run_row_mode) it
 // stores the next hash at the slot too, with the per-row counts, and the
 // next sort is a row resort (row_resort.hip), whose result is the (cell,
 // id) order of the separate updates; the run's first sort (keys by id,
