@@ -237,6 +237,12 @@ __global__ __launch_bounds__(256) void k_row_starts(RowTables T, const uint32_t*
   if (r < T.rows) T.count[r] = row_start_in(hash, n, T.rows, T.shift, r + 1u) - lo;
 }
 
+// Buckets of a tile whose lanes add together.  1M bed / 120,011 spheres on the
+// knot (nearly all of whose piles change row): 0: 9.9 / 5.6 us, 2: 8.1 / 5.7,
+// 4: 7.5 / 5.7, 8: 7.4 / 6.0, all: 7.5 / 8.0 (and 9.5 for 12,000 spheres, 4.8
+// with 4: a loop over up to 64 buckets).
+constexpr uint32_t kChgBuckets = 4;
+
 // One lane per current sorted entry k (keys[k] is the next key with
 // kMovedBit when the cell changes, hash[k] the current one), each wave over
 // kChgTiles consecutive 64-slot tiles with every tile's loads, then every
@@ -324,16 +330,19 @@ __global__ __launch_bounds__(256) void k_row_changers(RowTables T, const uint32_
       }
     }
   }
-  // one atomic per bucket and tile: the lowest lane of each bucket's lanes
-  // (its leader) adds their count, every lane takes the leader's result
-  // plus its rank among them; the leaders of both tiles add in one go
+  // one atomic per bucket and tile for the first few buckets: the lowest lane
+  // of each bucket's lanes (its leader) adds their count, every lane takes the
+  // leader's result plus its rank among them; lanes of further buckets add for
+  // themselves, all in one go
   uint32_t leader[kChgTiles], rank[kChgTiles], cnt[kChgTiles], at[kChgTiles];
 #pragma unroll
   for (uint32_t i = 0; i < kChgTiles; ++i) {
     leader[i] = lane;
-    rank[i] = cnt[i] = 0u;
+    rank[i] = 0u;
+    cnt[i] = 1u;
     uint64_t pending = __ballot(chg[i]);
-    while (pending != 0ull) {
+#pragma unroll 1
+    for (uint32_t b = 0; b < kChgBuckets && pending != 0ull; ++b) {
       const uint32_t l = lowest_lane(pending);
       const uint32_t bl = __builtin_amdgcn_readlane(bucket[i], l);
       const uint64_t peers = __ballot(chg[i] && bucket[i] == bl);
