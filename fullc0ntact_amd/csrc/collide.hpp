@@ -72,10 +72,10 @@ static_assert(kRowsBatch >= 1 && (uint32_t)kRowsBatch - 1u <= kSortedPosPad, "ro
 // Candidates whose loads are issued together in k_collide_v3.
 constexpr int kBatch = 4;
 // Polydisperse: spheres with more candidates than this are left to
-// k_collide_piles unread.  A step of 120,011 / 17,000 spheres on the knot: no
-// bound 87.2 / 70.4 us, 128: 85.0 / 68.8, 96: 111.6 / 65.1, 64: 213 / 63 (a
-// sphere of an ordinary log-normal bed has up to 100).
-constexpr uint32_t kPileCandidates = 128;
+// k_collide_piles unread.  A step of 20,000 / 120,011 / 200,000 spheres on the
+// knot (the more, the denser): 96: 59 / 101 / 187 us, 128: 62 / 77 / 112, 144:
+// 64 / 78 / 100, 160: 65 / 79 / 89; no bound, with one counter: 70 / 87 / -.
+constexpr uint32_t kPileCandidates = 144;
 
 // The cursor sphere of collideD (particles_kernel.cu:286-288): its pair
 // force (at rest, no attraction) added to the 27 cells' sum.

@@ -430,7 +430,7 @@ __global__ __launch_bounds__(kBlock, kCollideWavesPerSimd) void k_collide_v3(
               : collide_one_v3<kPoly, kBlock>(P, contactD2, k, pos0, vel0, rA, sortedPos,
                                               sortedVel, cellStart, cellEnd, n, s_list);
     if (kPoly && kRows && left) {
-      piles[2 + atomicAdd(&piles[0], 1u)] = k;
+      piles[kPilesList + atomicAdd(&piles[0], 1u)] = k;
     } else {
       key = collide_finish<kFuse>(P, B, p4, pos0, vel0, rA, force, k, index[k], newVel, pos, dt,
                                   invCell, oldKey, keysOut, slotOf, idOfSlot, slotKeys != 0,
@@ -458,11 +458,13 @@ __global__ __launch_bounds__(kBlock, kCollideWavesPerSimd) void k_collide_v3(
 // about five rounds here and of 90 in a lane of its own, which was the launch's
 // tail: 120,011 log-normal spheres settled on a knot, fused collide 189 us
 // with every candidate through the pair force in the lane, 133 us with lists
-// refilled in the lane, 61 us with this launch, 54 us with its shorter rounds
-// and the spheres of many candidates left unread.
+// refilled in the lane, 61 us with this launch; 50 us (36 + 14) with its
+// shorter rounds, the spheres of many candidates left unread and its blocks
+// reporting to 32 counters (to one: 5 us more for 512 blocks).
 // Equal radii keep the lane's own path: their lists overflow only while a
 // bed is compressed, and an empty launch costs about 2 us a step.
-constexpr unsigned kPileBlocks = 512;
+constexpr unsigned kPileBlocks = 768;  // three waves per SIMD (152 VGPRs)
+static_assert(kPileBlocks >= kPilesParts, "every part has a block");
 
 template <bool kFuse>
 __global__ __launch_bounds__(kBlock) void k_collide_piles(
@@ -479,7 +481,7 @@ __global__ __launch_bounds__(kBlock) void k_collide_piles(
   const uint32_t count = min(piles[0], n);
   for (uint32_t i = blockIdx.x * (kBlock / 64) + (uint32_t)w; i < count;
        i += gridDim.x * (kBlock / 64)) {
-    const uint32_t k = piles[2 + i];
+    const uint32_t k = piles[kPilesList + i];
     const float4 p4 = sortedPos[k], v4 = sortedVel[k];
     const v3f pos0 = xyz(p4), vel0 = xyz(v4);
     const float rA = p4.w, reach = rA + P.particleRadius;
@@ -581,11 +583,19 @@ __global__ __launch_bounds__(kBlock) void k_collide_piles(
     }
     __builtin_amdgcn_wave_barrier();
   }
-  // every block has read the count before it reports here
+  // every block has read the count before it reports here: to a counter that
+  // few share (one for all took 10 ns a block), whose last one reports on
   __syncthreads();
-  if (threadIdx.x == 0 && atomicAdd(&piles[1], 1u) == gridDim.x - 1u) {
-    piles[0] = 0u;
-    piles[1] = 0u;
+  if (threadIdx.x == 0) {
+    const uint32_t part = blockIdx.x % kPilesParts;
+    uint32_t* done = piles + 16u * (1u + part);
+    if (atomicAdd(done, 1u) == (gridDim.x - part + kPilesParts - 1u) / kPilesParts - 1u) {
+      *done = 0u;
+      if (atomicAdd(&piles[1], 1u) == kPilesParts - 1u) {
+        piles[0] = 0u;
+        piles[1] = 0u;
+      }
+    }
   }
 }
 

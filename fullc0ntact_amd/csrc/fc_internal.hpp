@@ -257,8 +257,10 @@ hipError_t launch_reorder(hipStream_t s, uint32_t* cellStart, uint32_t* cellEnd,
 // position; else outside (if given) holds `epoch` when launch_rows_state
 // found a sphere whose cell index lies outside the grid.
 // piles: [0] the number of spheres that a polydisperse collide left to
-// k_collide_piles, [1] its finished blocks (both zero between launches),
-// then their sorted indices (n words).
+// k_collide_piles, [1] and one word of each later 64-byte line up to the list
+// the blocks of that launch that are done (all zero between steps), from
+// [kPilesList] on the spheres.
+constexpr uint32_t kPilesParts = 32, kPilesList = 16u * (1u + kPilesParts);
 struct GatheredState {
   const uint2* sortedQ = nullptr;
   QuantFrame frame;

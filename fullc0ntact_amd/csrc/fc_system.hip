@@ -434,9 +434,9 @@ fc_status fc_system_set_polydisperse(fc_system* sys, int enable) {
   if (!sys) return set_error(FC_ERROR_INVALID_VALUE, "sys is NULL");
   FC_HIP_TRY(hipStreamSynchronize(sys->ctx->stream));
   if (enable && !sys->piles) {
-    const size_t words = (size_t)sys->n + 2;
+    const size_t words = (size_t)sys->n + kPilesList;
     FC_HIP_TRY(hipMalloc(&sys->piles, words * sizeof(uint32_t)));
-    FC_HIP_TRY(hipMemset(sys->piles, 0, 2 * sizeof(uint32_t)));
+    FC_HIP_TRY(hipMemset(sys->piles, 0, kPilesList * sizeof(uint32_t)));
   }
   sys->polydisperse = enable ? 1 : 0;
   drop_graph(sys);  // the captured step carries the radius mode in its kernels
