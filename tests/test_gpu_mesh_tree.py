@@ -112,3 +112,16 @@ def test_points_not_finite(gpu_ctx):
     sd, cp = mesh_signed_distance(gpu_ctx, v, f, p)
     rsd, rcp, _ = orc.mesh_sdf(v, f, p)
     assert np.array_equal(sd, rsd) and np.array_equal(cp, rcp)
+
+
+@pytest.mark.parametrize("name", ["knot512x16", "knot513x16"])
+def test_points_of_either_key(gpu_ctx, name):
+    """The largest mesh whose triangles are ordered by the short key (16,384)
+    and the next."""
+    from fullc0ntact_amd.distance_map import mesh_signed_distance
+    v, f = mesh(name)
+    q = np.random.default_rng(11).uniform(-0.8, 0.8, (300, 3))
+    q[:20] = v[:20]
+    print(name, len(f), flush=True)
+    sd, cp = mesh_signed_distance(gpu_ctx, v, f, q)
+    check(sd, cp, v, f, q, False)
