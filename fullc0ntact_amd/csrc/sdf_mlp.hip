@@ -257,7 +257,7 @@ __global__ __launch_bounds__(kTrainThreads) void k_sdf_grad_tiles(
     const float* __restrict__ params, const float* __restrict__ freq,
     const float* __restrict__ frame, const float* __restrict__ pts,
     const float* __restrict__ labels, uint32_t samplesPerBody, uint32_t batchStart,
-    uint32_t batchSize, uint32_t tilesPerBlock, float invM, float* __restrict__ partial,
+    uint32_t batchSize, uint32_t tilesPerBlock, float samples, float* __restrict__ partial,
     float* __restrict__ lossPartial) {
   __shared__ __attribute__((aligned(16))) float S[kTrainLds];
 
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(kTrainThreads) void k_sdf_grad_tiles(
     if (now) {
       const float err = (y + b4) - target;
       if (g == 0) lossAcc += err * err;
-      dy = 2.0f * err * invM;
+      dy = 2.0f * err / samples;  // (a rounded 1 / M puts the whole gradient off by its rounding)
     }
     if (g == 0) gb4 += dy;
 #pragma unroll
@@ -544,33 +544,38 @@ __global__ __launch_bounds__(kTrainThreads) void k_sdf_grad_tiles(
   }
 }
 
+// Sum of nblk values `stride` floats apart: eight running sums, whose loads
+// are in flight together, then a tree over them.  One running sum of 42 blocks'
+// partials had rounded to a relative 1e-7, more than the blocks themselves.
+__device__ __forceinline__ float sum_partials(const float* __restrict__ at, uint32_t nblk,
+                                              size_t stride) {
+  float s[8] = {};
+  uint32_t k = 0;
+  for (; k + 8 <= nblk; k += 8)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s[u] += at[(size_t)(k + u) * stride];
+#pragma unroll
+  for (int u = 0; u < 7; ++u)
+    if (k + u < nblk) s[u] += at[(size_t)(k + u) * stride];
+  return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
+
 // Sum of the block partials per parameter (fixed order), then either the
 // plain gradient (adam == 0) or an Adam step on the parameters.
 __global__ __launch_bounds__(kTB) void k_sdf_reduce_step(
     const float* __restrict__ partial, const float* __restrict__ lossPartial, uint32_t nblk,
     uint32_t B, float* __restrict__ grad, float* __restrict__ loss, int adam,
     float* __restrict__ params, float* __restrict__ m, float* __restrict__ v, float lr,
-    float corr1, float corr2, float invM) {
+    float corr1, float corr2, float samples) {
   const size_t idx = (size_t)blockIdx.x * kTB + threadIdx.x;
   if (idx >= (size_t)B * kSdfStride) return;
   const uint32_t b = (uint32_t)(idx / kSdfStride);
   const uint32_t p = (uint32_t)(idx % kSdfStride);
   if (p >= (uint32_t)kSdfParams) return;  // padding
-  float g = 0.0f;
-  const float* at = partial + (size_t)b * nblk * kSdfStride + p;
-  uint32_t k = 0;
-  for (; k + 8 <= nblk; k += 8) {  // eight loads in flight, added in order
-    float v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = at[(size_t)(k + u) * kSdfStride];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) g += v[u];
-  }
-  for (; k < nblk; ++k) g += at[(size_t)k * kSdfStride];
+  const float g = sum_partials(partial + (size_t)b * nblk * kSdfStride + p, nblk, kSdfStride);
   if (p == 0) {
-    float l = 0.0f;
-    for (uint32_t q = 0; q < nblk; ++q) l += lossPartial[(size_t)b * nblk + q];
-    loss[b] += l * invM;
+    const float l = sum_partials(lossPartial + (size_t)b * nblk, nblk, 1);
+    loss[b] += l / samples;
   }
   if (!adam) {
     grad[idx] = g;
@@ -1303,10 +1308,10 @@ fc_status sdf_step(fc_sdf* m, const float* pts, const float* labels, uint32_t sa
   if (perBlock > 8) perBlock = 8;
   const uint32_t nblk = (uint32_t)((tiles + perBlock - 1) / perBlock);
   FC_TRY(ensure_partials(m, (size_t)m->B * nblk * kSdfStride, (size_t)m->B * nblk));
-  const float invM = 1.0f / (float)batchSize;
+  const float samples = (float)batchSize;
   hipLaunchKernelGGL(k_sdf_grad_tiles, dim3(nblk, m->B), dim3(kTrainThreads), 0, st,
                      m->params, m->freq, m->frame, pts, labels, samplesPerBody, batchStart,
-                     batchSize, (uint32_t)perBlock, invM, m->partial, m->lossPartial);
+                     batchSize, (uint32_t)perBlock, samples, m->partial, m->lossPartial);
   FC_HIP_TRY(hipGetLastError());
   float c1 = 1.0f, c2 = 1.0f;
   if (adam) {
@@ -1318,7 +1323,7 @@ fc_status sdf_step(fc_sdf* m, const float* pts, const float* labels, uint32_t sa
   const size_t total = (size_t)m->B * kSdfStride;
   hipLaunchKernelGGL(k_sdf_reduce_step, dim3((unsigned)((total + kTB - 1) / kTB)), dim3(kTB), 0,
                      st, m->partial, m->lossPartial, nblk, m->B, m->grad, m->lossOut, adam,
-                     m->params, m->adamM, m->adamV, lr, c1, c2, invM);
+                     m->params, m->adamM, m->adamV, lr, c1, c2, samples);
   FC_HIP_TRY(hipGetLastError());
   return FC_SUCCESS;
 }

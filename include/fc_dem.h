@@ -276,7 +276,8 @@ fc_status fc_system_set_boundary(fc_system* sys, fc_boundary mode, const fc_dist
  * neighbour search and the contact pre-filter; the cell size must be at
  * least twice it); a larger pos.w is reported as FC_ERROR_INVALID_VALUE at
  * the next synchronising call.  With every pos.w equal to particleRadius
- * the results are bit-identical to the monodisperse step. */
+ * the results are bit-identical to the monodisperse step.  The first call
+ * that enables it allocates a list of 4 bytes per sphere. */
 fc_status fc_system_set_polydisperse(fc_system* sys, int enable);
 
 /* ------------------------------------------------------------------------- */
@@ -300,7 +301,11 @@ fc_status fc_distmap_create(fc_context* ctx, const int32_t cells[3], float cellS
  * signed distance (negative inside), closest point, normal = vertex - closest
  * point (DistanceMapMesh::ComputeDistance, distancegridcgal.hpp:36-71, with
  * the exact distance of D. Eberly's point-triangle method and the sign of the
- * generalized winding number instead of CGAL). */
+ * generalized winding number instead of CGAL).  Meshes of 128 to 2^22
+ * triangles that turn out closed are searched through a tree in the context's
+ * scratch (about 130 bytes a triangle, kept for the next call); other meshes,
+ * and any when the scratch cannot grow, triangle by triangle.  The results are
+ * the same bit for bit. */
 fc_status fc_distmap_build(fc_context* ctx, const double* vertices, uint32_t numVertices,
                            const uint32_t* triangles, uint32_t numTriangles,
                            const int32_t cells[3], float cellSize, const float bmin[3],
@@ -370,7 +375,10 @@ fc_status fc_integrate_system_distmap(fc_context* ctx, const fc_distmap* map, fl
                                       float* vel, float deltaTime, uint32_t numParticles);
 /* Exact signed distance (and closest point, may be NULL) of numPoints
  * points to a closed triangle mesh, all arrays on the device (binary64,
- * 3 per vertex/point, 3 indices per triangle; indices must be < numVertices). */
+ * 3 per vertex/point, 3 indices per triangle; indices must be < numVertices).
+ * Through the tree of fc_distmap_build (and 8 bytes of scratch a point, up to
+ * 2^22 points at a time) where that applies; inside a stream capture, where
+ * nothing may be allocated, triangle by triangle. */
 fc_status fc_mesh_signed_distance(fc_context* ctx, const double* vertices, uint32_t numVertices,
                                   const uint32_t* triangles, uint32_t numTriangles,
                                   const double* points, uint32_t numPoints, double* sdf,
