@@ -991,18 +991,22 @@ fc_status fc_distmap_query(fc_context* ctx, const fc_distmap* m, const float* po
   // From 2^17 points on two threads take a point (k_distmap_query_pairs);
   // fewer do not fill the card, and a thread each is up to 7 % faster: 100,000
   // points in 32^3 / 64^3 cells 5.3 / 7.5 us against 5.6 / 7.3, 200,000 in 32^3
-  // 8.5 against 8.3.  Up to 2^30 points a launch.
-  constexpr uint64_t kMost = 1ull << 30;
-  for (uint64_t at = 0; at < n; at += kMost) {
-    const uint32_t count = (uint32_t)std::min<uint64_t>(n - at, kMost);
-    const bool pairs = n >= (1u << 17);
-    hipLaunchKernelGGL(pairs ? k_distmap_query_pairs : k_distmap_query,
-                       dim3(grid_for(pairs ? 2 * (uint64_t)count : count, kBlock)), dim3(kBlock), 0,
-                       ctx->stream, distmap_view(m), points + 3 * at, count, dist + at,
-                       cp ? cp + 3 * at : nullptr, normal ? normal + 3 * at : nullptr);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return hip_error(e, "distmap query");
+  // 8.5 against 8.3.
+  if (n < (1u << 17)) {
+    hipLaunchKernelGGL(k_distmap_query, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, ctx->stream,
+                       distmap_view(m), points, n, dist, cp, normal);
+  } else {
+    constexpr uint64_t kMost = 1ull << 30;  // points of one launch
+    for (uint64_t at = 0; at < n; at += kMost) {
+      const uint32_t count = (uint32_t)std::min<uint64_t>(n - at, kMost);
+      hipLaunchKernelGGL(k_distmap_query_pairs, dim3(grid_for(2 * (uint64_t)count, kBlock)),
+                         dim3(kBlock), 0, ctx->stream, distmap_view(m), points + 3 * at, count,
+                         dist + at, cp ? cp + 3 * at : nullptr,
+                         normal ? normal + 3 * at : nullptr);
+    }
   }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return hip_error(e, "distmap query");
   return FC_SUCCESS;
 }
 
