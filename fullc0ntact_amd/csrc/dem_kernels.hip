@@ -959,6 +959,8 @@ bool collide_slot_keys(const fc_sim_params& P, uint32_t n) {
   return n > (uint32_t)RS_TILE && rows <= (1u << 18) && n <= 256u * rows;
 }
 
+bool collide_rows_optional(uint32_t n) { return n <= kSplitMaxSpheres; }
+
 bool collide_rows_state_pays(const fc_sim_params& P, uint32_t n) {
   return rows_walk_ok(P) && n > kSplitMaxSpheres && n < (1u << 27);
 }

@@ -306,6 +306,8 @@ bool collide_can_fuse(const fc_sim_params& P, uint32_t n);
 // Whether a run's fused collide stores the next key at the sorted slot
 // (then the run's later sorts are row resorts).
 bool collide_slot_keys(const fc_sim_params& P, uint32_t n);
+// Whether such a run may keep the key at the id and sort by radix instead.
+bool collide_rows_optional(uint32_t n);
 hipError_t launch_collide_fused(hipStream_t s, const fc_sim_params& P, const BoundaryArg& B,
                                 float4* pos, float4* vel,
                                 const float4* sortedPos, const float4* sortedVel,
@@ -453,8 +455,10 @@ struct fc_system {
   int polydisperse = 0;
   uint32_t* piles = nullptr;  // GatheredState::piles, once polydisperse
   // Row resort tables of multi-step runs (allocated by the first run that
-  // uses them).
+  // uses them), and whether there was no memory for those of a system that
+  // can do without (collide_rows_optional): its runs then sort by radix.
   fc::RowTables rowTables;
+  bool noRowTables = false;
   fc::BoundaryArg boundary_arg() const;
   fc::QuantFrame quant_frame() const;
   // whether integrate's box walls, with one radius, bound every position

@@ -181,7 +181,9 @@ int run_passes(const fc_sim_params& P) {
 // Whether a run's steps after its first sort resort the spheres row by row
 // (row_resort.hip) instead of radix-sorting them: then the fused collide
 // stores the next keys at the sorted slots.
-bool run_row_mode(const fc_system* sys) { return collide_slot_keys(sys->params, sys->n); }
+bool run_row_mode(const fc_system* sys) {
+  return !sys->noRowTables && collide_slot_keys(sys->params, sys->n);
+}
 
 fc_status enqueue_run_head(fc_system* sys, float dt, StageTimer* timer) {
   fc_context* ctx = sys->ctx;
@@ -575,7 +577,16 @@ fc_status fc_system_run(fc_system* sys, float deltaTime, uint32_t steps) {
     return FC_SUCCESS;
   }
   StageTimer* timer = ctx->timer.enabled ? &ctx->timer : nullptr;
-  if (run_row_mode(sys)) FC_TRY(ensure_row_tables(sys->rowTables, sys->params, sys->n));
+  if (run_row_mode(sys)) {
+    const fc_status s = ensure_row_tables(sys->rowTables, sys->params, sys->n);
+    if (s != FC_SUCCESS) {
+      // small systems can do without; the captured steps may not mix the two
+      if (!collide_rows_optional(sys->n)) return s;
+      (void)hipGetLastError();
+      sys->noRowTables = true;
+      drop_graph(sys);
+    }
+  }
   FC_TRY(enqueue_run_head(sys, deltaTime, timer));
   FC_TRY(enqueue_run_body(sys, deltaTime, /*clearInSort=*/false, /*last=*/false,
                           /*fromSlots=*/false, timer));
