@@ -869,11 +869,12 @@ static WrapCut wrap_cut(const fc_sim_params& P, const GatheredState& gs) {
   return w;
 }
 
-// Systems up to this many spheres take the row-split collide (k_collide_split).
-#ifndef FC_SPLIT_MAX_SPHERES
-#define FC_SPLIT_MAX_SPHERES 16384
-#endif
-constexpr uint32_t kSplitMaxSpheres = FC_SPLIT_MAX_SPHERES;
+// Systems up to this many spheres take the row-split collide
+// (k_collide_split): a step of a run of 20,000 / 32,000 / 48,000 spheres of
+// one radius with it 26.7 / 30.5 / 35.4 us, with the row-range kernel 31.7 /
+// 33.8 / 33.5; with radii of their own, piled on the knot, 20,000 / 26,000
+// 67.9 / 79.5 against 70.2 / 70.6.
+constexpr uint32_t kSplitMaxSpheres = 32768, kSplitMaxPoly = 16384;
 
 template <bool kFuse, bool kPoly>
 static void launch_v3(hipStream_t s, const GatheredState* gs, dim3 g, dim3 b,
@@ -887,7 +888,7 @@ static void launch_v3(hipStream_t s, const GatheredState* gs, dim3 g, dim3 b,
                       const RowHists* rows = nullptr) {
   // up to RS_TILE spheres the next sort counts ranks: no digit histogram
   if (n <= (uint32_t)RS_TILE) gHist = nullptr;
-  if (rows_walk_ok(P) && n <= kSplitMaxSpheres) {
+  if (rows_walk_ok(P) && n <= (kPoly ? kSplitMaxPoly : kSplitMaxSpheres)) {
     const uint32_t waves = (n + kSplitSpheresPerWave - 1) / kSplitSpheresPerWave;
     hipLaunchKernelGGL((k_collide_split<kFuse, kPoly>), dim3((waves + 3) / 4), b, 0, s, P, B, d2,
                        newVel, sortedPos, sortedVel, index, cellStart, cellEnd, n, pos, dt,
@@ -954,12 +955,12 @@ hipError_t launch_collide(hipStream_t s, const fc_sim_params& P, bool poly, uint
 // 53 / 56, 8^3 46 / 74 against 58 / 85, 4^3 143 / 1382 against 150 / 371.
 bool collide_slot_keys(const fc_sim_params& P, uint32_t n) {
   if (!rows_walk_ok(P) || !row_resort_grid_ok(P)) return false;
-  if (n > kSplitMaxSpheres) return true;
+  if (!collide_rows_optional(n)) return true;
   const uint64_t rows = (uint64_t)P.gridSize.y * P.gridSize.z;
   return n > (uint32_t)RS_TILE && rows <= (1u << 18) && n <= 256u * rows;
 }
 
-bool collide_rows_optional(uint32_t n) { return n <= kSplitMaxSpheres; }
+bool collide_rows_optional(uint32_t n) { return n <= 16384u; }
 
 bool collide_rows_state_pays(const fc_sim_params& P, uint32_t n) {
   return rows_walk_ok(P) && n > kSplitMaxSpheres && n < (1u << 27);

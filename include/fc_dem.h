@@ -182,7 +182,7 @@ fc_status fc_reorder_data_and_find_cell_start(fc_context* ctx, uint32_t* cellSta
 
 /* collide (particleSystem.cuh:52-59; collideD, particles_kernel.cu:256-293):
  * 27-cell spring-dashpot-shear force plus the collider sphere, written as
- * newVel[index[k]] = (vel + force, 0).  Above 16384 particles the context
+ * newVel[index[k]] = (vel + force, 0).  Above 32768 particles the context
  * first builds, in buffers of its own, each sorted particle's velocity with
  * its cell hash and its 16-bit coordinates (the arrays are assumed to come
  * from fc_reorder_data_and_find_cell_start of the hashes fc_calc_hash gives
