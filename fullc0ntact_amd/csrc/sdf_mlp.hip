@@ -1,7 +1,6 @@
 // Learned signed-distance surrogate (network in sdf_mlp.hpp): GPU training
 // by this file's own forward/backward kernels (FP32, deterministic), the
-// reference FP32 forward, and the BF16 MFMA inference kernel (FP32
-// accumulation) used to cull far-field boundary queries.
+// FP32 MFMA forward, and the BF16 MFMA inference kernel (FP32 accumulation) used to cull far-field boundary queries.
 #include "fc_internal.hpp"
 #include "distmap.hpp"
 #include "sdf_mlp.hpp"
@@ -94,13 +93,11 @@ constexpr int kTB = 256;  // inference block
 // The network in registers: under 256 of them.
 constexpr int kInferWavesPerSimd = 2;
 
-__device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + __expf(-z)); }
 // SiLU of the inference path: the hardware exp2 and reciprocal (about 1 ulp
-// each) instead of the IEEE division of the training arithmetic.
+// each) instead of the corrected reciprocal of the training arithmetic.
 __device__ __forceinline__ float silu_fast(float z) {
   return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.4426950408889634f));
 }
-__device__ __forceinline__ float silu(float z) { return z * sigmoidf_(z); }
 
 // sin(2 pi t) and cos(2 pi t) with the hardware's revolution-based
 // instructions after reducing t to [-1/2, 1/2].
@@ -122,53 +119,6 @@ __device__ __forceinline__ uint16_t bf16_rne(float f) {
   uint32_t u = __float_as_uint(f);
   u += 0x7fffu + ((u >> 16) & 1u);
   return (uint16_t)(u >> 16);
-}
-
-// ---------------------------------------------------------------------------
-// Reference FP32 forward, one lane per query.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kTB) void k_sdf_eval_f32(const float* __restrict__ params,
-                                                      const float* __restrict__ freq,
-                                                      const float* __restrict__ frame,
-                                                      const uint32_t* __restrict__ bodies,
-                                                      uint32_t numBodies,
-                                                      const float* __restrict__ pts, uint32_t n,
-                                                      float* __restrict__ out) {
-  const uint32_t q = blockIdx.x * kTB + threadIdx.x;
-  if (q >= n) return;
-  const uint32_t b = bodies ? bodies[q] : 0u;
-  if (b >= numBodies) {
-    out[q] = __int_as_float(0x7fc00000);
-    return;
-  }
-  const float* P = params + (size_t)b * kSdfStride;
-  const float* F = freq + (size_t)b * kSdfFreqs * 3;
-  const float* fr = frame + (size_t)b * 4;
-  float x, y, z;
-  sdf_norm(fr, pts[3 * q], pts[3 * q + 1], pts[3 * q + 2], x, y, z);
-  float f[kSdfIn];
-  for (int k = 0; k < kSdfFreqs; ++k) {
-    const float t = F[3 * k] * x + F[3 * k + 1] * y + F[3 * k + 2] * z;
-    sincos_rev(t, f[k], f[kSdfFreqs + k]);
-  }
-  float h[kSdfHidden], g[kSdfHidden];
-  for (int o = 0; o < kSdfHidden; ++o) {
-    float a = P[kSdfOffB1 + o];
-    for (int i = 0; i < kSdfIn; ++i) a += f[i] * P[kSdfOffW1 + i * kSdfHidden + o];
-    h[o] = silu(a);
-  }
-  for (int o = 0; o < kSdfHidden; ++o) {
-    float a = P[kSdfOffB2 + o];
-    for (int i = 0; i < kSdfHidden; ++i) a += h[i] * P[kSdfOffW2 + i * kSdfHidden + o];
-    g[o] = silu(a);
-  }
-  float yv = P[kSdfOffB4];
-  for (int o = 0; o < kSdfHidden; ++o) {
-    float a = P[kSdfOffB3 + o];
-    for (int i = 0; i < kSdfHidden; ++i) a += g[i] * P[kSdfOffW3 + i * kSdfHidden + o];
-    yv += silu(a) * P[kSdfOffW4 + o];
-  }
-  out[q] = yv * fr[3];
 }
 
 // ---------------------------------------------------------------------------
@@ -668,6 +618,7 @@ __device__ __forceinline__ bf16x8 feature_operand(const float* f, float x, float
 // those and three waves per SIMD: their latency is longer than what they
 // save).
 struct SdfNet {
+  static constexpr int kTable = 0;  // words of LDS a wave
   bf16x8 frag[kSdfFrags];
   floatx4 bias[3][4], w4[4];  // of rows 16 ob + 4g .. + 3
   float f[12];                // of frequencies 4g .. 4g + 3
@@ -675,7 +626,8 @@ struct SdfNet {
 
   __device__ __forceinline__ void load(const uint16_t* __restrict__ packed,
                                        const float* __restrict__ params,
-                                       const float* __restrict__ freq, uint32_t net, int lane) {
+                                       const float* __restrict__ freq, uint32_t net, int lane,
+                                       float*) {
     const int g = lane >> 4;
     const float* P = params + (size_t)net * kSdfStride;
     const float* F = freq + (size_t)net * kSdfFreqs * 3 + 12 * g;
@@ -774,12 +726,106 @@ __device__ __forceinline__ float sdf_tile_mfma_loaded(const uint16_t* __restrict
   return yv + P[kSdfOffB4];
 }
 
+// The network in binary32 on the 16x16x4 FP32 MFMA (sums are chains of fused
+// multiply-adds), laid out as in the training kernel: a layer's output
+// registers are the next one's B operand.  The weights' operands stay in
+// registers (160), biases and the last layer in a table of the wave's in LDS.
+//
+// Bound by the FP32 units, which matrix and vector instructions share: 160
+// MFMAs of 32 cycles and 48 activations a lane for each tile.  Calls with a
+// lane a query, its layers in scratch memory, and with this: 500,003 queries of
+// 8 networks in order 1,466 and 117 us, in random order 5,326 and 888 (a tile
+// then runs once per network in it); 1,000 queries 528 and 12 us.  Relative
+// error against binary64 4.7e-7 and 4.5e-7.
+struct SdfNet32 {
+  static constexpr int kTable = 4 * kSdfHidden;  // b1, b2, b3, w4
+  float w1[32], w2[64], w3[64];  // [16 outputs ob][step 4 ob' + r]: input 16 ob' + 4 g + r
+  float f[12];                   // of frequencies 4g .. 4g + 3
+  float b4;
+  const float* table;
+
+  __device__ __forceinline__ void load(const uint16_t*, const float* __restrict__ params,
+                                       const float* __restrict__ freq, uint32_t net, int lane,
+                                       float* tab) {
+    const int g = lane >> 4, c = lane & 15;
+    const float* P = params + (size_t)net * kSdfStride;
+    const float* F = freq + (size_t)net * kSdfFreqs * 3 + 12 * g;
+    const float* W = P + 4 * g * kSdfHidden + c;
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob) {
+#pragma unroll
+      for (int st = 0; st < 8; ++st)
+        w1[8 * ob + st] = W[kSdfOffW1 + (16 * (st >> 2) + (st & 3)) * kSdfHidden + 16 * ob];
+#pragma unroll
+      for (int st = 0; st < 16; ++st) {
+        const int in = (16 * (st >> 2) + (st & 3)) * kSdfHidden + 16 * ob;
+        w2[16 * ob + st] = W[kSdfOffW2 + in];
+        w3[16 * ob + st] = W[kSdfOffW3 + in];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 12; ++j) f[j] = F[j];
+    b4 = P[kSdfOffB4];
+    const float b1 = P[kSdfOffB1 + lane], b2 = P[kSdfOffB2 + lane], b3 = P[kSdfOffB3 + lane],
+                v4 = P[kSdfOffW4 + lane];
+    __builtin_amdgcn_wave_barrier();
+    tab[lane] = b1;
+    tab[kSdfHidden + lane] = b2;
+    tab[2 * kSdfHidden + lane] = b3;
+    tab[3 * kSdfHidden + lane] = v4;
+    __builtin_amdgcn_wave_barrier();
+    table = tab + 4 * g;
+  }
+
+  __device__ __forceinline__ float eval(float x, float y, float z) const {
+    float act[16];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      sincos_rev(f[3 * j] * x + f[3 * j + 1] * y + f[3 * j + 2] * z, act[j], act[4 + j]);
+    layer<8>(w1, 0, act);
+    layer<16>(w2, 1, act);
+    layer<16>(w3, 2, act);
+    float yv = 0.0f;
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob) {
+      const float4 w = ld4(table + 3 * kSdfHidden + 16 * ob);
+      yv = __builtin_fmaf(act[4 * ob], w.x, yv);
+      yv = __builtin_fmaf(act[4 * ob + 1], w.y, yv);
+      yv = __builtin_fmaf(act[4 * ob + 2], w.z, yv);
+      yv = __builtin_fmaf(act[4 * ob + 3], w.w, yv);
+    }
+    yv += __shfl_xor(yv, 16);
+    yv += __shfl_xor(yv, 32);
+    return yv + b4;
+  }
+
+ private:
+  template <int kSteps>
+  __device__ __forceinline__ void layer(const float* w, int L, float (&act)[16]) const {
+    floatx4 z[4];
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob)
+      z[ob] = *reinterpret_cast<const floatx4*>(table + L * kSdfHidden + 16 * ob);
+#pragma unroll
+    for (int st = 0; st < kSteps; ++st)
+#pragma unroll
+      for (int ob = 0; ob < 4; ++ob)
+        z[ob] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[kSteps * ob + st], act[st], z[ob], 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      float d;
+      silu_grad(z[e >> 2][e & 3], act[e], d);  // (its derivative is not used)
+    }
+  }
+};
+
 // Wave-level inference.  A wave takes a run of 16-query tiles, four at a
 // time: lane l reads and normalises query l of the 64, so each is divided once
 // and not once per lane group, and writes its distance.  Queries of one tile
 // that belong to different bodies are run once per distinct body; the network
 // is read where it changes.  out = y * halfExtent (NaN for a body id out of
 // range).
+template <class Net>
 __global__ __launch_bounds__(kTB, kInferWavesPerSimd) void k_sdf_infer(
     const uint16_t* __restrict__ packed, const float* __restrict__ params,
     const float* __restrict__ freq, const float* __restrict__ frame,
@@ -792,7 +838,8 @@ __global__ __launch_bounds__(kTB, kInferWavesPerSimd) void k_sdf_infer(
   // contiguous runs of tiles per wave: consecutive tiles share a network
   const uint32_t t0 = (uint32_t)((uint64_t)tiles * wave / nWaves),
                  t1 = (uint32_t)((uint64_t)tiles * (wave + 1) / nWaves);
-  SdfNet net;
+  __shared__ __attribute__((aligned(16))) float s_table[kTB / 64][Net::kTable > 0 ? Net::kTable : 1];
+  Net net;
   uint32_t cur = 0xffffffffu;
   for (uint32_t t = t0; t < t1; t += 4) {
     const size_t q = (size_t)t * 16 + lane;
@@ -817,7 +864,7 @@ __global__ __launch_bounds__(kTB, kInferWavesPerSimd) void k_sdf_infer(
         const uint32_t lead =
             (uint32_t)__builtin_amdgcn_readlane((int)body, __ffsll((unsigned long long)mask) - 1);
         if (lead != cur) {
-          net.load(packed, params, freq, lead, lane);
+          net.load(packed, params, freq, lead, lane, s_table[threadIdx.x >> 6]);
           cur = lead;
         }
         const float yv = net.eval(tx, ty, tz);
@@ -1173,7 +1220,7 @@ __global__ __launch_bounds__(kTB, kInferWavesPerSimd) void k_sdf_map_margin(
   const uint32_t dx = (uint32_t)col & 3u, dy = ((uint32_t)col >> 2) & 1u, dz = (uint32_t)col >> 3;
   const float* fr = frame + (size_t)net * 4;
   SdfNet mlp;
-  mlp.load(packed, params, freq, net, lane);
+  mlp.load(packed, params, freq, net, lane, nullptr);
   float over = -INFINITY, slope = 0.0f, err = 0.0f;
   uint32_t count = 0;
   for (uint64_t blk = wave; blk < blocks; blk += nWaves) {
@@ -1493,13 +1540,12 @@ fc_status fc_sdf_eval(fc_sdf* m, const uint32_t* bodies, const float* points, ui
   if (!points || !out) return set_error(FC_ERROR_INVALID_VALUE, "NULL array");
   hipStream_t st = m->ctx->stream;
   if (precision == FC_SDF_FP32) {
-    hipLaunchKernelGGL(k_sdf_eval_f32, dim3((n + kTB - 1) / kTB), dim3(kTB), 0, st, m->params,
-                       m->freq, m->frame, bodies, m->B, points, n, out);
+    hipLaunchKernelGGL(k_sdf_infer<SdfNet32>, dim3(mfma_blocks(n)), dim3(kTB), 0, st, nullptr,
+                       m->params, m->freq, m->frame, bodies, m->B, points, n, out);
   } else if (precision == FC_SDF_BF16) {
     FC_TRY(sdf_pack(m));
-    const uint32_t blocks = mfma_blocks(n);
-    hipLaunchKernelGGL(k_sdf_infer, dim3(blocks), dim3(kTB), 0, st, m->packed, m->params,
-                       m->freq, m->frame, bodies, m->B, points, n, out);
+    hipLaunchKernelGGL(k_sdf_infer<SdfNet>, dim3(mfma_blocks(n)), dim3(kTB), 0, st, m->packed,
+                       m->params, m->freq, m->frame, bodies, m->B, points, n, out);
   } else {
     return set_error(FC_ERROR_INVALID_VALUE, "precision must be FC_SDF_FP32 or FC_SDF_BF16");
   }

@@ -75,3 +75,31 @@ def test_inference_is_the_same_in_parts(gpu_ctx, n):
     parts = [s.eval(pts[i:i + 1000], bodies[i:i + 1000], BF16) for i in range(0, n, 1000)]
     assert np.array_equal(y.view(np.uint32), np.concatenate(parts).view(np.uint32))
     s.close()
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 63, 65, 1000, 32769])
+def test_fp32_inference_tiles(gpu_ctx, n):
+    """The binary32 network at the same edges, mixed tiles and ids out of
+    range, and with a query that is not a number beside others."""
+    from fullc0ntact_amd.sdf import FP32, SdfSurrogate
+    print(n, flush=True)
+    rng = np.random.default_rng(n)
+    s = SdfSurrogate(gpu_ctx, rng.uniform(-0.1, 0.1, (3, 3)), rng.uniform(0.8, 1.2, 3), seed=7)
+    p, f, fr = s.params()
+    p = p + rng.normal(0.0, 0.03, p.shape).astype(np.float32)
+    s.set_params(p)
+    pts = rng.uniform(-0.8, 0.8, (n, 3)).astype(np.float32)
+    bodies = np.where(np.arange(n) < n // 2, 2, rng.integers(0, 4, n)).astype(np.uint32)
+    lost = (np.arange(n) % 29) == 11
+    pts[lost, 1] = np.nan
+    y = s.eval(pts, bodies, FP32)
+    assert np.array_equal(np.isnan(y), lost | (bodies == 3))
+    for b in range(3):
+        m = (bodies == b) & ~lost
+        if m.any():
+            ref = orc.sdf_forward(p[b], f[b], fr[b], pts[m])
+            scale = np.max(np.abs(orc.sdf_forward(p[b], f[b], fr[b], pts[~lost][:512])))
+            # the bound of the whole-network test: binary32 sums of 64 terms a
+            # layer and the hardware sine and cosine (2e-6 of a turn)
+            assert np.max(np.abs(y[m] - ref)) <= 1e-4 * max(scale, 0.1), b
+    s.close()
