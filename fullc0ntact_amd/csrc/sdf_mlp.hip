@@ -1,6 +1,7 @@
 // Learned signed-distance surrogate (network in sdf_mlp.hpp): GPU training
 // by this file's own forward/backward kernels (FP32, deterministic), the
-// FP32 MFMA forward, and the BF16 MFMA inference kernel (FP32 accumulation) used to cull far-field boundary queries.
+// FP32 MFMA forward, and the BF16 MFMA inference kernel (FP32 accumulation)
+// used to cull far-field boundary queries.
 #include "fc_internal.hpp"
 #include "distmap.hpp"
 #include "sdf_mlp.hpp"
