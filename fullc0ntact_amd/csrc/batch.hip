@@ -62,6 +62,7 @@ struct fc_batch {
   hipGraph_t graph = nullptr;
   hipGraphExec_t graphExec = nullptr;
   float graphDt = 0.0f;
+  uint32_t graphSort = 0, runGraphSort = 0;  // the sort scratch's generation at each capture
   // Row resort of a multi-step run's steady steps (rows: S x gridSize.y x
   // gridSize.z, each gridSize.x consecutive keys)
   fc::RowTables rowTables;
@@ -495,6 +496,7 @@ fc_status capture_batch_graph(fc_batch* b, float dt) {
     return hip_error(e, "hipGraphInstantiate");
   }
   b->graphDt = dt;
+  b->graphSort = b->ctx->sort.generation;
   return FC_SUCCESS;
 }
 
@@ -617,6 +619,7 @@ fc_status capture_batch_run_graph(fc_batch* b, float dt) {
     return hip_error(e, "hipGraphInstantiate");
   }
   b->runGraphDt = dt;
+  b->runGraphSort = b->ctx->sort.generation;
   return FC_SUCCESS;
 }
 
@@ -641,7 +644,9 @@ fc_status enqueue_batch_run(fc_batch* b, float dt, uint32_t steps) {
   FC_TRY(enqueue_batch_run_step(b, dt, /*fromSlots=*/false, /*last=*/steps == 1));
   if (steps == 1) return FC_SUCCESS;
   uint32_t middle = steps - 2;
-  if (middle >= kBatchRunSteps && (!b->runGraphExec || b->runGraphDt != dt))
+  // (another call on the context may have grown the sort scratch)
+  if (middle >= kBatchRunSteps && (!b->runGraphExec || b->runGraphDt != dt ||
+                                   b->runGraphSort != ctx->sort.generation))
     FC_TRY(capture_batch_run_graph(b, dt));
   for (; middle >= kBatchRunSteps; middle -= kBatchRunSteps)
     FC_HIP_TRY(hipGraphLaunch(b->runGraphExec, st));
@@ -865,7 +870,8 @@ fc_status fc_batch_run(fc_batch* b, float deltaTime, uint32_t steps) {
     FC_TRY(enqueue_batch_update(b, deltaTime));
     ++i;
   }
-  if (i < steps && (!b->graphExec || b->graphDt != deltaTime))
+  if (i < steps && (!b->graphExec || b->graphDt != deltaTime ||
+                    b->graphSort != b->ctx->sort.generation))
     FC_TRY(capture_batch_graph(b, deltaTime));
   for (; i < steps; ++i) FC_HIP_TRY(hipGraphLaunch(b->graphExec, b->ctx->stream));
   return FC_SUCCESS;

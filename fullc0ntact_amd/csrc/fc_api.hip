@@ -147,6 +147,7 @@ fc_status ensure_sort_capacity(fc_context* ctx, size_t n) {
       s.groupStatusCapacity >= lookback_groups(tiles) * RS_RADIX)
     return FC_SUCCESS;
   FC_HIP_TRY(hipStreamSynchronize(ctx->stream));
+  ++s.generation;
   hipFree(s.keysA);
   hipFree(s.valsA);
   hipFree(s.keysB);

@@ -91,6 +91,9 @@ struct SortScratch {
   size_t groupStatusCapacity = 0;    // in words
   uint32_t* histogram = nullptr;     // [RS_MAX_PASSES][RS_HIST_COPIES][RS_RADIX]
   uint32_t* counters = nullptr;      // [RSC_COUNT]
+  // Counts the reallocations of the arrays above (ensure_sort_capacity):
+  // steps captured under another number hold addresses that are gone.
+  uint32_t generation = 0;
 };
 
 struct StageTimer;
@@ -445,6 +448,7 @@ struct fc_system {
   hipGraphExec_t graphExec[2] = {nullptr, nullptr};
   float graphDt = 0.0f;
   fc_sim_params graphParams{};
+  uint32_t graphSort = 0;  // the sort scratch's generation at the capture
   // Boundary of the integrate stage.
   fc_boundary boundary = FC_BOUNDARY_BOX;
   const fc_distmap* boundaryMap = nullptr;

@@ -345,6 +345,7 @@ fc_status capture_graph(fc_system* sys, float dt) {
   }
   sys->graphDt = dt;
   sys->graphParams = sys->params;
+  sys->graphSort = sys->ctx->sort.generation;
   return FC_SUCCESS;
 }
 
@@ -596,7 +597,9 @@ fc_status fc_system_run(fc_system* sys, float deltaTime, uint32_t steps) {
       for (uint32_t i = 0; i < middle; ++i)
         FC_TRY(enqueue_run_body(sys, deltaTime, true, false, true, timer));
     } else {
+      // another call on the context may have grown the sort scratch
       if (!sys->graphExec[0] || sys->graphDt != deltaTime ||
+          sys->graphSort != ctx->sort.generation ||
           std::memcmp(&sys->graphParams, &sys->params, sizeof(fc_sim_params)) != 0) {
         FC_TRY(capture_graph(sys, deltaTime));
       }

@@ -1,0 +1,39 @@
+"""The device memory that the library's launches and captured graphs name, on
+the CPU: tests/cpp/host_memory_check.cpp stands in for the HIP runtime and fails
+on a launch or a replay that names freed memory."""
+from __future__ import annotations
+
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from fullc0ntact_amd import build
+
+ROOT = Path(__file__).resolve().parents[1]
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("host_memory") / "host_memory_check"
+    cmd = [build.hipcc(), "-x", "hip", "--offload-host-only", "-std=c++17", "-O1",
+           f"-I{ROOT / 'include'}", f"-I{build.CSRC}",
+           str(ROOT / "tests" / "cpp" / "host_memory_check.cpp"), f"-L{build.PKG}", "-lfc_dem",
+           f"-Wl,-rpath,{build.PKG}", "-rdynamic", "-o", str(exe)]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    return exe
+
+
+def holds(program, scenario):
+    r = subprocess.run([str(program), scenario], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, f"{scenario}: {r.stdout}{r.stderr}"
+
+
+# Runs before and after calls that grow the context's sort scratch (labels, a
+# map, a larger system, a larger sort): up to 4,096 spheres, over that by radix
+# sort, batches that sort by radix in updates and in runs, and by rows.
+@pytest.mark.parametrize("scenario", ["system-small", "system-radix", "batch-cells",
+                                      "batch-radix", "batch-rows"])
+def test_captured_steps_and_grown_scratch(program, scenario):
+    holds(program, scenario)
