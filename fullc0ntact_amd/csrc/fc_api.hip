@@ -16,6 +16,7 @@ fc_status set_error(fc_status s, const std::string& msg) {
 }
 
 fc_status hip_error(hipError_t e, const char* what) {
+  (void)hipGetLastError();  // reported here: not once more by the next launch
   std::string msg = std::string(what) + ": " + hipGetErrorString(e);
   if (e == hipErrorOutOfMemory || e == hipErrorMemoryAllocation)
     return set_error(FC_ERROR_OUT_OF_MEMORY, msg);

@@ -373,7 +373,21 @@ int batch_runs(fc_uint3 grid) {
   return 0;
 }
 
+// An error that a call has returned is that call's alone.
+int errors_once() {
+  fc_context* c = context();
+  fc_system *s = nullptr, *other = nullptr;
+  OK(fc_system_create(c, 4096, fc_uint3{64, 64, 64}, &s));
+  rt().most = 0;
+  REQUIRE(fc_system_create(c, 4096, fc_uint3{64, 64, 64}, &other) == FC_ERROR_OUT_OF_MEMORY);
+  rt().most = ~(size_t)0;
+  OK(fc_system_update(s, 0.5f));
+  OK(fc_system_run(s, 0.5f, 20));
+  return 0;
+}
+
 int run(const std::string& name) {
+  if (name == "errors-once") return errors_once();
   if (name == "system-small") return system_runs(4096, fc_uint3{64, 64, 64}, "k_small_rank");
   if (name == "system-radix") return system_runs(8000, fc_uint3{4, 1024, 512}, "k_rs_scatter");
   if (name == "batch-cells") return batch_runs(fc_uint3{64, 64, 2});

@@ -37,3 +37,7 @@ def holds(program, scenario):
                                       "batch-radix", "batch-rows"])
 def test_captured_steps_and_grown_scratch(program, scenario):
     holds(program, scenario)
+
+
+def test_an_error_is_returned_once(program):
+    holds(program, "errors-once")
