@@ -140,15 +140,7 @@ void StageTimer::destroy() {
 // ---------------------------------------------------------------------------
 // Sort scratch management
 // ---------------------------------------------------------------------------
-fc_status ensure_sort_capacity(fc_context* ctx, size_t n) {
-  SortScratch& s = ctx->sort;
-  size_t tiles = (n + RS_TILE - 1) / RS_TILE;
-  if (tiles == 0) tiles = 1;
-  if (s.capacity >= n && s.statusCapacity >= tiles * RS_RADIX &&
-      s.groupStatusCapacity >= lookback_groups(tiles) * RS_RADIX)
-    return FC_SUCCESS;
-  FC_HIP_TRY(hipStreamSynchronize(ctx->stream));
-  ++s.generation;
+static void free_sort_arrays(SortScratch& s) {
   hipFree(s.keysA);
   hipFree(s.valsA);
   hipFree(s.keysB);
@@ -158,21 +150,61 @@ fc_status ensure_sort_capacity(fc_context* ctx, size_t n) {
   s.keysA = s.valsA = s.keysB = s.valsB = nullptr;
   s.status = s.groupStatus = nullptr;
   s.capacity = s.statusCapacity = s.groupStatusCapacity = 0;
-  size_t cap = std::max<size_t>(n, RS_TILE);
-  FC_HIP_TRY(hipMalloc(&s.keysA, cap * sizeof(uint32_t)));
-  FC_HIP_TRY(hipMalloc(&s.valsA, cap * sizeof(uint32_t)));
-  FC_HIP_TRY(hipMalloc(&s.keysB, cap * sizeof(uint32_t)));
-  FC_HIP_TRY(hipMalloc(&s.valsB, cap * sizeof(uint32_t)));
-  size_t words = ((cap + RS_TILE - 1) / RS_TILE) * RS_RADIX;
-  FC_HIP_TRY(hipMalloc(&s.status, words * sizeof(uint64_t)));
-  FC_HIP_TRY(hipMemset(s.status, 0, words * sizeof(uint64_t)));
-  const size_t gwords = lookback_groups((cap + RS_TILE - 1) / RS_TILE) * RS_RADIX;
-  FC_HIP_TRY(hipMalloc(&s.groupStatus, gwords * sizeof(uint64_t)));
-  FC_HIP_TRY(hipMemset(s.groupStatus, 0, gwords * sizeof(uint64_t)));
+}
+
+// The arrays for sorts of up to `cap` pairs into s, which holds none; none on
+// failure either.
+static hipError_t alloc_sort_arrays(SortScratch& s, size_t cap, hipStream_t stream) {
+  const size_t tiles = (cap + RS_TILE - 1) / RS_TILE;
+  const size_t words = tiles * RS_RADIX, gwords = lookback_groups(tiles) * RS_RADIX;
+  hipError_t e = hipMalloc(&s.keysA, cap * sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMalloc(&s.valsA, cap * sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMalloc(&s.keysB, cap * sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMalloc(&s.valsB, cap * sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMalloc(&s.status, words * sizeof(uint64_t));
+  if (e == hipSuccess) e = hipMalloc(&s.groupStatus, gwords * sizeof(uint64_t));
+  if (e == hipSuccess) e = hipMemsetAsync(s.status, 0, words * sizeof(uint64_t), stream);
+  if (e == hipSuccess) e = hipMemsetAsync(s.groupStatus, 0, gwords * sizeof(uint64_t), stream);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // handled here: no later launch is to report it
+    free_sort_arrays(s);
+    return e;
+  }
   s.capacity = cap;
   s.statusCapacity = words;
   s.groupStatusCapacity = gwords;
-  return FC_SUCCESS;
+  return hipSuccess;
+}
+
+// A growth that finds no memory leaves the context what it had: its systems
+// and batches were created with it and never ask again.
+fc_status ensure_sort_capacity(fc_context* ctx, size_t n) {
+  SortScratch& s = ctx->sort;
+  size_t tiles = (n + RS_TILE - 1) / RS_TILE;
+  if (tiles == 0) tiles = 1;
+  if (s.capacity >= n && s.statusCapacity >= tiles * RS_RADIX &&
+      s.groupStatusCapacity >= lookback_groups(tiles) * RS_RADIX)
+    return FC_SUCCESS;
+  FC_HIP_TRY(hipStreamSynchronize(ctx->stream));
+  const size_t cap = std::max<size_t>(n, RS_TILE), had = s.capacity;
+  SortScratch next;
+  next.histogram = s.histogram;
+  next.counters = s.counters;
+  next.generation = s.generation + 1;
+  hipError_t e = alloc_sort_arrays(next, cap, ctx->stream);
+  if (e == hipSuccess) {
+    free_sort_arrays(s);
+    s = next;
+    return FC_SUCCESS;
+  }
+  if (had != 0) {
+    // no room beside the old arrays: in their place, or else they come back
+    free_sort_arrays(s);
+    ++s.generation;
+    e = alloc_sort_arrays(s, cap, ctx->stream);
+    if (e != hipSuccess) (void)alloc_sort_arrays(s, had, ctx->stream);
+  }
+  return e == hipSuccess ? FC_SUCCESS : hip_error(e, "sort scratch");
 }
 
 // The context's stage timer when timing is enabled (fc_context_enable_timing),
@@ -328,12 +360,7 @@ fc_status fc_context_destroy(fc_context* ctx) {
   if (ctx->stream) hipStreamSynchronize(ctx->stream);
   ctx->timer.destroy();
   SortScratch& s = ctx->sort;
-  hipFree(s.keysA);
-  hipFree(s.valsA);
-  hipFree(s.keysB);
-  hipFree(s.valsB);
-  hipFree(s.status);
-  hipFree(s.groupStatus);
+  free_sort_arrays(s);
   hipFree(s.histogram);
   hipFree(s.counters);
   hipFree(ctx->devFlags);

@@ -473,6 +473,7 @@ hipError_t launch_sort_small(hipStream_t stream, SortScratch& s, const uint32_t*
                              const SortGather& gather) {
   if (n == 0) return hipSuccess;
   if (n > (uint32_t)RS_TILE || passes < 1 || passes > RS_MAX_PASSES) return hipErrorInvalidValue;
+  if (s.capacity < n) return hipErrorInvalidValue;
   // The keys are cells, below numCells: (key << 12) | index fits 32 bits
   // for keys of up to 20 bits.
   int bits = key_bits_for_cells(numCells);

@@ -41,6 +41,7 @@ struct Runtime {
   std::map<uintptr_t, Block> blocks;  // addresses are never given out twice
   uintptr_t next = kFirst;
   size_t inUse = 0, most = ~(size_t)0;     // hipMalloc fails beyond `most` bytes in use
+  size_t failing = 0;                      // nor for this size exactly
   hipError_t last = hipSuccess;
   hipError_t memsetError = hipSuccess;     // what the next hipMemset returns
   std::map<const void*, std::string> names;
@@ -169,7 +170,7 @@ hipError_t hipLaunchCooperativeKernel(const void*, dim3, dim3, void**, unsigned,
 }
 hipError_t hipMalloc(void** p, size_t size) {
   *p = nullptr;
-  if (size > rt().most || rt().inUse > rt().most - size) return result(hipErrorOutOfMemory);
+  if ((size == rt().failing && size) || size > rt().most || rt().inUse > rt().most - size) return result(hipErrorOutOfMemory);
   const uintptr_t at = rt().next;
   rt().next += (size + 4096 + 255) & ~(size_t)255;
   rt().blocks[at] = Block{size, true};
@@ -307,14 +308,16 @@ T* device(size_t count) {
   return static_cast<T*>(p);
 }
 
-// A mesh call with more points than any system here has spheres.
+// Calls that need more sort scratch than any system below has spheres.
+constexpr uint32_t kLabels = 65536, kMapTriangles = 8192, kSystem = 100000, kSort = 200000;
+
 fc_status labels(fc_context* c) {
-  const uint32_t nv = 3072, nt = 6144, np = 65536;
+  const uint32_t nv = 3072, nt = 6144, np = kLabels;
   return fc_mesh_signed_distance(c, device<double>(3 * nv), nv, device<uint32_t>(3 * nt), nt,
                                  device<double>(3 * np), np, device<double>(np), nullptr);
 }
 fc_status build_map(fc_context* c) {
-  const uint32_t nv = 4096, nt = 8192;
+  const uint32_t nv = 4096, nt = kMapTriangles;
   std::vector<double> v(3 * nv, 0.5);
   std::vector<uint32_t> f(3 * nt);
   for (uint32_t i = 0; i < 3 * nt; ++i) f[i] = i % nv;
@@ -327,11 +330,11 @@ fc_status build_map(fc_context* c) {
 }
 fc_status larger_system(fc_context* c) {
   fc_system* s = nullptr;
-  return fc_system_create(c, 100000, fc_uint3{64, 64, 64}, &s);
+  return fc_system_create(c, kSystem, fc_uint3{64, 64, 64}, &s);
 }
 fc_status larger_sort(fc_context* c) {
-  const uint32_t n = 200000;
-  return fc_sort_particles(c, device<uint32_t>(n), device<uint32_t>(n), n);
+  static uint32_t *k = device<uint32_t>(kSort), *v = device<uint32_t>(kSort);
+  return fc_sort_particles(c, k, v, kSort);
 }
 using Growth = fc_status (*)(fc_context*);
 const Growth kGrowths[] = {labels, build_map, larger_system, larger_sort};
@@ -386,8 +389,66 @@ int errors_once() {
   return 0;
 }
 
+// A call that finds no memory for its scratch: the mesh calls do without, the
+// others say so, and the context's systems and batches run on.
+int growth_fails(uint32_t n, fc_uint3 grid) {
+  for (Growth grow : kGrowths) {
+    fc_context* c = context();
+    fc_system* s = nullptr;
+    const uint32_t counts[2] = {700, 900};
+    (void)larger_sort(context());  // (its arrays)
+    fc_batch* b = nullptr;
+    OK(fc_system_create(c, n, grid, &s));
+    OK(fc_batch_create(c, 2, counts, fc_uint3{64, 64, 2}, &b));
+    OK(fc_system_run(s, 0.5f, 20));
+    OK(fc_batch_run(b, 0.5f, 20));
+    const bool mesh = grow == labels || grow == build_map;
+    rt().failing = 4 * (grow == labels ? kLabels
+                                       : (grow == build_map ? kMapTriangles
+                                                            : (grow == larger_system ? kSystem : kSort)));
+    rt().launched.clear();
+    REQUIRE(grow(c) == (mesh ? FC_SUCCESS : FC_ERROR_OUT_OF_MEMORY));
+    rt().failing = 0;
+    REQUIRE(!launched("k_tree_leaves") && launched("k_mesh_sdf") == mesh);
+    OK(fc_system_update(s, 0.5f));
+    OK(fc_system_run(s, 0.5f, 20));
+    OK(fc_batch_update(b, 0.5f));
+    OK(fc_batch_run(b, 0.5f, 20));
+    OK(grow(c));
+    REQUIRE(!mesh || launched("k_tree_leaves"));
+    OK(fc_system_run(s, 0.5f, 20));
+    OK(fc_batch_run(b, 0.5f, 20));
+  }
+  return 0;
+}
+
+// Room for the larger scratch only in the place of the smaller; and room for
+// neither, where the steps return an error.
+int no_room_for_both() {
+  fc_context* c = context();
+  fc_system* s = nullptr;
+  OK(fc_system_create(c, 4096, fc_uint3{64, 64, 64}, &s));
+  OK(fc_system_run(s, 0.5f, 20));
+  const uint32_t n = 8192;
+  uint32_t *k = device<uint32_t>(n), *v = device<uint32_t>(n);
+  rt().most = rt().inUse + 16 * n;  // (the arrays take 16 n bytes and the look-back words)
+  OK(fc_sort_particles(c, k, v, n));
+  OK(fc_system_run(s, 0.5f, 20));
+  rt().most = 0;
+  REQUIRE(fc_sort_particles(c, k, v, n + 1) == FC_ERROR_OUT_OF_MEMORY);
+  REQUIRE(fc_system_update(s, 0.5f) == FC_ERROR_HIP);
+  REQUIRE(fc_system_run(s, 0.5f, 20) == FC_ERROR_HIP);
+  rt().most = ~(size_t)0;
+  OK(fc_sort_particles(c, k, v, n));
+  OK(fc_system_run(s, 0.5f, 20));
+  return 0;
+}
+
 int run(const std::string& name) {
   if (name == "errors-once") return errors_once();
+  if (name == "growth-fails-small") return growth_fails(4096, fc_uint3{64, 64, 64});
+  if (name == "growth-fails-radix") return growth_fails(8000, fc_uint3{4, 1024, 512});
+  if (name == "no-room-for-both") return no_room_for_both();
   if (name == "system-small") return system_runs(4096, fc_uint3{64, 64, 64}, "k_small_rank");
   if (name == "system-radix") return system_runs(8000, fc_uint3{4, 1024, 512}, "k_rs_scatter");
   if (name == "batch-cells") return batch_runs(fc_uint3{64, 64, 2});

@@ -41,3 +41,8 @@ def test_captured_steps_and_grown_scratch(program, scenario):
 
 def test_an_error_is_returned_once(program):
     holds(program, "errors-once")
+# A growth without memory: the callers' systems and batches keep their scratch.
+@pytest.mark.parametrize("scenario", ["growth-fails-small", "growth-fails-radix",
+                                      "no-room-for-both"])
+def test_growth_that_fails(program, scenario):
+    holds(program, scenario)
