@@ -628,7 +628,12 @@ fc_status enqueue_batch_run(fc_batch* b, float dt, uint32_t steps) {
   hipStream_t st = ctx->stream;
   const uint64_t cells = (uint64_t)b->S * b->C;
   const bool rowMode = batch_row_mode(b);
-  if (rowMode) FC_TRY(ensure_row_tables(b->rowTables, batch_row_grid(b), b->n));
+  if (rowMode) {
+    bool remade = false;
+    const fc_status s = ensure_row_tables(b->rowTables, batch_row_grid(b), b->n, &remade);
+    if (remade) drop_batch_graph(b);  // the captured steps hold the tables
+    FC_TRY(s);
+  }
   // head: integrate + hash from the ids, clearing the previous cells
   const uint32_t* prev = nullptr;
   if (b->tablesTrackHash) {

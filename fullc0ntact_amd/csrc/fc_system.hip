@@ -579,13 +579,15 @@ fc_status fc_system_run(fc_system* sys, float deltaTime, uint32_t steps) {
   }
   StageTimer* timer = ctx->timer.enabled ? &ctx->timer : nullptr;
   if (run_row_mode(sys)) {
-    const fc_status s = ensure_row_tables(sys->rowTables, sys->params, sys->n);
+    bool remade = false;
+    const fc_status s = ensure_row_tables(sys->rowTables, sys->params, sys->n, &remade);
+    // the captured steps hold the tables (a shape of as many cells may have
+    // come and gone without a capture), or ran without them
+    if (remade) drop_graph(sys);
     if (s != FC_SUCCESS) {
-      // small systems can do without; the captured steps may not mix the two
-      if (!collide_rows_optional(sys->n)) return s;
+      if (!collide_rows_optional(sys->n)) return s;  // small systems can do without
       (void)hipGetLastError();
       sys->noRowTables = true;
-      drop_graph(sys);
     }
   }
   FC_TRY(enqueue_run_head(sys, deltaTime, timer));

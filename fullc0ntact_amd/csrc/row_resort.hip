@@ -701,13 +701,15 @@ RowHists row_hists(const RowTables& T) {
   return h;
 }
 
-fc_status ensure_row_tables(RowTables& T, const fc_sim_params& P, uint32_t n) {
+fc_status ensure_row_tables(RowTables& T, const fc_sim_params& P, uint32_t n, bool* remade) {
+  *remade = false;
   uint32_t shift = 0;
   while ((1u << shift) < P.gridSize.x) ++shift;
   const uint32_t rows = P.gridSize.y * P.gridSize.z;
   const uint32_t groups = (rows + (1u << kRowGroupShift) - 1u) >> kRowGroupShift;
   if (T.block != nullptr && T.rows == rows && T.shift == shift && T.capacity >= n)
     return FC_SUCCESS;
+  *remade = true;
   free_row_tables(T);
   // count, startNext [rows + 1]; chgStart [rows x copies + 1]; rowList
   // [2 rows, 16-byte]; groupWords [3 groups, 64-bit]; listCount, epoch [2];

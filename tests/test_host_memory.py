@@ -41,8 +41,15 @@ def test_captured_steps_and_grown_scratch(program, scenario):
 
 def test_an_error_is_returned_once(program):
     holds(program, "errors-once")
+
+
 # A growth without memory: the callers' systems and batches keep their scratch.
 @pytest.mark.parametrize("scenario", ["growth-fails-small", "growth-fails-radix",
                                       "no-room-for-both"])
 def test_growth_that_fails(program, scenario):
+    holds(program, scenario)
+
+
+@pytest.mark.parametrize("scenario", ["row-tables-small", "row-tables"])
+def test_captured_steps_and_new_row_tables(program, scenario):
     holds(program, scenario)
