@@ -460,8 +460,9 @@ struct fc_system {
   int polydisperse = 0;
   uint32_t* piles = nullptr;  // GatheredState::piles, once polydisperse
   // Row resort tables of multi-step runs (allocated by the first run that
-  // uses them), and whether there was no memory for those of a system that
-  // can do without (collide_rows_optional): its runs then sort by radix.
+  // uses them), and whether there was no memory for those of this grid and
+  // the system can do without (collide_rows_optional): its runs then sort by
+  // radix until the grid changes.
   fc::RowTables rowTables;
   bool noRowTables = false;
   fc::BoundaryArg boundary_arg() const;

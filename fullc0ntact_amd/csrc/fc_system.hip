@@ -510,6 +510,8 @@ fc_status fc_system_set_params(fc_system* sys, const fc_sim_params* params) {
     drop_graph(sys);
     FC_TRY(alloc_tables(sys, params->numCells));
   }
+  if (std::memcmp(&params->gridSize, &sys->params.gridSize, sizeof(fc_uint3)) != 0)
+    sys->noRowTables = false;  // other tables: they may fit
   sys->params = *params;
   return FC_SUCCESS;
 }
@@ -585,8 +587,8 @@ fc_status fc_system_run(fc_system* sys, float deltaTime, uint32_t steps) {
     // come and gone without a capture), or ran without them
     if (remade) drop_graph(sys);
     if (s != FC_SUCCESS) {
-      if (!collide_rows_optional(sys->n)) return s;  // small systems can do without
-      (void)hipGetLastError();
+      // small systems can do without
+      if (s != FC_ERROR_OUT_OF_MEMORY || !collide_rows_optional(sys->n)) return s;
       sys->noRowTables = true;
     }
   }

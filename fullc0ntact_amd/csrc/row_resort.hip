@@ -749,7 +749,11 @@ fc_status ensure_row_tables(RowTables& T, const fc_sim_params& P, uint32_t n, bo
   T.shift = shift;
   T.groups = groups;
   T.capacity = n;
-  FC_HIP_TRY(hipMemset(T.block, 0, words * sizeof(uint32_t)));
+  const hipError_t e = hipMemset(T.block, 0, words * sizeof(uint32_t));
+  if (e != hipSuccess) {
+    free_row_tables(T);  // (else the next call would take them as they are)
+    return hip_error(e, "row tables");
+  }
   return FC_SUCCESS;
 }
 

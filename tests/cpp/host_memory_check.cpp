@@ -399,6 +399,43 @@ int row_tables(uint32_t n) {
   return 0;
 }
 
+// Runs of a system that can do without row tables, while there is no memory
+// for them, after a grid change with memory, and with another error.
+int no_row_tables() {
+  fc_context* c = context();
+  fc_system* s = nullptr;
+  OK(fc_system_create(c, 8000, fc_uint3{64, 64, 64}, &s));
+  rt().most = rt().inUse;
+  OK(fc_system_run(s, 0.5f, 20));
+  REQUIRE(launched("k_rs_scatter") && !launched("k_row_sort") && !launched("k_row_reset"));
+  OK(fc_system_run(s, 0.5f, 20));  // no second attempt at the same grid
+  rt().most = ~(size_t)0;
+  OK(fc_system_run(s, 0.5f, 20));
+  REQUIRE(!launched("k_row_sort"));
+  fc_sim_params p;
+  OK(fc_system_get_params(s, &p));
+  p.spring *= 2.0f;
+  OK(fc_system_set_params(s, &p));
+  OK(fc_system_run(s, 0.5f, 20));
+  REQUIRE(!launched("k_row_sort"));
+  p.gridSize = fc_uint3{128, 32, 64};
+  OK(fc_system_set_params(s, &p));
+  rt().launched.clear();
+  OK(fc_system_run(s, 0.5f, 20));
+  REQUIRE(launched("k_row_sort"));
+  // an error that is not for want of memory is the caller's to see, and the
+  // next run has its tables again
+  p.gridSize = fc_uint3{32, 64, 128};
+  OK(fc_system_set_params(s, &p));
+  rt().memsetError = hipErrorLaunchFailure;
+  REQUIRE(fc_system_run(s, 0.5f, 20) == FC_ERROR_HIP);
+  rt().launched.clear();
+  const size_t blocks = rt().blocks.size();
+  OK(fc_system_run(s, 0.5f, 20));
+  REQUIRE(launched("k_row_sort") && rt().blocks.size() > blocks);  // none that were not cleared
+  return 0;
+}
+
 // An error that a call has returned is that call's alone.
 int errors_once() {
   fc_context* c = context();
@@ -470,6 +507,7 @@ int no_room_for_both() {
 int run(const std::string& name) {
   if (name == "row-tables-small") return row_tables(8000);
   if (name == "row-tables") return row_tables(40000);
+  if (name == "no-row-tables") return no_row_tables();
   if (name == "errors-once") return errors_once();
   if (name == "growth-fails-small") return growth_fails(4096, fc_uint3{64, 64, 64});
   if (name == "growth-fails-radix") return growth_fails(8000, fc_uint3{4, 1024, 512});

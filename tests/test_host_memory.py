@@ -53,3 +53,7 @@ def test_growth_that_fails(program, scenario):
 @pytest.mark.parametrize("scenario", ["row-tables-small", "row-tables"])
 def test_captured_steps_and_new_row_tables(program, scenario):
     holds(program, scenario)
+
+
+def test_runs_without_row_tables(program):
+    holds(program, "no-row-tables")
