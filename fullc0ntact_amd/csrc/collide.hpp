@@ -651,6 +651,13 @@ __device__ __forceinline__ void collide_row_cells(const fc_sim_params& P, v3f in
   }
   const uint32_t b1 = len[0], b2 = b1 + len[1], total = b2 + len[2];
   const uint32_t q1 = st[1] - b1, q2 = st[2] - b2;  // modulo 2^32
+  // The current cell's sum runs on until the first candidate of the next cell
+  // that has one.  Adding each force to its cell's sum by selects instead cost
+  // 5 % where cells are full and a third in a row of hundreds: 16,000 spheres
+  // in a heap of 6^3 cells, an update 150 -> 144 us (146 with a loop per cell,
+  // two candidates a round); 4,096 in one row of 16 cells 491 -> 445 (379).
+  const uint32_t next1 = b1 < total ? b1 : 0xffffffffu, next2 = b2 < total ? b2 : 0xffffffffu;
+  v3f sum = make_v3(0.0f, 0.0f, 0.0f);
 #pragma unroll 1
   for (uint32_t t = 0; t < total; t += kRowBatch) {
     float4 pj[kRowBatch], vj[kRowBatch];
@@ -665,18 +672,31 @@ __device__ __forceinline__ void collide_row_cells(const fc_sim_params& P, v3f in
     }
 #pragma unroll
     for (int u = 0; u < kRowBatch; ++u) {
+      const uint32_t tu = t + (uint32_t)u;
+      if (tu == next1 || tu == next2) {
+        if (tu == next1) {
+          cf[0] = sum;
+          sum = make_v3(0.0f, 0.0f, 0.0f);
+        }
+        if (tu == next2) {
+          cf[1] = sum;
+          sum = make_v3(0.0f, 0.0f, 0.0f);
+        }
+      }
       if (jj[u] != k) {
-        const uint32_t tu = t + (uint32_t)u;
         const v3f f = collide_spheres_fast(pos, xyz(pj[u]), vel, xyz(vj[u]), rA,
                                            kPoly ? pj[u].w : rA, P.spring, P.damping, P.shear,
                                            P.attraction);
-        const int c = tu < b1 ? 0 : (tu < b2 ? 1 : 2);
-#pragma unroll
-        for (int x = 0; x < 3; ++x)
-          if (c == x) cf[x] = make_v3(cf[x].x + f.x, cf[x].y + f.y, cf[x].z + f.z);
+        sum = make_v3(sum.x + f.x, sum.y + f.y, sum.z + f.z);
       }
     }
   }
+  if (b2 < total)
+    cf[2] = sum;
+  else if (b1 < total)
+    cf[1] = sum;
+  else
+    cf[0] = sum;
 }
 
 }  // namespace fc
