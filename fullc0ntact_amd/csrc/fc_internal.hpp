@@ -373,11 +373,12 @@ struct RowTables {
   uint32_t* count = nullptr;      // [rows] spheres per row in the current order
   uint32_t* startNext = nullptr;  // [rows + 1] row starts of the next order
   uint32_t* chgStart = nullptr;   // [rows x copies + 1] bucket starts of the row changers
-  // [rows][2] one entry per row that holds spheres in the next order, in row
-  // order: {row, next start, next count, current start}, {current count,
-  // changers' first bucket start, changers moving in, 0}
+  // [entries][2] one entry per row that holds spheres in the next order (a
+  // long row has several), in row order: {row, next start, next count, current
+  // start}, {current count, changers' first bucket start, changers moving in,
+  // part of the row}
   uint4* rowList = nullptr;
-  uint64_t* groupWords = nullptr; // [groups][3] per 256-row group: spheres, changers, rows (epoch-tagged)
+  uint64_t* groupWords = nullptr; // [groups][3] per 256-row group: spheres, changers, entries (epoch-tagged)
   uint32_t* listCount = nullptr;  // [1] entries of rowList
   uint32_t* epoch = nullptr;      // [1] steps resorted (tags the group words)
   uint32_t* zeroed = nullptr;     // the counts below, zero between steps

@@ -22,10 +22,10 @@
 //                     cell are already in (cell, id) order; the others (the
 //                     movers, few) are ranked among themselves, and each
 //                     member's place is its rank in its own list plus the
-//                     number of the other list below it.  Rows beyond LDS,
-//                     or with many movers, are ranked by counting.  The
-//                     members are written at the row's start with the
-//                     gathered state and the new cell tables.
+//                     number of the other list below it.  Rows beyond LDS
+//                     are shared out to several blocks.  The members are
+//                     written at the row's start with the gathered state
+//                     and the new cell tables.
 //
 // This replaces the radix passes and the cell-bounds kernel of those
 // steps; the first sort of a run (keys in id order) stays a radix sort.
@@ -35,19 +35,35 @@ namespace fc {
 namespace {
 
 constexpr int kScanThreads = 256;
-// The row sort: one row per 128-thread block (9 KB of LDS, 82 VGPRs: 10
+// The row sort: one row per 128-thread block (11 KB of LDS, 83 VGPRs: 10
 // blocks per CU) over a fixed grid of 8192 blocks, so that the ~3800
 // occupied rows of a 1M-sphere bed are in flight together (each row is a
 // chain of dependent loads; capping the kernel at 64 or 72 VGPRs for more
-// blocks per CU made it slower).
+// blocks per CU made it slower).  Five waves per SIMD: with six a step of the
+// settled 1M bed takes 24.7 instead of 23.7 us here, 1,000,000 spheres at
+// random in a 256^3 grid 90 instead of 105.  Long rows wait for the end of the
+// kernel, which keeps their registers out of the loop over the others (100,000
+// at random in 128^3 28.0 us with them inside it, 25.9 so).
 constexpr int kSortThreads = 128;
+constexpr int kSortWavesPerSimd = 5;
 constexpr uint32_t kRowCap = 768;      // members of a row held in LDS
-constexpr uint32_t kMoverCap = 256;    // movers ranked by counting
+constexpr uint32_t kRowPart = 384;     // members of a part of a longer row
+constexpr uint32_t kMoverCap = 256;    // movers ranked among themselves
 constexpr uint32_t kPerThread = kRowCap / kSortThreads;
 constexpr uint32_t kMoversPerThread = kMoverCap / kSortThreads;
 constexpr uint32_t kSortBlocks = 8192; // grid of the row sort
 static_assert(kRowCap % kSortThreads == 0 && kMoverCap % kSortThreads == 0, "whole per-thread shares");
 constexpr uint64_t kNoMember = ~0ull;
+// A row of more than kRowCap members is shared out in parts of about kRowPart
+// members, a block and a list entry each (sort_part).
+constexpr uint32_t kRowBins = 256;     // ranges of a row's cells, two per thread
+constexpr uint32_t kSmallBin = 384;    // ranges of up to so many are taken together
+constexpr uint32_t kNoBin = ~0u;
+static_assert(kRowPart - 1 + kSmallBin <= kRowCap, "a part's small ranges fit LDS");
+static_assert(kRowBins == 2 * kSortThreads, "two ranges per thread");
+__device__ __forceinline__ uint32_t row_parts(uint32_t members) {
+  return members <= kRowCap ? (members != 0u ? 1u : 0u) : (members + kRowPart - 1u) / kRowPart;
+}
 static_assert(kScanThreads == (1 << kRowGroupShift), "one row per scan thread");
 
 // Exclusive scan of one value per thread over a kThreads-thread block;
@@ -103,7 +119,7 @@ static_assert(kRowCopies == 8, "two 16-byte words of counters per row");
 constexpr uint32_t kScanSpinLimit = 1u << 22;
 
 // One block per 256-row group, one row per thread.  The block publishes
-// its group's totals (spheres, changers, occupied rows), each tagged with
+// its group's totals (spheres, changers, list entries), each tagged with
 // this step's epoch, then adds the totals of the earlier groups as they
 // appear (every group publishes before it waits, and waits only on earlier
 // ones; the wait is bounded and reported).  Each row then takes its start
@@ -111,7 +127,8 @@ constexpr uint32_t kScanSpinLimit = 1u << 22;
 // its changers' bucket start; every occupied row gets its entry in row
 // order (next start and count, current start and count, the changers'
 // first bucket start and number), so that the row sort reads one entry
-// per row; the counters are zeroed for the next producer.
+// per row, a row beyond LDS one for each of its parts; the counters are
+// zeroed for the next producer.
 __global__ __launch_bounds__(kScanThreads) void k_row_scan(RowTables T, uint32_t* devFlags) {
   __shared__ uint32_t s_wave[3][kScanThreads / 64];
   const uint32_t g = blockIdx.x;
@@ -135,7 +152,8 @@ __global__ __launch_bounds__(kScanThreads) void k_row_scan(RowTables T, uint32_t
   uint32_t th, tc, to;
   uint32_t ph = block_exclusive_scan(h, s_wave[0], &th);
   uint32_t pc = block_exclusive_scan(c, s_wave[1], &tc);
-  uint32_t po = block_exclusive_scan(h != 0u ? 1u : 0u, s_wave[2], &to);
+  const uint32_t parts = row_parts(h);
+  uint32_t po = block_exclusive_scan(parts, s_wave[2], &to);
   uint64_t* pub = T.groupWords + (size_t)g * 3;
   if (threadIdx.x == 0) {
     const uint64_t tag = (uint64_t)epoch << 32;
@@ -177,9 +195,9 @@ __global__ __launch_bounds__(kScanThreads) void k_row_scan(RowTables T, uint32_t
   if (in) {
     T.startNext[r] = ph;
     T.count[r] = h;
-    if (h != 0u) {
-      T.rowList[2 * (size_t)po] = make_uint4(r, ph, h, curStart);
-      T.rowList[2 * (size_t)po + 1] = make_uint4(curCount, pc, c, 0u);
+    for (uint32_t q = 0; q < parts; ++q) {
+      T.rowList[2 * (size_t)(po + q)] = make_uint4(r, ph, h, curStart);
+      T.rowList[2 * (size_t)(po + q) + 1] = make_uint4(curCount, pc, c, q);
     }
     uint32_t st[kRowCopies];
 #pragma unroll
@@ -198,7 +216,7 @@ __global__ __launch_bounds__(kScanThreads) void k_row_scan(RowTables T, uint32_t
     // the last thread's prefixes plus its own counts are the totals
     T.startNext[T.rows] = ph + h;  // past the last row: the sphere count
     T.chgStart[(size_t)T.rows * kRowCopies] = pc;
-    *T.listCount = po + (h != 0u ? 1u : 0u);
+    *T.listCount = po + parts;
   }
 }
 
@@ -387,12 +405,14 @@ __device__ __forceinline__ void emit_member(const RowOutputs& O, uint32_t q, uin
   if (lastOfCell) O.cellEnd[key] = q + 1u;
 }
 
-// Writes the row's m members, in order in s_key/s_slot, from position o0:
-// each thread loads the state of up to kEmitBatch members before it stores
-// any, so the gathers' latencies overlap.
+// Writes the m members in s_key/s_slot, a cell's one after the other in order,
+// the i-th (of cell x) to position place(i, x): each thread loads the state of
+// up to kEmitBatch members before it stores any, so the gathers' latencies
+// overlap.
 constexpr uint32_t kEmitBatch = 4;
+template <class Place>
 __device__ __forceinline__ void emit_row(const RowOutputs& O, const uint64_t* s_key,
-                                         const uint32_t* s_slot, uint32_t o0, uint32_t m,
+                                         const uint32_t* s_slot, Place place, uint32_t m,
                                          uint32_t rowBase) {
   for (uint32_t base = 0; base < m; base += kSortThreads * kEmitBatch) {
     float4 p[kEmitBatch], v[kEmitBatch];
@@ -412,7 +432,7 @@ __device__ __forceinline__ void emit_row(const RowOutputs& O, const uint64_t* s_
       const uint64_t ck = s_key[i];
       const uint32_t x = (uint32_t)(ck >> 32);
       const uint32_t key = rowBase | x;
-      const uint32_t q = o0 + i;
+      const uint32_t q = place(i, x);
       O.hash[q] = key;
       O.index[q] = (uint32_t)ck;
       O.sortedPos[q] = p[t];
@@ -462,54 +482,237 @@ __device__ __forceinline__ uint32_t count_below(const uint64_t* s_key, uint32_t 
   return a;
 }
 
-// The members of row r (more than LDS holds, or too many movers to rank):
-// each member's place is the number of members below it, counted over the
-// candidates staged through LDS in kRowCap chunks.  O(m x candidates).
-__device__ void rank_by_counting(const RowTables& T, const uint32_t* keys,
-                                 const uint32_t* idOfSlot, const RowOutputs& O, uint32_t r,
-                                 uint32_t o0, uint32_t m, uint32_t a0, uint32_t A, uint32_t c0,
-                                 uint32_t C, uint64_t* s_key, uint32_t* s_wave,
-                                 uint32_t* devFlags) {
-  const uint32_t tid = threadIdx.x;
-  const uint32_t rowBase = r << T.shift;
-  const uint32_t U = A + C;
-  uint32_t members = 0;
-  for (uint32_t tb = 0; tb < U; tb += kSortThreads) {
-    const uint32_t u = tb + tid;
-    uint32_t slot = 0;
-    const uint64_t mine = u < U ? candidate(T, keys, idOfSlot, r, a0, A, c0, u, &slot) : kNoMember;
-    uint32_t below = 0, sameBelow = 0, sameAbove = 0;
-    for (uint32_t w = 0; w < U; w += kRowCap) {
+// LDS of a part of a long row.
+struct PartShared {
+  uint32_t start[kRowBins + 1];  // members before each range of cells
+  uint32_t at[kRowBins];         // counts; then places in the pool
+  uint64_t large[4];             // ranges taken one by one, as lane masks
+  uint32_t count;
+};
+
+// The members of one range of cells that LDS does not hold: each one's place is
+// the number of the range's members below it.  The parts that the range reaches
+// into take a share of the candidates each, against all of them, staged
+// through LDS; O(members^2), as the pair forces of such cells are.
+template <bool kOneCell>
+__device__ __forceinline__ void rank_by_counting(const RowTables& T, const uint32_t* keys,
+                                              const uint32_t* idOfSlot, const RowOutputs& O,
+                                              uint32_t r, uint32_t o0, uint32_t a0, uint32_t A,
+                                              uint32_t c0, uint32_t C, uint32_t part,
+                                              uint32_t bin, uint32_t binShift, uint64_t* s_key,
+                                              PartShared& S) {
+  constexpr uint32_t kMine = 4;
+  const uint32_t tid = threadIdx.x, rowBase = r << T.shift, U = A + C;
+  const uint32_t first = S.start[bin], members = S.start[bin + 1] - first;
+  const uint32_t p0 = first / kRowPart, share = (first + members - 1u) / kRowPart - p0 + 1u;
+  const uint32_t from = (uint32_t)((uint64_t)U * (part - p0) / share);
+  const uint32_t to = (uint32_t)((uint64_t)U * (part - p0 + 1u) / share);
+  auto member = [&](uint32_t u, uint32_t end, uint32_t* slot) {
+    const uint64_t k =
+        u < end ? candidate(T, keys, idOfSlot, r, a0, A, c0, u, slot) : kNoMember;
+    return k != kNoMember && (uint32_t)(k >> 32) >> binShift == bin ? k : kNoMember;
+  };
+  for (uint32_t b = from; b < to; b += kMine * kSortThreads) {
+    uint64_t mine[kMine];
+    uint32_t slot[kMine], below[kMine], sameBelow[kMine], sameAbove[kMine];
+#pragma unroll
+    for (uint32_t v = 0; v < kMine; ++v) {
+      slot[v] = below[v] = sameBelow[v] = sameAbove[v] = 0u;
+      mine[v] = member(b + v * kSortThreads + tid, to, &slot[v]);
+    }
+    for (uint32_t g0 = 0; g0 < U; g0 += kRowCap) {
+      __syncthreads();  // the pool's readers
+      if (tid == 0) S.count = 0u;
       __syncthreads();
-      for (uint32_t i = tid; i < kRowCap; i += kSortThreads) {
-        uint32_t sl;
-        s_key[i] =
-            w + i < U ? candidate(T, keys, idOfSlot, r, a0, A, c0, w + i, &sl) : kNoMember;
+#pragma unroll
+      for (uint32_t t = 0; t < kPerThread; ++t) {
+        uint32_t ignored;
+        const uint64_t k = member(g0 + t * kSortThreads + tid, U, &ignored);
+        if (k != kNoMember) s_key[atomicAdd(&S.count, 1u)] = k;
       }
       __syncthreads();
-      if (mine != kNoMember) {
-        const uint32_t xm = (uint32_t)(mine >> 32);
-        for (uint32_t i = 0; i < kRowCap; ++i) {
-          const uint64_t o = s_key[i];
-          if (o == kNoMember) continue;
-          below += o < mine ? 1u : 0u;
-          const bool same = (uint32_t)(o >> 32) == xm;
-          sameBelow += (same && o < mine) ? 1u : 0u;
-          sameAbove += (same && o > mine) ? 1u : 0u;
+      const uint32_t have = S.count;
+#pragma unroll 4
+      for (uint32_t i = 0; i < have; ++i) {
+        const uint64_t o = s_key[i];
+#pragma unroll
+        for (uint32_t v = 0; v < kMine; ++v) {
+          if (kOneCell) {  // ordered by their ids alone
+            below[v] += (uint32_t)o < (uint32_t)mine[v] ? 1u : 0u;
+          } else {
+            const bool same = (uint32_t)(o >> 32) == (uint32_t)(mine[v] >> 32);
+            below[v] += o < mine[v] ? 1u : 0u;
+            sameBelow[v] += same && o < mine[v] ? 1u : 0u;
+            sameAbove[v] += same && o > mine[v] ? 1u : 0u;
+          }
         }
       }
     }
-    if (mine != kNoMember) {
-      ++members;
-      if (below < m)
-        emit_member(O, o0 + below, rowBase | (uint32_t)(mine >> 32), (uint32_t)mine, slot,
-                    sameBelow == 0u, sameAbove == 0u);
-      else
-        atomicOr(devFlags, DEVERR_ROW_COUNT);
+#pragma unroll
+    for (uint32_t v = 0; v < kMine; ++v) {
+      if (mine[v] == kNoMember) continue;
+      const bool firstOfCell = kOneCell ? below[v] == 0u : sameBelow[v] == 0u;
+      const bool lastOfCell = kOneCell ? below[v] + 1u == members : sameAbove[v] == 0u;
+      emit_member(O, o0 + first + below[v], rowBase | (uint32_t)(mine[v] >> 32),
+                  (uint32_t)mine[v], slot[v], firstOfCell, lastOfCell);
     }
   }
-  if (block_sum<kSortThreads>(members, s_wave) != m && tid == 0)
-    atomicOr(devFlags, DEVERR_ROW_COUNT);
+}
+
+// The pool's `mine` members, range by range (S.at: the end of each range in the
+// pool), to their places: a member's place in its range is the number of the
+// range's members below it.
+__device__ __forceinline__ void place_pool(const RowOutputs& O, uint32_t o0, uint32_t mine,
+                                           uint32_t binShift, uint32_t rowBase, uint64_t* s_key,
+                                           uint32_t* s_slot, const PartShared& S) {
+  const uint32_t tid = threadIdx.x;
+  auto begin_of = [&](uint32_t x) {
+    const uint32_t b = x >> binShift;
+    return S.at[b] - (S.start[b + 1u] - S.start[b]);
+  };
+  uint64_t key[kPerThread];
+  uint32_t slot[kPerThread], to[kPerThread];
+#pragma unroll
+  for (uint32_t t = 0; t < kPerThread; ++t) {
+    const uint32_t i = tid + t * kSortThreads;
+    key[t] = kNoMember;
+    slot[t] = to[t] = 0u;
+    if (i < mine) {
+      key[t] = s_key[i];
+      slot[t] = s_slot[i];
+      const uint32_t x = (uint32_t)(key[t] >> 32), begin = begin_of(x), end = S.at[x >> binShift];
+      to[t] = begin;
+#pragma unroll 4
+      for (uint32_t k = begin; k < end; ++k) to[t] += s_key[k] < key[t] ? 1u : 0u;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t t = 0; t < kPerThread; ++t)
+    if (tid + t * kSortThreads < mine) {
+      s_key[to[t]] = key[t];
+      s_slot[to[t]] = slot[t];
+    }
+  __syncthreads();
+  emit_row(
+      O, s_key, s_slot,
+      [&](uint32_t i, uint32_t x) { return o0 + S.start[x >> binShift] + (i - begin_of(x)); },
+      mine, rowBase);
+}
+
+// Part `part` of a row of more than kRowCap members (several spheres to a
+// cell, or very long rows).  Every part counts the row's members by kRowBins
+// ranges of cells and takes those that begin in its kRowPart places: the small
+// ones together, larger ones one by one, as long as LDS holds them.  Each
+// costs a pass over the row's candidates.  A step of a run of 5,000 spheres in
+// one row of 64 cells, of 16,000 in eight, and of 16,000 with log-normal radii
+// on the floor of an 8^3 grid: with a block for the whole row, each member
+// counted against all of it, 12,300 / 2,450 / 660 us, with this 197 / 84 / 143
+// (with the radix sort 165 / 90 / 134).
+__device__ __forceinline__ void sort_part(const RowTables& T, const uint32_t* keys,
+                                          const uint32_t* idOfSlot, const RowOutputs& O,
+                                          uint32_t r, uint32_t o0, uint32_t m, uint32_t a0,
+                                          uint32_t A, uint32_t c0, uint32_t C, uint32_t part,
+                                          uint64_t* s_key, uint32_t* s_slot, uint32_t* s_wave,
+                                          PartShared& S, uint32_t* devFlags) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const uint32_t U = A + C, rowBase = r << T.shift, inRow = (1u << T.shift) - 1u;
+  const uint32_t binShift = (1u << T.shift) > kRowBins ? T.shift - 8u : 0u;
+  static_assert(kRowBins == 1u << 8, "binShift");
+  // ---- members of each range
+  S.at[2u * tid] = S.at[2u * tid + 1u] = 0u;
+  __syncthreads();
+  for (uint32_t g0 = 0; g0 < U; g0 += kRowCap) {
+    uint32_t key[kPerThread];
+#pragma unroll
+    for (uint32_t t = 0; t < kPerThread; ++t) {
+      const uint32_t u = g0 + t * kSortThreads + tid;
+      key[t] = ~0u;  // no row's: keys are below 2^30
+      if (u < U) key[t] = u < A ? keys[a0 + u] & ~kMovedBit : T.chgList[c0 + (u - A)].y;
+    }
+#pragma unroll
+    for (uint32_t t = 0; t < kPerThread; ++t)
+      if (key[t] >> T.shift == r) atomicAdd(&S.at[(key[t] & inRow) >> binShift], 1u);
+  }
+  __syncthreads();
+  const uint32_t n0 = S.at[2u * tid], n1 = S.at[2u * tid + 1u];
+  uint32_t total, small;
+  const uint32_t s0 = block_exclusive_scan<kSortThreads>(n0 + n1, s_wave, &total), s1 = s0 + n0;
+  if (total != m) {  // the counts and the members disagree: write nothing
+    if (tid == 0) atomicOr(devFlags, DEVERR_ROW_COUNT);
+    return;
+  }
+  S.start[2u * tid] = s0;
+  S.start[2u * tid + 1u] = s1;
+  if (tid == 0) S.start[kRowBins] = m;
+  // ---- this part's ranges: those that begin in it, and the ones beyond LDS
+  // that reach into it
+  const uint32_t lo = part * kRowPart, hi = lo + kRowPart;
+  const bool in0 = s0 >= lo && s0 < hi, in1 = s1 >= lo && s1 < hi;
+  const uint64_t large0 = __ballot(n0 > kRowCap ? s0 < hi && s0 + n0 > lo : n0 > kSmallBin && in0);
+  const uint64_t large1 = __ballot(n1 > kRowCap ? s1 < hi && s1 + n1 > lo : n1 > kSmallBin && in1);
+  if (lane == 0u) {
+    S.large[2u * wave] = large0;
+    S.large[2u * wave + 1u] = large1;
+  }
+  const uint32_t small0 = in0 && n0 <= kSmallBin ? n0 : 0u;
+  const uint32_t small1 = in1 && n1 <= kSmallBin ? n1 : 0u;
+  __syncthreads();  // (and the first scan's readers of s_wave)
+  const uint32_t l0 = block_exclusive_scan<kSortThreads>(small0 + small1, s_wave, &small);
+  S.at[2u * tid] = small0 != 0u ? l0 : kNoBin;
+  S.at[2u * tid + 1u] = small1 != 0u ? l0 + small0 : kNoBin;
+  __syncthreads();
+  // the members of the ranges that S.at gives a place, to the pool, in any order
+  auto gather = [&] {
+    for (uint32_t g0 = 0; g0 < U; g0 += kRowCap) {
+      uint64_t key[kPerThread];
+      uint32_t slot[kPerThread];
+#pragma unroll
+      for (uint32_t t = 0; t < kPerThread; ++t) {
+        const uint32_t u = g0 + t * kSortThreads + tid;
+        slot[t] = 0u;
+        key[t] = u < U ? candidate(T, keys, idOfSlot, r, a0, A, c0, u, &slot[t]) : kNoMember;
+      }
+#pragma unroll
+      for (uint32_t t = 0; t < kPerThread; ++t) {
+        if (key[t] == kNoMember) continue;
+        uint32_t* at = &S.at[(uint32_t)(key[t] >> 32) >> binShift];
+        if (*at == kNoBin) continue;
+        const uint32_t p = atomicAdd(at, 1u);
+        if (p < kRowCap) {
+          s_key[p] = key[t];
+          s_slot[p] = slot[t];
+        }
+      }
+    }
+    __syncthreads();
+  };
+  if (small != 0u) {
+    gather();
+    place_pool(O, o0, small, binShift, rowBase, s_key, s_slot, S);
+  }
+  for (uint32_t w = 0; w < 4u; ++w) {
+    for (uint64_t todo = S.large[w]; todo != 0ull; todo &= todo - 1ull) {
+      const uint32_t bin = 128u * (w >> 1) + 2u * lowest_lane(todo) + (w & 1u);
+      const uint32_t members = S.start[bin + 1u] - S.start[bin];
+      if (members > kRowCap) {
+        if (binShift == 0u)
+          rank_by_counting<true>(T, keys, idOfSlot, O, r, o0, a0, A, c0, C, part, bin, binShift,
+                                 s_key, S);
+        else
+          rank_by_counting<false>(T, keys, idOfSlot, O, r, o0, a0, A, c0, C, part, bin, binShift,
+                                  s_key, S);
+        continue;
+      }
+      __syncthreads();  // the last range's readers
+      S.at[2u * tid] = S.at[2u * tid + 1u] = kNoBin;
+      __syncthreads();
+      if (tid == 0) S.at[bin] = 0u;
+      __syncthreads();
+      gather();
+      place_pool(O, o0, members, binShift, rowBase, s_key, s_slot, S);
+    }
+  }
 }
 
 // The next keys carry kMovedBit; the sorted hashes are written to O.hash
@@ -518,7 +721,7 @@ __device__ void rank_by_counting(const RowTables& T, const uint32_t* keys,
 // list length, as the launch has at most one block per row), then its
 // current range's keys and ids together with its incomers' records, then,
 // after the merge in LDS, the members' state.
-__global__ __launch_bounds__(kSortThreads) void k_row_sort(
+__global__ __launch_bounds__(kSortThreads, kSortWavesPerSimd) void k_row_sort(
     RowTables T, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ idOfSlot,
     RowOutputs O, uint32_t* devFlags) {
   // pool: the stayers in order from the front, the movers from the back;
@@ -528,10 +731,12 @@ __global__ __launch_bounds__(kSortThreads) void k_row_sort(
   __shared__ uint32_t s_wave[kSortThreads / 64];
   __shared__ uint32_t s_count[kPerThread][kSortThreads / 64];  // stayers per chunk and wave
   __shared__ uint32_t s_movers;
+  __shared__ PartShared s_part;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   uint4 e0 = T.rowList[2 * (size_t)blockIdx.x], e1 = T.rowList[2 * (size_t)blockIdx.x + 1];
   const uint32_t listed = *T.listCount;
   if (blockIdx.x == 0 && tid == 0) *T.epoch += 1u;  // the scan of this step is done
+  bool longRows = false;  // this block has parts of long rows, taken at the end
   for (uint32_t j = blockIdx.x; j < listed; j += gridDim.x) {
     if (j != blockIdx.x) {
       e0 = T.rowList[2 * (size_t)j];
@@ -542,7 +747,7 @@ __global__ __launch_bounds__(kSortThreads) void k_row_sort(
     const uint32_t rowBase = r << T.shift;
     __syncthreads();  // the previous row's LDS reads are done
     if (m > kRowCap) {
-      rank_by_counting(T, keys, idOfSlot, O, r, o0, m, a0, A, c0, C, s_key, s_wave, devFlags);
+      longRows = true;
       continue;
     }
     // gather, kRowCap candidates at a time (one group for every row of at
@@ -677,12 +882,45 @@ __global__ __launch_bounds__(kSortThreads) void k_row_sort(
           s_slot[mr[t]] = ms[t];
         }
     } else {
-      // many movers (a transient): count instead
-      rank_by_counting(T, keys, idOfSlot, O, r, o0, m, a0, A, c0, C, s_key, s_wave, devFlags);
-      continue;
+      // many movers (a pile that moves as a whole): every member's place is
+      // the number of members below it
+      uint64_t key[kPerThread];
+      uint32_t sl[kPerThread], to[kPerThread];
+#pragma unroll
+      for (uint32_t t = 0; t < kPerThread; ++t) {
+        const uint32_t i = tid + t * kSortThreads;
+        key[t] = kNoMember;
+        sl[t] = to[t] = 0u;
+        if (i < m) {
+          const uint32_t at = i < stayers ? i : mBase + (i - stayers);
+          key[t] = s_key[at];
+          sl[t] = s_slot[at];
+        }
+      }
+      for (uint32_t q = 0; q < m; ++q) {
+        const uint64_t o = s_key[q < stayers ? q : mBase + (q - stayers)];
+#pragma unroll
+        for (uint32_t t = 0; t < kPerThread; ++t) to[t] += o < key[t] ? 1u : 0u;
+      }
+      __syncthreads();
+#pragma unroll
+      for (uint32_t t = 0; t < kPerThread; ++t)
+        if (tid + t * kSortThreads < m) {
+          s_key[to[t]] = key[t];
+          s_slot[to[t]] = sl[t];
+        }
     }
     __syncthreads();
-    emit_row(O, s_key, s_slot, o0, m, rowBase);
+    emit_row(O, s_key, s_slot, [o0](uint32_t i, uint32_t) { return o0 + i; }, m, rowBase);
+  }
+  if (!longRows) return;
+  for (uint32_t j = blockIdx.x; j < listed; j += gridDim.x) {
+    e0 = T.rowList[2 * (size_t)j];
+    e1 = T.rowList[2 * (size_t)j + 1];
+    if (e0.z <= kRowCap) continue;
+    __syncthreads();  // the previous row's LDS reads are done
+    sort_part(T, keys, idOfSlot, O, e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w, s_key, s_slot,
+              s_wave, s_part, devFlags);
   }
 }
 
@@ -712,14 +950,15 @@ fc_status ensure_row_tables(RowTables& T, const fc_sim_params& P, uint32_t n, bo
   *remade = true;
   free_row_tables(T);
   // count, startNext [rows + 1]; chgStart [rows x copies + 1]; rowList
-  // [2 rows, 16-byte]; groupWords [3 groups, 64-bit]; listCount, epoch [2];
+  // [2 entries, 16-byte]; groupWords [3 groups, 64-bit]; listCount, epoch [2];
   // rowHist, chgHist, chgCursor [rows x copies] (zeroed); chgList [n, 16-byte]
   // every array up to the counters starts on a 64-word (256-byte) boundary,
   // chgList on a 32-byte one
   const size_t cells = (size_t)rows * kRowCopies;
   auto up = [](size_t x) { return (x + 63) & ~(size_t)63; };
   const size_t zeroWords = 3 * cells;
-  const size_t words = 2 * up(rows + 1) + up(cells + 1) + up(8 * (size_t)rows) +
+  const size_t entries = (size_t)rows + n / kRowPart;  // a long row has one for each part
+  const size_t words = 2 * up(rows + 1) + up(cells + 1) + up(8 * entries) +
                        up(6 * (size_t)groups) + up(2) + zeroWords + 4 * (size_t)(n ? n : 1);
   FC_HIP_TRY(hipMalloc(&T.block, words * sizeof(uint32_t)));
   uint32_t* w = T.block;
@@ -730,7 +969,7 @@ fc_status ensure_row_tables(RowTables& T, const fc_sim_params& P, uint32_t n, bo
   T.chgStart = w;
   w += up(cells + 1);
   T.rowList = reinterpret_cast<uint4*>(w);
-  w += up(8 * (size_t)rows);
+  w += up(8 * entries);
   T.groupWords = reinterpret_cast<uint64_t*>(w);
   w += up(6 * (size_t)groups);
   T.listCount = w;
