@@ -158,12 +158,15 @@ struct SortGather {
 // clearHash: when given, the first pass also resets to EMPTY every cell of
 // cellStart/cellEnd that starts a run in the sorted array clearHash (the
 // previous update's cells); requires a pass count >= 2 (minPasses).
+// skip: a device word, written before the sort's launches; where it is not
+// zero they return at once and the outputs stay as they are.
 hipError_t radix_sort_pairs(hipStream_t stream, SortScratch& s, uint32_t* devFlags,
                             const uint32_t* keysIn, const uint32_t* valsIn,
                             uint32_t* keysOut, uint32_t* valsOut, uint32_t n, int bits,
                             StageTimer* timer, bool histogramReady = false, int minPasses = 1,
                             const uint32_t* clearHash = nullptr, uint32_t* cellStart = nullptr,
-                            uint32_t* cellEnd = nullptr, const SortGather* gather = nullptr);
+                            uint32_t* cellEnd = nullptr, const SortGather* gather = nullptr,
+                            const uint32_t* skip = nullptr);
 // Sort of n <= RS_TILE pairs by counting, in two launches that also do the
 // cell-table work of a system step: every key's rank in the stable order
 // (one wave per key over all keys staged in LDS) into keysA/valsA of the

@@ -62,7 +62,7 @@ __global__ void k_mesh_info_init(MeshInfo* I) {
     I->hi[threadIdx.x] = 0ull;
   }
   if (threadIdx.x < 2) I->edges[threadIdx.x] = 0ull;
-  if (threadIdx.x == 0) I->bad = I->pad = 0u;
+  if (threadIdx.x == 0) I->bad = I->open = 0u;
 }
 
 __device__ __forceinline__ void load_corners(const double* __restrict__ verts, uint32_t nv,
@@ -196,10 +196,13 @@ inline int mesh_order_bits(uint32_t nt) { return nt <= (1u << 14) ? 15 : kOrderB
 __global__ __launch_bounds__(kBlock) void k_mesh_order(const double* __restrict__ verts,
                                                         uint32_t nv,
                                                         const uint32_t* __restrict__ tris,
-                                                        uint32_t nt,
-                                                        const MeshInfo* __restrict__ I, int bits,
-                                                        uint32_t* __restrict__ keys) {
+                                                        uint32_t nt, MeshInfo* __restrict__ I,
+                                                        int bits, uint32_t* __restrict__ keys) {
   const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+  // An open mesh is left to the brute force: the sorts and searches that follow
+  // end at once (131 triangles, 200 points: 173 us a call with the whole tree
+  // built in vain, 143 so; 65,536 points 198 and 155).
+  if (t == 0 && !mesh_closed(*I)) I->open = 1u;
   if (t >= nt) return;
   double v[9];
   uint32_t vi[3];
@@ -241,7 +244,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_leaves(const double* __restrict
   }
   TreeTri T;
   uint32_t vi[3];
-  const uint32_t t = order[p];
+  const uint32_t t = min(order[p], nt - 1u);  // (an open mesh's was not written)
   load_corners(verts, nv, tris, t, T.v, vi);
   T.id = t;
   tri[p] = T;
@@ -887,7 +890,7 @@ hipError_t launch_mesh_tree(fc_context* ctx, const double* verts, uint32_t nv,
   hipError_t e = hipGetLastError();
   if (e == hipSuccess)
     e = radix_sort_pairs(s, ctx->sort, ctx->devFlags, keys, nullptr, keys, order, nt, bits,
-                         nullptr);
+                         nullptr, false, 1, nullptr, nullptr, nullptr, nullptr, &info->open);
   if (e != hipSuccess) return e;
   const uint32_t padded = (nt + 7u) & ~7u;
   hipLaunchKernelGGL(k_tree_leaves, dim3((padded + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
@@ -945,7 +948,8 @@ hipError_t launch_tree_points(fc_context* ctx, const MeshTree& T, const double* 
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
       e = radix_sort_pairs(s, ctx->sort, ctx->devFlags, keys, nullptr, keys, order, n,
-                           kOrderBits, nullptr);
+                           kOrderBits, nullptr, false, 1, nullptr, nullptr, nullptr, nullptr,
+                           &T.info->open);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_tree_signs, dim3((n + kRaysPerWave - 1) / kRaysPerWave), dim3(kLanes), 0,
                        s, T, p, n, order, sdf + at);

@@ -16,7 +16,8 @@ namespace fc {
 struct MeshInfo {
   unsigned long long lo[3], hi[3];
   unsigned long long edges[2];
-  uint32_t bad, pad;
+  uint32_t bad;
+  uint32_t open;  // 1 when mesh_closed is false (k_mesh_order)
 };
 
 // A triangle in tree order: its corners and its number in the mesh.

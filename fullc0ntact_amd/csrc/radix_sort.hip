@@ -84,7 +84,9 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, uint64_t active) {
 // Standalone digit-0 histogram (used when the keys come from the caller).
 __global__ __launch_bounds__(RS_THREADS) void k_rs_histogram(
     const uint32_t* __restrict__ keys, uint32_t n, int passes, int bits,
-    uint32_t* __restrict__ gHist, uint32_t* counters, uint32_t* devFlags) {
+    uint32_t* __restrict__ gHist, uint32_t* counters, uint32_t* devFlags,
+    const uint32_t* __restrict__ skip) {
+  if (skip != nullptr && *skip != 0u) return;
   __shared__ uint32_t s_hist[RS_RADIX];
   for (int i = threadIdx.x; i < RS_RADIX; i += RS_THREADS) s_hist[i] = 0u;
   histogram_producer_prologue(gHist, passes, counters);
@@ -125,7 +127,9 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
     uint32_t* __restrict__ keysOut, uint32_t* __restrict__ valsOut, uint32_t n, int pass,
     int passes, uint32_t* gHist, uint64_t* status, uint64_t* groupStatus, uint32_t* counters,
     uint32_t* devFlags, const uint32_t* __restrict__ clearHash, uint32_t* __restrict__ cellStart,
-    uint32_t* __restrict__ cellEnd, SortGather ga, int ticketed) {
+    uint32_t* __restrict__ cellEnd, SortGather ga, int ticketed,
+    const uint32_t* __restrict__ skip) {
+  if (skip != nullptr && *skip != 0u) return;
   constexpr uint32_t kTile = (uint32_t)RS_THREADS * kItems;
   constexpr uint32_t kTileWaveKeys = 64u * kItems;
   __shared__ uint32_t s_keys[kTile];
@@ -513,7 +517,8 @@ hipError_t radix_sort_pairs(hipStream_t stream, SortScratch& s, uint32_t* devFla
                             const uint32_t* keysIn, const uint32_t* valsIn, uint32_t* keysOut,
                             uint32_t* valsOut, uint32_t n, int bits, StageTimer* timer,
                             bool histogramReady, int minPasses, const uint32_t* clearHash,
-                            uint32_t* cellStart, uint32_t* cellEnd, const SortGather* gather) {
+                            uint32_t* cellStart, uint32_t* cellEnd, const SortGather* gather,
+                            const uint32_t* skip) {
   if (n == 0) return hipSuccess;
   const bool inPlace = keysIn == keysOut || (valsIn != nullptr && valsIn == valsOut);
   int passes = radix_passes(bits, inPlace);
@@ -536,7 +541,7 @@ hipError_t radix_sort_pairs(hipStream_t stream, SortScratch& s, uint32_t* devFla
     if (histBlocks > (uint32_t)RS_MAX_HIST_BLOCKS) histBlocks = RS_MAX_HIST_BLOCKS;
     if (timer) timer->begin(stream, "sort_histogram");
     hipLaunchKernelGGL(k_rs_histogram, dim3(histBlocks), dim3(RS_THREADS), 0, stream, keysIn, n,
-                       passes, bits, s.histogram, s.counters, devFlags);
+                       passes, bits, s.histogram, s.counters, devFlags, skip);
     e = hipGetLastError();
     if (timer) timer->end(stream);
     if (e != hipSuccess) return e;
@@ -568,12 +573,12 @@ hipError_t radix_sort_pairs(hipStream_t stream, SortScratch& s, uint32_t* devFla
       hipLaunchKernelGGL(k_rs_scatter<2 * RS_ITEMS>, dim3(numTiles), dim3(RS_THREADS), 0, stream,
                          kin, vin, kout, vout, n, p, passes, s.histogram, s.status,
                          s.groupStatus, s.counters, devFlags, p == 0 ? clearHash : nullptr,
-                         cellStart, cellEnd, ga, ticketed);
+                         cellStart, cellEnd, ga, ticketed, skip);
     else
       hipLaunchKernelGGL(k_rs_scatter<RS_ITEMS>, dim3(numTiles), dim3(RS_THREADS), 0, stream,
                          kin, vin, kout, vout, n, p, passes, s.histogram, s.status,
                          s.groupStatus, s.counters, devFlags, p == 0 ? clearHash : nullptr,
-                         cellStart, cellEnd, ga, ticketed);
+                         cellStart, cellEnd, ga, ticketed, skip);
     e = hipGetLastError();
     if (timer) timer->end(stream);
     if (e != hipSuccess) return e;

@@ -50,3 +50,37 @@ def test_runs_around_a_call(n, grid, call):
         s.close()
     ps.close()
     ctx.close()
+
+
+def test_open_and_closed_meshes_in_turn():
+    """The sorts of an open mesh end at once; those of the meshes and systems
+    after it on the same scratch are as ever."""
+    from fullc0ntact_amd import Context, ParticleSystem, make_params
+    from fullc0ntact_amd.distance_map import mesh_signed_distance
+    rng = np.random.default_rng(5)
+    ctx = Context(0)
+    n, grid = 6000, (4, 1024, 512)  # sorts by radix
+    P = make_params(n, grid[0], 1.0 / 64.0, gridSize=grid, numCells=int(np.prod(grid)))
+    pos = np.ones((n, 4), np.float32)
+    pos[:, :3] = rng.uniform(-0.95, 0.95, (n, 3))
+    vel = np.zeros((n, 4), np.float32)
+    ps = ParticleSystem(n, grid, context=ctx)
+    ps.m_params = P
+    ps.setArray(ps.POSITION, pos, 0, n)
+    ps.setArray(ps.VELOCITY, vel, 0, n)
+    st = orc.State(pos, vel, P.numCells)
+    for nu, nv, cut in ((16, 4, 0), (33, 4, 1), (33, 4, 0), (40, 8, 5), (64, 8, 0)):
+        v, f = meshes.torus_knot(2, 3, nu, nv, radius=0.2, scale=0.3)
+        f = f[:len(f) - cut]
+        q = rng.uniform(-1.0, 1.0, (9000, 3))
+        print(len(f), cut, flush=True)
+        sd, cp = mesh_signed_distance(ctx, v, f, q)
+        rsd, rcp, _ = orc.mesh_sdf(v, f, q)
+        far = np.abs(rsd) > 1e-14
+        assert np.array_equal(sd[far], rsd[far]) and np.array_equal(cp, rcp)
+        ps.run(0.5, 11)
+        for _ in range(11):
+            st.update(0.5, orc.params_from(P))
+        _compare_system(ps, st)
+    ps.close()
+    ctx.close()
