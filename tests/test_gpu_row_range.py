@@ -100,3 +100,12 @@ def test_either_side_of_the_line(gpu_ctx, n):
     nv = Stages(gpu_ctx, P).collide(sp, sv, i, cs, ce, vel)
     onv = orc.collide(sp, sv, i, cs, ce, OP, newVel4=vel)
     assert np.array_equal(bits(nv), bits(onv))
+
+
+def test_flat_grid_at_the_walls(gpu_ctx, many):
+    walls.test_system_at_the_walls(gpu_ctx, (32, 4, 8))
+
+
+@pytest.mark.parametrize("pile", [2, 63, 64, 200])
+def test_moving_piles_of_other_sizes(gpu_ctx, many, pile):
+    walls.test_piles_that_move_as_a_whole(gpu_ctx, pile)
