@@ -630,7 +630,7 @@ fc_status enqueue_batch_run(fc_batch* b, float dt, uint32_t steps) {
   const bool rowMode = batch_row_mode(b);
   if (rowMode) {
     bool remade = false;
-    const fc_status s = ensure_row_tables(b->rowTables, batch_row_grid(b), b->n, &remade);
+    const fc_status s = ensure_row_tables(b->rowTables, batch_row_grid(b), b->n, st, &remade);
     if (remade) drop_batch_graph(b);  // the captured steps hold the tables
     FC_TRY(s);
   }

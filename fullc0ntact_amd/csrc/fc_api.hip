@@ -343,10 +343,11 @@ fc_status fc_context_create(int device, fc_context** out) {
             hipMalloc(&s.counters, RSC_COUNT * sizeof(uint32_t)) == hipSuccess &&
             hipMalloc(&s.histogram, (size_t)RS_HIST_COPIES * RS_MAX_PASSES * RS_RADIX *
                                         sizeof(uint32_t)) == hipSuccess &&
-            hipMemset(s.histogram, 0, (size_t)RS_HIST_COPIES * RS_MAX_PASSES * RS_RADIX *
-                                          sizeof(uint32_t)) == hipSuccess &&
-            hipMemset(ctx->devFlags, 0, 2 * sizeof(uint32_t)) == hipSuccess &&
-            hipMemset(s.counters, 0, RSC_COUNT * sizeof(uint32_t)) == hipSuccess;
+            hipMemsetAsync(s.histogram, 0, (size_t)RS_HIST_COPIES * RS_MAX_PASSES * RS_RADIX *
+                                               sizeof(uint32_t), ctx->stream) == hipSuccess &&
+            hipMemsetAsync(ctx->devFlags, 0, 2 * sizeof(uint32_t), ctx->stream) == hipSuccess &&
+            hipMemsetAsync(s.counters, 0, RSC_COUNT * sizeof(uint32_t), ctx->stream) ==
+                hipSuccess;
   if (!ok) {
     fc_context_destroy(ctx);
     return set_error(FC_ERROR_OUT_OF_MEMORY, "context allocation failed");

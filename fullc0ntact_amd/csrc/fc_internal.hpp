@@ -411,8 +411,10 @@ struct RowOutputs {
 constexpr uint64_t kMaxRows = 1ull << 22;
 bool row_resort_grid_ok(const fc_sim_params& P);
 RowHists row_hists(const RowTables& T);
-// *remade: the tables are new ones, steps captured before hold others.
-fc_status ensure_row_tables(RowTables& T, const fc_sim_params& P, uint32_t n, bool* remade);
+// Clears new tables on s.  *remade: the tables are new ones, steps captured
+// before hold others.
+fc_status ensure_row_tables(RowTables& T, const fc_sim_params& P, uint32_t n, hipStream_t s,
+                            bool* remade);
 void free_row_tables(RowTables& T);
 hipError_t launch_row_clear(hipStream_t s, const RowTables& T);
 hipError_t launch_row_scan(hipStream_t s, const RowTables& T, uint32_t* devFlags);

@@ -439,7 +439,8 @@ fc_status fc_system_set_polydisperse(fc_system* sys, int enable) {
   if (enable && !sys->piles) {
     const size_t words = (size_t)sys->n + kPilesList;
     FC_HIP_TRY(hipMalloc(&sys->piles, words * sizeof(uint32_t)));
-    FC_HIP_TRY(hipMemset(sys->piles, 0, kPilesList * sizeof(uint32_t)));
+    // (on the stream that runs the kernels: it does not wait for the null stream)
+    FC_HIP_TRY(hipMemsetAsync(sys->piles, 0, kPilesList * sizeof(uint32_t), sys->ctx->stream));
   }
   sys->polydisperse = enable ? 1 : 0;
   drop_graph(sys);  // the captured step carries the radius mode in its kernels
@@ -470,8 +471,10 @@ fc_status fc_system_create(fc_context* ctx, uint32_t numParticles, fc_uint3 grid
   if (e == hipSuccess) e = hipMalloc(&sys->keys, n * sizeof(uint32_t));
   if (e == hipSuccess) e = hipMalloc(&sys->slotOf, n * sizeof(uint32_t));
   if (e == hipSuccess) e = hipMalloc(&sys->idOfSlot, n * sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMemset(sys->pos, 0, n * sizeof(float4));
-  if (e == hipSuccess) e = hipMemset(sys->vel, 0, n * sizeof(float4));
+  if (e == hipSuccess) e = hipMemsetAsync(sys->pos, 0, n * sizeof(float4), ctx->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(sys->vel, 0, n * sizeof(float4), ctx->stream);
+  // (done when the caller has the arrays: they may be written from elsewhere)
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
     free_system_buffers(sys);
     delete sys;
@@ -582,7 +585,7 @@ fc_status fc_system_run(fc_system* sys, float deltaTime, uint32_t steps) {
   StageTimer* timer = ctx->timer.enabled ? &ctx->timer : nullptr;
   if (run_row_mode(sys)) {
     bool remade = false;
-    const fc_status s = ensure_row_tables(sys->rowTables, sys->params, sys->n, &remade);
+    const fc_status s = ensure_row_tables(sys->rowTables, sys->params, sys->n, ctx->stream, &remade);
     // the captured steps hold the tables (a shape of as many cells may have
     // come and gone without a capture), or ran without them
     if (remade) drop_graph(sys);

@@ -939,7 +939,8 @@ RowHists row_hists(const RowTables& T) {
   return h;
 }
 
-fc_status ensure_row_tables(RowTables& T, const fc_sim_params& P, uint32_t n, bool* remade) {
+fc_status ensure_row_tables(RowTables& T, const fc_sim_params& P, uint32_t n, hipStream_t s,
+                            bool* remade) {
   *remade = false;
   uint32_t shift = 0;
   while ((1u << shift) < P.gridSize.x) ++shift;
@@ -988,7 +989,7 @@ fc_status ensure_row_tables(RowTables& T, const fc_sim_params& P, uint32_t n, bo
   T.shift = shift;
   T.groups = groups;
   T.capacity = n;
-  const hipError_t e = hipMemset(T.block, 0, words * sizeof(uint32_t));
+  const hipError_t e = hipMemsetAsync(T.block, 0, words * sizeof(uint32_t), s);
   if (e != hipSuccess) {
     free_row_tables(T);  // (else the next call would take them as they are)
     return hip_error(e, "row tables");

@@ -43,7 +43,8 @@ struct Runtime {
   size_t inUse = 0, most = ~(size_t)0;     // hipMalloc fails beyond `most` bytes in use
   size_t failing = 0;                      // nor for this size exactly
   hipError_t last = hipSuccess;
-  hipError_t memsetError = hipSuccess;     // what the next hipMemset returns
+  hipError_t memsetError = hipSuccess;     // what the next clear returns
+  int unordered = 0;                       // clears on the null stream
   std::map<const void*, std::string> names;
   Graph* capturing = nullptr;
   struct { dim3 grid, block; size_t shared; hipStream_t stream; } config;
@@ -190,11 +191,17 @@ hipError_t hipFree(void* p) {
   return hipSuccess;
 }
 hipError_t hipMemset(void*, int, size_t) {
+  ++rt().unordered;
   const hipError_t e = rt().memsetError;
   rt().memsetError = hipSuccess;
   return result(e);
 }
-hipError_t hipMemsetAsync(void*, int, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipMemsetAsync(void*, int, size_t, hipStream_t) {
+  if (rt().capturing) rt().fault = "hipMemsetAsync inside a capture";
+  const hipError_t e = rt().memsetError;
+  rt().memsetError = hipSuccess;
+  return result(e);
+}
 hipError_t hipMemcpyAsync(void* dst, const void*, size_t size, hipMemcpyKind kind, hipStream_t) {
   if (kind == hipMemcpyDeviceToHost) std::memset(dst, 0, size);
   return hipSuccess;
@@ -436,6 +443,20 @@ int no_row_tables() {
   return 0;
 }
 
+// The contexts' streams do not wait for the null stream: what a kernel reads is
+// cleared on the stream that launches it.
+int clears() {
+  fc_context* c = context();
+  fc_system* s = nullptr;
+  OK(fc_system_create(c, 20000, fc_uint3{64, 64, 64}, &s));
+  OK(fc_system_set_polydisperse(s, 1));
+  OK(fc_system_run(s, 0.5f, 20));
+  REQUIRE(launched("k_collide_piles") && launched("k_row_sort"));
+  OK(labels(c));
+  REQUIRE(rt().unordered == 0);
+  return 0;
+}
+
 // An error that a call has returned is that call's alone.
 int errors_once() {
   fc_context* c = context();
@@ -508,6 +529,7 @@ int run(const std::string& name) {
   if (name == "row-tables-small") return row_tables(8000);
   if (name == "row-tables") return row_tables(40000);
   if (name == "no-row-tables") return no_row_tables();
+  if (name == "clears") return clears();
   if (name == "errors-once") return errors_once();
   if (name == "growth-fails-small") return growth_fails(4096, fc_uint3{64, 64, 64});
   if (name == "growth-fails-radix") return growth_fails(8000, fc_uint3{4, 1024, 512});

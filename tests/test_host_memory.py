@@ -57,3 +57,7 @@ def test_captured_steps_and_new_row_tables(program, scenario):
 
 def test_runs_without_row_tables(program):
     holds(program, "no-row-tables")
+
+
+def test_memory_is_cleared_on_the_stream_that_reads_it(program):
+    holds(program, "clears")
