@@ -295,6 +295,9 @@ constexpr int kTriTile = 128;
 // Blocks walk the points with the grid's stride, so that a launch that finds
 // nothing to do is short.
 constexpr unsigned kSdfMaxBlocks = 4096;
+// A builder's copy of its mesh of up to so many bytes stays in the context's
+// scratch for the next one.
+constexpr size_t kMeshCopyKept = (size_t)256 << 20;
 
 template <bool kLattice>
 __global__ __launch_bounds__(kBlock) void k_mesh_sdf(
@@ -885,14 +888,17 @@ fc_status fc_distmap_build(fc_context* ctx, const double* vertices, uint32_t num
   }
   m->cellSize = cellSize;
   hipStream_t st = ctx->stream;
-  // the mesh's copy lies in the context's scratch, after the tree
+  // the mesh's copy lies in the context's scratch, after the tree; a large one
+  // (the tree's own part is bounded by its 2^22 triangles) is not kept there
   const size_t vb = (size_t)numVertices * 3 * sizeof(double),
                tb = (size_t)numTriangles * 3 * sizeof(uint32_t);
+  const bool keep = vb + tb <= kMeshCopyKept;
   const bool tree = mesh_tree_pays(numTriangles, m->V) && tree_lattice_fits(cells, b, cs);
   const size_t at = tree ? mesh_tree_bytes(numTriangles) : 0;
   hipError_t e = hipSuccess;
   void* own = nullptr;
-  const bool kept = tree_scratch(ctx, tree ? numTriangles : 0, at + vb + tb);
+  const bool scratch = tree_scratch(ctx, tree ? numTriangles : 0, at + (keep ? vb + tb : 0));
+  const bool kept = scratch && keep;
   if (!kept) e = hipMalloc(&own, vb + tb);
   double* dv = reinterpret_cast<double*>(kept ? static_cast<char*>(ctx->meshScratch) + at
                                               : static_cast<char*>(own));
@@ -901,7 +907,7 @@ fc_status fc_distmap_build(fc_context* ctx, const double* vertices, uint32_t num
   if (e == hipSuccess) e = hipMemcpyAsync(dt, triangles, tb, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = upload_axes(m, ax, st);
   MeshTree T;
-  if (e == hipSuccess && tree && kept) {
+  if (e == hipSuccess && tree && scratch) {
     e = launch_mesh_tree(ctx, dv, numVertices, dt, numTriangles, ctx->meshScratch, &T);
     if (e == hipSuccess)
       e = launch_tree_lattice(st, T, dv, numVertices, dt, numTriangles, m->cells, b, cs, m->cpd,

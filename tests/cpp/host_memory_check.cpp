@@ -457,6 +457,27 @@ int clears() {
   return 0;
 }
 
+// The copy of a mesh too large for the tree goes with the call that made it.
+int large_meshes() {
+  fc_context* c = context();
+  OK(build_map(c));
+  const size_t before = rt().inUse;
+  std::vector<double> v((size_t)3 << 24, 0.5);  // 400 MB
+  std::vector<uint32_t> f(3 * kMapTriangles);
+  for (uint32_t i = 0; i < f.size(); ++i) f[i] = i;
+  const int32_t cells[3] = {8, 8, 8};
+  const float lo[3] = {-1.0f, -1.0f, -1.0f};
+  for (uint32_t triangles : {12u, kMapTriangles}) {
+    fc_distmap* m = nullptr;
+    rt().launched.clear();
+    OK(fc_distmap_build(c, v.data(), 1u << 24, f.data(), triangles, cells, 0.25f, lo, &m));
+    REQUIRE(launched("k_tree_leaves") == (triangles > 12));
+    OK(fc_distmap_destroy(m));
+    REQUIRE(rt().inUse < before + (64u << 20));
+  }
+  return 0;
+}
+
 // An error that a call has returned is that call's alone.
 int errors_once() {
   fc_context* c = context();
@@ -530,6 +551,7 @@ int run(const std::string& name) {
   if (name == "row-tables") return row_tables(40000);
   if (name == "no-row-tables") return no_row_tables();
   if (name == "clears") return clears();
+  if (name == "large-meshes") return large_meshes();
   if (name == "errors-once") return errors_once();
   if (name == "growth-fails-small") return growth_fails(4096, fc_uint3{64, 64, 64});
   if (name == "growth-fails-radix") return growth_fails(8000, fc_uint3{4, 1024, 512});

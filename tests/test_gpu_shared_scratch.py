@@ -84,3 +84,19 @@ def test_open_and_closed_meshes_in_turn():
         _compare_system(ps, st)
     ps.close()
     ctx.close()
+
+
+def test_map_of_a_mesh_that_is_not_kept(gpu_ctx):
+    """A mesh whose copy is too large for the context's scratch (vertices that
+    no triangle names) gives the same map."""
+    from fullc0ntact_amd.distance_map import DistanceMap
+    v, f = meshes.torus_knot(2, 3, 64, 8, radius=0.2, scale=0.3)
+    lay = []
+    for pad in (0, (256 << 20) // 24):
+        w = np.concatenate([v, np.zeros((pad, 3))])
+        print(len(w), flush=True)
+        m = DistanceMap.from_mesh(gpu_ctx, w, f, (15, 16, 17), 0.125, (-1.0, -1.0, -1.0))
+        lay.append(m.download())
+        m.close()
+    for k in lay[0]:
+        assert np.array_equal(lay[0][k], lay[1][k]), k

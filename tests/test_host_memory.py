@@ -61,3 +61,7 @@ def test_runs_without_row_tables(program):
 
 def test_memory_is_cleared_on_the_stream_that_reads_it(program):
     holds(program, "clears")
+
+
+def test_large_meshes_are_not_kept(program):
+    holds(program, "large-meshes")
