@@ -330,6 +330,8 @@ void generate_initial_state(float* pos, float* vel, uint32_t n, fc_particle_conf
                             uint64_t seed, float r, float jitterFrac, float velAmp);
 // Grows the context's sort scratch to hold n keys (synchronises first).
 fc_status ensure_sort_capacity(fc_context* ctx, size_t n);
+// An error when a grid change found no memory for any cell tables.
+fc_status need_tables(const fc_system* sys);
 // Synchronises the context stream and converts the device error word.
 fc_status check_device_flags(fc_context* ctx);
 fc_sim_params default_params(uint32_t numParticles, fc_uint3 gridSize);

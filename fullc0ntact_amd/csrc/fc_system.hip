@@ -73,14 +73,37 @@ void drop_graph(fc_system* sys) {
   }
 }
 
+hipError_t alloc_pair(uint32_t** a, uint32_t** b, uint32_t count) {
+  hipError_t e = hipMalloc(a, (size_t)count * sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMalloc(b, (size_t)count * sizeof(uint32_t));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // handled by the caller
+    hipFree(*a);
+    *a = *b = nullptr;
+  }
+  return e;
+}
+
+// Cell tables for numCells.  Without memory for them the system keeps those of
+// its parameters (sys->params).
 fc_status alloc_tables(fc_system* sys, uint32_t numCells) {
-  hipFree(sys->cellStart);
-  hipFree(sys->cellEnd);
-  sys->cellStart = sys->cellEnd = nullptr;
-  FC_HIP_TRY(hipMalloc(&sys->cellStart, (size_t)numCells * sizeof(uint32_t)));
-  FC_HIP_TRY(hipMalloc(&sys->cellEnd, (size_t)numCells * sizeof(uint32_t)));
-  sys->tablesTrackHash = false;
-  return FC_SUCCESS;
+  uint32_t *start = nullptr, *end = nullptr;
+  hipError_t e = alloc_pair(&start, &end, numCells);
+  const bool had = sys->cellStart != nullptr;
+  if (e == hipSuccess || had) {
+    hipFree(sys->cellStart);
+    hipFree(sys->cellEnd);
+    sys->cellStart = start;
+    sys->cellEnd = end;
+    sys->tablesTrackHash = false;
+  }
+  if (e != hipSuccess && had) {
+    // no room beside the old ones: in their place, or else they come back
+    e = alloc_pair(&sys->cellStart, &sys->cellEnd, numCells);
+    if (e != hipSuccess)
+      (void)alloc_pair(&sys->cellStart, &sys->cellEnd, sys->params.numCells);
+  }
+  return e == hipSuccess ? FC_SUCCESS : hip_error(e, "cell tables");
 }
 
 // One update(dt) (particleSystem.cpp:222-284): integrate -> calcHash ->
@@ -91,6 +114,7 @@ fc_status enqueue_update(fc_system* sys, float dt, StageTimer* timer) {
   hipStream_t st = ctx->stream;
   const fc_sim_params& P = sys->params;
   const uint32_t n = sys->n;
+  FC_TRY(need_tables(sys));
   hipError_t e = hipSuccess;
   const uint32_t* prev = nullptr;
   if (sys->tablesTrackHash) {
@@ -191,6 +215,7 @@ fc_status enqueue_run_head(fc_system* sys, float dt, StageTimer* timer) {
   const fc_sim_params& P = sys->params;
   const uint32_t n = sys->n;
   const int passes = run_passes(P);
+  FC_TRY(need_tables(sys));
   hipError_t e = hipSuccess;
   const uint32_t* prev = nullptr;
   if (sys->tablesTrackHash) {
@@ -351,6 +376,12 @@ fc_status capture_graph(fc_system* sys, float dt) {
 
 }  // namespace
 
+fc_status need_tables(const fc_system* sys) {
+  if (sys->cellStart != nullptr) return FC_SUCCESS;
+  return set_error(FC_ERROR_OUT_OF_MEMORY, "the system has no cell tables: set its parameters "
+                                           "again when there is memory for them");
+}
+
 // reset(CONFIG_GRID / CONFIG_RANDOM) (particleSystem.cpp:380-444) into host
 // float4 arrays with a SplitMix64 stream: CONFIG_GRID is the s^3 lattice of
 // spacing 2r from -1+r (s = smallest integer with s^3 >= n) jittered by
@@ -508,7 +539,7 @@ uint32_t fc_system_num_particles(const fc_system* sys) { return sys ? sys->n : 0
 fc_status fc_system_set_params(fc_system* sys, const fc_sim_params* params) {
   if (!sys || !params) return set_error(FC_ERROR_INVALID_VALUE, "NULL argument");
   FC_TRY(validate_params(*params));
-  if (params->numCells != sys->params.numCells) {
+  if (params->numCells != sys->params.numCells || sys->cellStart == nullptr) {
     FC_HIP_TRY(hipStreamSynchronize(sys->ctx->stream));
     drop_graph(sys);
     FC_TRY(alloc_tables(sys, params->numCells));
@@ -639,6 +670,7 @@ fc_status fc_system_device_arrays(fc_system* sys, float** pos, float** vel, floa
 fc_status fc_system_dump_grid(fc_system* sys, uint32_t* maxParticlesPerCell,
                               uint32_t* occupiedCells) {
   if (!sys) return set_error(FC_ERROR_INVALID_VALUE, "sys is NULL");
+  FC_TRY(need_tables(sys));
   const uint32_t C = sys->params.numCells;
   std::vector<uint32_t> cs(C), ce(C);
   FC_HIP_TRY(hipMemcpyAsync(cs.data(), sys->cellStart, (size_t)C * 4, hipMemcpyDeviceToHost,

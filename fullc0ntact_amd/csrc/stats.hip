@@ -198,6 +198,7 @@ fc_status fc_system_contact_histogram(fc_system* sys, uint32_t* hist, uint32_t n
   if (!sys || !hist) return set_error(FC_ERROR_INVALID_VALUE, "NULL argument");
   if (nbins == 0 || nbins > kStatMaxBins)
     return set_error(FC_ERROR_INVALID_VALUE, "nbins must be in [1, 4096]");
+  FC_TRY(need_tables(sys));
   fc_context* ctx = sys->ctx;
   FC_TRY(ensure_stats_scratch(ctx));
   uint32_t* dHist = stats_hist(ctx);

@@ -118,6 +118,8 @@ Node node_of(const std::string& name, void** args) {
       // the rank sort's staging arrays are always there
       if (pointer && p == 0 && n.kernel == "k_small_rank" && i >= 6)
         rt().fault = "k_small_rank without its scratch";
+      if (pointer && p == 0 && n.kernel.rfind("k_collide_", 0) == 0 && (i == 7 || i == 8))
+        rt().fault = n.kernel + " without cell tables";
     }
   }
   return n;
@@ -478,6 +480,44 @@ int large_meshes() {
   return 0;
 }
 
+// A grid for whose cell tables there is no memory is refused, and the system
+// runs on with the one that it has; or says so, if even that one is gone.
+int no_cell_tables(uint32_t n) {
+  fc_context* c = context();
+  fc_system* s = nullptr;
+  OK(fc_system_create(c, n, fc_uint3{64, 64, 64}, &s));
+  OK(fc_system_run(s, 0.5f, 20));
+  fc_sim_params a, b;
+  OK(fc_system_get_params(s, &a));
+  b = a;
+  b.gridSize = fc_uint3{256, 256, 256};
+  b.numCells = 1u << 24;
+  rt().failing = 4u << 24;
+  REQUIRE(fc_system_set_params(s, &b) == FC_ERROR_OUT_OF_MEMORY);
+  rt().failing = 0;
+  OK(fc_system_update(s, 0.5f));
+  OK(fc_system_run(s, 0.5f, 20));
+  rt().most = rt().inUse + (4u << 24);  // room in the place of the old tables only
+  OK(fc_system_set_params(s, &a));
+  b.gridSize = fc_uint3{128, 64, 64};
+  b.numCells = 1u << 19;
+  rt().most = rt().inUse + (2u << 20);
+  OK(fc_system_set_params(s, &b));
+  rt().most = ~(size_t)0;
+  OK(fc_system_run(s, 0.5f, 20));
+  rt().most = 0;
+  REQUIRE(fc_system_set_params(s, &a) == FC_ERROR_OUT_OF_MEMORY);
+  REQUIRE(fc_system_update(s, 0.5f) == FC_ERROR_OUT_OF_MEMORY);
+  REQUIRE(fc_system_run(s, 0.5f, 20) == FC_ERROR_OUT_OF_MEMORY);
+  uint32_t most, occupied, hist[8];
+  REQUIRE(fc_system_dump_grid(s, &most, &occupied) == FC_ERROR_OUT_OF_MEMORY);
+  REQUIRE(fc_system_contact_histogram(s, hist, 8) == FC_ERROR_OUT_OF_MEMORY);
+  rt().most = ~(size_t)0;
+  OK(fc_system_set_params(s, &a));
+  OK(fc_system_run(s, 0.5f, 20));
+  return 0;
+}
+
 // An error that a call has returned is that call's alone.
 int errors_once() {
   fc_context* c = context();
@@ -552,6 +592,8 @@ int run(const std::string& name) {
   if (name == "no-row-tables") return no_row_tables();
   if (name == "clears") return clears();
   if (name == "large-meshes") return large_meshes();
+  if (name == "no-cell-tables-small") return no_cell_tables(3000);
+  if (name == "no-cell-tables") return no_cell_tables(40000);
   if (name == "errors-once") return errors_once();
   if (name == "growth-fails-small") return growth_fails(4096, fc_uint3{64, 64, 64});
   if (name == "growth-fails-radix") return growth_fails(8000, fc_uint3{4, 1024, 512});

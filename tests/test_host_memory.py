@@ -65,3 +65,8 @@ def test_memory_is_cleared_on_the_stream_that_reads_it(program):
 
 def test_large_meshes_are_not_kept(program):
     holds(program, "large-meshes")
+
+
+@pytest.mark.parametrize("scenario", ["no-cell-tables-small", "no-cell-tables"])
+def test_grids_without_memory(program, scenario):
+    holds(program, scenario)
