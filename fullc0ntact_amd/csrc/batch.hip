@@ -506,11 +506,11 @@ fc_status capture_batch_graph(fc_batch* b, float dt) {
 // resort's cost is a chain of dependent loads per row, and a scene's grid
 // rows hold few spheres (about 20 on the freshly dropped 64^3 ensemble):
 // per ensemble step, 1 grid row per row measured 1.876 ms, 4 1.391 ms,
-// 8 1.323 ms (radix passes: 1.663 ms); 16 and 32 (4.6 and 9.1 ms) put
-// rows past the row sort's LDS capacity (768 members) into its counting
-// path.  A settled bed (about 2.2 spheres per occupied cell, some 140 per
-// 64-cell grid row) would do that to 8 as well; 4 keeps such rows near
-// 570 members.
+// 8 1.323 ms (radix passes: 1.663 ms).  16 and 32 (4.6 and 9.1 ms while one
+// block ranked such a row by counting) put rows past the row sort's LDS
+// capacity (768 members).  A settled bed (about 2.2 spheres per occupied
+// cell, some 140 per 64-cell grid row) would do that to 8 as well; 4 keeps
+// such rows near 570 members.
 constexpr uint32_t kBatchRowGridRows = 4;
 
 fc_sim_params batch_row_grid(const fc_batch* b) {

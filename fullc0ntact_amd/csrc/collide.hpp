@@ -72,9 +72,12 @@ static_assert(kRowsBatch >= 1 && (uint32_t)kRowsBatch - 1u <= kSortedPosPad, "ro
 // Candidates whose loads are issued together in k_collide_v3.
 constexpr int kBatch = 4;
 // Polydisperse: spheres with more candidates than this are left to
-// k_collide_piles unread.  A step of 20,000 / 120,011 / 200,000 spheres on the
-// knot (the more, the denser): 96: 59 / 101 / 187 us, 128: 62 / 77 / 112, 144:
-// 64 / 78 / 100, 160: 65 / 79 / 89; no bound, with one counter: 70 / 87 / -.
+// k_collide_piles unread.  A step of a run of 20,000 / 50,000 / 120,011 /
+// 200,000 spheres on the knot (the more, the denser; medians over two states):
+// 112: 60 / 67 / 90 / 156 us, 144: 60 / 70 / 80 / 104, 160: 60 / 71 / 81 / 94,
+// 176: 60 / 72 / 83 / 93, 192: 60 / 73 / 84 / 94, 256: 60 / 75 / 87 / 96, no
+// bound 60 / 75 / 88 / 97.  No one bound is best at every density: 144 is
+// within 5 % of the best up to 120,011 and 12 % over it at 200,000.
 constexpr uint32_t kPileCandidates = 144;
 
 // The cursor sphere of collideD (particles_kernel.cu:286-288): its pair

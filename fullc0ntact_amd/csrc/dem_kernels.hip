@@ -951,12 +951,14 @@ hipError_t launch_collide(hipStream_t s, const fc_sim_params& P, bool poly, uint
 // Whether a run's fused collide stores the next key at the sorted slot for a
 // row resort, on a grid whose row tables fit; up to RS_TILE spheres a step
 // sorts by counting ranks.  Small systems leave grids of many rows (the scan
-// reads every row) and of few (a row beyond the resort's LDS is ranked by
-// counting) to the radix sort, which carries the key at the id and the slot
-// map.  A step of 8,000 / 16,000 spheres with the resort against the radix
-// sort: 64^3 grid 27 / 29 us against 45 / 47, 256^3 30 / 34 against 45 / 48,
-// 64 x 512 x 512 37 / 39 against 45 / 47, 64 x 1024 x 1024 69 / 70 against
-// 53 / 56, 8^3 46 / 74 against 58 / 85, 4^3 143 / 1382 against 150 / 371.
+// reads every row) and of few (their rows are beyond the resort's LDS and go
+// to it in parts) to the radix sort, which carries the key at the id and the
+// slot map.  A step of 8,000 / 16,000 spheres at random with the resort against
+// the radix sort: 64^3 grid 29 / 30 us against 48 / 48, 64 x 512 x 512 38 / 40
+// against 48 / 49, 64 x 1024 x 1024 70 / 72 against 55 / 56, 64 x 8 x 8
+// 26 / 32 against 38 / 43, 64 x 4 x 4 35 / 80 against 43 / 60, 8^3 44 / 75
+// against 56 / 87, 4^3 165 / 462 against 174 / 391; all on the floor of an 8^3
+// grid 160 / 334 against 157 / 317.
 bool collide_slot_keys(const fc_sim_params& P, uint32_t n) {
   if (!rows_walk_ok(P) || !row_resort_grid_ok(P)) return false;
   if (!collide_rows_optional(n)) return true;

@@ -569,7 +569,7 @@ fc_status alloc_map(fc_context* ctx, const int32_t cells[3], fc_distmap** out) {
   m->ctx = ctx;
   for (int a = 0; a < 3; ++a) m->cells[a] = cells[a];
   m->V = V;
-  // one allocation: the axes (map_axes' layout), then the vertices' arrays
+  // one allocation: the axes (axis_offset's layout), then the vertices' arrays
   const size_t axes = axis_offset(m, 3);
   const hipError_t e = hipMalloc(&m->block, axes * sizeof(float) + 2 * V * sizeof(float4));
   if (e == hipSuccess) {

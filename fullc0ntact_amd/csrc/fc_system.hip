@@ -301,7 +301,7 @@ fc_status enqueue_run_body(fc_system* sys, float dt, bool clearInSort, bool last
     if (timer) timer->end(st);
     if (e != hipSuccess) return hip_error(e, "row sort");
   } else if (n <= (uint32_t)RS_TILE) {
-    // One block sorts, gathers and writes the cell tables.
+    // Two launches sort by counting, gather and write the cell tables.
     if (timer) timer->begin(st, "sort_small");
     e = launch_sort_small(st, ctx->sort, sys->keys, valsIn, sys->hash, valsOut, n, passes,
                           clearHash, sys->cellStart, sys->cellEnd, P.numCells, ga);

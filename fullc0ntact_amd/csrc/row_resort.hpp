@@ -15,11 +15,12 @@ constexpr uint32_t kRowGroupShift = 8;  // rows per group of the two-level scan:
 // (hashes are below 2^30 wherever the row resort runs).
 constexpr uint32_t kMovedBit = 0x80000000u;
 
-// The per-row counters come in kRowCopies copies, [row][copy]: the counts
-// of the sphere at sorted slot k go to copy (k >> 8) % kRowCopies, so the
+// The per-row counters come in kRowCopies copies, [row][copy], so that the
 // many waves that count into one row at the same moment spread their
-// atomics over several addresses.  The changer pass takes the same copy
-// for slot k, and the scan gives every (row, copy) its own bucket range.
+// atomics over several addresses.  A row changer at sorted slot k is counted
+// in copy (k >> 8) % kRowCopies of its new row: the scan gives every
+// (row, copy) its own bucket range, and the changer pass takes the same copy
+// for slot k.  Of the counts of all keys only the sum over the copies is used.
 constexpr uint32_t kRowCopies = 8;
 
 __device__ __forceinline__ uint32_t row_copy(uint32_t slot) {
@@ -42,10 +43,10 @@ __device__ __forceinline__ uint32_t lowest_lane(uint64_t m) {
 }
 
 // Adds this wave's next keys to the row counts; `slot` is the lane's sorted
-// slot (the lanes of a wave hold 64 consecutive slots of one 256-slot
-// tile) and `oldKey` the key of the cell the sphere is in now.  A run of
-// lanes with the same row adds its count with one atomic.  Every lane of
-// the wave must call it.
+// slot (ascending over the wave's valid lanes; they may stand in two 256-slot
+// tiles) and `oldKey` the key of the cell the sphere is in now.  A run of
+// lanes with the same row adds its count with one atomic, to its first lane's
+// copy.  Every lane of the wave must call it.
 __device__ __forceinline__ void row_histograms(const RowHists& rh, uint32_t slot, uint32_t key,
                                                uint32_t oldKey, bool valid) {
   const uint32_t lane = threadIdx.x & 63u;

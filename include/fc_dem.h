@@ -223,7 +223,9 @@ fc_status fc_system_destroy(fc_system* sys);
 uint32_t fc_system_num_particles(const fc_system* sys);
 
 /* m_params writes/reads (the set* setters of particleSystem.h:64-72 are
- * field writes on a copy; see fc_particle_system.hpp). */
+ * field writes on a copy; see fc_particle_system.hpp).  Another number of
+ * cells allocates its tables; without memory for them the call fails and the
+ * system keeps its parameters. */
 fc_status fc_system_set_params(fc_system* sys, const fc_sim_params* params);
 fc_status fc_system_get_params(const fc_system* sys, fc_sim_params* params);
 
@@ -246,7 +248,10 @@ fc_status fc_system_reset(fc_system* sys, fc_particle_config config, uint64_t se
 /* update(deltaTime) (particleSystem.cpp:222-284). */
 fc_status fc_system_update(fc_system* sys, float deltaTime);
 /* steps consecutive update(deltaTime) calls.  Results are bit-identical to
- * calling fc_system_update steps times. */
+ * calling fc_system_update steps times.  The first run of more than 4,096
+ * spheres on a grid shape allocates the row tables of its sort (about 170
+ * bytes per grid row and 16 per sphere; systems of up to 16,384 spheres do
+ * without when there is no memory for them). */
 fc_status fc_system_run(fc_system* sys, float deltaTime, uint32_t steps);
 
 /* Device pointers of the system's buffers (for zero-copy consumers).  Any
@@ -303,9 +308,9 @@ fc_status fc_distmap_create(fc_context* ctx, const int32_t cells[3], float cellS
  * the exact distance of D. Eberly's point-triangle method and the sign of the
  * generalized winding number instead of CGAL).  Meshes of 128 to 2^22
  * triangles that turn out closed are searched through a tree in the context's
- * scratch (about 130 bytes a triangle, kept for the next call); other meshes,
- * and any when the scratch cannot grow, triangle by triangle.  The results are
- * the same bit for bit. */
+ * scratch (about 130 bytes a triangle, and the mesh's own copy up to 256 MB,
+ * kept for the next call); other meshes, and any when the scratch cannot grow,
+ * triangle by triangle.  The results are the same bit for bit. */
 fc_status fc_distmap_build(fc_context* ctx, const double* vertices, uint32_t numVertices,
                            const uint32_t* triangles, uint32_t numTriangles,
                            const int32_t cells[3], float cellSize, const float bmin[3],

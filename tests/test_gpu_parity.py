@@ -678,8 +678,9 @@ def _edge_pairs(rng, n_pairs, r, poly):
 
 @pytest.mark.parametrize("poly", [False, True])
 def test_system_collide_contact_distance_edges(gpu_ctx, poly):
-    # The system path's row-range collide drops candidates on 16-bit
-    # fixed-point coordinates before the exact test; no pair the reference
+    # The row-split collide of 5,000 spheres (test_gpu_contact_edges.py: the
+    # row-range one, which drops candidates on 16-bit fixed-point coordinates
+    # before the exact test); no pair the reference
     # counts as touching may be lost, anywhere in the box.  With no gravity
     # and zero velocities the integrate leaves every position as placed.
     from fullc0ntact_amd import ParticleSystem
@@ -741,8 +742,9 @@ def test_system_list_overflow_fallback(gpu_ctx, poly):
     # row-range fallback, beside list-path lanes in the same waves.  Updates
     # and a graph-launched run must equal the oracle bit for bit.  With poly
     # the radii come from pos.w (U(0.6 r, r)), through the fallback's
-    # polydisperse branch.  Over 16384 spheres, so that the row-range
-    # kernel (not the row-split one of small systems) runs.
+    # polydisperse branch.  Over 16384 spheres, so that with poly the
+    # row-range kernel runs (with one radius the row-split one does up to
+    # 32768: test_gpu_row_range.py).
     from fullc0ntact_amd import ParticleSystem
     grid, r = 64, 1.0 / 64.0
     rng = np.random.default_rng(44)

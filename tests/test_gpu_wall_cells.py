@@ -1,6 +1,7 @@
 """The collide's neighbour walk where cell indices wrap, and its overflowing
-lists, against the oracle bit for bit (over 16,384 spheres: the row-range
-kernel).
+lists, against the oracle bit for bit (20,000 spheres: with one radius the
+row-split kernel, with radii of their own the row-range one;
+test_gpu_row_range.py repeats the former at 40,000).
 
  - A grid that covers the box exactly: every wall sphere has neighbour cells
    on the opposite side, which the walls put out of contact.
