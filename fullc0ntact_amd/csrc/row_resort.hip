@@ -607,7 +607,7 @@ __device__ __forceinline__ void place_pool(const RowOutputs& O, uint32_t o0, uin
 // costs a pass over the row's candidates.  A step of a run of 5,000 spheres in
 // one row of 64 cells, of 16,000 in eight, and of 16,000 with log-normal radii
 // on the floor of an 8^3 grid: with a block for the whole row, each member
-// counted against all of it, 12,300 / 2,450 / 660 us, with this 197 / 84 / 143
+// counted against all of it, 12,300 / 2,450 / 660 us, with this 172 / 84 / 134
 // (with the radix sort 165 / 90 / 134).
 __device__ __forceinline__ void sort_part(const RowTables& T, const uint32_t* keys,
                                           const uint32_t* idOfSlot, const RowOutputs& O,
